@@ -1568,8 +1568,11 @@ __global__ __launch_bounds__(256) void k_svd_write(double* __restrict__ base, co
 // numerically zero, columns t < limit: starting from unit vectors, classical
 // Gram-Schmidt twice against all earlier columns (the dot products of one
 // pass in one step, thread per column; the update thread per row), keeping
-// the first candidate whose residual norm exceeds 1/2.  One work-group per
-// sector.
+// the first candidate whose residual norm exceeds 0.7 / sqrt(ell): the
+// residuals' squares sum to the number of missing columns, so one of the ell
+// candidates always does (1/2 was out of reach when few columns are missing:
+// every candidate was tried and the columns stayed zero).  One work-group
+// per sector.
 __global__ __launch_bounds__(256) void k_svd_complete(double* __restrict__ base,
                                                       const CompleteTask* __restrict__ ts) {
   __shared__ double sh[256];
@@ -1613,7 +1616,7 @@ __global__ __launch_bounds__(256) void k_svd_complete(double* __restrict__ base,
       double acc = 0.0;
       for (int l = tid; l < ell; l += blockDim.x) acc += v[l] * v[l];
       const double nrm = sqrt(wg_sum(acc, sh));
-      if (nrm > 0.5) {
+      if (nrm * nrm * double(ell) > 0.49) {
         for (int l = tid; l < ell; l += blockDim.x) Z[int64_t(l) * k + t] = v[l] / nrm;
         __syncthreads();
         break;
