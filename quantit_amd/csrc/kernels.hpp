@@ -209,17 +209,14 @@ void svd_complete(hipStream_t s, double* base, const CompleteTask* tasks, int n)
 void svd_shift(hipStream_t s, double* base, const SvdSector* secs, int nsec);
 void fill_i32(hipStream_t s, int32_t* p, int n, int32_t v);
 
-// Single-work-group one-sided Jacobi with the whole sector in LDS
-// (descriptors: see SmallJacobi in svd_jacobi.hip).
+// One k x k matrix of the one-work-group kernels.
 struct SmallJacobi {
-  int64_t y_off, w_off;  // Y (ell x k, column-major, ld ldy), W (ldw x ldw, column-major)
+  int64_t y_off, w_off;  // input (ell x k, column-major, ld ldy), output (ldw x ldw, column-major)
   int32_t ell, k, ldy, ldw;
   int32_t flag_idx;       // flags[flag_idx]: result count of the kernel (-1: none)
   int32_t aux_idx;        // flags[aux_idx]: second count (gram_eig; -1: none)
 };
-void jacobi_small(hipStream_t s, double* base, const void* descs, int n, int* flags, double tol, int max_sweeps,
-                  size_t lds_bytes);
-size_t jacobi_small_lds_limit();
+size_t gram_eig_lds_limit();  // largest dynamic LDS per work-group (bytes)
 // Eigenvectors of k x k Gram matrices (SmallJacobi with ell = k): W written
 // k x k at w_off with leading dimension ldw; flags[flag_idx] = pairs of G
 // failing the orthogonality test (0: W = I).  precond: pivoted-Cholesky
@@ -236,6 +233,23 @@ void gs_step(hipStream_t s, double* base, const void* descs, int n, int kmax);
 // Orthogonality test of G (SmallJacobi: y_off = G, k, ldy; flag_idx/aux_idx
 // as for gram_eig).
 void gram_check(hipStream_t s, const double* base, const void* descs, int n, int* flags, double tol, int kmax);
+// Work item of one round of the two-sided block Jacobi on G (gram_rounds.hip):
+// the solve of block pair a, tile (a, b) of G (a <= b), or rows
+// [64 b, 64 b + 64) of X's column pair a.
+enum GramKind : int32_t { kGramSolve = 0, kGramApplyG = 1, kGramApplyX = 2 };
+struct GramRound {
+  int64_t g0, g1;  // two kp x kp buffers; a sweep starts from the Gram matrix in g0
+  int64_t x;       // X, k x kp column-major, leading dimension k
+  int64_t q, d;    // 2 x (nb / 2) row-major 32 x 32 blocks each: rotations and rotated blocks, by round parity
+  int32_t k, nb, flag, kind;
+  int32_t a, b;
+};
+// Launch `round` (0 .. max nb - 1) of a sweep.  counters[flag] receives the
+// pairs of the fresh G over the tolerance (complete after round 1: a sector
+// left at 0 has converged and takes no further part); skip: the previous
+// sweep's counters or null.
+void gram_round(hipStream_t s, double* base, const GramRound* work, int nwork, int round, int* counters,
+                const int* skip, double tol);
 struct CholPanel {
   int64_t g_off;      // G (k x k, ld k), updated between panels
   int64_t l_off;      // L (k x k, ld k, zeroed), rows in the original order
@@ -253,7 +267,7 @@ struct GramVec {
   int64_t x_off, w_off, scratch_off;  // scratch: 3k doubles
   int32_t k, ldx, ldw, pad;
 };
-void gram_vectors(hipStream_t s, double* base, const void* descs, int n, int kmax);  // largest dynamic LDS per work-group (bytes)
+void gram_vectors(hipStream_t s, double* base, const void* descs, int n, int kmax);
 
 // Global truncation (sources/btensor_linalg.cpp:657-755,
 // sources/LinearAlgebra.cpp:57-75): singular values of nsec sectors stored

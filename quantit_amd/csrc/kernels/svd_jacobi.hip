@@ -562,113 +562,6 @@ __device__ double wg_sum(double v, double* sh) {
   return r;
 }
 
-// ---- single-work-group Jacobi for sectors that fit in LDS -------------------
-// One work-group per sector holds Y (ell x ke, ke = k rounded up to even) in
-// LDS and runs cyclic one-sided Jacobi sweeps (circle ordering over single
-// columns) until a sweep rotates nothing.  Each column pair is handled by a
-// group of gsz lanes that reduce the three dot products with shuffles and
-// rotate the pair in LDS; W (ldw x ldw, column-major, global) accumulates the
-// rotations.  Y is written back at the end; flags[flag_idx] receives the
-// number of rotations of the first sweep.
-constexpr int kSmallThreads = 1024;
-
-__global__ __launch_bounds__(kSmallThreads) void k_jacobi_small(double* __restrict__ base,
-                                                                const SmallJacobi* __restrict__ js,
-                                                                int* __restrict__ flags, double tol, int max_sweeps) {
-  extern __shared__ double lds[];
-  __shared__ int nrot[2];
-  __shared__ int first;
-  const SmallJacobi J = js[blockIdx.x];
-  const int ell = J.ell, k = J.k;
-  const int ke = k + (k & 1);
-  double* Yg = base + J.y_off;
-  double* W = base + J.w_off;
-  const int tid = threadIdx.x;
-  // load Y (padding column zero) and set W to the identity
-  for (int64_t e = tid; e < int64_t(ell) * ke; e += blockDim.x) {
-    const int r = int(e % ell), c = int(e / ell);
-    lds[e] = c < k ? Yg[int64_t(c) * J.ldy + r] : 0.0;
-  }
-  for (int64_t e = tid; e < int64_t(J.ldw) * J.ldw; e += blockDim.x)
-    W[e] = (e % J.ldw == e / J.ldw) ? 1.0 : 0.0;
-  if (tid == 0) {
-    first = -1;
-    nrot[0] = nrot[1] = 0;
-  }
-  __syncthreads();
-  const int npairs = ke / 2;
-  int gsz = 64;
-  while (gsz > 1 && gsz * npairs > int(blockDim.x)) gsz >>= 1;
-  const int pi = tid / gsz, li = tid % gsz, pstride = int(blockDim.x) / gsz;
-  for (int sweep = 0; sweep < max_sweeps && ke >= 2; ++sweep) {
-    int* cnt = &nrot[sweep & 1];
-    for (int r = 0; r < ke - 1; ++r) {
-      for (int p = pi; p < npairs; p += pstride) {
-        const int a0 = circle_block(p, r, ke), b0 = circle_block(ke - 1 - p, r, ke);
-        const int a = min(a0, b0), b = max(a0, b0);
-        double* ya = lds + int64_t(a) * ell;
-        double* yb = lds + int64_t(b) * ell;
-        double al = 0.0, be = 0.0, ga = 0.0;
-#pragma unroll 4
-        for (int l = li; l < ell; l += gsz) {
-          const double x = ya[l], y = yb[l];
-          al += x * x;
-          be += y * y;
-          ga += x * y;
-        }
-        for (int off = gsz >> 1; off > 0; off >>= 1) {
-          al += __shfl_xor(al, off, gsz);
-          be += __shfl_xor(be, off, gsz);
-          ga += __shfl_xor(ga, off, gsz);
-        }
-        if (al > 0.0 && be > 0.0 && fabs(ga) > tol * sqrt(al) * sqrt(be)) {
-          const double zeta = (be - al) / (2.0 * ga);
-          const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-          const double c = 1.0 / sqrt(1.0 + t * t), sn = c * t;
-#pragma unroll 4
-          for (int l = li; l < ell; l += gsz) {
-            const double x = ya[l], y = yb[l];
-            ya[l] = c * x - sn * y;
-            yb[l] = sn * x + c * y;
-          }
-          double* wa = W + int64_t(a) * J.ldw;
-          double* wb = W + int64_t(b) * J.ldw;
-#pragma unroll 4
-          for (int l = li; l < k; l += gsz) {
-            const double x = wa[l], y = wb[l];
-            wa[l] = c * x - sn * y;
-            wb[l] = sn * x + c * y;
-          }
-          if (li == 0) atomicAdd(cnt, 1);
-        }
-      }
-      __syncthreads();
-    }
-    // cnt is final after the last barrier; the other counter is cleared for
-    // the next sweep before anyone can touch it (it is only used after the
-    // next sweep's first barrier)
-    const int n = *cnt;
-    if (tid == 0) {
-      if (first < 0) first = n;
-      nrot[(sweep + 1) & 1] = 0;
-    }
-    __syncthreads();
-    if (n == 0) break;
-  }
-  for (int64_t e = tid; e < int64_t(ell) * k; e += blockDim.x) {
-    const int r = int(e % ell), c = int(e / ell);
-    Yg[int64_t(c) * J.ldy + r] = lds[e];
-  }
-  if (tid == 0 && J.flag_idx >= 0) flags[J.flag_idx] = first < 0 ? 0 : first;
-}
-
-void jacobi_small(hipStream_t st, double* base, const void* descs, int n, int* flags, double tol, int max_sweeps,
-                  size_t lds_bytes) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_jacobi_small, dim3(n), dim3(kSmallThreads), lds_bytes, st, base,
-                     static_cast<const SmallJacobi*>(descs), flags, tol, max_sweeps);
-}
-
 // ---- eigenvectors of a Gram matrix by one-sided Jacobi without accumulation --
 // One work-group per k x k Gram matrix G (k <= kGramEigMaxK) held in LDS.
 //
@@ -680,7 +573,8 @@ void jacobi_small(hipStream_t st, double* base, const void* descs, int n, int* f
 //    flags[flag_idx] = pairs failing both; flags[J.aux_idx] (when >= 0) = pairs
 //    converged only in the absolute sense.  No failing pair: W = I exactly.
 // 2. Preconditioning (precond != 0): pivoted Cholesky P^T G P = R^T R in
-//    place (diagonal pivoting, stops at a non-positive pivot), X = R^T.  This
+//    place (diagonal pivoting; from a non-positive pivot on, the factor of a
+//    diagonal below G's rounding), X = R^T.  This
 //    is the QR-with-pivoting preconditioner of Drmac and Veselic (SIAM J.
 //    Matrix Anal. Appl. 29, 2008) applied through G: on graded spectra the
 //    Jacobi below then needs a few sweeps instead of tens.  Without it X = G.
@@ -1006,9 +900,9 @@ __device__ __forceinline__ void wl_sweeps(double* X, int k, double tol_rot, int 
 // are those of the register-tile form (the largest remaining diagonal,
 // smallest index on ties; l = G(:, p) / sqrt(G(p, p)); every update the same
 // fused multiply-add), so L is the same to the bit; column j of X receives l
-// in the original row order.  Returns the rank.
+// in the original row order, pivoted[i] whether row i was a pivot.  Returns the rank.
 template <int KM>
-__device__ __forceinline__ int chol_wave(double* X, int k) {
+__device__ __forceinline__ int chol_wave(double* X, int* pivoted, int k) {
   __shared__ double lb[64];  // the step's column l, one entry per lane
   __shared__ double cp[64];  // the pivot's row of the trailing matrix
   const int lane = threadIdx.x & 63;
@@ -1063,6 +957,7 @@ __device__ __forceinline__ int chol_wave(double* X, int k) {
     for (int c = 0; c < KM; ++c) g[c] -= l * lb[c];
     __builtin_amdgcn_wave_barrier();  // every read of lb precedes the next step's writes
   }
+  if (row) pivoted[lane] = used;
   return rk;
 }
 
@@ -1151,7 +1046,7 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
     int rk = k;
     if (k <= 64) {
       if (tid < 64) {
-        const int r = k <= 32 ? chol_wave<32>(X, k) : chol_wave<64>(X, k);
+        const int r = k <= 32 ? chol_wave<32>(X, perm, k) : chol_wave<64>(X, perm, k);
         if (tid == 0) rk_sh = r;
       }
       __syncthreads();
@@ -1256,8 +1151,24 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
         }
       }
     }
-    // columns from the rank on are zero; perm back to the identity
+    // Columns from the rank on: small multiples of the unit vectors of the rows
+    // without a pivot, the factor of G + delta^2 I there with delta^2 = 2^-54
+    // of the largest diagonal, below the rounding of G.  The Jacobi sweeps
+    // then make the null space's basis with all others (a numpy model takes
+    // the same number of sweeps or one more); completing zero columns one by
+    // one took 640 of 1780 us for two sectors of k = 98 with spectra over ten
+    // decades.  G = 0 leaves zero columns.
     for (int e = rk * k + tid; e < k * k; e += blockDim.x) X[e] = 0.0;
+    double top = 0.0;
+    if (rk > 0 && rk < k)
+      for (int i = 0; i < k; ++i) top = fmax(top, fabs(X[i]));  // sqrt of the largest diagonal
+    __syncthreads();
+    if (rk > 0 && tid < k && !perm[tid]) {
+      int c = rk;
+      for (int i = 0; i < tid; ++i) c += perm[i] ? 0 : 1;
+      X[c * k + tid] = top * 0x1p-27;
+    }
+    __syncthreads();
     for (int i = tid; i < ke; i += blockDim.x) perm[i] = i;
     __syncthreads();
   }
@@ -1412,14 +1323,12 @@ size_t gram_eig_lds_bytes(int k) {
   return size_t(int64_t(k) * ke + 3 * ke + 16) * sizeof(double) + size_t(ke) * sizeof(int);
 }
 
-size_t jacobi_small_lds_limit() {
+size_t gram_eig_lds_limit() {
   static const size_t limit = [] {
     int dev = 0;
     int v = 0;
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) v = 65536;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_jacobi_small),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, v - 64);
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gram_eig),
                               hipFuncAttributeMaxDynamicSharedMemorySize, v - 64);
     return size_t(v);

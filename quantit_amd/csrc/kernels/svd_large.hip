@@ -280,6 +280,20 @@ __global__ __launch_bounds__(kLargeThreads) void k_pchol_panel(double* __restric
     Lp[e] = col[e];
     if (j0 + t < k) L[int64_t(j0 + t) * k + i] = col[e];
   }
+  if (rank > 0 && rank < k) {
+    // the factor of G + delta^2 I on the rows without a pivot, as in k_gram_eig
+    __syncthreads();  // the zero columns copied above are overwritten
+    const double* first = j0 == 0 ? col : L;
+    double top = 0.0;
+    for (int i = lane; i < k; i += 64) top = fmax(top, fabs(first[i]));
+    for (int off = 32; off > 0; off >>= 1) top = fmax(top, __shfl_xor(top, off));
+    for (int i = tid; i < k; i += blockDim.x) {
+      if (used[i]) continue;
+      int c = rank;
+      for (int j = 0; j < i; ++j) c += used[j] ? 0 : 1;
+      L[int64_t(c) * k + i] = top * 0x1p-27;
+    }
+  }
 }
 
 __global__ __launch_bounds__(256) void k_pchol_init(double* __restrict__ base, const CholPanel* __restrict__ ps) {

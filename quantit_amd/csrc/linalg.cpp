@@ -299,15 +299,94 @@ int jacobi_sweeps(Context* ctx, double* ab, const std::vector<kern::SvdSector>& 
   return sweeps;
 }
 
+// One Gram eigenproblem of gram_sweeps: X (k x kp, kp = 16 nb, zero columns
+// from k on) whose columns are driven orthogonal; g0, g1: kp x kp, q, d: 2 x
+// (nb / 2) blocks of 32 x 32, all element offsets from the arena base.
+struct GramProblem {
+  int64_t x, g0, g1, q, d;
+  int32_t k, nb;
+};
+
+// Two-sided block Jacobi sweeps (gram_rounds.hip) over the problems until
+// every pair of columns passes the relative test, or max_sweeps.  A sweep is
+// one Gram GEMM and max nb launches; its convergence counts are complete
+// after the second launch, so the host reads them while the next few run and
+// enqueues the rest of the sweep only if some problem still rotates.
+int gram_sweeps(Context* ctx, double* ab, const std::vector<GramProblem>& ps, double tol, int max_sweeps,
+                int* capped) {
+  const int n = int(ps.size());
+  if (n == 0 || max_sweeps <= 0) return 0;
+  BufPtr cnt = ctx->alloc(size_t(2 * n) * sizeof(int32_t));
+  int32_t* d_cnt[2] = {reinterpret_cast<int32_t*>(cnt->cptr()), reinterpret_cast<int32_t*>(cnt->cptr()) + n};
+  ctx->reserve_read(size_t(n));
+  std::vector<kern::GramRound> work;
+  std::vector<kern::GemmOut> outs;
+  std::vector<kern::GemmPair> prs;
+  int max_nb = 0;
+  // solves first (the launch's critical path), then the widest tiles' work
+  for (int kind : {kern::kGramSolve, kern::kGramApplyG, kern::kGramApplyX})
+    for (int i = 0; i < n; ++i) {
+      const auto& p = ps[i];
+      const int half = p.nb / 2, rows = (p.k + 63) / 64;
+      max_nb = std::max(max_nb, p.nb);
+      kern::GramRound w{p.g0, p.g1, p.x, p.q, p.d, p.k, p.nb, i, kind, 0, 0};
+      for (w.a = 0; w.a < half; ++w.a) {
+        const int b0 = kind == kern::kGramApplyG ? w.a : 0;
+        const int b1 = kind == kern::kGramSolve ? 1 : kind == kern::kGramApplyG ? half : rows;
+        for (w.b = b0; w.b < b1; ++w.b) work.push_back(w);
+      }
+    }
+  for (int i = 0; i < n; ++i) {
+    const auto& p = ps[i];
+    kern::GemmPair g{};  // G = X^T X over the k real columns
+    g.a_off = g.b_off = p.x;
+    g.a_rs = g.b_cs = p.k;
+    g.a_cs = g.b_rs = 1;
+    g.K = p.k;
+    outs.push_back({p.g0, p.k, p.k, int32_t(prs.size()), int32_t(prs.size() + 1), p.nb * kern::kSvdBlock, 0});
+    prs.push_back(g);
+  }
+  const kern::GramRound* d_work = ctx->upload_vec(work);
+  const GemmLaunch gram = prepare_gemm(ctx, outs, prs);
+  constexpr int kAhead = 6;  // launches enqueued before the host waits for the counts
+  for (int sweep = 0;; ++sweep) {
+    const int slot = sweep & 1;
+    kern::fill_i32(ctx->stream(), d_cnt[slot], n, 0);
+    run_gemm(ctx, ab, gram, "svd_sweep_gram");
+    auto rounds = [&](int r0, int r1) {
+      for (int r = r0; r < r1; ++r) {
+        KernelTimer kt(*ctx, "svd_gram_round");
+        kern::gram_round(ctx->stream(), ab, d_work, int(work.size()), r, d_cnt[slot],
+                         sweep ? d_cnt[slot ^ 1] : nullptr, tol);
+      }
+    };
+    rounds(0, 2);
+    QTT_HIP(hipMemcpyAsync(ctx->read_slot(slot), d_cnt[slot], size_t(n) * sizeof(int32_t), hipMemcpyDeviceToHost,
+                           ctx->stream()));
+    QTT_HIP(hipEventRecord(ctx->read_event(slot), ctx->stream()));
+    const int ahead = std::min(max_nb, kAhead);
+    rounds(2, ahead);
+    ctx->wait_event(ctx->read_event(slot));
+    const int32_t* h = ctx->read_slot(slot);
+    int left = 0;
+    for (int i = 0; i < n; ++i) left += h[i] != 0;
+    if (left == 0) return sweep;
+    if (sweep >= max_sweeps) {
+      if (capped) *capped += left;
+      return sweep;
+    }
+    rounds(ahead, max_nb);
+  }
+}
+
 // Gathers the sector matrices of a rank-2 tensor and runs the batched Jacobi
 // SVD (eigh_mode: shifted symmetric eigen-decomposition) on device.
 //
-// Sectors much longer than wide (ell >= 2 kp) are first preconditioned by
-// Gram iterations: G = Y^T Y (kp x kp, MFMA GEMM), its eigenvectors W_g by the
-// same block Jacobi on G, Y <- Y W_g and W <- W W_g, repeated until the
-// Jacobi on G rotates nothing in its first sweep, i.e. the columns of Y are
-// orthogonal to the tolerance.  Every step is an exact orthogonal transform
-// of Y, so the singular values still come from the column norms of Y.
+// Sectors run Gram iterations: G = Y^T Y (MFMA GEMM), its eigenvectors W_g,
+// Y <- Y W_g and W <- W W_g, repeated until G is diagonal to the tolerance,
+// i.e. the columns of Y are orthogonal.  Every step is an exact orthogonal
+// transform of Y, so the singular values still come from the column norms of
+// Y.  eigh solves A + c I once in the Gram matrix's place.
 Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool eigh_mode,
                     bool defer_complete = false) {
   Context* ctx = t.ctx;
@@ -427,11 +506,10 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
   const double tol = 8.0 * std::sqrt(double(std::max(max_ell, 16))) * DBL_EPSILON;
   const int inner = env_int("QTT_SVD_INNER_SWEEPS", 1);
   const int max_sweeps = env_int("QTT_SVD_MAX_SWEEPS", 30);
-  const size_t lds_limit = kern::jacobi_small_lds_limit();
+  const size_t lds_limit = kern::gram_eig_lds_limit();
   const size_t lds_margin = 256;
-  auto lds_bytes = [](int64_t ell, int64_t k) { return size_t(ell * (k + (k & 1))) * sizeof(double); };
   const bool use_small = env_int("QTT_SVD_SMALL", 1) != 0;
-  std::vector<char> done(ns, 0), big_only(ns, 0);
+  std::vector<char> done(ns, 0);
   B.wide.assign(ns, 0);
   std::vector<BufPtr> keep;  // Gram and ping-pong buffers live until the finalize is enqueued
 
@@ -449,7 +527,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
   const int eig_max_k = std::min(kern::kGramEigMaxK, env_int("QTT_SVD_EIG_MAX_K", kern::kGramEigMaxK));
   for (int i = 0; i < ns; ++i) {
     const auto& s = B.secs[i];
-    if (eigh_mode || !use_small || s.k < 1) continue;
+    if (!use_small || s.k < 1) continue;
     if (s.k <= eig_max_k && kern::gram_eig_lds_bytes(s.k) + lds_margin <= lds_limit) {
       wide.push_back(i);
     } else if (size_t(s.k) * (4 + kern::kPcholExtra) * sizeof(double) <= pchol_limit &&
@@ -469,7 +547,8 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
             ? int(std::min<size_t>(32, pchol_limit / (size_t(kmax_large) * sizeof(double)) - kern::kPcholExtra))
             : 0;
     int64_t elems = 0;
-    std::vector<int64_t> go(nw), gwo(nw), y2o(nw), w2o(nw), lo(nw, -1), lpo(nw, -1), sco(nw, -1), sto(nw, -1);
+    std::vector<int64_t> go(nw), gwo(nw), y2o(nw), w2o(nw), lo(nw, -1), lpo(nw, -1), sco(nw, -1), sto(nw, -1),
+        pgo(nw, -1), pqo(nw, -1);
     size_t lds_need = 0;
     for (int q = 0; q < nw; ++q) {
       const auto& s = B.secs[wide[q]];
@@ -492,6 +571,10 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         elems += 3 * k;
         sto[q] = elems;  // ints
         elems += (k + 2) / 2 + 1;
+        pgo[q] = elems;  // the sweeps' two G buffers
+        elems += 2 * kp * kp;
+        pqo[q] = elems;  // rotations and rotated blocks, two parities each
+        elems += int64_t(4) * (s.nb / 2) * 1024;
       } else {
         lds_need = std::max(lds_need, kern::gram_eig_lds_bytes(s.k));
       }
@@ -641,6 +724,10 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
           c.dst_cs = 1;
           add_chunks(zt, int(z.size()), int64_t(c.cols));
           z.push_back(c);
+          c.dst_off = gb + pgo[q];  // G's padding stays zero under the sweeps
+          c.cols = int32_t(kp * kp);
+          add_chunks(zt, int(z.size()), int64_t(c.cols));
+          z.push_back(c);
         }
         KernelTimer kt(*ctx, "svd_init");
         auto [dz, dzt] = ctx->upload_pack(z, zt);
@@ -677,29 +764,50 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         }
         if (j0 + pnb < kact) run_gemm(ctx, ab, upd, "svd_pchol_update", -1.0, 1.0);
       }
-      std::vector<kern::SvdSector> gsec;
-      std::vector<int> all;
+      std::vector<GramProblem> ps;
       std::vector<kern::GramVec> vd;
       for (int q : qs) {
         const auto& s = B.secs[wide[q]];
-        kern::SvdSector g = s;
-        g.y_off = gb + lo[q];
-        g.w_off = -1;  // the eigenvectors come from the normalised columns
-        g.ell = s.k;
-        g.flag_idx = int32_t(gsec.size());
-        all.push_back(int(gsec.size()));
-        gsec.push_back(g);
+        const int64_t kp = int64_t(s.nb) * kern::kSvdBlock;
+        ps.push_back({gb + lo[q], gb + pgo[q], gb + pgo[q] + kp * kp, gb + pqo[q],
+                      gb + pqo[q] + int64_t(2) * (s.nb / 2) * 1024, s.k, s.nb});
         vd.push_back({gb + lo[q], gb + gwo[q], gb + sco[q], s.k, s.k, s.k, 0});
       }
-      jacobi_sweeps(ctx, ab, gsec, all, tol, inner, max_sweeps, nullptr, &B.unconverged);
+      // well inside tol: couplings d left between the columns come back in the
+      // next Gram matrix as d (sigma_i^2 + sigma_j^2), against tol sigma_i
+      // sigma_max; stopping at tol itself repeats the iteration up to its cap
+      gram_sweeps(ctx, ab, ps, tol / 8.0, max_sweeps, &B.unconverged);
       int kv = 0;
       for (auto& v : vd) kv = std::max(kv, v.k);
       KernelTimer kt(*ctx, "svd_vectors");
       kern::gram_vectors(ctx->stream(), ab, ctx->upload_vec(vd), int(vd.size()), kv);
     };
-    const int max_it = env_int("QTT_SVD_GRAM_ITERS", 6);
+    // eigh: A + c I is positive (semi-)definite, so it takes the Gram matrix's
+    // place once: its eigenvectors are A's, and the column norms of (A + c I) W
+    // are the shifted eigenvalues.
+    const int max_it = eigh_mode ? 1 : env_int("QTT_SVD_GRAM_ITERS", 6);
     for (int it = 0; it < max_it && !act.empty(); ++it) {
-      gram_of(act);
+      if (eigh_mode) {
+        std::vector<kern::Copy2D> cg;
+        std::vector<kern::ChunkTask> ct;
+        for (int q : act) {
+          const auto& s = B.secs[wide[q]];
+          kern::Copy2D c{};
+          c.src_off = s.y_off;
+          c.dst_off = gb + go[q];
+          c.rows = 1;
+          c.cols = int32_t(int64_t(s.k) * s.k);
+          c.src_cs = c.dst_cs = 1;
+          c.alpha = 1.0;
+          add_chunks(ct, int(cg.size()), int64_t(c.cols));
+          cg.push_back(c);
+        }
+        KernelTimer kt(*ctx, "svd_init");
+        auto [dc, dt] = ctx->upload_pack(cg, ct);
+        kern::copy2d(ctx->stream(), ab, dc, dt, int(ct.size()));
+      } else {
+        gram_of(act);
+      }
       std::vector<int> act_s, act_l;
       for (int q : act) (large[wide[q]] ? act_l : act_s).push_back(q);
       // small sectors: test and solve in one work-group each.  Beside large
@@ -728,7 +836,9 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       // large sectors: test first (the solve is a long chain of launches); the
       // flag read also covers the small solver launched above
       int cd_launched = 0;
-      if (!act_l.empty()) {
+      if (!act_l.empty() && eigh_mode) {
+        solve_large(act_l);
+      } else if (!act_l.empty()) {
         cd_launched = 1;
         std::vector<kern::SmallJacobi> cd;
         int kc = 0;
@@ -756,7 +866,8 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       rotate(act);
       B.sweeps += 1;
     }
-    for (int q : act) big_only[wide[q]] = 1;  // keeps its accumulated W: multi-WG path only
+    if (eigh_mode)
+      for (int q : act) done[wide[q]] = 1;
     // Sectors converged with residual couplings below the absolute floor:
     // two first-order Gram-Schmidt passes Y <- Y T (longer columns first)
     // make the short columns orthogonal; W is unchanged, and the dropped
@@ -793,31 +904,13 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       for (int q : corr) std::swap(B.secs[wide[q]].y_off, alt_y[q]);
     }
   }
-  // ---- Jacobi on everything not yet orthogonal --------------------------------
-  std::vector<int> rest_small, rest_big;
-  size_t small_need = 0;
-  for (int i = 0; i < ns; ++i) {
-    if (done[i]) continue;
-    const auto& s = B.secs[i];
-    if (use_small && !big_only[i] && lds_bytes(s.ell, s.k) + lds_margin <= lds_limit) {
-      rest_small.push_back(i);
-      small_need = std::max(small_need, lds_bytes(s.ell, s.k));
-    } else {
-      rest_big.push_back(i);
-    }
-  }
-  if (!rest_small.empty()) {
-    std::vector<kern::SmallJacobi> jd;
-    for (int i : rest_small) {
-      const auto& s = B.secs[i];
-      jd.push_back({s.y_off, s.w_off, s.ell, s.k, s.ell, s.nb * kern::kSvdBlock, -1, 0});
-    }
-    KernelTimer kt(*ctx, "svd_small");
-    kern::jacobi_small(ctx->stream(), ab, ctx->upload_vec(jd), int(jd.size()), nullptr, tol, max_sweeps,
-                       small_need);
-  }
-  for (int i : rest_big) B.wide[i] = 1;
-  B.sweeps += jacobi_sweeps(ctx, ab, B.secs, rest_big, tol, inner, max_sweeps, nullptr, &B.unconverged);
+  // ---- Jacobi on everything not yet orthogonal: sectors wider than the panel
+  // Cholesky's LDS holds, and what the Gram iterations left ------------------
+  std::vector<int> rest;
+  for (int i = 0; i < ns; ++i)
+    if (!done[i] && B.secs[i].k > 0) rest.push_back(i);
+  for (int i : rest) B.wide[i] = 1;
+  B.sweeps += jacobi_sweeps(ctx, ab, B.secs, rest, tol, inner, max_sweeps, nullptr, &B.unconverged);
   // ---- finalize --------------------------------------------------------------
   std::vector<int4> wt;
   for (int i = 0; i < ns; ++i) {
