@@ -24,6 +24,9 @@ COMMON = [
     f"--offload-arch={ARCH}",
     # packed FP32 instructions stay disabled in every device object
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # MFMA results in ordinary registers: with the default the GEMM loops copy
+    # their accumulators to and from the matrix registers every k step
+    "-mllvm", "-amdgpu-mfma-vgpr-form",
 ]
 
 

@@ -32,25 +32,24 @@ struct GemmTile {
   int16_t tm, tn;  // tile coordinates inside the output block
 };
 constexpr int kGemmTile = 64;
-
-void gemm_f64(hipStream_t s, double* base, const GemmTile* tiles, int ntiles, const GemmOut* outs,
-              const GemmPair* pairs, double alpha, double beta);
-// Tile variants of the FP64 grouped GEMM (same bits as gemm_f64; a tile's
-// tm, tn count in units of the variant's TM x TN).  kTile64 is gemm_f64.
-// kTile64k32 is the double-buffered 64 x 64 tile with 32-deep k steps.
-enum GemmVariant : int {
-  kTile64 = 0,
-  kTile64db = 1,
-  kTile128x64 = 2,
-  kTile64x128 = 3,
-  kTile128 = 4,
-  kTile64k32 = 5,
-  kGemmVariants = 6
-};
-constexpr int kVariantTM[kGemmVariants] = {64, 64, 128, 64, 128, 64};
-constexpr int kVariantTN[kGemmVariants] = {64, 64, 64, 128, 128, 64};
-void gemm_f64_variant(hipStream_t s, int variant, double* base, const GemmTile* tiles, int ntiles,
-                      const GemmOut* outs, const GemmPair* pairs, double alpha, double beta);
+// How the operands of a launch are contiguous: bit 0 A in k (else in m), bit 1
+// B in n (else in k), common to all its pairs; kLayoutAny: in no common way.
+enum GemmLayout : int { kLayoutAny = -1 };
+GemmLayout gemm_layout(const GemmPair* pairs, size_t n, const GemmOut* outs, size_t nouts);
+// The grouped FP64 GEMM with 64 x 64 or 32 x 32 tiles (tile; a tile's tm, tn
+// count in its own units).  Launches of kLayoutAny take 64 x 64 tiles.
+void gemm_f64(hipStream_t s, int tile, GemmLayout lay, double* base, const GemmTile* tiles, int ntiles,
+              const GemmOut* outs, const GemmPair* pairs, double alpha, double beta);
+// Tile choices of the tuning table and of QTT_GEMM_VARIANT, by number: 5 is
+// the 32 x 32 tile, every other number the 64 x 64 one (0 the general kernel;
+// 2 to 4 are numbers of wider tiles in tables of older builds).
+enum GemmVariant : int { kTileAny = 0, kTile64 = 1, kTile32 = 5, kGemmVariants = 6 };
+inline int variant_tile(int v) { return v == kTile32 ? 32 : 64; }
+// Tile of a launch that is not timed: 32 x 32 below this many 64 x 64 tiles
+// (three per CU), where the longest tile and the idle CUs decide: 225 tiles
+// 165 us against 216, 218 tiles 23.7 against 28.8; from 1024 tiles on the 64 x
+// 64 tile is ahead (318 us against 439 at 1024, 112 against 137 at 5707).
+constexpr int64_t kTile64Min = 768;
 
 // Size of the file-scope device scratch (kernels/gemm.hip) that the
 // allocation-free contraction takes its packed operands, split-K partials

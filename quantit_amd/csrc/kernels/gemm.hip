@@ -1,18 +1,17 @@
 // Grouped block-sparse GEMM for gfx950 (CDNA4).
 //
-// One work-group computes one 64x64 tile of one output block and walks that
+// One work-group computes one tile of one output block and walks that
 // block's list of (A_p, B_p) pairs in order, so every output block is written
 // exactly once with a fixed accumulation order (no atomics: results do not
 // depend on what else runs on the device).  The permute gather of the
 // reference's permute_bl (sources/btensor.cpp:1843-1894) is folded into the
 // tile loads through per-pair (row, column) element strides.
 //
-// FP64 path: v_mfma_f64_16x16x4_f64.  Each of the 4 waves owns a 32x32
-// quadrant = 2x2 MFMA tiles; LDS holds a 64x16 A tile and a 16x64 B tile
-// (k-major, row pitch 80 doubles so the two 16-lane halves of a 32-lane
-// LDS read phase fall in opposite bank halves).
+// The split-FP32 kernel's waves own 32x32 quadrants = 2x2 MFMA tiles; LDS holds
+// a 64x16 A tile and a 16x64 B tile (k-major, row pitch 80).
 #include <map>
 #include <mutex>
+#include <type_traits>
 
 #include "../kernels.hpp"
 
@@ -96,72 +95,6 @@ __device__ __forceinline__ void load_tiles(const double* __restrict__ A, const d
   }
 }
 
-// Register-staged variant of load_tiles for the FP64 kernel: fetch() issues
-// the global loads of one (A, B) k-tile into registers, stash() writes them to
-// LDS, so the loads of tile t+1 overlap the MFMAs of tile t.
-struct Regs {
-  double a[4], b[4];
-};
-
-__device__ __forceinline__ void fetch(const double* __restrict__ base, const GemmPair& pr, int M, int N, int m0,
-                                      int n0, int k0, int tid, Regs& r) {
-  const double* A = base + pr.a_off;
-  const double* B = base + pr.b_off;
-  const int K = pr.K;
-  if (pr.a_cs == 1) {
-    const int m = tid >> 2, kq = (tid & 3) * 4, gm = m0 + m;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gk = k0 + kq + j;
-      r.a[j] = (gm < M && gk < K) ? A[int64_t(gm) * pr.a_rs + gk] : 0.0;
-    }
-  } else {
-    const int k = tid >> 4, mq = (tid & 15) * 4, gk = k0 + k;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gm = m0 + mq + j;
-      r.a[j] = (gm < M && gk < K) ? A[int64_t(gm) * pr.a_rs + int64_t(gk) * pr.a_cs] : 0.0;
-    }
-  }
-  if (pr.b_cs == 1) {
-    const int k = tid >> 4, nq = (tid & 15) * 4, gk = k0 + k;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + nq + j;
-      r.b[j] = (gn < N && gk < K) ? B[int64_t(gk) * pr.b_rs + gn] : 0.0;
-    }
-  } else {
-    const int n = tid >> 2, kq = (tid & 3) * 4, gn = n0 + n;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gk = k0 + kq + j;
-      r.b[j] = (gn < N && gk < K) ? B[int64_t(gk) * pr.b_rs + int64_t(gn) * pr.b_cs] : 0.0;
-    }
-  }
-}
-
-__device__ __forceinline__ void stash(const GemmPair& pr, int tid, const Regs& r, double (*As)[LDP],
-                                      double (*Bs)[LDP]) {
-  if (pr.a_cs == 1) {
-    const int m = tid >> 2, kq = (tid & 3) * 4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) As[kq + j][m] = r.a[j];
-  } else {
-    const int k = tid >> 4, mq = (tid & 15) * 4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) As[k][mq + j] = r.a[j];
-  }
-  if (pr.b_cs == 1) {
-    const int k = tid >> 4, nq = (tid & 15) * 4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) Bs[k][nq + j] = r.b[j];
-  } else {
-    const int n = tid >> 2, kq = (tid & 3) * 4;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) Bs[kq + j][n] = r.b[j];
-  }
-}
-
 // Output element (row, col) of 16x16 MFMA tile register r in lane l:
 //   v_mfma_f64_16x16x4_f64: row = 4*r + l/16, col = l%16
 //   v_mfma_f32_16x16x4_f32: row = 4*(l/16) + r, col = l%16
@@ -186,74 +119,224 @@ __device__ __forceinline__ void store_tile(double* __restrict__ C, const GemmOut
       }
 }
 
-__global__ __launch_bounds__(256) void k_gemm_f64(double* __restrict__ base, const GemmTile* __restrict__ tiles,
-                                                  const GemmOut* __restrict__ outs,
-                                                  const GemmPair* __restrict__ pairs, double alpha, double beta) {
-  __shared__ double As[BK][LDP];
-  __shared__ double Bs[BK][LDP];
-  const GemmTile t = tiles[blockIdx.x];
-  const GemmOut o = outs[t.out];
-  const int m0 = t.tm * BM, n0 = t.tn * BN;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  v4d acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+// ---- FP64 grouped GEMM, contiguous operands -----------------------------------
+// One work-group computes a T x T tile (4 waves in 2 x 2); k in steps of 16
+// through a double-buffered LDS, one barrier a step, the next step's loads in
+// flight under the MFMAs of the current one.  An operand is contiguous in k
+// (KC) or in its rows, the same for every pair of the launch, so a thread
+// loads 16 bytes at a time (8-byte aligned: a global load needs 4) and the LDS
+// tile keeps the operand's own order: row by row (pitch 18) or k by k (pitch
+// T + 16), both free of bank conflicts for the MFMA reads.
+//
+// v_mfma_f64_16x16x4 takes 64 cycles and shares the FP64 units with every
+// vector instruction, so the loop keeps those out: loads are a scalar base
+// that moves with k and per-thread offsets fixed for a pair, the two LDS
+// buffers are unrolled to immediate offsets, and edges are dealt with only in
+// the steps that have one.  A thread's pair of rows (or of k) past the edge is
+// moved back inside the block; what it holds is put right on the way to LDS,
+// after the loads have been waited for.
+//
+// 2048^3 product: 53.6 TFLOP/s (at about 2.1 GHz; 47.7 with the offsets formed
+// every step, 40.1 for the general kernel below, which loads 8 bytes at a time
+// with a bounds check each).  T = 32 for launches with few tiles: a quarter of
+// the matrix work per step and four times the work-groups (two 146^3 Gram
+// products 6.3 us against 10.4 for T = 64, six of 149 .. 492: 23.7 against 28.8).
+//
+// Every output element accumulates over k in the same order whatever the tile
+// (4-wide MFMA chunks from each pair's k = 0, pairs in list order), so all
+// tiles give the same bits.
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef double v2d8 __attribute__((ext_vector_type(2), aligned(8)));
+constexpr int KS = 16;      // k per step
+constexpr int PK = KS + 2;  // LDS pitch of a row kept in k order
 
-  // flattened (pair, k-tile) iteration with one tile of register prefetch
-  int p = o.pair_begin, k0 = 0;
-  while (p < o.pair_end && pairs[p].K <= 0) ++p;
-  if (p < o.pair_end) {
-    GemmPair pr = pairs[p];
-    Regs cur;
-    fetch(base, pr, o.M, o.N, m0, n0, 0, tid, cur);
-    while (true) {
-      stash(pr, tid, cur, As, Bs);
-      __syncthreads();
-      // advance to the next tile and prefetch it
-      int np = p, nk = k0 + BK;
-      GemmPair npr = pr;
-      if (nk >= pr.K) {
-        nk = 0;
-        ++np;
-        while (np < o.pair_end && pairs[np].K <= 0) ++np;
-        if (np < o.pair_end) npr = pairs[np];
-      }
-      const bool more = np < o.pair_end;
-      Regs nxt;
-      if (more) fetch(base, npr, o.M, o.N, m0, n0, nk, tid, nxt);
+template <int T, bool KC>
+struct GemmOperand {
+  static constexpr int kElems = KC ? T * PK : KS * (T + 16);
+  static constexpr int kRow = KC ? PK : 1, kK = KC ? 1 : T + 16;  // LDS strides
+  static constexpr int E = T * KS / 512;         // 16-byte loads per thread and step
+  static constexpr int L = T / 2, KR = 256 / L;  // row order: threads per k, k per pass
+  v2d v[E];
+  uint32_t off[E];  // byte offsets from (row 0, first k of the step)
+  bool edge = false, swap = false;
+
+  static __device__ __forceinline__ int first_row(int R, int r0, int tid) {
+    return min(r0 + (tid % L) * 2, R < 2 ? 0 : R - 2);
+  }
+  static __device__ __forceinline__ int64_t step(int64_t ld) { return KC ? KS * 8 : KS * 8 * ld; }
+  // a new pair: element (r, k) at r * ld + k (KC) or k * ld + r
+  __device__ __forceinline__ void begin(int64_t ld, int R, int r0, int tid) {
+    if constexpr (KC) {
 #pragma unroll
-      for (int kk = 0; kk < BK; kk += 4) {
-        const int kr = kk + (lane >> 4), c = lane & 15;
-        const double a0 = As[kr][wm + c], a1 = As[kr][wm + 16 + c];
-        const double b0 = Bs[kr][wn + c], b1 = Bs[kr][wn + 16 + c];
-        acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-      }
-      __syncthreads();
-      if (!more) break;
-      p = np;
-      k0 = nk;
-      pr = npr;
-      cur = nxt;
+      for (int u = 0; u < E; ++u)
+        off[u] = (uint32_t(min(r0 + (tid >> 3) + 32 * u, R - 1)) * uint32_t(ld) + (tid & 7) * 2) * 8u;
+    } else {
+      edge = r0 + T > R;
+      const int r = first_row(R, r0, tid);
+      swap = r0 + (tid % L) * 2 != r;  // the block's last row, second of its pair here
+#pragma unroll
+      for (int u = 0; u < E; ++u) off[u] = (uint32_t(tid / L + KR * u) * uint32_t(ld) + uint32_t(r)) * 8u;
     }
   }
-  store_tile<true>(base + o.c_off, o, m0, n0, wm, wn, lane, acc, alpha, beta);
+  // p: (row 0, first k of the step); kleft: valid k from there
+  __device__ __forceinline__ void fetch(const char* __restrict__ p, int64_t ld, int R, int r0, int kleft, int tid) {
+    if (kleft >= KS && (KC || R >= 2)) {
+#pragma unroll
+      for (int u = 0; u < E; ++u) v[u] = *reinterpret_cast<const v2d8*>(p + off[u]);
+      return;
+    }
+    uint32_t o[E];
+    if constexpr (KC) {
+      const int k = min((tid & 7) * 2, kleft < 2 ? 0 : kleft - 2);
+#pragma unroll
+      for (int u = 0; u < E; ++u)
+        o[u] = (uint32_t(min(r0 + (tid >> 3) + 32 * u, R - 1)) * uint32_t(ld) + uint32_t(k)) * 8u;
+    } else {
+      const int r = first_row(R, r0, tid);
+#pragma unroll
+      for (int u = 0; u < E; ++u)
+        o[u] = (uint32_t(min(tid / L + KR * u, kleft - 1)) * uint32_t(ld) + uint32_t(r)) * 8u;
+    }
+    if (KC ? kleft < 2 : R < 2) {  // a single k or row: nothing beside it to load
+#pragma unroll
+      for (int u = 0; u < E; ++u) v[u].x = v[u].y = *reinterpret_cast<const double*>(p + o[u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < E; ++u) v[u] = *reinterpret_cast<const v2d8*>(p + o[u]);
+    }
+  }
+  __device__ __forceinline__ void stash(double* __restrict__ s, int kleft, int tid) const {
+    if constexpr (KC) {
+      const int k = (tid & 7) * 2;
+      double* d = s + (tid >> 3) * PK + k;
+#pragma unroll
+      for (int u = 0; u < E; ++u) {
+        v2d x = v[u];
+        if (kleft < KS && k + 1 >= kleft) {
+          x.x = k < kleft ? x.y : 0.0;
+          x.y = 0.0;
+        }
+        *reinterpret_cast<v2d*>(d + 32 * u * PK) = x;
+      }
+    } else {
+      double* d = s + (tid / L) * (T + 16) + (tid % L) * 2;
+#pragma unroll
+      for (int u = 0; u < E; ++u) {
+        v2d x = v[u];
+        if (edge && swap) x.x = x.y;
+        if (kleft < KS && tid / L + KR * u >= kleft) x = v2d{0.0, 0.0};
+        *reinterpret_cast<v2d*>(d + KR * u * (T + 16)) = x;
+      }
+    }
+  }
+};
+
+// AK: A contiguous in k (else in m); BN: B contiguous in n (else in k).
+template <int T, bool AK, bool BN>
+__global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, const GemmTile* __restrict__ tiles,
+                                                   const GemmOut* __restrict__ outs,
+                                                   const GemmPair* __restrict__ pairs, double alpha, double beta) {
+  using OpA = GemmOperand<T, AK>;
+  using OpB = GemmOperand<T, !BN>;
+  constexpr int F = T / 32;  // 16 x 16 MFMA tiles per wave and dimension
+  __shared__ __align__(16) double As[2 * OpA::kElems];
+  __shared__ __align__(16) double Bs[2 * OpB::kElems];
+  const GemmTile t = tiles[blockIdx.x];
+  const GemmOut o = outs[t.out];
+  const int m0 = t.tm * T, n0 = t.tn * T;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+  const int cl = lane & 15, kq = lane >> 4;
+  v4d acc[F][F];
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  int p = o.pair_begin;
+  while (p < o.pair_end && pairs[p].K <= 0) ++p;
+  if (p < o.pair_end) {
+    OpA ga;
+    OpB gb;
+    const char *pa, *pb;
+    int64_t lda, ldb;
+    int kleft;
+    auto begin = [&] {
+      const GemmPair pr = pairs[p];
+      pa = reinterpret_cast<const char*>(base + pr.a_off);
+      pb = reinterpret_cast<const char*>(base + pr.b_off);
+      lda = AK ? pr.a_rs : pr.a_cs;
+      ldb = BN ? pr.b_rs : pr.b_cs;
+      kleft = pr.K;
+      ga.begin(lda, o.M, m0, tid);
+      gb.begin(ldb, o.N, n0, tid);
+    };
+    auto fetch = [&] {
+      ga.fetch(pa, lda, o.M, m0, kleft, tid);
+      gb.fetch(pb, ldb, o.N, n0, kleft, tid);
+    };
+    begin();
+    fetch();
+    const int ao = (wm + cl) * OpA::kRow + kq * OpA::kK, bo = (wn + cl) * OpB::kRow + kq * OpB::kK;
+    auto step = [&](auto buf) {
+      double* sa = As + decltype(buf)::value * OpA::kElems;
+      double* sb = Bs + decltype(buf)::value * OpB::kElems;
+      const int have = kleft;
+      // this buffer's last readers passed the barrier of the step between
+      ga.stash(sa, have, tid);
+      gb.stash(sb, have, tid);
+      bool more = true;
+      kleft -= KS;
+      pa += OpA::step(lda);
+      pb += OpB::step(ldb);
+      if (kleft <= 0) {
+        ++p;
+        while (p < o.pair_end && pairs[p].K <= 0) ++p;
+        more = p < o.pair_end;
+        if (more) begin();
+      }
+      if (more) fetch();
+      __syncthreads();
+#pragma unroll
+      for (int kk = 0; kk < KS; kk += 4)
+        if (kk < have) {  // uniform: chunks past a pair's end are zeros
+          double a[F], b[F];
+#pragma unroll
+          for (int i = 0; i < F; ++i) a[i] = sa[ao + i * 16 * OpA::kRow + kk * OpA::kK];
+#pragma unroll
+          for (int j = 0; j < F; ++j) b[j] = sb[bo + j * 16 * OpB::kRow + kk * OpB::kK];
+#pragma unroll
+          for (int i = 0; i < F; ++i)
+#pragma unroll
+            for (int j = 0; j < F; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+      return more;
+    };
+    while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
+    }
+  }
+  double* C = base + o.c_off;
+#pragma unroll
+  for (int i = 0; i < F; ++i)
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = m0 + wm + i * 16 + 4 * r + kq;  // f64 MFMA output layout
+        const int col = n0 + wn + j * 16 + cl;
+        if (row < o.M && col < o.N) {
+          double* pc = C + int64_t(row) * o.ldc + col;
+          double v = alpha * acc[i][j][r];
+          if (beta != 0.0) v += beta * (*pc);
+          *pc = v;
+        }
+      }
 }
 
-// ---- tile variants of the FP64 grouped GEMM ---------------------------------
-// TM x TN output tile per work-group (4 waves in 2 x 2, each (TM/2) x (TN/2)
-// as (TM/32) x (TN/32) MFMA 16x16 tiles), k in steps of KD (16 or 32)
-// through a double-buffered LDS: the global loads of step t+1 are in
-// registers while the MFMAs of step t run, then written to the other buffer,
-// one barrier per step.  Every output element accumulates over k in the same
-// order as k_gemm_f64 (4-wide MFMA chunks from each pair's k = 0, pairs in
-// list order; the zero padding of a pair's last step adds exact zeros), so
-// all variants give the same bits.
+// ---- FP64 grouped GEMM, any strides --------------------------------------------
+// The same tile for launches whose pairs are not contiguous in one common way
+// (blocks with unit-length legs beside permuted ones): 8-byte loads with a
+// bounds check each, double-buffered LDS k by k.
 template <int TM, int TN, int KD>
 struct TileRegs {
   double a[TM * KD / 256], b[TN * KD / 256];
@@ -560,41 +643,45 @@ void gemm_rows(hipStream_t s, double* base, const RowTask* tasks, int ntasks, co
   hipLaunchKernelGGL(k_gemm_rows, dim3(ntasks), dim3(kRowsPerTask), 0, s, base, tasks, outs, pairs, alpha, beta);
 }
 
-void gemm_f64(hipStream_t s, double* base, const GemmTile* tiles, int ntiles, const GemmOut* outs,
-              const GemmPair* pairs, double alpha, double beta) {
-  if (ntiles <= 0) return;
-  hipLaunchKernelGGL(k_gemm_f64, dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha, beta);
+GemmLayout gemm_layout(const GemmPair* pairs, size_t n, const GemmOut* outs, size_t nouts) {
+  bool ak = true, am = true, bk = true, bn = true;
+  for (size_t o = 0; o < nouts; ++o)
+    for (int32_t q = outs[o].pair_begin; q < outs[o].pair_end && size_t(q) < n; ++q) {
+      const GemmPair& p = pairs[q];
+      if (p.K <= 0) continue;
+      // one k or one row: that dimension's stride is never used; the threads'
+      // offsets are 32-bit byte counts (whole rows, or 16 k of all rows)
+      const int64_t M = outs[o].M, N = outs[o].N, lim = int64_t(1) << 29;
+      ak &= (p.a_cs == 1 || p.K == 1) && M * p.a_rs + KS < lim;
+      am &= (p.a_rs == 1 || M == 1) && KS * p.a_cs + M < lim;
+      bk &= (p.b_rs == 1 || p.K == 1) && N * p.b_cs + KS < lim;
+      bn &= (p.b_cs == 1 || N == 1) && KS * p.b_rs + N < lim;
+    }
+  if (!(ak || am) || !(bk || bn)) return kLayoutAny;
+  return GemmLayout((ak ? 1 : 0) | (bn ? 2 : 0));
 }
 
-void gemm_f64_variant(hipStream_t s, int variant, double* base, const GemmTile* tiles, int ntiles,
-                      const GemmOut* outs, const GemmPair* pairs, double alpha, double beta) {
-  if (ntiles <= 0) return;
-  switch (variant) {
-    case kTile64:
-      hipLaunchKernelGGL(k_gemm_f64, dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha, beta);
-      break;
-    case kTile64db:
-      hipLaunchKernelGGL((k_gemm_f64t<64, 64, 16>), dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha, beta);
-      break;
-    case kTile128x64:
-      hipLaunchKernelGGL((k_gemm_f64t<128, 64, 16>), dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha,
-                         beta);
-      break;
-    case kTile64x128:
-      hipLaunchKernelGGL((k_gemm_f64t<64, 128, 16>), dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha,
-                         beta);
-      break;
-    case kTile128:
-      hipLaunchKernelGGL((k_gemm_f64t<128, 128, 16>), dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha,
-                         beta);
-      break;
-    case kTile64k32:
-      hipLaunchKernelGGL((k_gemm_f64t<64, 64, 32>), dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha,
-                         beta);
-      break;
-    default:
-      break;
+template <int T>
+static void gemm_contiguous(hipStream_t s, GemmLayout lay, double* base, const GemmTile* tiles, int ntiles,
+                            const GemmOut* outs, const GemmPair* pairs, double alpha, double beta) {
+  const dim3 g(ntiles), b(256);
+  switch (int(lay)) {
+    case 0: hipLaunchKernelGGL((k_gemm_f64c<T, false, false>), g, b, 0, s, base, tiles, outs, pairs, alpha, beta); break;
+    case 1: hipLaunchKernelGGL((k_gemm_f64c<T, true, false>), g, b, 0, s, base, tiles, outs, pairs, alpha, beta); break;
+    case 2: hipLaunchKernelGGL((k_gemm_f64c<T, false, true>), g, b, 0, s, base, tiles, outs, pairs, alpha, beta); break;
+    default: hipLaunchKernelGGL((k_gemm_f64c<T, true, true>), g, b, 0, s, base, tiles, outs, pairs, alpha, beta); break;
   }
+}
+
+void gemm_f64(hipStream_t s, int tile, GemmLayout lay, double* base, const GemmTile* tiles, int ntiles,
+              const GemmOut* outs, const GemmPair* pairs, double alpha, double beta) {
+  if (ntiles <= 0) return;
+  if (lay == kLayoutAny)
+    hipLaunchKernelGGL((k_gemm_f64t<64, 64, 16>), dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha, beta);
+  else if (tile == 32)
+    gemm_contiguous<32>(s, lay, base, tiles, ntiles, outs, pairs, alpha, beta);
+  else
+    gemm_contiguous<64>(s, lay, base, tiles, ntiles, outs, pairs, alpha, beta);
 }
 
 void gemm_split(hipStream_t s, double* base, const GemmTile* tiles, int ntiles, const GemmOut* outs,

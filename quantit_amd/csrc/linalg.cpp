@@ -95,18 +95,27 @@ struct GemmLaunch {
   const kern::GemmOut* outs = nullptr;
   const kern::GemmPair* pairs = nullptr;
   int ntiles = 0;
+  int tile = kern::kGemmTile;
+  kern::GemmLayout lay = kern::kLayoutAny;
 };
 
 GemmLaunch prepare_gemm(Context* ctx, const std::vector<kern::GemmOut>& outs,
                         const std::vector<kern::GemmPair>& pairs) {
+  GemmLaunch g;
+  g.lay = kern::gemm_layout(pairs.data(), pairs.size(), outs.data(), outs.size());
+  auto count = [&](int t) {
+    int64_t n = 0;
+    for (const auto& o : outs) n += int64_t((o.M + t - 1) / t) * ((o.N + t - 1) / t);
+    return n;
+  };
+  if (g.lay != kern::kLayoutAny && count(64) < kern::kTile64Min) g.tile = 32;
   std::vector<kern::GemmTile> tiles;
+  tiles.reserve(size_t(count(g.tile)));
   for (size_t o = 0; o < outs.size(); ++o) {
-    const int tm = (outs[o].M + kern::kGemmTile - 1) / kern::kGemmTile;
-    const int tn = (outs[o].N + kern::kGemmTile - 1) / kern::kGemmTile;
+    const int tm = (outs[o].M + g.tile - 1) / g.tile, tn = (outs[o].N + g.tile - 1) / g.tile;
     for (int i = 0; i < tm; ++i)
       for (int j = 0; j < tn; ++j) tiles.push_back({int32_t(o), int16_t(i), int16_t(j)});
   }
-  GemmLaunch g;
   if (tiles.empty()) return g;
   std::tie(g.tiles, g.outs, g.pairs) = ctx->upload_pack(tiles, outs, pairs);
   g.ntiles = int(tiles.size());
@@ -117,7 +126,7 @@ void run_gemm(Context* ctx, double* ab, const GemmLaunch& g, const char* name, d
               double beta = 0.0) {
   if (g.ntiles == 0) return;
   KernelTimer kt(*ctx, name);
-  kern::gemm_f64(ctx->stream(), ab, g.tiles, g.ntiles, g.outs, g.pairs, alpha, beta);
+  kern::gemm_f64(ctx->stream(), g.tile, g.lay, ab, g.tiles, g.ntiles, g.outs, g.pairs, alpha, beta);
 }
 
 void launch_gemm(Context* ctx, double* ab, const std::vector<kern::GemmOut>& outs,

@@ -78,7 +78,7 @@ struct KeyEnt {
 // ---- GEMM tile-variant tuning table (process-wide) -----------------------------
 // A contraction's shape class: log2 of the work-weighted mean M and N of its
 // MFMA outputs and of its 64 x 64 tile count.  Classes with fewer than
-// kTuneMinTiles tiles always take the 64 x 64 tile (latency-bound).
+// kTuneMinTiles tiles always take the 32 x 32 tile (latency-bound).
 constexpr int64_t kTuneMinTiles = 64;
 
 struct TuneTable {
@@ -109,7 +109,7 @@ std::string gemm_shape_key(const std::vector<kern::GemmOut>& outs, const std::ve
 }
 
 // Variant for a class.  QTT_GEMM_VARIANT=<n> forces one; QTT_GEMM_TUNE=0
-// disables tuning (64 x 64 unless the table has an entry).  *tune is set
+// disables tuning (the rule of kTile64Min unless the table has an entry).  *tune is set
 // when the caller should time the variants now (unknown class, tuning on,
 // timing allowed).
 int gemm_variant_for(const std::string& key, int64_t tiles, bool may_time, bool* tune) {
@@ -118,7 +118,7 @@ int gemm_variant_for(const std::string& key, int64_t tiles, bool may_time, bool*
     const int v = std::atoi(f);
     if (v >= 0 && v < kern::kGemmVariants) return v;
   }
-  if (tiles < kTuneMinTiles) return kern::kTile64;
+  if (tiles < kTuneMinTiles) return kern::kTile32;
   {
     TuneTable& t = tune_table();
     std::lock_guard<std::mutex> lk(t.mu);
@@ -127,7 +127,7 @@ int gemm_variant_for(const std::string& key, int64_t tiles, bool may_time, bool*
   }
   const char* e = std::getenv("QTT_GEMM_TUNE");
   *tune = may_time && !(e && std::atoi(e) == 0);
-  return kern::kTile64;
+  return tiles < kern::kTile64Min ? kern::kTile32 : kern::kTile64;
 }
 
 void gemm_variant_record(const std::string& key, int v) {
@@ -256,7 +256,8 @@ struct TdPlan::Launch {
   const kern::ChunkTask* sum_tasks = nullptr;
   int nsum_tasks = 0;
   bool split_fp32 = false;
-  int variant = 0;  // FP64 tile variant (kern::GemmVariant)
+  int tile = kern::kGemmTile;  // FP64 tile edge
+  kern::GemmLayout lay = kern::kLayoutAny;
   const char* gemm_name = "gemm_f64";
 };
 
@@ -284,7 +285,7 @@ void td_run(Context* ctx, const TdPlan::Launch& l, bool timed) {
     kern::gemm_split(ctx->stream(), ab, l.tiles, l.ntiles, l.outs, l.pairs, 1.0, 0.0);
   } else {
     auto kt = timer(l.gemm_name);
-    kern::gemm_f64_variant(ctx->stream(), l.variant, ab, l.tiles, l.ntiles, l.outs, l.pairs, 1.0, 0.0);
+    kern::gemm_f64(ctx->stream(), l.tile, l.lay, ab, l.tiles, l.ntiles, l.outs, l.pairs, 1.0, 0.0);
   }
   if (l.nsum_tasks) {
     auto kt = timer("gemm_split_k_sum");
@@ -750,14 +751,13 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
   std::vector<int> ord(launch_outs.size());
   std::iota(ord.begin(), ord.end(), 0);
   std::stable_sort(ord.begin(), ord.end(), [&](int x, int y) { return launch_work[x] > launch_work[y]; });
-  // MFMA tiles of a TM x TN variant, longest work first, row by row
-  auto tiles_of = [&](int variant) {
-    const int TM = kern::kVariantTM[variant], TN = kern::kVariantTN[variant];
+  // MFMA tiles of edge T, longest work first, row by row
+  auto tiles_of = [&](int T) {
     std::vector<kern::GemmTile> tl;
     for (int o : ord) {
       if (size_t(o) < outs.size() && (narrow[size_t(o)] || split_block[size_t(o)])) continue;
-      const int tm = (launch_outs[o].M + TM - 1) / TM;
-      const int tn = (launch_outs[o].N + TN - 1) / TN;
+      const int tm = (launch_outs[o].M + T - 1) / T;
+      const int tn = (launch_outs[o].N + T - 1) / T;
       for (int i = 0; i < tm; ++i)
         for (int j = 0; j < tn; ++j) tl.push_back({int32_t(o), int16_t(i), int16_t(j)});
     }
@@ -768,19 +768,24 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
       const int rpt = kern::rows_per_task(gouts[o].N);
       for (int r0 = 0; r0 < gouts[o].M; r0 += rpt) row_tasks.push_back({int32_t(o), int32_t(r0)});
     }
-  // tile variant: from the tuning table for this contraction's shape class;
-  // a class not seen yet is timed over every variant when the call may
-  // time (not inside plans or the allocation-free path), else the 64 x 64
-  // tile runs
+  // tile: from the tuning table for this contraction's shape class; a class
+  // not seen yet is timed when the call may time (not inside plans or the
+  // allocation-free path), else kTile64Min decides.  Pairs without a common
+  // contiguous dimension take the general kernel.
   const bool f64_tiles = ctx->precision == Precision::FP64 && !per_block;
-  int variant = kern::kTile64;
   std::string tune_key;
   bool tune_now = false;
-  if (f64_tiles) {
+  if (f64_tiles && !all_narrow) {
     tune_key = gemm_shape_key(launch_outs, launch_work, mfma_tiles);
-    variant = gemm_variant_for(tune_key, mfma_tiles, work.timed(), &tune_now);
+    const int variant = gemm_variant_for(tune_key, mfma_tiles, work.timed(), &tune_now);
+    if (variant != kern::kTileAny)
+      lch.lay = kern::gemm_layout(gpairs.data(), gpairs.size(), launch_outs.data(), launch_outs.size());
+    if (lch.lay == kern::kLayoutAny)
+      tune_now = false;
+    else
+      lch.tile = kern::variant_tile(variant);
   }
-  tiles = tiles_of(tune_now ? int(kern::kTile64) : variant);
+  tiles = tiles_of(lch.tile);
   if (stats) {
     stats->flops += flops;
     stats->bytes += bytes;
@@ -811,12 +816,13 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     }
     td_pack(ctx, lch, true);
     if (one.empty()) return out;
+    const kern::GemmLayout lay = kern::gemm_layout(gpairs.data(), gpairs.size(), one.data(), one.size());
     auto [d_one, d_tl, d_pairs] = ctx->upload_pack(one, tl, gpairs);
     for (size_t l = 0; l < launches.size(); ++l) {
       const bool first = l == 0 || one[l].c_off != one[l - 1].c_off;
       KernelTimer kt(*ctx, "gemm_per_block");
-      kern::gemm_f64(ctx->stream(), ab, d_tl + launches[l].first, launches[l].second, d_one, d_pairs, 1.0,
-                     first ? 0.0 : 1.0);
+      kern::gemm_f64(ctx->stream(), kern::kGemmTile, lay, ab, d_tl + launches[l].first, launches[l].second, d_one,
+                     d_pairs, 1.0, first ? 0.0 : 1.0);
     }
     return out;
   }
@@ -829,38 +835,40 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
   lch.nrows = int(row_tasks.size());
   lch.nsum_tasks = int(sum_tasks.size());
   lch.split_fp32 = ctx->precision == Precision::SPLIT_FP32;
-  lch.variant = variant;
   lch.gemm_name = ctx->gemm_label ? ctx->gemm_label : (lch.split_fp32 ? "gemm_split" : "gemm_f64");
   if (tune_now) {
-    // operands ready, then every variant timed on the real launch (each
-    // writes the same output bits); the fastest is recorded and used
+    // operands ready, then both tiles timed on the real launch (each writes
+    // the same output bits); the faster is recorded and used
     td_pack(ctx, lch, false);
     lch.nptasks = 0;
     float best_ms = 0.f;
+    int best = kern::kTile64;
     hipEvent_t e0, e1;
     QTT_HIP(hipEventCreate(&e0));
     QTT_HIP(hipEventCreate(&e1));
-    for (int v = 0; v < kern::kGemmVariants; ++v) {
-      std::vector<kern::GemmTile> tl = tiles_of(v);
+    for (int v : {kern::kTile64, kern::kTile32}) {
+      const int T = kern::variant_tile(v);
+      std::vector<kern::GemmTile> tl = tiles_of(T);
       const kern::GemmTile* dt = ctx->upload_vec(tl);
       float ms = 0.f;
       for (int rep = 0; rep < 2; ++rep) {
         QTT_HIP(hipEventRecord(e0, ctx->stream()));
-        kern::gemm_f64_variant(ctx->stream(), v, ab, dt, int(tl.size()), lch.outs, lch.pairs, 1.0, 0.0);
+        kern::gemm_f64(ctx->stream(), T, lch.lay, ab, dt, int(tl.size()), lch.outs, lch.pairs, 1.0, 0.0);
         QTT_HIP(hipEventRecord(e1, ctx->stream()));
         QTT_HIP(hipEventSynchronize(e1));
         QTT_HIP(hipEventElapsedTime(&ms, e0, e1));
       }
-      if (v == 0 || ms < best_ms) {
+      if (v == kern::kTile64 || ms < best_ms) {
         best_ms = ms;
-        lch.variant = v;
+        best = v;
+        lch.tile = T;
         lch.tiles = dt;
         lch.ntiles = int(tl.size());
       }
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    gemm_variant_record(tune_key, lch.variant);
+    gemm_variant_record(tune_key, best);
   }
   if (plan)
     *plan = lch;
