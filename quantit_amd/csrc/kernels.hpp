@@ -47,8 +47,8 @@ enum GemmVariant : int { kTileAny = 0, kTile64 = 1, kTile32 = 5, kGemmVariants =
 inline int variant_tile(int v) { return v == kTile32 ? 32 : 64; }
 // Tile of a launch that is not timed: 32 x 32 below this many 64 x 64 tiles
 // (three per CU), where the longest tile and the idle CUs decide: 225 tiles
-// 165 us against 216, 218 tiles 23.7 against 28.8; from 1024 tiles on the 64 x
-// 64 tile is ahead (318 us against 439 at 1024, 112 against 137 at 5707).
+// 161 us against 245, 218 tiles 24.4 against 33.1; from 1024 tiles on the 64 x
+// 64 tile is ahead (323 us against 430 at 1024, 107 against 136 at 5707).
 constexpr int64_t kTile64Min = 768;
 
 // Size of the file-scope device scratch (kernels/gemm.hip) that the

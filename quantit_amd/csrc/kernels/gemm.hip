@@ -136,6 +136,12 @@ __device__ __forceinline__ void store_tile(double* __restrict__ C, const GemmOut
 // moved back inside the block; what it holds is put right on the way to LDS,
 // after the loads have been waited for.
 //
+// Products of a ragged tile that have no element in the block are left out:
+// 8101 tiles over blocks of 1 .. 1000 rows 188 us against 214, 5707 tiles of a
+// matvec 107 against 112 (a tile still loads whole, so its time does not fall
+// with its products when few tiles are in flight: 225 tiles 245 us against 216,
+// which run at T = 32 below kTile64Min).
+//
 // 2048^3 product: 53.6 TFLOP/s (at about 2.1 GHz; 47.7 with the offsets formed
 // every step, 40.1 for the general kernel below, which loads 8 bytes at a time
 // with a bounds check each).  T = 32 for launches with few tiles: a quarter of
@@ -245,7 +251,12 @@ __global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, co
   const GemmOut o = outs[t.out];
   const int m0 = t.tm * T, n0 = t.tn * T;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * (T / 2), wn = (wave & 1) * (T / 2);
+  // a wave takes every other 16 x 16 product of the tile in each dimension, so
+  // what a ragged edge leaves of a tile is spread over all four; mi x nj of
+  // its F x F have elements in the block
+  const int wm = (wave >> 1) * 16, wn = (wave & 1) * 16;
+  const int mi = __builtin_amdgcn_readfirstlane(min(F, (o.M - m0 - wm + 31) / 32));
+  const int nj = __builtin_amdgcn_readfirstlane(min(F, (o.N - n0 - wn + 31) / 32));
   const int cl = lane & 15, kq = lane >> 4;
   v4d acc[F][F];
 #pragma unroll
@@ -277,7 +288,7 @@ __global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, co
     begin();
     fetch();
     const int ao = (wm + cl) * OpA::kRow + kq * OpA::kK, bo = (wn + cl) * OpB::kRow + kq * OpB::kK;
-    auto step = [&](auto buf) {
+    auto step = [&](auto buf, auto whole) {
       double* sa = As + decltype(buf)::value * OpA::kElems;
       double* sb = Bs + decltype(buf)::value * OpB::kElems;
       const int have = kleft;
@@ -296,23 +307,44 @@ __global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, co
       }
       if (more) fetch();
       __syncthreads();
+      auto multiply = [&](auto fi, auto fj) {
+        constexpr int FI = decltype(fi)::value, FJ = decltype(fj)::value;
 #pragma unroll
-      for (int kk = 0; kk < KS; kk += 4)
-        if (kk < have) {  // uniform: chunks past a pair's end are zeros
-          double a[F], b[F];
+        for (int kk = 0; kk < KS; kk += 4)
+          if (kk < have) {  // uniform: chunks past a pair's end are zeros
+            double a[FI], b[FJ];
 #pragma unroll
-          for (int i = 0; i < F; ++i) a[i] = sa[ao + i * 16 * OpA::kRow + kk * OpA::kK];
+            for (int i = 0; i < FI; ++i) a[i] = sa[ao + i * 32 * OpA::kRow + kk * OpA::kK];
 #pragma unroll
-          for (int j = 0; j < F; ++j) b[j] = sb[bo + j * 16 * OpB::kRow + kk * OpB::kK];
+            for (int j = 0; j < FJ; ++j) b[j] = sb[bo + j * 32 * OpB::kRow + kk * OpB::kK];
 #pragma unroll
-          for (int i = 0; i < F; ++i)
+            for (int i = 0; i < FI; ++i)
 #pragma unroll
-            for (int j = 0; j < F; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
+              for (int j = 0; j < FJ; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+          }
+      };
+      constexpr std::integral_constant<int, F> all{};
+      constexpr std::integral_constant<int, 1> one{};
+      if (decltype(whole)::value || (mi == F && nj == F)) {
+        multiply(all, all);
+      } else if constexpr (F == 2) {
+        if (mi == 1 && nj == 2) multiply(one, all);
+        if (mi == 2 && nj == 1) multiply(all, one);
+        if (mi == 1 && nj == 1) multiply(one, one);
+      }
       return more;
     };
-    while (step(std::integral_constant<int, 0>{}) && step(std::integral_constant<int, 1>{})) {
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    // a loop of their own for tiles inside the block: the choice of products
+    // in every step costs them 7 %
+    if (o.M - m0 >= T && o.N - n0 >= T) {
+      while (step(even, std::true_type{}) && step(odd, std::true_type{})) {
+      }
+    } else {
+      while (step(even, std::false_type{}) && step(odd, std::false_type{})) {
+      }
     }
   }
   double* C = base + o.c_off;
@@ -322,8 +354,8 @@ __global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, co
     for (int j = 0; j < F; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm + i * 16 + 4 * r + kq;  // f64 MFMA output layout
-        const int col = n0 + wn + j * 16 + cl;
+        const int row = m0 + wm + i * 32 + 4 * r + kq;  // f64 MFMA output layout
+        const int col = n0 + wn + j * 32 + cl;
         if (row < o.M && col < o.N) {
           double* pc = C + int64_t(row) * o.ldc + col;
           double v = alpha * acc[i][j][r];
