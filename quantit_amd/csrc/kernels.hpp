@@ -25,7 +25,7 @@ struct GemmOut {
 struct GemmPair {
   int64_t a_off, b_off;
   int64_t a_rs, a_cs, b_rs, b_cs;
-  int32_t K, pad;
+  int32_t K, k0;  // k0: summed K of the output's pairs before this one (gemm_rows)
 };
 struct GemmTile {
   int32_t out;
@@ -63,16 +63,18 @@ hipError_t noalloc_scratch_address(int device, void** out);
 // chunk and are folded into FP64 accumulators after every chunk.
 void gemm_split(hipStream_t s, double* base, const GemmTile* tiles, int ntiles, const GemmOut* outs,
                 const GemmPair* pairs, double alpha, double beta);
-// Output blocks with at most kRowsMaxN columns and a short summed K: one
-// thread per output row (B staged in LDS), the pairs in order, k ascending
-// (one FP64 FMA chain per element).  A task is kRowsPerTask consecutive rows
-// of one output block.
-constexpr int kRowsMaxN = 16, kRowsMaxK = 128, kRowsPerTask = 256;
+// Output blocks with at most kRowsMaxN columns and a short summed K.  A task is
+// 64 or 128 (task_rows) consecutive rows of one output block: 64 while the
+// work-groups all fit on the chip at once (30 blocks of 300 rows, K 128: 8.6 us
+// against 9.9; 72 k rows 4.1 against 4.2), above that 128, whose longer streams
+// hide more (760 k rows of 7 and 12 columns, K 33: 46.8 us against 52.3, 85.6
+// for one thread a row; 1 M rows, N 3, K 5: 16.2 against 21.6 and 18.2).
+constexpr int kRowsMaxN = 16, kRowsMaxK = 128;
 struct RowTask {
   int32_t out, row0;
 };
-inline int rows_per_task(int) { return kRowsPerTask; }
-void gemm_rows(hipStream_t s, double* base, const RowTask* tasks, int ntasks, const GemmOut* outs,
+inline int rows_per_task(int64_t rows) { return rows < 64 * 2048 ? 64 : 128; }
+void gemm_rows(hipStream_t s, double* base, const RowTask* tasks, int ntasks, int task_rows, const GemmOut* outs,
                const GemmPair* pairs, double alpha, double beta);
 
 // ---- data movement ----------------------------------------------------------

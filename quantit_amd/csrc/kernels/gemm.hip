@@ -615,64 +615,107 @@ __global__ __launch_bounds__(256) void k_gemm_split(double* __restrict__ base, c
   store_tile<false>(base + o.c_off, o, m0, n0, wm, wn, lane, acc, alpha, beta);
 }
 
-// Narrow outputs (N <= kRowsMaxN, summed K <= kRowsMaxK): an MFMA tile
-// would be mostly padding there.  One thread per output row: B of every
-// pair (at most kRowsMaxK x kRowsMaxN) is staged in LDS once per work-group,
-// each thread streams its row of A (lanes read consecutive rows when A's row
-// stride is 1) and keeps the N accumulators in registers.  Every element is
-// one FP64 FMA chain over the pairs in order, k ascending.
-__global__ __launch_bounds__(kRowsPerTask) void k_gemm_rows(double* __restrict__ base,
-                                                             const RowTask* __restrict__ tasks,
-                                                             const GemmOut* __restrict__ outs,
-                                                             const GemmPair* __restrict__ pairs, double alpha,
-                                                             double beta) {
-  __shared__ double Bs[kRowsMaxK * kRowsMaxN];
+// Narrow outputs (N <= kRowsMaxN, summed K <= kRowsMaxK): an MFMA tile of the
+// kernels above would be mostly padding there, and these launches are short:
+// the chain of dependent loads decides, then the streaming of A.  A wave takes
+// RT x 16 rows and all columns as v_mfma_f64_16x16x4 products of the transposed
+// operands (a store then holds four columns of 16 rows, contiguous for N <= 4),
+// the operands straight from global memory, the next two chunks in flight.  The k of all pairs form one list, so a
+// pair of one or two k wastes nothing; where each k lives goes to LDS first.
+// Twelve blocks of 4 .. 15 rows and columns, K 48: 4.7 us against 34.7 for a
+// thread per row with B in LDS, whose loads came four at a time.
+// Every element is one chain over the pairs in order, k ascending.
+struct RowK {
+  int64_t a_off, a_rs, b_off, b_cs;
+};
+template <int RT>
+__global__ __launch_bounds__(256) void k_gemm_rows(double* __restrict__ base, const RowTask* __restrict__ tasks,
+                                                   const GemmOut* __restrict__ outs,
+                                                   const GemmPair* __restrict__ pairs, double alpha, double beta) {
+  __shared__ RowK ks[kRowsMaxK];
   const RowTask t = tasks[blockIdx.x];
   const GemmOut o = outs[t.out];
-  int kb = 0;
-  for (int p = o.pair_begin; p < o.pair_end; ++p) {
-    const GemmPair pr = pairs[p];
-    const double* B = base + pr.b_off;
-    for (int e = int(threadIdx.x); e < pr.K * o.N; e += blockDim.x) {
-      const int k = e / o.N, n = e - k * o.N;
-      Bs[(kb + k) * kRowsMaxN + n] = B[int64_t(k) * pr.b_rs + int64_t(n) * pr.b_cs];
-    }
-    kb += pr.K;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int np = o.pair_end - o.pair_begin;
+  int ksum = 0;
+  if (np > 0) {
+    const GemmPair last = pairs[o.pair_end - 1];
+    ksum = last.k0 + last.K;
+  }
+  for (int q = tid >> 4; q < np; q += 16) {
+    const GemmPair pr = pairs[o.pair_begin + q];
+    for (int k = tid & 15; k < pr.K; k += 16)
+      ks[pr.k0 + k] = {pr.a_off + k * pr.a_cs, pr.a_rs, pr.b_off + k * pr.b_rs, pr.b_cs};
   }
   __syncthreads();
-  const int m = t.row0 + int(threadIdx.x);
-  if (m >= o.M) return;
-  double acc[kRowsMaxN];
+  const int m0 = t.row0 + (tid >> 6) * 16 * RT;
+  if (m0 >= o.M || o.N <= 0) return;
+  const int cl = lane & 15, kq = lane >> 4;
+  const int64_t n = min(cl, o.N - 1);
+  int64_t m[RT];
 #pragma unroll
-  for (int n = 0; n < kRowsMaxN; ++n) acc[n] = 0.0;
-  kb = 0;
-  for (int p = o.pair_begin; p < o.pair_end; ++p) {
-    const GemmPair pr = pairs[p];
-    const double* A = base + pr.a_off + int64_t(m) * pr.a_rs;
-#pragma unroll 4
-    for (int k = 0; k < pr.K; ++k) {
-      const double a = A[int64_t(k) * pr.a_cs];
-      const double* bk = Bs + (kb + k) * kRowsMaxN;
+  for (int i = 0; i < RT; ++i) m[i] = min(m0 + 16 * i + cl, o.M - 1);
+  v4d acc[RT];
 #pragma unroll
-      for (int n = 0; n < kRowsMaxN; ++n)
-        if (n < o.N) acc[n] = fma(a, bk[n], acc[n]);
+  for (int i = 0; i < RT; ++i) acc[i] = v4d{0.0, 0.0, 0.0, 0.0};
+  // chunk c: k = 4 c .. 4 c + 3 of the list, one per lane quarter; loads past
+  // the list's end repeat its last k, and their values are dropped
+  auto load = [&](int c, double (&a)[RT], double& b) {
+    const RowK e = ks[min(4 * c + kq, ksum - 1)];
+    b = base[e.b_off + n * e.b_cs];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) a[i] = base[e.a_off + m[i] * e.a_rs];
+  };
+  auto multiply = [&](int c, double (&a)[RT], double b) {
+    if (4 * c + 4 > ksum) {
+      const bool in = 4 * c + kq < ksum;
+      b = in ? b : 0.0;
+#pragma unroll
+      for (int i = 0; i < RT; ++i) a[i] = in ? a[i] : 0.0;
     }
-    kb += pr.K;
+#pragma unroll
+    for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a[i], acc[i], 0, 0, 0);
+  };
+  if (ksum > 0) {
+    const int nc = (ksum + 3) / 4;
+    double a0[RT], a1[RT], b0, b1;
+    load(0, a0, b0);
+    load(1, a1, b1);
+    if (nc <= 2) {
+      multiply(0, a0, b0);
+      if (nc == 2) multiply(1, a1, b1);
+    } else {
+      for (int c = 0; c < nc; c += 2) {
+        multiply(c, a0, b0);
+        load(c + 2, a0, b0);
+        if (c + 1 < nc) multiply(c + 1, a1, b1);
+        load(c + 3, a1, b1);
+      }
+    }
   }
-  double* C = base + o.c_off + int64_t(m) * o.ldc;
 #pragma unroll
-  for (int n = 0; n < kRowsMaxN; ++n)
-    if (n < o.N) {
-      double v = alpha * acc[n];
-      if (beta != 0.0) v += beta * C[n];
-      C[n] = v;
+  for (int i = 0; i < RT; ++i) {
+    const int row = m0 + 16 * i + cl;
+    double* C = base + o.c_off + int64_t(row) * o.ldc;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int col = 4 * r + kq;  // f64 MFMA output layout, transposed
+      if (row < o.M && col < o.N) {
+        double v = alpha * acc[i][r];
+        if (beta != 0.0) v += beta * C[col];
+        C[col] = v;
+      }
     }
+  }
 }
 
-void gemm_rows(hipStream_t s, double* base, const RowTask* tasks, int ntasks, const GemmOut* outs,
+void gemm_rows(hipStream_t s, double* base, const RowTask* tasks, int ntasks, int task_rows, const GemmOut* outs,
                const GemmPair* pairs, double alpha, double beta) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(k_gemm_rows, dim3(ntasks), dim3(kRowsPerTask), 0, s, base, tasks, outs, pairs, alpha, beta);
+  if (task_rows == 128)
+    hipLaunchKernelGGL(k_gemm_rows<2>, dim3(ntasks), dim3(256), 0, s, base, tasks, outs, pairs, alpha, beta);
+  else
+    hipLaunchKernelGGL(k_gemm_rows<1>, dim3(ntasks), dim3(256), 0, s, base, tasks, outs, pairs, alpha, beta);
 }
 
 GemmLayout gemm_layout(const GemmPair* pairs, size_t n, const GemmOut* outs, size_t nouts) {

@@ -247,7 +247,7 @@ struct TdPlan::Launch {
   const kern::ChunkTask* ptasks = nullptr;
   int nptasks = 0;
   const kern::RowTask* rows = nullptr;
-  int nrows = 0;
+  int nrows = 0, task_rows = 64;
   const kern::GemmTile* tiles = nullptr;
   int ntiles = 0;
   const kern::GemmOut* outs = nullptr;
@@ -278,7 +278,7 @@ void td_run(Context* ctx, const TdPlan::Launch& l, bool timed) {
   td_pack(ctx, l, timed);
   if (l.nrows) {
     auto kt = timer("gemm_rows");
-    kern::gemm_rows(ctx->stream(), ab, l.rows, l.nrows, l.outs, l.pairs, 1.0, 0.0);
+    kern::gemm_rows(ctx->stream(), ab, l.rows, l.nrows, l.task_rows, l.outs, l.pairs, 1.0, 0.0);
   }
   if (l.split_fp32) {
     auto kt = timer(l.gemm_name);
@@ -642,6 +642,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
       gp.b_rs = y.rs;
       gp.b_cs = y.cs;
       gp.K = int32_t(x.K);
+      gp.k0 = int32_t(ksum);
       gpairs.push_back(gp);
       ksum += x.K;
       flops += 2.0 * double(M) * double(N) * double(x.K);
@@ -763,10 +764,14 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     }
     return tl;
   };
+  if (all_narrow) {
+    int64_t rows = 0;
+    for (auto& o : gouts) rows += o.M;
+    lch.task_rows = kern::rows_per_task(rows);
+  }
   for (int o : ord)
     if (size_t(o) < outs.size() && narrow[size_t(o)]) {
-      const int rpt = kern::rows_per_task(gouts[o].N);
-      for (int r0 = 0; r0 < gouts[o].M; r0 += rpt) row_tasks.push_back({int32_t(o), int32_t(r0)});
+      for (int64_t r0 = 0; r0 < gouts[o].M; r0 += lch.task_rows) row_tasks.push_back({int32_t(o), int32_t(r0)});
     }
   // tile: from the tuning table for this contraction's shape class; a class
   // not seen yet is timed when the call may time (not inside plans or the

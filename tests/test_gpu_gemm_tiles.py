@@ -74,3 +74,27 @@ def test_pairs_without_a_common_layout(ctx, monkeypatch, variant):
         out = from_dev(to_dev(ctx, A).tensordot(to_dev(ctx, B), da, db))
         ref = np.tensordot(A.to_dense(), B.to_dense(), (da, db))
         assert np.array_equal(out.to_dense(), ref), (da, db)
+
+
+@pytest.mark.parametrize("rows", [1, 15, 17, 64, 65, 129, 40_000])
+def test_narrow_products_are_exact(ctx, rows):
+    """The row kernel: several pairs to an output, summed K over no whole
+    chunks of four, every column count, both task sizes (the last entry has
+    more than 2^17 rows in all); infinite neighbours stay out."""
+    rng = np.random.default_rng(rows)
+    for ks, cols in (([1], [1, 2]), ([1, 2, 2], [3, 4, 5, 16]), ([5, 60, 63], [7, 12])):
+        m = [rows, 1 + rows // 2]
+        A = BTensor(G1, [m, ks], [[(0,)] * len(m), [(0,)] * len(ks)], (0,))
+        B = BTensor(G1, [ks, cols], [[(0,)] * len(ks), [(0,)] * len(cols)], (0,))
+        for i, r in enumerate(m):
+            for j, k in enumerate(ks):
+                A.blocks[(i, j)] = rng.integers(-9, 10, (r, k)).astype(float)
+        for j, k in enumerate(ks):
+            for i, n in enumerate(cols):
+                B.blocks[(j, i)] = rng.integers(-9, 10, (k, n)).astype(float)
+        inf = np.inf
+        A.blocks[(1, len(ks) - 1)][:] = inf  # reaches the second row block only
+        out = from_dev(to_dev(ctx, A).tensordot(to_dev(ctx, B), [1], [0]))
+        for c in range(len(cols)):
+            ref = sum(A.blocks[(0, j)] @ B.blocks[(j, c)] for j in range(len(ks)))
+            assert np.array_equal(out.blocks[(0, c)], ref), (ks, cols[c])
