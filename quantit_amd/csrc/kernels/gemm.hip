@@ -212,27 +212,27 @@ struct GemmOperand {
     }
   }
   __device__ __forceinline__ void stash(double* __restrict__ s, int kleft, int tid) const {
-    if constexpr (KC) {
-      const int k = (tid & 7) * 2;
-      double* d = s + (tid >> 3) * PK + k;
+    constexpr int step = KC ? 32 * PK : KR * (T + 16);
+    double* d = s + (KC ? (tid >> 3) * PK + (tid & 7) * 2 : (tid / L) * (T + 16) + (tid % L) * 2);
+    if (kleft >= KS && !edge) {
 #pragma unroll
-      for (int u = 0; u < E; ++u) {
-        v2d x = v[u];
-        if (kleft < KS && k + 1 >= kleft) {
+      for (int u = 0; u < E; ++u) *reinterpret_cast<v2d*>(d + u * step) = v[u];
+      return;
+    }
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+      v2d x = v[u];
+      if constexpr (KC) {
+        const int k = (tid & 7) * 2;
+        if (k + 1 >= kleft) {
           x.x = k < kleft ? x.y : 0.0;
           x.y = 0.0;
         }
-        *reinterpret_cast<v2d*>(d + 32 * u * PK) = x;
+      } else {
+        if (swap) x.x = x.y;
+        if (tid / L + KR * u >= kleft) x = v2d{0.0, 0.0};
       }
-    } else {
-      double* d = s + (tid / L) * (T + 16) + (tid % L) * 2;
-#pragma unroll
-      for (int u = 0; u < E; ++u) {
-        v2d x = v[u];
-        if (edge && swap) x.x = x.y;
-        if (kleft < KS && tid / L + KR * u >= kleft) x = v2d{0.0, 0.0};
-        *reinterpret_cast<v2d*>(d + KR * u * (T + 16)) = x;
-      }
+      *reinterpret_cast<v2d*>(d + u * step) = x;
     }
   }
 };
@@ -307,6 +307,7 @@ __global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, co
       }
       if (more) fetch();
       __syncthreads();
+      const double *ap = sa + ao, *bp = sb + bo;
       auto multiply = [&](auto fi, auto fj) {
         constexpr int FI = decltype(fi)::value, FJ = decltype(fj)::value;
 #pragma unroll
@@ -314,9 +315,9 @@ __global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, co
           if (kk < have) {  // uniform: chunks past a pair's end are zeros
             double a[FI], b[FJ];
 #pragma unroll
-            for (int i = 0; i < FI; ++i) a[i] = sa[ao + i * 32 * OpA::kRow + kk * OpA::kK];
+            for (int i = 0; i < FI; ++i) a[i] = ap[i * 32 * OpA::kRow + kk * OpA::kK];
 #pragma unroll
-            for (int j = 0; j < FJ; ++j) b[j] = sb[bo + j * 32 * OpB::kRow + kk * OpB::kK];
+            for (int j = 0; j < FJ; ++j) b[j] = bp[j * 32 * OpB::kRow + kk * OpB::kK];
 #pragma unroll
             for (int i = 0; i < FI; ++i)
 #pragma unroll
@@ -329,9 +330,12 @@ __global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, co
       if (decltype(whole)::value || (mi == F && nj == F)) {
         multiply(all, all);
       } else if constexpr (F == 2) {
-        if (mi == 1 && nj == 2) multiply(one, all);
-        if (mi == 2 && nj == 1) multiply(all, one);
-        if (mi == 1 && nj == 1) multiply(one, one);
+        if (mi == 1 && nj == 2)
+          multiply(one, all);
+        else if (mi == 2 && nj == 1)
+          multiply(all, one);
+        else if (mi == 1 && nj == 1)
+          multiply(one, one);
       }
       return more;
     };
