@@ -310,8 +310,7 @@ BTensor clone(const BTensor& t) {
   }
   if (!tasks.empty()) {
     KernelTimer kt(*t.ctx, "copy2d");
-    auto [dd, dt] = t.ctx->upload_pack(cp, tasks);
-    kern::copy2d(t.ctx->stream(), ab, dd, dt, int(tasks.size()));
+    kern::copy2d(t.ctx->stream(), ab, t.ctx->lists(cp, tasks), int(tasks.size()));
   }
   return out;
 }
@@ -382,8 +381,7 @@ BTensor permute(const BTensor& t, const std::vector<int64_t>& in_perm) {
   }
   if (!tasks.empty()) {
     KernelTimer kt(*t.ctx, "permute_copy");
-    auto [dd, dt] = t.ctx->upload_pack(descs, tasks);
-    kern::permute_copy(t.ctx->stream(), ab, dd, dt, int(tasks.size()));
+    kern::permute_copy(t.ctx->stream(), ab, t.ctx->lists(descs, tasks), int(tasks.size()));
   }
   return out;
 }

@@ -101,8 +101,7 @@ BTensor mul(const BTensor& x_in, const BTensor& y_in) {
   }
   if (!tasks.empty()) {
     KernelTimer kt(*ctx, "ew_mul");
-    auto [up_descs, up_tasks] = ctx->upload_pack(descs, tasks);
-    kern::ew_binary(ctx->stream(), ab, up_descs, up_tasks, int(tasks.size()), 0, 0.0);
+    kern::ew_binary(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), 0, 0.0);
   }
   return out;
 }
@@ -137,8 +136,7 @@ BTensor div_scalar_tensor(const BTensor& x, const BTensor& s, double min_abs) {
   }
   if (!tasks.empty()) {
     KernelTimer kt(*ctx, "ew_div");
-    auto [up_descs, up_tasks] = ctx->upload_pack(descs, tasks);
-    kern::ew_binary(ctx->stream(), ab, up_descs, up_tasks, int(tasks.size()), 1,
+    kern::ew_binary(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), 1,
                     min_abs);
   }
   return out;
@@ -192,8 +190,7 @@ BTensor merge_axpby(const BTensor& x, int64_t a_off, double a, const BTensor& y,
   }
   if (!tasks.empty()) {
     KernelTimer kt(*ctx, "axpby");
-    auto [up_descs, up_tasks] = ctx->upload_pack(descs, tasks);
-    kern::axpby(ctx->stream(), ab, up_descs, up_tasks, int(tasks.size()), a_off, a,
+    kern::axpby(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), a_off, a,
                 b_off, b);
   }
   return out;
@@ -260,8 +257,7 @@ BTensor full_dot(const BTensor& x, const BTensor& y, bool sqrt_out) {
   out.allocate({BIdx{}});
   BufPtr partial = ctx->alloc(std::max<size_t>(tasks.size(), 1) * sizeof(double));
   KernelTimer kt(*ctx, "dot");
-  kern::dot(ctx->stream(), ab, tasks.empty() ? nullptr : ctx->upload_vec(descs),
-            tasks.empty() ? nullptr : ctx->upload_vec(tasks), int(tasks.size()), partial->dptr() - ab,
+  kern::dot(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), partial->dptr() - ab,
             out.ptr(out.blocks[0]) - ab, sqrt_out);
   return out;
 }
@@ -296,8 +292,7 @@ BTensor fill_like(Context* ctx, const Shape& s, double value) {
     std::vector<kern::ChunkTask> tasks;
     add_chunks(tasks, 0, n);
     KernelTimer kt(*ctx, "fill");
-    auto [up_cp, up_tasks] = ctx->upload_pack(cp, tasks);
-    kern::copy2d(ctx->stream(), ab, up_cp, up_tasks, int(tasks.size()));
+    kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
   }
   return out;
 }

@@ -10,6 +10,49 @@
 namespace qtt {
 namespace kern {
 
+// ---- descriptor lists of a launch --------------------------------------------
+// A launch reads its descriptors either from device memory or, when they are
+// short, from its own arguments (a kernel takes up to 4 KB).  An upload is a
+// dispatch of its own in front of every launch: upload and a small kernel 5.2
+// us back to back (4.8 of the host), with 3 KB of arguments 3.0 (2.7), without
+// descriptors 2.7 (2.3).
+constexpr size_t kArgListBytes = 3584;
+struct ArgLists {
+  alignas(16) char b[kArgListBytes];
+  template <class T>
+  __device__ __forceinline__ const T* list(uint32_t at = 0) const {
+    return reinterpret_cast<const T*>(b + at);
+  }
+};
+struct DevLists {
+  const char* p;
+  // constant while the kernel runs: uniform reads stay scalar loads
+  template <class T>
+  __device__ __forceinline__ const T* list(uint32_t at = 0) const {
+    using Const = const __attribute__((address_space(4))) char;
+    return (const T*)((Const*)p + at);
+  }
+};
+// The lists of one launch, list i at byte at[i].
+struct Lists {
+  const char* dev = nullptr;  // null: in arg
+  uint32_t at[6] = {0, 0, 0, 0, 0, 0};
+  ArgLists arg;
+  Lists() {}
+};
+// Launches the DevLists or the ArgLists instance of a kernel over its lists.
+template <class D, class A, class... X>
+void launch_lists(D dev, A arg, const Lists& l, dim3 grid, dim3 block, size_t lds, hipStream_t s, double* base,
+                  X... x) {
+  if (l.dev)
+    hipLaunchKernelGGL(dev, grid, block, lds, s, base, DevLists{l.dev}, x...);
+  else
+    hipLaunchKernelGGL(arg, grid, block, lds, s, base, l.arg, x...);
+}
+// Copy of pinned host memory into device memory by a kernel (both 16-byte
+// aligned): the runtime's own copy takes 20 us from 64 KB on, this 6.
+void stage_copy(hipStream_t s, void* dst, const void* src, size_t bytes);
+
 // ---- grouped block GEMM ---------------------------------------------------
 // C_out = alpha * sum_p A_p * B_p + beta * C_out for every output block, the
 // pairs of one output block taken in list order (the reference's mm +
@@ -36,10 +79,11 @@ constexpr int kGemmTile = 64;
 // B in n (else in k), common to all its pairs; kLayoutAny: in no common way.
 enum GemmLayout : int { kLayoutAny = -1 };
 GemmLayout gemm_layout(const GemmPair* pairs, size_t n, const GemmOut* outs, size_t nouts);
+// Lists of the GEMM launches: GemmTile, GemmOut, GemmPair, RowTask.
 // The grouped FP64 GEMM with 64 x 64 or 32 x 32 tiles (tile; a tile's tm, tn
 // count in its own units).  Launches of kLayoutAny take 64 x 64 tiles.
-void gemm_f64(hipStream_t s, int tile, GemmLayout lay, double* base, const GemmTile* tiles, int ntiles,
-              const GemmOut* outs, const GemmPair* pairs, double alpha, double beta);
+void gemm_f64(hipStream_t s, int tile, GemmLayout lay, double* base, const Lists& l, int ntiles, double alpha,
+              double beta);
 // Tile choices of the tuning table and of QTT_GEMM_VARIANT, by number: 5 is
 // the 32 x 32 tile, every other number the 64 x 64 one (0 the general kernel;
 // 2 to 4 are numbers of wider tiles in tables of older builds).
@@ -61,8 +105,7 @@ hipError_t noalloc_scratch_address(int device, void** out);
 // hi/lo split FP32 MFMA: each operand x = hi + lo (hi = fp32(x), lo =
 // fp32(x - hi)); products hi*hi + hi*lo + lo*hi accumulate in FP32 per K
 // chunk and are folded into FP64 accumulators after every chunk.
-void gemm_split(hipStream_t s, double* base, const GemmTile* tiles, int ntiles, const GemmOut* outs,
-                const GemmPair* pairs, double alpha, double beta);
+void gemm_split(hipStream_t s, double* base, const Lists& l, int ntiles, double alpha, double beta);
 // Output blocks with at most kRowsMaxN columns and a short summed K.  A task is
 // 64 or 128 (task_rows) consecutive rows of one output block: 64 while the
 // work-groups all fit on the chip at once (30 blocks of 300 rows, K 128: 8.6 us
@@ -74,8 +117,7 @@ struct RowTask {
   int32_t out, row0;
 };
 inline int rows_per_task(int64_t rows) { return rows < 64 * 2048 ? 64 : 128; }
-void gemm_rows(hipStream_t s, double* base, const RowTask* tasks, int ntasks, int task_rows, const GemmOut* outs,
-               const GemmPair* pairs, double alpha, double beta);
+void gemm_rows(hipStream_t s, double* base, const Lists& l, int ntasks, int task_rows, double alpha, double beta);
 
 // ---- data movement ----------------------------------------------------------
 // Row-major copy of a permuted view: dst element with multi-index j over
@@ -94,7 +136,8 @@ struct ChunkTask {
 // a 256-thread group, so a task is a few dependent memory round trips and a
 // launch spreads over many work-groups.
 constexpr int kChunk = 2048;
-void permute_copy(hipStream_t s, double* base, const PermDesc* descs, const ChunkTask* tasks, int ntasks);
+// The lists of these launches: descriptors, ChunkTasks.
+void permute_copy(hipStream_t s, double* base, const Lists& l, int ntasks);
 
 // 2-D strided copy dst[r*dst_rs + c*dst_cs] = alpha * src[r*src_rs + c*src_cs];
 // src_off < 0 fills the destination with the value alpha.
@@ -104,13 +147,14 @@ struct Copy2D {
   int32_t rows, cols;
   double alpha;
 };
-void copy2d(hipStream_t s, double* base, const Copy2D* descs, const ChunkTask* tasks, int ntasks);
+void copy2d(hipStream_t s, double* base, const Lists& l, int ntasks);
 struct SumParts {
   int64_t dst_off, src_off, n;
   int32_t parts, pad;
 };
 // dst = sum of `parts` consecutive arrays of n doubles at src (fixed order).
-void sum_parts(hipStream_t s, double* base, const SumParts* descs, const ChunkTask* tasks, int ntasks);
+// The two lists are those from `first` on.
+void sum_parts(hipStream_t s, double* base, const Lists& l, int ntasks, int first = 0);
 
 // ---- elementwise / reductions ---------------------------------------------
 // out = x (op) y with y broadcast: mode 0 y scalar, 1 y vector along the last
@@ -121,14 +165,14 @@ struct EwDesc {
   int64_t x_off, y_off, out_off, numel;
   int32_t ncol, mode;
 };
-void ew_binary(hipStream_t s, double* base, const EwDesc* descs, const ChunkTask* tasks, int ntasks, int op,
+void ew_binary(hipStream_t s, double* base, const Lists& l, int ntasks, int op,
                double min_abs);
 // out = a*x + b*y; x_off or y_off < 0 means that operand is absent.  a and b
 // are read from device scalars when a_off/b_off >= 0, else the host values.
 struct AxpbyDesc {
   int64_t x_off, y_off, out_off, numel;
 };
-void axpby(hipStream_t s, double* base, const AxpbyDesc* descs, const ChunkTask* tasks, int ntasks, int64_t a_off,
+void axpby(hipStream_t s, double* base, const Lists& l, int ntasks, int64_t a_off,
            double a, int64_t b_off, double b);
 // Deterministic dot product over matched block pairs: one partial per chunk
 // task, then a fixed-order tree reduction into base[out_off].  With sqrt_out
@@ -136,7 +180,7 @@ void axpby(hipStream_t s, double* base, const AxpbyDesc* descs, const ChunkTask*
 struct DotDesc {
   int64_t x_off, y_off, numel;
 };
-void dot(hipStream_t s, double* base, const DotDesc* descs, const ChunkTask* tasks, int ntasks,
+void dot(hipStream_t s, double* base, const Lists& l, int ntasks,
          int64_t partial_off, int64_t out_off, bool sqrt_out);
 // eig2x2Mat (sources/dmrg.cpp:543-572) on device scalars a0, a1, b; writes
 // E, o, n to out[0..3) and sets flags[0] = 1 on NaN.
@@ -179,7 +223,7 @@ struct SvdSector {
   int64_t shift_off;        // device double holding c (eigh mode)
 };
 constexpr int kSvdBlock = 16;  // columns per Jacobi block
-void svd_init_w(hipStream_t s, double* base, const SvdSector* secs, int nsec);
+void svd_init_w(hipStream_t s, double* base, const Lists& secs, int nsec);
 // One round of the block Jacobi tournament; max_ell = largest row count
 // among the sectors (picks the LDS-resident kernel when the block pair fits).
 // cross_after0: rounds after the first of a sweep rotate only the pairs
@@ -195,8 +239,7 @@ void svd_round(hipStream_t s, double* base, const RoundWork* work, int nwork, in
                const int* skip, double tol, int inner_sweeps, int max_ell, int cross_after0);
 // norms + ranks (one work-group per sector) and the tiled transposed scatter
 // of the (sector, part, row0, col0) tasks into U / V.
-void svd_finalize(hipStream_t s, double* base, const SvdSector* secs, const SvdSector* host_secs, int nsec,
-                  const int4* tasks, int ntasks);
+void svd_finalize(hipStream_t s, double* base, const Lists& l, const SvdSector* host_secs, int nsec, int ntasks);
 // Orthonormal completion of the Z-side columns (Z: ell x k row-major, values
 // S descending) whose singular value is numerically zero, for columns
 // t < limit only: a truncation that keeps `limit` columns never reads the
@@ -205,9 +248,9 @@ struct CompleteTask {
   int64_t z_off, s_off, v_off, p_off;
   int32_t ell, k, limit, pad;
 };
-void svd_complete(hipStream_t s, double* base, const CompleteTask* tasks, int n);
+void svd_complete(hipStream_t s, double* base, const Lists& tasks, int n);
 // eigh mode: c = ||A||_F per sector, stored at shift_off, and Y += c I.
-void svd_shift(hipStream_t s, double* base, const SvdSector* secs, int nsec);
+void svd_shift(hipStream_t s, double* base, const Lists& secs, int nsec);
 void fill_i32(hipStream_t s, int32_t* p, int n, int32_t v);
 
 // One k x k matrix of the one-work-group kernels.
@@ -223,17 +266,17 @@ size_t gram_eig_lds_limit();  // largest dynamic LDS per work-group (bytes)
 // failing the orthogonality test (0: W = I).  precond: pivoted-Cholesky
 // preconditioning.
 constexpr int kGramEigMaxK = 140;
-void gram_eig(hipStream_t s, double* base, const void* descs, int n, int* flags, double tol, int max_sweeps,
+void gram_eig(hipStream_t s, double* base, const Lists& descs, int n, int* flags, double tol, int max_sweeps,
               int precond, size_t lds_bytes);
 size_t gram_eig_lds_bytes(int k);
 // First-order Gram-Schmidt factor T (k x k at w_off) from the Gram matrix at
 // y_off (SmallJacobi with ell = k).
-void gs_step(hipStream_t s, double* base, const void* descs, int n, int kmax);
+void gs_step(hipStream_t s, double* base, const Lists& descs, int n, int kmax);
 
 // ---- Gram eigenvectors for wide sectors (G in device memory) ---------------
 // Orthogonality test of G (SmallJacobi: y_off = G, k, ldy; flag_idx/aux_idx
 // as for gram_eig).
-void gram_check(hipStream_t s, const double* base, const void* descs, int n, int* flags, double tol, int kmax);
+void gram_check(hipStream_t s, double* base, const Lists& descs, int n, int* flags, double tol, int kmax);
 // Work item of one round of the two-sided block Jacobi on G (gram_rounds.hip):
 // the solve of block pair a, tile (a, b) of G (a <= b), or rows
 // [64 b, 64 b + 64) of X's column pair a.
@@ -268,14 +311,14 @@ struct GramVec {
   int64_t x_off, w_off, scratch_off;  // scratch: 3k doubles
   int32_t k, ldx, ldw, pad;
 };
-void gram_vectors(hipStream_t s, double* base, const void* descs, int n, int kmax);
+void gram_vectors(hipStream_t s, double* base, const Lists& descs, int n, int kmax);
 
 // Global truncation (sources/btensor_linalg.cpp:657-755,
 // sources/LinearAlgebra.cpp:57-75): singular values of nsec sectors stored
 // descending at s_off[i] with k[i] entries, s_pos[i] = k[0] + ... + k[i-1];
 // writes kept[i].
-void truncate_select(hipStream_t s, double* base, const int64_t* s_offs, const int32_t* ks, const int64_t* s_pos,
-                     int nsec, int64_t scratch_off, int64_t total, double tol, double pow, int64_t min_size,
+// lists: s_off, s_pos, k
+void truncate_select(hipStream_t s, double* base, const Lists& l, int nsec, int64_t scratch_off, int64_t total, double tol, double pow, int64_t min_size,
                      int64_t max_size, int32_t* kept, double* thr_out);
 
 }  // namespace kern

@@ -1,15 +1,17 @@
 // Data movement, elementwise and reduction kernels (HBM-bound).  Work is
 // split into (descriptor, chunk) tasks of kChunk elements so a launch always
 // has many work-groups regardless of how uneven the blocks are.
+#include <algorithm>
+
 #include "../kernels.hpp"
 
 namespace qtt {
 namespace kern {
 
-__global__ __launch_bounds__(256) void k_permute(double* __restrict__ base, const PermDesc* __restrict__ descs,
-                                                 const ChunkTask* __restrict__ tasks) {
-  const ChunkTask t = tasks[blockIdx.x];
-  const PermDesc d = descs[t.desc];
+template <class L>
+__global__ __launch_bounds__(256) void k_permute(double* __restrict__ base, L l, uint32_t tasks) {
+  const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
+  const PermDesc d = l.template list<PermDesc>()[t.desc];
   const int64_t start = int64_t(t.chunk) * kChunk;
   const int64_t end = min(start + int64_t(kChunk), d.numel);
   const double* src = base + d.src_off;
@@ -26,15 +28,15 @@ __global__ __launch_bounds__(256) void k_permute(double* __restrict__ base, cons
   }
 }
 
-void permute_copy(hipStream_t s, double* base, const PermDesc* descs, const ChunkTask* tasks, int ntasks) {
+void permute_copy(hipStream_t s, double* base, const Lists& l, int ntasks) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(k_permute, dim3(ntasks), dim3(256), 0, s, base, descs, tasks);
+  launch_lists(k_permute<DevLists>, k_permute<ArgLists>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[1]);
 }
 
-__global__ __launch_bounds__(256) void k_copy2d(double* __restrict__ base, const Copy2D* __restrict__ descs,
-                                                const ChunkTask* __restrict__ tasks) {
-  const ChunkTask t = tasks[blockIdx.x];
-  const Copy2D d = descs[t.desc];
+template <class L>
+__global__ __launch_bounds__(256) void k_copy2d(double* __restrict__ base, L l, uint32_t tasks) {
+  const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
+  const Copy2D d = l.template list<Copy2D>()[t.desc];
   const int64_t numel = int64_t(d.rows) * d.cols;
   const int64_t start = int64_t(t.chunk) * kChunk;
   const int64_t end = min(start + int64_t(kChunk), numel);
@@ -55,10 +57,11 @@ __global__ __launch_bounds__(256) void k_copy2d(double* __restrict__ base, const
 
 // dst[i] = sum over s < parts of src[s * n + i] (fixed order): the reduction of
 // split-K partial products.  desc = {dst_off, src_off, n, parts}.
-__global__ __launch_bounds__(256) void k_sum_parts(double* __restrict__ base, const SumParts* __restrict__ descs,
-                                                   const ChunkTask* __restrict__ tasks) {
-  const ChunkTask t = tasks[blockIdx.x];
-  const SumParts d = descs[t.desc];
+template <class L>
+__global__ __launch_bounds__(256) void k_sum_parts(double* __restrict__ base, L l, uint32_t descs,
+                                                   uint32_t tasks) {
+  const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
+  const SumParts d = l.template list<SumParts>(descs)[t.desc];
   const int64_t i0 = int64_t(t.chunk) * kChunk;
   const int64_t i1 = i0 + kChunk < d.n ? i0 + kChunk : d.n;
   for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
@@ -68,20 +71,21 @@ __global__ __launch_bounds__(256) void k_sum_parts(double* __restrict__ base, co
   }
 }
 
-void sum_parts(hipStream_t s, double* base, const SumParts* descs, const ChunkTask* tasks, int ntasks) {
+void sum_parts(hipStream_t s, double* base, const Lists& l, int ntasks, int first) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(k_sum_parts, dim3(ntasks), dim3(256), 0, s, base, descs, tasks);
+  launch_lists(k_sum_parts<DevLists>, k_sum_parts<ArgLists>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[first],
+               l.at[first + 1]);
 }
 
-void copy2d(hipStream_t s, double* base, const Copy2D* descs, const ChunkTask* tasks, int ntasks) {
+void copy2d(hipStream_t s, double* base, const Lists& l, int ntasks) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(k_copy2d, dim3(ntasks), dim3(256), 0, s, base, descs, tasks);
+  launch_lists(k_copy2d<DevLists>, k_copy2d<ArgLists>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[1]);
 }
 
-__global__ __launch_bounds__(256) void k_ew_binary(double* __restrict__ base, const EwDesc* __restrict__ descs,
-                                                   const ChunkTask* __restrict__ tasks, int op, double min_abs) {
-  const ChunkTask t = tasks[blockIdx.x];
-  const EwDesc d = descs[t.desc];
+template <class L>
+__global__ __launch_bounds__(256) void k_ew_binary(double* __restrict__ base, L l, uint32_t tasks, int op, double min_abs) {
+  const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
+  const EwDesc d = l.template list<EwDesc>()[t.desc];
   const int64_t start = int64_t(t.chunk) * kChunk;
   const int64_t end = min(start + int64_t(kChunk), d.numel);
   const double* x = base + d.x_off;
@@ -102,17 +106,17 @@ __global__ __launch_bounds__(256) void k_ew_binary(double* __restrict__ base, co
   }
 }
 
-void ew_binary(hipStream_t s, double* base, const EwDesc* descs, const ChunkTask* tasks, int ntasks, int op,
+void ew_binary(hipStream_t s, double* base, const Lists& l, int ntasks, int op,
                double min_abs) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(k_ew_binary, dim3(ntasks), dim3(256), 0, s, base, descs, tasks, op, min_abs);
+  launch_lists(k_ew_binary<DevLists>, k_ew_binary<ArgLists>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[1], op, min_abs);
 }
 
-__global__ __launch_bounds__(256) void k_axpby(double* __restrict__ base, const AxpbyDesc* __restrict__ descs,
-                                               const ChunkTask* __restrict__ tasks, int64_t a_off, double a,
+template <class L>
+__global__ __launch_bounds__(256) void k_axpby(double* __restrict__ base, L l, uint32_t tasks, int64_t a_off, double a,
                                                int64_t b_off, double b) {
-  const ChunkTask t = tasks[blockIdx.x];
-  const AxpbyDesc d = descs[t.desc];
+  const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
+  const AxpbyDesc d = l.template list<AxpbyDesc>()[t.desc];
   const int64_t start = int64_t(t.chunk) * kChunk;
   const int64_t end = min(start + int64_t(kChunk), d.numel);
   const double av = a_off >= 0 ? base[a_off] : a;
@@ -135,10 +139,10 @@ __global__ __launch_bounds__(256) void k_axpby(double* __restrict__ base, const 
   }
 }
 
-void axpby(hipStream_t s, double* base, const AxpbyDesc* descs, const ChunkTask* tasks, int ntasks, int64_t a_off,
+void axpby(hipStream_t s, double* base, const Lists& l, int ntasks, int64_t a_off,
            double a, int64_t b_off, double b) {
   if (ntasks <= 0) return;
-  hipLaunchKernelGGL(k_axpby, dim3(ntasks), dim3(256), 0, s, base, descs, tasks, a_off, a, b_off, b);
+  launch_lists(k_axpby<DevLists>, k_axpby<ArgLists>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[1], a_off, a, b_off, b);
 }
 
 // Block-wide sum in fixed order (deterministic).
@@ -155,11 +159,11 @@ __device__ double block_sum(double v, double* sh) {
   return r;
 }
 
-__global__ __launch_bounds__(256) void k_dot_partial(double* __restrict__ base, const DotDesc* __restrict__ descs,
-                                                     const ChunkTask* __restrict__ tasks, int64_t partial_off) {
+template <class L>
+__global__ __launch_bounds__(256) void k_dot_partial(double* __restrict__ base, L l, uint32_t tasks, int64_t partial_off) {
   __shared__ double sh[256];
-  const ChunkTask t = tasks[blockIdx.x];
-  const DotDesc d = descs[t.desc];
+  const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
+  const DotDesc d = l.template list<DotDesc>()[t.desc];
   const int64_t start = int64_t(t.chunk) * kChunk;
   const int64_t end = min(start + int64_t(kChunk), d.numel);
   const double* x = base + d.x_off;
@@ -179,10 +183,10 @@ __global__ __launch_bounds__(256) void k_dot_final(double* __restrict__ base, in
   if (threadIdx.x == 0) base[out_off] = sqrt_out ? sqrt(r) : r;
 }
 
-void dot(hipStream_t s, double* base, const DotDesc* descs, const ChunkTask* tasks, int ntasks, int64_t partial_off,
+void dot(hipStream_t s, double* base, const Lists& l, int ntasks, int64_t partial_off,
          int64_t out_off, bool sqrt_out) {
   if (ntasks > 0)
-    hipLaunchKernelGGL(k_dot_partial, dim3(ntasks), dim3(256), 0, s, base, descs, tasks, partial_off);
+    launch_lists(k_dot_partial<DevLists>, k_dot_partial<ArgLists>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[1], partial_off);
   hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(256), 0, s, base, partial_off, ntasks, out_off, int(sqrt_out));
 }
 
@@ -224,6 +228,21 @@ __global__ __launch_bounds__(256) void k_normalize(double* __restrict__ base, in
 void normalize(hipStream_t s, double* base, int64_t off, int64_t n) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_normalize, dim3(1), dim3(256), 0, s, base, off, n);
+}
+
+// The last thread of the grid copies what is left of a whole 16 bytes.
+__global__ __launch_bounds__(256) void k_stage_copy(uint4* __restrict__ dst, const uint4* __restrict__ src, size_t n,
+                                                    int tail) {
+  const size_t step = size_t(gridDim.x) * blockDim.x, i0 = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (size_t i = i0; i < n; i += step) dst[i] = src[i];
+  if (i0 == step - 1)
+    for (int b = 0; b < tail; ++b) reinterpret_cast<char*>(dst + n)[b] = reinterpret_cast<const char*>(src + n)[b];
+}
+
+void stage_copy(hipStream_t s, void* dst, const void* src, size_t bytes) {
+  const size_t n = bytes / 16, g = (n + 255) / 256;
+  hipLaunchKernelGGL(k_stage_copy, dim3(unsigned(std::min<size_t>(std::max<size_t>(g, 1), 1024))), dim3(256), 0, s,
+                     static_cast<uint4*>(dst), static_cast<const uint4*>(src), n, int(bytes % 16));
 }
 
 }  // namespace kern

@@ -238,10 +238,12 @@ struct GemmOperand {
 };
 
 // AK: A contiguous in k (else in m); BN: B contiguous in n (else in k).
-template <int T, bool AK, bool BN>
-__global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, const GemmTile* __restrict__ tiles,
-                                                   const GemmOut* __restrict__ outs,
-                                                   const GemmPair* __restrict__ pairs, double alpha, double beta) {
+template <class L, int T, bool AK, bool BN>
+__global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, L l, uint32_t at_tiles,
+                                                   uint32_t at_outs, uint32_t at_pairs, double alpha, double beta) {
+  const GemmTile* tiles = l.template list<GemmTile>(at_tiles);
+  const GemmOut* outs = l.template list<GemmOut>(at_outs);
+  const GemmPair* pairs = l.template list<GemmPair>(at_pairs);
   using OpA = GemmOperand<T, AK>;
   using OpB = GemmOperand<T, !BN>;
   constexpr int F = T / 32;  // 16 x 16 MFMA tiles per wave and dimension
@@ -449,10 +451,12 @@ __device__ __forceinline__ void stash_t(const GemmPair& pr, int tid, const TileR
   }
 }
 
-template <int TM, int TN, int KD>
-__global__ __launch_bounds__(256) void k_gemm_f64t(double* __restrict__ base, const GemmTile* __restrict__ tiles,
-                                                   const GemmOut* __restrict__ outs,
-                                                   const GemmPair* __restrict__ pairs, double alpha, double beta) {
+template <class L, int TM, int TN, int KD>
+__global__ __launch_bounds__(256) void k_gemm_f64t(double* __restrict__ base, L l, uint32_t at_tiles,
+                                                   uint32_t at_outs, uint32_t at_pairs, double alpha, double beta) {
+  const GemmTile* tiles = l.template list<GemmTile>(at_tiles);
+  const GemmOut* outs = l.template list<GemmOut>(at_outs);
+  const GemmPair* pairs = l.template list<GemmPair>(at_pairs);
   constexpr int WM = TM / 2, WN = TN / 2, FI = WM / 16, FJ = WN / 16;
   __shared__ double As[2][KD][TM + 16];
   __shared__ double Bs[2][KD][TN + 16];
@@ -558,10 +562,12 @@ __global__ __launch_bounds__(256) void k_gemm_f64t(double* __restrict__ base, co
       }
 }
 
-__global__ __launch_bounds__(256) void k_gemm_split(double* __restrict__ base, const GemmTile* __restrict__ tiles,
-                                                    const GemmOut* __restrict__ outs,
-                                                    const GemmPair* __restrict__ pairs, double alpha,
-                                                    double beta) {
+template <class L>
+__global__ __launch_bounds__(256) void k_gemm_split(double* __restrict__ base, L l, uint32_t at_tiles,
+                                                   uint32_t at_outs, uint32_t at_pairs, double alpha, double beta) {
+  const GemmTile* tiles = l.template list<GemmTile>(at_tiles);
+  const GemmOut* outs = l.template list<GemmOut>(at_outs);
+  const GemmPair* pairs = l.template list<GemmPair>(at_pairs);
   __shared__ float Ah[BK][LDP], Al[BK][LDP];
   __shared__ float Bh[BK][LDP], Bl[BK][LDP];
   const GemmTile t = tiles[blockIdx.x];
@@ -632,10 +638,12 @@ __global__ __launch_bounds__(256) void k_gemm_split(double* __restrict__ base, c
 struct RowK {
   int64_t a_off, a_rs, b_off, b_cs;
 };
-template <int RT>
-__global__ __launch_bounds__(256) void k_gemm_rows(double* __restrict__ base, const RowTask* __restrict__ tasks,
-                                                   const GemmOut* __restrict__ outs,
-                                                   const GemmPair* __restrict__ pairs, double alpha, double beta) {
+template <class L, int RT>
+__global__ __launch_bounds__(256) void k_gemm_rows(double* __restrict__ base, L l, uint32_t at_tasks,
+                                                   uint32_t at_outs, uint32_t at_pairs, double alpha, double beta) {
+  const RowTask* tasks = l.template list<RowTask>(at_tasks);
+  const GemmOut* outs = l.template list<GemmOut>(at_outs);
+  const GemmPair* pairs = l.template list<GemmPair>(at_pairs);
   __shared__ RowK ks[kRowsMaxK];
   const RowTask t = tasks[blockIdx.x];
   const GemmOut o = outs[t.out];
@@ -713,13 +721,14 @@ __global__ __launch_bounds__(256) void k_gemm_rows(double* __restrict__ base, co
   }
 }
 
-void gemm_rows(hipStream_t s, double* base, const RowTask* tasks, int ntasks, int task_rows, const GemmOut* outs,
-               const GemmPair* pairs, double alpha, double beta) {
+void gemm_rows(hipStream_t s, double* base, const Lists& l, int ntasks, int task_rows, double alpha, double beta) {
   if (ntasks <= 0) return;
   if (task_rows == 128)
-    hipLaunchKernelGGL(k_gemm_rows<2>, dim3(ntasks), dim3(256), 0, s, base, tasks, outs, pairs, alpha, beta);
+    launch_lists(k_gemm_rows<DevLists, 2>, k_gemm_rows<ArgLists, 2>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[3],
+                 l.at[1], l.at[2], alpha, beta);
   else
-    hipLaunchKernelGGL(k_gemm_rows<1>, dim3(ntasks), dim3(256), 0, s, base, tasks, outs, pairs, alpha, beta);
+    launch_lists(k_gemm_rows<DevLists, 1>, k_gemm_rows<ArgLists, 1>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[3],
+                 l.at[1], l.at[2], alpha, beta);
 }
 
 GemmLayout gemm_layout(const GemmPair* pairs, size_t n, const GemmOut* outs, size_t nouts) {
@@ -740,33 +749,39 @@ GemmLayout gemm_layout(const GemmPair* pairs, size_t n, const GemmOut* outs, siz
   return GemmLayout((ak ? 1 : 0) | (bn ? 2 : 0));
 }
 
+template <int T, bool AK, bool BN>
+static void gemm_contiguous(hipStream_t s, double* base, const Lists& l, int ntiles, double alpha, double beta) {
+  launch_lists(k_gemm_f64c<DevLists, T, AK, BN>, k_gemm_f64c<ArgLists, T, AK, BN>, l, dim3(ntiles), dim3(256), 0, s,
+               base, l.at[0], l.at[1], l.at[2], alpha, beta);
+}
+
 template <int T>
-static void gemm_contiguous(hipStream_t s, GemmLayout lay, double* base, const GemmTile* tiles, int ntiles,
-                            const GemmOut* outs, const GemmPair* pairs, double alpha, double beta) {
-  const dim3 g(ntiles), b(256);
+static void gemm_contiguous(hipStream_t s, GemmLayout lay, double* base, const Lists& l, int ntiles, double alpha,
+                            double beta) {
   switch (int(lay)) {
-    case 0: hipLaunchKernelGGL((k_gemm_f64c<T, false, false>), g, b, 0, s, base, tiles, outs, pairs, alpha, beta); break;
-    case 1: hipLaunchKernelGGL((k_gemm_f64c<T, true, false>), g, b, 0, s, base, tiles, outs, pairs, alpha, beta); break;
-    case 2: hipLaunchKernelGGL((k_gemm_f64c<T, false, true>), g, b, 0, s, base, tiles, outs, pairs, alpha, beta); break;
-    default: hipLaunchKernelGGL((k_gemm_f64c<T, true, true>), g, b, 0, s, base, tiles, outs, pairs, alpha, beta); break;
+    case 0: gemm_contiguous<T, false, false>(s, base, l, ntiles, alpha, beta); break;
+    case 1: gemm_contiguous<T, true, false>(s, base, l, ntiles, alpha, beta); break;
+    case 2: gemm_contiguous<T, false, true>(s, base, l, ntiles, alpha, beta); break;
+    default: gemm_contiguous<T, true, true>(s, base, l, ntiles, alpha, beta); break;
   }
 }
 
-void gemm_f64(hipStream_t s, int tile, GemmLayout lay, double* base, const GemmTile* tiles, int ntiles,
-              const GemmOut* outs, const GemmPair* pairs, double alpha, double beta) {
+void gemm_f64(hipStream_t s, int tile, GemmLayout lay, double* base, const Lists& l, int ntiles, double alpha,
+              double beta) {
   if (ntiles <= 0) return;
   if (lay == kLayoutAny)
-    hipLaunchKernelGGL((k_gemm_f64t<64, 64, 16>), dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha, beta);
+    launch_lists(k_gemm_f64t<DevLists, 64, 64, 16>, k_gemm_f64t<ArgLists, 64, 64, 16>, l, dim3(ntiles), dim3(256), 0,
+                 s, base, l.at[0], l.at[1], l.at[2], alpha, beta);
   else if (tile == 32)
-    gemm_contiguous<32>(s, lay, base, tiles, ntiles, outs, pairs, alpha, beta);
+    gemm_contiguous<32>(s, lay, base, l, ntiles, alpha, beta);
   else
-    gemm_contiguous<64>(s, lay, base, tiles, ntiles, outs, pairs, alpha, beta);
+    gemm_contiguous<64>(s, lay, base, l, ntiles, alpha, beta);
 }
 
-void gemm_split(hipStream_t s, double* base, const GemmTile* tiles, int ntiles, const GemmOut* outs,
-                const GemmPair* pairs, double alpha, double beta) {
+void gemm_split(hipStream_t s, double* base, const Lists& l, int ntiles, double alpha, double beta) {
   if (ntiles <= 0) return;
-  hipLaunchKernelGGL(k_gemm_split, dim3(ntiles), dim3(256), 0, s, base, tiles, outs, pairs, alpha, beta);
+  launch_lists(k_gemm_split<DevLists>, k_gemm_split<ArgLists>, l, dim3(ntiles), dim3(256), 0, s, base, l.at[0],
+               l.at[1], l.at[2], alpha, beta);
 }
 
 // Scratch of the allocation-free contraction (packed operands, split-K

@@ -36,8 +36,9 @@ constexpr int GP = NB2 + 1;         // LDS pitch of G and Q
 
 // W = I (kp x kp) for every sector; gridDim.y work-groups share a sector,
 // one column per wave-step.
-__global__ void k_svd_init_w(double* __restrict__ base, const SvdSector* __restrict__ secs) {
-  const SvdSector s = secs[blockIdx.x];
+template <class L>
+__global__ void k_svd_init_w(double* __restrict__ base, L l) {
+  const SvdSector s = l.template list<SvdSector>()[blockIdx.x];
   const int kp = s.nb * kSvdBlock;
   double* W = base + s.w_off;
   const int wave = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -46,9 +47,9 @@ __global__ void k_svd_init_w(double* __restrict__ base, const SvdSector* __restr
     for (int r = lane; r < kp; r += 64) W[int64_t(c) * kp + r] = (r == c) ? 1.0 : 0.0;
 }
 
-void svd_init_w(hipStream_t st, double* base, const SvdSector* secs, int nsec) {
+void svd_init_w(hipStream_t st, double* base, const Lists& secs, int nsec) {
   if (nsec <= 0) return;
-  hipLaunchKernelGGL(k_svd_init_w, dim3(nsec, 16), dim3(256), 0, st, base, secs);
+  launch_lists(k_svd_init_w<DevLists>, k_svd_init_w<ArgLists>, secs, dim3(nsec, 16), dim3(256), 0, st, base);
 }
 
 __device__ __forceinline__ int circle_block(int pos, int round, int nb) {
@@ -961,14 +962,15 @@ __device__ __forceinline__ int chol_wave(double* X, int* pivoted, int k) {
   return rk;
 }
 
+template <class L>
 __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict__ base,
-                                                            const SmallJacobi* __restrict__ js,
+                                                            L l,
                                                             int* __restrict__ flags, double tol, int max_sweeps,
                                                             int precond) {
   extern __shared__ double lds[];
   __shared__ int nrot[2];
   __shared__ int nviol, nabs, best;
-  const SmallJacobi J = js[blockIdx.x];
+  const SmallJacobi J = l.template list<SmallJacobi>()[blockIdx.x];
   const int k = J.k;
   const int ke = k + (k & 1);
   const int tid = threadIdx.x;
@@ -1279,8 +1281,9 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
 // longer than column j (ties: lower index), so Z T removes from every column
 // its components along the longer ones.  T is written k x k at w_off
 // (leading dimension ldw).  One work-group per matrix.
-__global__ __launch_bounds__(256) void k_gs_step(double* __restrict__ base, const SmallJacobi* __restrict__ js) {
-  const SmallJacobi J = js[blockIdx.x];
+template <class L>
+__global__ __launch_bounds__(256) void k_gs_step(double* __restrict__ base, L l) {
+  const SmallJacobi J = l.template list<SmallJacobi>()[blockIdx.x];
   const int k = J.k;
   const int j0 = blockIdx.y * 8;  // eight columns of T per work-group
   if (j0 >= k) return;
@@ -1303,17 +1306,16 @@ __global__ __launch_bounds__(256) void k_gs_step(double* __restrict__ base, cons
   }
 }
 
-void gs_step(hipStream_t st, double* base, const void* descs, int n, int kmax) {
+void gs_step(hipStream_t st, double* base, const Lists& descs, int n, int kmax) {
   if (n <= 0 || kmax <= 0) return;
-  hipLaunchKernelGGL(k_gs_step, dim3(n, (kmax + 7) / 8), dim3(256), 0, st, base,
-                     static_cast<const SmallJacobi*>(descs));
+  launch_lists(k_gs_step<DevLists>, k_gs_step<ArgLists>, descs, dim3(n, (kmax + 7) / 8), dim3(256), 0, st, base);
 }
 
-void gram_eig(hipStream_t st, double* base, const void* descs, int n, int* flags, double tol, int max_sweeps,
+void gram_eig(hipStream_t st, double* base, const Lists& descs, int n, int* flags, double tol, int max_sweeps,
               int precond, size_t lds_bytes) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_gram_eig, dim3(n), dim3(kGramEigThreads), lds_bytes, st, base,
-                     static_cast<const SmallJacobi*>(descs), flags, tol, max_sweeps, precond);
+  launch_lists(k_gram_eig<DevLists>, k_gram_eig<ArgLists>, descs, dim3(n), dim3(kGramEigThreads), lds_bytes, st, base, flags,
+               tol, max_sweeps, precond);
 }
 
 // X, nrm, vec, hh and perm, and 16 doubles beyond them: the wave-local loads
@@ -1329,8 +1331,9 @@ size_t gram_eig_lds_limit() {
     int v = 0;
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) v = 65536;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gram_eig),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, v - 64);
+    for (const void* f : {reinterpret_cast<const void*>(&k_gram_eig<DevLists>),
+                          reinterpret_cast<const void*>(&k_gram_eig<ArgLists>)})
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, v - 64);
     return size_t(v);
   }();
   return limit;
@@ -1344,8 +1347,9 @@ size_t gram_eig_lds_limit() {
 // in descending order (ties broken by column index) and the sorted values.
 // Column norms of Y: grid (sector, chunk of 16 columns); each wave sums
 // four columns at once (four independent loads per row step).
-__global__ __launch_bounds__(256) void k_svd_colnorms(double* __restrict__ base, const SvdSector* __restrict__ secs) {
-  const SvdSector s = secs[blockIdx.x];
+template <class L>
+__global__ __launch_bounds__(256) void k_svd_colnorms(double* __restrict__ base, L l) {
+  const SvdSector s = l.template list<SvdSector>()[blockIdx.x];
   const int k = s.k, ell = s.ell, kp = s.nb * kSvdBlock;
   const int c0 = blockIdx.y * 16 + (threadIdx.x >> 6) * 4;
   if (c0 >= k) return;
@@ -1381,11 +1385,12 @@ __global__ __launch_bounds__(256) void k_svd_colnorms(double* __restrict__ base,
 // that ranks values 64 y ... 64 y + 63 against all k, compared from LDS 1024
 // at a time.
 constexpr int kNormsWave = 64;
+template <class L>
 __global__ __launch_bounds__(kNormsWave) void k_svd_norms(double* __restrict__ base,
-                                                           const SvdSector* __restrict__ secs) {
+                                                           L l) {
   constexpr int kChunk = 1024;
   __shared__ double chunk[kChunk];
-  const SvdSector s = secs[blockIdx.x];
+  const SvdSector s = l.template list<SvdSector>()[blockIdx.x];
   const int k = s.k, kp = s.nb * kSvdBlock;
   const int j0 = blockIdx.y * kNormsWave;
   if (j0 >= k) return;  // uniform
@@ -1421,13 +1426,13 @@ __global__ __launch_bounds__(kNormsWave) void k_svd_norms(double* __restrict__ b
 // columns, transposed through LDS so both the reads and the writes are
 // coalesced.  task = (sector, part, row0, col0); part 0: Y -> Z side
 // (columns divided by their norm, zero when numerically null), part 1: W.
-__global__ __launch_bounds__(256) void k_svd_write(double* __restrict__ base, const SvdSector* __restrict__ secs,
-                                                   const int4* __restrict__ tasks) {
+template <class L>
+__global__ __launch_bounds__(256) void k_svd_write(double* __restrict__ base, L l, uint32_t tasks) {
   __shared__ double tile[64][65];
   __shared__ int perm[64];
   __shared__ double scl[64];
-  const int4 t = tasks[blockIdx.x];
-  const SvdSector s = secs[t.x];
+  const int4 t = l.template list<int4>(tasks)[blockIdx.x];
+  const SvdSector s = l.template list<SvdSector>()[t.x];
   const int k = s.k, kp = s.nb * kSvdBlock;
   const double* aux = base + s.w_off + int64_t(kp) * kp;
   const double* sig = aux;
@@ -1482,11 +1487,12 @@ __global__ __launch_bounds__(256) void k_svd_write(double* __restrict__ base, co
 // candidates always does (1/2 was out of reach when few columns are missing:
 // every candidate was tried and the columns stayed zero).  One work-group
 // per sector.
+template <class L>
 __global__ __launch_bounds__(256) void k_svd_complete(double* __restrict__ base,
-                                                      const CompleteTask* __restrict__ ts) {
+                                                      L l) {
   __shared__ double sh[256];
   __shared__ int first_sh;
-  const CompleteTask T = ts[blockIdx.x];
+  const CompleteTask T = l.template list<CompleteTask>()[blockIdx.x];
   const int k = T.k, ell = T.ell, lim = T.limit < k ? T.limit : k;
   if (lim <= 0) return;
   const double* S = base + T.s_off;
@@ -1534,24 +1540,26 @@ __global__ __launch_bounds__(256) void k_svd_complete(double* __restrict__ base,
   }
 }
 
-void svd_complete(hipStream_t st, double* base, const CompleteTask* tasks, int n) {
+void svd_complete(hipStream_t st, double* base, const Lists& tasks, int n) {
   if (n <= 0) return;
-  hipLaunchKernelGGL(k_svd_complete, dim3(n), dim3(256), 0, st, base, tasks);
+  launch_lists(k_svd_complete<DevLists>, k_svd_complete<ArgLists>, tasks, dim3(n), dim3(256), 0, st, base);
 }
 
-void svd_finalize(hipStream_t st, double* base, const SvdSector* secs, const SvdSector* host_secs, int nsec,
-                  const int4* tasks, int ntasks) {
+void svd_finalize(hipStream_t st, double* base, const Lists& l, const SvdSector* host_secs, int nsec, int ntasks) {
   if (nsec <= 0) return;
   int kmax = 1;
   for (int i = 0; i < nsec; ++i) kmax = std::max(kmax, host_secs[i].k);
-  hipLaunchKernelGGL(k_svd_colnorms, dim3(nsec, (kmax + 15) / 16), dim3(256), 0, st, base, secs);
-  hipLaunchKernelGGL(k_svd_norms, dim3(nsec, (kmax + kNormsWave - 1) / kNormsWave), dim3(kNormsWave), 0, st, base, secs);
-  if (ntasks > 0) hipLaunchKernelGGL(k_svd_write, dim3(ntasks), dim3(256), 0, st, base, secs, tasks);
+  launch_lists(k_svd_colnorms<DevLists>, k_svd_colnorms<ArgLists>, l, dim3(nsec, (kmax + 15) / 16), dim3(256), 0, st, base);
+  launch_lists(k_svd_norms<DevLists>, k_svd_norms<ArgLists>, l, dim3(nsec, (kmax + kNormsWave - 1) / kNormsWave),
+               dim3(kNormsWave), 0, st, base);
+  if (ntasks > 0)
+    launch_lists(k_svd_write<DevLists>, k_svd_write<ArgLists>, l, dim3(ntasks), dim3(256), 0, st, base, l.at[1]);
 }
 
-__global__ __launch_bounds__(256) void k_svd_shift(double* __restrict__ base, const SvdSector* __restrict__ secs) {
+template <class L>
+__global__ __launch_bounds__(256) void k_svd_shift(double* __restrict__ base, L l) {
   __shared__ double sh[256];
-  const SvdSector s = secs[blockIdx.x];
+  const SvdSector s = l.template list<SvdSector>()[blockIdx.x];
   double* Y = base + s.y_off;
   const int64_t n = int64_t(s.ell) * s.k;
   double acc = 0.0;
@@ -1561,9 +1569,9 @@ __global__ __launch_bounds__(256) void k_svd_shift(double* __restrict__ base, co
   if (threadIdx.x == 0) base[s.shift_off] = c;
 }
 
-void svd_shift(hipStream_t st, double* base, const SvdSector* secs, int nsec) {
+void svd_shift(hipStream_t st, double* base, const Lists& secs, int nsec) {
   if (nsec <= 0) return;
-  hipLaunchKernelGGL(k_svd_shift, dim3(nsec), dim3(256), 0, st, base, secs);
+  launch_lists(k_svd_shift<DevLists>, k_svd_shift<ArgLists>, secs, dim3(nsec), dim3(256), 0, st, base);
 }
 
 __global__ void k_fill_i32(int32_t* p, int n, int32_t v) {
@@ -1580,15 +1588,17 @@ void fill_i32(hipStream_t st, int32_t* p, int n, int32_t v) {
 // The values of all sectors are gathered, sorted descending (bitonic, in LDS
 // when 2^ceil(log2 total) doubles fit, else in the scratch area) and the cut
 // is found by the reference's sequential tail accumulation.
-template <bool IN_LDS>
-__global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, const int64_t* __restrict__ s_offs,
-                                                   const int32_t* __restrict__ ks, const int64_t* __restrict__ s_pos,
+template <class L, bool IN_LDS>
+__global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, L l, uint32_t at_pos, uint32_t at_ks,
                                                    int nsec, int64_t scratch_off,
                                                    int64_t total, double tol, double pw, int64_t min_size,
                                                    int64_t max_size, int32_t* __restrict__ kept,
                                                    double* __restrict__ thr_out) {
   extern __shared__ double vl[];
   __shared__ double thr_sh;
+  const int64_t* s_offs = l.template list<int64_t>();
+  const int64_t* s_pos = l.template list<int64_t>(at_pos);
+  const int32_t* ks = l.template list<int32_t>(at_ks);
   double* v = IN_LDS ? vl : base + scratch_off;
   int64_t n2 = 1;
   while (n2 < total) n2 <<= 1;
@@ -1673,8 +1683,7 @@ __global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, co
   }
 }
 
-void truncate_select(hipStream_t st, double* base, const int64_t* s_offs, const int32_t* ks, const int64_t* s_pos,
-                     int nsec, int64_t scratch_off, int64_t total, double tol, double pw, int64_t min_size,
+void truncate_select(hipStream_t st, double* base, const Lists& l, int nsec, int64_t scratch_off, int64_t total, double tol, double pw, int64_t min_size,
                      int64_t max_size, int32_t* kept, double* thr_out) {
   int64_t n2 = 1;
   while (n2 < total) n2 <<= 1;
@@ -1684,16 +1693,17 @@ void truncate_select(hipStream_t st, double* base, const int64_t* s_offs, const 
     int dev = 0, v = 0;
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) v = 65536;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_truncate<true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, v - 256);
+    for (const void* f : {reinterpret_cast<const void*>(&k_truncate<DevLists, true>),
+                          reinterpret_cast<const void*>(&k_truncate<ArgLists, true>)})
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, v - 256);
     return size_t(v) - 256;
   }();
   if (lds <= limit)
-    hipLaunchKernelGGL(k_truncate<true>, dim3(1), dim3(1024), lds, st, base, s_offs, ks, s_pos, nsec, scratch_off,
-                       total, tol, pw, min_size, max_size, kept, thr_out);
+    launch_lists(k_truncate<DevLists, true>, k_truncate<ArgLists, true>, l, dim3(1), dim3(1024), lds, st, base, l.at[1],
+                 l.at[2], nsec, scratch_off, total, tol, pw, min_size, max_size, kept, thr_out);
   else
-    hipLaunchKernelGGL(k_truncate<false>, dim3(1), dim3(1024), 0, st, base, s_offs, ks, s_pos, nsec, scratch_off,
-                       total, tol, pw, min_size, max_size, kept, thr_out);
+    launch_lists(k_truncate<DevLists, false>, k_truncate<ArgLists, false>, l, dim3(1), dim3(1024), 0, st, base, l.at[1],
+                 l.at[2], nsec, scratch_off, total, tol, pw, min_size, max_size, kept, thr_out);
 }
 
 }  // namespace kern

@@ -63,9 +63,10 @@ __device__ __forceinline__ double fast_rsqrt_pc(double x) {
 
 constexpr int kLargeThreads = 1024;
 
-__global__ void k_gram_check_zero(const SmallJacobi* __restrict__ js, int n, int* __restrict__ flags) {
+template <class L>
+__global__ void k_gram_check_zero(double*, L l, int n, int* __restrict__ flags) {
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    const SmallJacobi J = js[i];
+    const SmallJacobi J = l.template list<SmallJacobi>()[i];
     if (J.flag_idx >= 0) flags[J.flag_idx] = 0;
     if (J.aux_idx >= 0) flags[J.aux_idx] = 0;
   }
@@ -76,13 +77,13 @@ __global__ void k_gram_check_zero(const SmallJacobi* __restrict__ js, int n, int
 // beforehand.  Work-group y of a sector takes the columns c = y (mod
 // gridDim.y); the diagonal sits in LDS (dynamic, k doubles); wave w scans the
 // upper part of its w-th, (w + 16)-th, ... column with coalesced reads.
-__global__ __launch_bounds__(kLargeThreads) void k_gram_check(const double* __restrict__ base,
-                                                              const SmallJacobi* __restrict__ js,
-                                                              int* __restrict__ flags, double tol) {
+template <class L>
+__global__ __launch_bounds__(kLargeThreads) void k_gram_check(double* __restrict__ base, L l, int* __restrict__ flags,
+                                                              double tol) {
   extern __shared__ double dg[];
   __shared__ double sh[kLargeThreads];
   __shared__ int nv, na;
-  const SmallJacobi J = js[blockIdx.x];
+  const SmallJacobi J = l.template list<SmallJacobi>()[blockIdx.x];
   const int k = J.k;
   const double* G = base + J.y_off;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwave = blockDim.x >> 6;
@@ -120,23 +121,23 @@ __global__ __launch_bounds__(kLargeThreads) void k_gram_check(const double* __re
   }
 }
 
-void gram_check(hipStream_t st, const double* base, const void* descs, int n, int* flags, double tol, int kmax) {
+void gram_check(hipStream_t st, double* base, const Lists& descs, int n, int* flags, double tol, int kmax) {
   if (n <= 0) return;
   static const size_t limit = [] {
     int dev = 0, v = 0;
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) v = 65536;
     const size_t l = size_t(v) - kLargeThreads * sizeof(double) - 64;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gram_check),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, int(l));
+    for (const void* f : {reinterpret_cast<const void*>(&k_gram_check<DevLists>),
+                          reinterpret_cast<const void*>(&k_gram_check<ArgLists>)})
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, int(l));
     return l;
   }();
   const size_t lds = size_t(kmax) * sizeof(double);
   if (lds > limit) throw std::runtime_error("gram check: sector wider than the LDS holds");
   const int ny = std::max(1, std::min(8, kmax / 64));  // about 64 columns per work-group
-  hipLaunchKernelGGL(k_gram_check_zero, dim3(1), dim3(256), 0, st, static_cast<const SmallJacobi*>(descs), n, flags);
-  hipLaunchKernelGGL(k_gram_check, dim3(n, ny), dim3(kLargeThreads), lds, st, base,
-                     static_cast<const SmallJacobi*>(descs), flags, tol);
+  launch_lists(k_gram_check_zero<DevLists>, k_gram_check_zero<ArgLists>, descs, dim3(1), dim3(256), 0, st, base, n, flags);
+  launch_lists(k_gram_check<DevLists>, k_gram_check<ArgLists>, descs, dim3(n, ny), dim3(kLargeThreads), lds, st, base, flags, tol);
 }
 
 // One panel [j0, j0 + nb) of the pivoted Cholesky of G (already updated by
@@ -334,9 +335,10 @@ size_t pchol_lds_limit() {
 // projection passes), one work-group per sector, and returns at once when
 // there are none.  W is written at w_off with leading dimension ldw;
 // scratch_off: 3k doubles (norms, two work vectors).
+template <class L>
 __global__ __launch_bounds__(kLargeThreads) void k_gram_vec_norm(double* __restrict__ base,
-                                                                 const GramVec* __restrict__ js) {
-  const GramVec J = js[blockIdx.x];
+                                                                 L l) {
+  const GramVec J = l.template list<GramVec>()[blockIdx.x];
   const int k = J.k;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c0 = blockIdx.y * 64 + wave * 4;
@@ -376,11 +378,12 @@ __global__ __launch_bounds__(kLargeThreads) void k_gram_vec_norm(double* __restr
   }
 }
 
+template <class L>
 __global__ __launch_bounds__(kLargeThreads) void k_gram_vectors(double* __restrict__ base,
-                                                                const GramVec* __restrict__ js) {
+                                                                L l) {
   __shared__ double sh[kLargeThreads];
   __shared__ int best, nzero;
-  const GramVec J = js[blockIdx.x];
+  const GramVec J = l.template list<GramVec>()[blockIdx.x];
   const int k = J.k;
   const int tid = threadIdx.x;
   double* W = base + J.w_off;
@@ -437,12 +440,11 @@ __global__ __launch_bounds__(kLargeThreads) void k_gram_vectors(double* __restri
   }
 }
 
-void gram_vectors(hipStream_t st, double* base, const void* descs, int n, int kmax) {
+void gram_vectors(hipStream_t st, double* base, const Lists& descs, int n, int kmax) {
   if (n <= 0 || kmax <= 0) return;
-  hipLaunchKernelGGL(k_gram_vec_norm, dim3(n, (kmax + 63) / 64), dim3(kLargeThreads), 0, st, base,
-                     static_cast<const GramVec*>(descs));
-  hipLaunchKernelGGL(k_gram_vectors, dim3(n), dim3(kLargeThreads), 0, st, base,
-                     static_cast<const GramVec*>(descs));
+  launch_lists(k_gram_vec_norm<DevLists>, k_gram_vec_norm<ArgLists>, descs, dim3(n, (kmax + 63) / 64), dim3(kLargeThreads),
+               0, st, base);
+  launch_lists(k_gram_vectors<DevLists>, k_gram_vectors<ArgLists>, descs, dim3(n), dim3(kLargeThreads), 0, st, base);
 }
 
 }  // namespace kern

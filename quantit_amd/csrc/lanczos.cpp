@@ -69,8 +69,7 @@ void launch_copies(Context* ctx, double* ab, const std::vector<kern::Copy2D>& cp
                    const std::vector<kern::ChunkTask>& tasks, const char* name) {
   if (tasks.empty()) return;
   KernelTimer kt(*ctx, name);
-  auto [dc, dt] = ctx->upload_pack(cp, tasks);
-  kern::copy2d(ctx->stream(), ab, dc, dt, int(tasks.size()));
+  kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
 }
 
 kern::Copy2D flat_copy(int64_t src, int64_t dst, int64_t ne) {

@@ -88,19 +88,17 @@ struct Batched {
   std::vector<kern::CompleteTask> complete;
 };
 
-// A grouped GEMM whose descriptors are on the device (one staging copy), so
-// it can be launched several times.
+// A grouped GEMM ready to launch; one that is launched several times keeps
+// its descriptors on the device.
 struct GemmLaunch {
-  const kern::GemmTile* tiles = nullptr;
-  const kern::GemmOut* outs = nullptr;
-  const kern::GemmPair* pairs = nullptr;
+  kern::Lists lists;
   int ntiles = 0;
   int tile = kern::kGemmTile;
   kern::GemmLayout lay = kern::kLayoutAny;
 };
 
 GemmLaunch prepare_gemm(Context* ctx, const std::vector<kern::GemmOut>& outs,
-                        const std::vector<kern::GemmPair>& pairs) {
+                        const std::vector<kern::GemmPair>& pairs, bool repeated) {
   GemmLaunch g;
   g.lay = kern::gemm_layout(pairs.data(), pairs.size(), outs.data(), outs.size());
   auto count = [&](int t) {
@@ -117,7 +115,7 @@ GemmLaunch prepare_gemm(Context* ctx, const std::vector<kern::GemmOut>& outs,
       for (int j = 0; j < tn; ++j) tiles.push_back({int32_t(o), int16_t(i), int16_t(j)});
   }
   if (tiles.empty()) return g;
-  std::tie(g.tiles, g.outs, g.pairs) = ctx->upload_pack(tiles, outs, pairs);
+  g.lists = repeated ? ctx->device_lists(tiles, outs, pairs) : ctx->lists(tiles, outs, pairs);
   g.ntiles = int(tiles.size());
   return g;
 }
@@ -126,13 +124,13 @@ void run_gemm(Context* ctx, double* ab, const GemmLaunch& g, const char* name, d
               double beta = 0.0) {
   if (g.ntiles == 0) return;
   KernelTimer kt(*ctx, name);
-  kern::gemm_f64(ctx->stream(), g.tile, g.lay, ab, g.tiles, g.ntiles, g.outs, g.pairs, alpha, beta);
+  kern::gemm_f64(ctx->stream(), g.tile, g.lay, ab, g.lists, g.ntiles, alpha, beta);
 }
 
 void launch_gemm(Context* ctx, double* ab, const std::vector<kern::GemmOut>& outs,
                  const std::vector<kern::GemmPair>& pairs, const char* name, double alpha = 1.0,
                  double beta = 0.0) {
-  run_gemm(ctx, ab, prepare_gemm(ctx, outs, pairs), name, alpha, beta);
+  run_gemm(ctx, ab, prepare_gemm(ctx, outs, pairs, false), name, alpha, beta);
 }
 
 int env_int(const char* name, int dflt) {
@@ -252,7 +250,7 @@ int jacobi_sweeps(Context* ctx, double* ab, const std::vector<kern::SvdSector>& 
     }
     launch_gemm(ctx, ab, outs, prs, "svd_sweep_check_gram");
     KernelTimer kt(*ctx, "svd_sweep_check");
-    kern::gram_check(ctx->stream(), ab, ctx->upload_vec(cd), int(cd.size()), d_chk, tol, kc);
+    kern::gram_check(ctx->stream(), ab, ctx->lists(cd), int(cd.size()), d_chk, tol, kc);
     return true;
   };
   const bool use_check = env_int("QTT_SVD_SWEEP_CHECK", 1) != 0;
@@ -356,7 +354,7 @@ int gram_sweeps(Context* ctx, double* ab, const std::vector<GramProblem>& ps, do
     prs.push_back(g);
   }
   const kern::GramRound* d_work = ctx->upload_vec(work);
-  const GemmLaunch gram = prepare_gemm(ctx, outs, prs);
+  const GemmLaunch gram = prepare_gemm(ctx, outs, prs, true);
   constexpr int kAhead = 6;  // launches enqueued before the host waits for the counts
   for (int sweep = 0;; ++sweep) {
     const int slot = sweep & 1;
@@ -465,8 +463,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
   }
   if (!tasks.empty()) {
     KernelTimer kt(*ctx, "svd_zero");
-    auto [dc, dt] = ctx->upload_pack(cp, tasks);
-    kern::copy2d(ctx->stream(), ab, dc, dt, int(tasks.size()));
+    kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
   }
   cp.clear();
   tasks.clear();
@@ -500,12 +497,11 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
   }
   if (!tasks.empty()) {
     KernelTimer kt(*ctx, "svd_gather");
-    auto [dc, dt] = ctx->upload_pack(cp, tasks);
-    kern::copy2d(ctx->stream(), ab, dc, dt, int(tasks.size()));
+    kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
   }
   if (ns == 0) return B;
   {
-    auto* d_secs = ctx->upload_vec(B.secs);
+    const kern::Lists d_secs = ctx->lists(B.secs);
     KernelTimer kt(*ctx, "svd_init");
     kern::svd_init_w(ctx->stream(), ab, d_secs, ns);
     if (eigh_mode) kern::svd_shift(ctx->stream(), ab, d_secs, ns);
@@ -611,9 +607,8 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         wi.push_back(w);
       }
       KernelTimer kt(*ctx, "svd_init");
-      auto [dz, dzt] = ctx->upload_pack(z, zt);
-      kern::copy2d(ctx->stream(), ab, dz, dzt, int(zt.size()));
-      kern::svd_init_w(ctx->stream(), ab, ctx->upload_vec(wi), nw);
+      kern::copy2d(ctx->stream(), ab, ctx->lists(z, zt), int(zt.size()));
+      kern::svd_init_w(ctx->stream(), ab, ctx->lists(wi), nw);
     }
     std::vector<int64_t> alt_y(nw), alt_w(nw);
     for (int q = 0; q < nw; ++q) {
@@ -671,8 +666,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       launch_gemm(ctx, ab, outs, prs, "svd_gram");
       if (!st.empty()) {
         KernelTimer kt(*ctx, "svd_gram_sum");
-        auto [ds, dst] = ctx->upload_pack(sums, st);
-        kern::sum_parts(ctx->stream(), ab, ds, dst, int(st.size()));
+        kern::sum_parts(ctx->stream(), ab, ctx->lists(sums, st), int(st.size()));
       }
     };
     auto read_flags = [&] { ctx->read_small(h_flags.data(), d_flags, size_t(2 * nw) * sizeof(int32_t)); };
@@ -739,8 +733,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
           z.push_back(c);
         }
         KernelTimer kt(*ctx, "svd_init");
-        auto [dz, dzt] = ctx->upload_pack(z, zt);
-        kern::copy2d(ctx->stream(), ab, dz, dzt, int(zt.size()));
+        kern::copy2d(ctx->stream(), ab, ctx->lists(z, zt), int(zt.size()));
       }
       int kact = 0;
       for (int q : qs) kact = std::max(kact, B.secs[wide[q]].k);
@@ -765,7 +758,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       }
       const auto* d_pd = ctx->upload_vec(pd);
       kern::pchol_init(ctx->stream(), ab, d_pd, int(pd.size()));
-      const GemmLaunch upd = prepare_gemm(ctx, outs, prs);
+      const GemmLaunch upd = prepare_gemm(ctx, outs, prs, true);
       for (int j0 = 0; j0 < kact; j0 += pnb) {
         {
           KernelTimer kt(*ctx, "svd_pchol");
@@ -789,7 +782,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       int kv = 0;
       for (auto& v : vd) kv = std::max(kv, v.k);
       KernelTimer kt(*ctx, "svd_vectors");
-      kern::gram_vectors(ctx->stream(), ab, ctx->upload_vec(vd), int(vd.size()), kv);
+      kern::gram_vectors(ctx->stream(), ab, ctx->lists(vd), int(vd.size()), kv);
     };
     // eigh: A + c I is positive (semi-)definite, so it takes the Gram matrix's
     // place once: its eigenvectors are A's, and the column norms of (A + c I) W
@@ -812,8 +805,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
           cg.push_back(c);
         }
         KernelTimer kt(*ctx, "svd_init");
-        auto [dc, dt] = ctx->upload_pack(cg, ct);
-        kern::copy2d(ctx->stream(), ab, dc, dt, int(ct.size()));
+        kern::copy2d(ctx->stream(), ab, ctx->lists(cg, ct), int(ct.size()));
       } else {
         gram_of(act);
       }
@@ -836,7 +828,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         std::stable_sort(jd.begin(), jd.end(),
                          [](const kern::SmallJacobi& a, const kern::SmallJacobi& b) { return a.k > b.k; });
         static const char* const kEigNames[] = {"svd_eig", "svd_eig_it1", "svd_eig_it2", "svd_eig_it3+"};
-        const auto* d_jd = ctx->upload_vec(jd);
+        const kern::Lists d_jd = ctx->lists(jd);
         if (overlap) ctx->fork();
         KernelTimer kt(*ctx, kEigNames[std::min(it, 3)]);
         kern::gram_eig(overlap ? ctx->side_stream() : ctx->stream(), ab, d_jd, int(jd.size()), d_flags, tol,
@@ -858,7 +850,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         }
         {
           KernelTimer kt(*ctx, "svd_check");
-          kern::gram_check(ctx->stream(), ab, ctx->upload_vec(cd), int(cd.size()), d_flags, tol, kc);
+          kern::gram_check(ctx->stream(), ab, ctx->lists(cd), int(cd.size()), d_flags, tol, kc);
         }
         read_flags();  // the small sectors' flags may not be written yet when overlapped
         retire(act_l);
@@ -892,7 +884,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       }
       {
         KernelTimer kt(*ctx, "svd_gs");
-        kern::gs_step(ctx->stream(), ab, ctx->upload_vec(gd), int(gd.size()), kg);
+        kern::gs_step(ctx->stream(), ab, ctx->lists(gd), int(gd.size()), kg);
       }
       std::vector<kern::GemmOut> outs;
       std::vector<kern::GemmPair> prs;
@@ -932,8 +924,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
   }
   {
     KernelTimer kt(*ctx, "svd_finalize");
-    kern::svd_finalize(ctx->stream(), ab, ctx->upload_vec(B.secs), B.secs.data(), ns, ctx->upload_vec(wt),
-                       int(wt.size()));
+    kern::svd_finalize(ctx->stream(), ab, ctx->lists(B.secs, wt), B.secs.data(), ns, int(wt.size()));
   }
   if (!eigh_mode) {
     for (const auto& s : B.secs) {
@@ -951,7 +942,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
     }
     if (!defer_complete) {
       KernelTimer kt(*ctx, "svd_complete");
-      kern::svd_complete(ctx->stream(), ab, ctx->upload_vec(B.complete), int(B.complete.size()));
+      kern::svd_complete(ctx->stream(), ab, ctx->lists(B.complete), int(B.complete.size()));
       B.complete.clear();
     }
   }
@@ -1177,9 +1168,7 @@ BTensor truncate_units(BTensor&& d_in, const std::vector<BTensor*>& units, size_
   const int64_t clamp = std::numeric_limits<int64_t>::max();
   {
     KernelTimer kt(*ctx, "truncate_select");
-    auto [up_s_offs, up_ks, up_pos] = ctx->upload_pack(s_offs, ks, s_pos);
-    kern::truncate_select(ctx->stream(), ab, up_s_offs, up_ks, up_pos, nd,
-                          scratch->dptr() - ab, total, tol, pw, int64_t(std::min<size_t>(min_size, size_t(clamp))),
+    kern::truncate_select(ctx->stream(), ab, ctx->lists(s_offs, s_pos, ks), nd, scratch->dptr() - ab, total, tol, pw, int64_t(std::min<size_t>(min_size, size_t(clamp))),
                           int64_t(std::min<size_t>(max_size, size_t(clamp))), d_kept, d_thr);
   }
   std::vector<int32_t> kept(nd);
@@ -1249,8 +1238,7 @@ BTensor truncate_units(BTensor&& d_in, const std::vector<BTensor*>& units, size_
     }
     if (!tasks.empty()) {
       KernelTimer kt(*ctx, "truncate_copy");
-      auto [dc, dt] = ctx->upload_pack(cp, tasks);
-      kern::copy2d(ctx->stream(), ab, dc, dt, int(tasks.size()));
+      kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
     }
     return out;
   };
@@ -1325,8 +1313,7 @@ SvdResult svd_matrix(const BTensor& t, bool some, bool compute_uv) {
     }
     if (!zt.empty()) {
       KernelTimer kt(*ctx, "svd_zero_uv");
-      auto [dz, dzt] = ctx->upload_pack(z, zt);
-      kern::copy2d(ctx->stream(), ab, dz, dzt, int(zt.size()));
+      kern::copy2d(ctx->stream(), ab, ctx->lists(z, zt), int(zt.size()));
     }
   }
   return r;
@@ -1361,7 +1348,7 @@ SvdResult svd_truncated(const BTensor& t, size_t split, double tol, size_t min_s
       c.p_off += so;
     }
     KernelTimer kt(*ctx, "svd_complete");
-    kern::svd_complete(ctx->stream(), arena_base(ctx), ctx->upload_vec(run), int(run.size()));
+    kern::svd_complete(ctx->stream(), arena_base(ctx), ctx->lists(run), int(run.size()));
   };
   out.d = truncate_units(std::move(out.d), {&out.U, &out.V}, max_size, min_size, tol, pw, complete_kept);
   return out;

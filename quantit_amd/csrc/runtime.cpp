@@ -109,8 +109,8 @@ Context::~Context() {
   if (stream_) (void)hipStreamDestroy(stream_);
 }
 
-// Reserves `bytes` of the staging ring at *pos and fills its host half.
-char* Context::stage_host(const void* data, size_t bytes, size_t* pos) {
+// Reserves `bytes` of the staging ring at *pos; returns its host half.
+char* Context::stage_host(size_t bytes, size_t* pos) {
   size_t need = round_up(bytes ? bytes : 1);
   if (need > stage_cap_) throw OutOfMemory("descriptor upload larger than the staging ring");
   if (stage_pos_ + need > stage_cap_) {
@@ -121,24 +121,39 @@ char* Context::stage_host(const void* data, size_t bytes, size_t* pos) {
     stage_pos_ = 0;
   }
   *pos = stage_pos_;
-  char* h = host_stage_ + stage_pos_;
-  if (bytes) std::memcpy(h, data, bytes);
   stage_pos_ += need;
-  return h;
+  return host_stage_ + *pos;
+}
+
+// Above this the copy is a kernel (stage_copy); below, the two are alike.
+static constexpr size_t kStageKernelBytes = size_t(16) << 10;
+
+// The device half of the ring at pos, after the host half's copy to it.
+char* Context::stage_send(size_t pos, size_t bytes) {
+  char* d = dev_stage_->cptr() + pos;
+  if (bytes > kStageKernelBytes)
+    kern::stage_copy(stream_, d, host_stage_ + pos, bytes);
+  else if (bytes)
+    QTT_HIP(hipMemcpyAsync(d, host_stage_ + pos, bytes, hipMemcpyHostToDevice, stream_));
+  return d;
 }
 
 void* Context::upload(const void* data, size_t bytes) {
   size_t pos = 0;
-  char* h = stage_host(data, bytes, &pos);
-  char* d = dev_stage_->cptr() + pos;
-  if (bytes) QTT_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream_));
-  return d;
+  char* h = stage_host(bytes, &pos);
+  if (bytes) std::memcpy(h, data, bytes);
+  return stage_send(pos, bytes);
 }
 
 void Context::stage_to(void* dev_dst, const void* data, size_t bytes) {
+  if (!bytes) return;
   size_t pos = 0;
-  char* h = stage_host(data, bytes, &pos);
-  if (bytes) QTT_HIP(hipMemcpyAsync(dev_dst, h, bytes, hipMemcpyHostToDevice, stream_));
+  char* h = stage_host(bytes, &pos);
+  std::memcpy(h, data, bytes);
+  if (bytes > kStageKernelBytes && reinterpret_cast<uintptr_t>(dev_dst) % 16 == 0)
+    kern::stage_copy(stream_, dev_dst, h, bytes);
+  else
+    QTT_HIP(hipMemcpyAsync(dev_dst, h, bytes, hipMemcpyHostToDevice, stream_));
 }
 
 void Context::fork() {

@@ -11,6 +11,7 @@
 #include <tuple>
 #include <vector>
 
+#include "kernels.hpp"
 #include "qtt_common.hpp"
 
 namespace qtt {
@@ -92,24 +93,16 @@ class Context {
   T* upload_vec(const std::vector<T>& v) {
     return static_cast<T*>(upload(v.data(), v.size() * sizeof(T)));
   }
-  // Several descriptor lists in one staging copy (one host-to-device
-  // transfer instead of one per list); each list starts 16-byte aligned.
+  // The descriptor lists of one launch, each 16-byte aligned: in the launch's
+  // arguments where they fit, else in one staging copy.  device_lists: always
+  // a staging copy, for lists that several launches read.
   template <class... T>
-  std::tuple<T*...> upload_pack(const std::vector<T>&... v) {
-    constexpr size_t kA = 16;
-    const size_t sizes[] = {v.size() * sizeof(T)...};
-    size_t offs[sizeof...(T)], total = 0;
-    for (size_t i = 0; i < sizeof...(T); ++i) {
-      offs[i] = total;
-      total += (sizes[i] + kA - 1) / kA * kA;
-    }
-    std::vector<char> buf(total ? total : 1);
-    const void* src[] = {static_cast<const void*>(v.data())...};
-    for (size_t i = 0; i < sizeof...(T); ++i)
-      if (sizes[i]) std::memcpy(buf.data() + offs[i], src[i], sizes[i]);
-    char* d = static_cast<char*>(upload(buf.data(), total));
-    size_t i = 0;
-    return std::tuple<T*...>{reinterpret_cast<T*>(d + offs[i++])...};
+  kern::Lists lists(const std::vector<T>&... v) {
+    return make_lists(true, v...);
+  }
+  template <class... T>
+  kern::Lists device_lists(const std::vector<T>&... v) {
+    return make_lists(false, v...);
   }
   // Copies host bytes through the pinned staging ring to any device address
   // (stream-ordered; no allocation).
@@ -200,7 +193,26 @@ class Context {
   hipEvent_t read_ev_[2] = {nullptr, nullptr};
   hipEvent_t sync_ev_ = nullptr;
   void* noalloc_scratch_ = nullptr;
-  char* stage_host(const void* data, size_t bytes, size_t* pos);
+  char* stage_host(size_t bytes, size_t* pos);
+  char* stage_send(size_t pos, size_t bytes);
+  template <class... T>
+  kern::Lists make_lists(bool in_args, const std::vector<T>&... v) {
+    kern::Lists l;
+    const size_t sizes[] = {v.size() * sizeof(T)...};
+    const void* src[] = {static_cast<const void*>(v.data())...};
+    size_t total = 0, pos = 0;
+    for (size_t i = 0; i < sizeof...(T); ++i) {
+      l.at[i] = uint32_t(total);
+      total += (sizes[i] + 15) / 16 * 16;
+    }
+    if (total > UINT32_MAX) throw OutOfMemory("descriptor lists larger than 4 GiB");
+    const bool arg = in_args && total <= kern::kArgListBytes;
+    char* h = arg ? l.arg.b : stage_host(total, &pos);
+    for (size_t i = 0; i < sizeof...(T); ++i)
+      if (sizes[i]) std::memcpy(h + l.at[i], src[i], sizes[i]);
+    if (!arg) l.dev = stage_send(pos, total);
+    return l;
+  }
 };
 
 // RAII helper: brackets one launch with events when profiling is enabled.

@@ -146,6 +146,8 @@ class TdWork {
   // device copy of host bytes, ordered on the context stream before the
   // work enqueued afterwards
   virtual void* put(const void* src, size_t bytes) = 0;
+  // the context, when the launch follows at once and is not repeated
+  virtual Context* launches_once() const { return nullptr; }
   virtual bool timed() const = 0;
 };
 
@@ -158,6 +160,7 @@ class ArenaWork : public TdWork {
     return keep_.back()->dptr() - reinterpret_cast<double*>(ctx_->arena().base());
   }
   void* put(const void* src, size_t bytes) override { return ctx_->upload(src, bytes); }
+  Context* launches_once() const override { return ctx_; }
   bool timed() const override { return true; }
 
  private:
@@ -194,23 +197,24 @@ class StaticWork : public TdWork {
   size_t pos_ = 0;
 };
 
-// Several descriptor lists in one copy; each list starts 16-byte aligned.
+// The descriptor lists of a launch: in its arguments where the call launches
+// once, else in one copy to where the work keeps them.
 template <class... T>
-std::tuple<T*...> put_pack(TdWork& w, const std::vector<T>&... v) {
-  constexpr size_t kA = 16;
+kern::Lists put_lists(TdWork& w, const std::vector<T>&... v) {
+  if (Context* c = w.launches_once()) return c->lists(v...);
+  kern::Lists l;
   const size_t sizes[] = {v.size() * sizeof(T)...};
-  size_t offs[sizeof...(T)], total = 0;
+  size_t total = 0;
   for (size_t i = 0; i < sizeof...(T); ++i) {
-    offs[i] = total;
-    total += (sizes[i] + kA - 1) / kA * kA;
+    l.at[i] = uint32_t(total);
+    total += (sizes[i] + 15) / 16 * 16;
   }
   std::vector<char> buf(total ? total : 1);
   const void* src[] = {static_cast<const void*>(v.data())...};
   for (size_t i = 0; i < sizeof...(T); ++i)
-    if (sizes[i]) std::memcpy(buf.data() + offs[i], src[i], sizes[i]);
-  char* d = static_cast<char*>(w.put(buf.data(), total));
-  size_t i = 0;
-  return std::tuple<T*...>{reinterpret_cast<T*>(d + offs[i++])...};
+    if (sizes[i]) std::memcpy(buf.data() + l.at[i], src[i], sizes[i]);
+  l.dev = static_cast<char*>(w.put(buf.data(), total));
+  return l;
 }
 
 BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int64_t>& da_in,
@@ -241,19 +245,13 @@ class PersistWork : public TdWork {
 }  // namespace
 
 // Kernel arguments of one contraction: permute-packs, narrow-row tasks, MFMA
-// tiles, split-K sums (device descriptor pointers).
+// tiles, split-K sums.
 struct TdPlan::Launch {
-  const kern::PermDesc* pdesc = nullptr;
-  const kern::ChunkTask* ptasks = nullptr;
+  kern::Lists pack;  // PermDesc, ChunkTask
   int nptasks = 0;
-  const kern::RowTask* rows = nullptr;
+  kern::Lists lists;  // GemmTile, GemmOut, GemmPair, RowTask, SumParts, ChunkTask
   int nrows = 0, task_rows = 64;
-  const kern::GemmTile* tiles = nullptr;
   int ntiles = 0;
-  const kern::GemmOut* outs = nullptr;
-  const kern::GemmPair* pairs = nullptr;
-  const kern::SumParts* sums = nullptr;
-  const kern::ChunkTask* sum_tasks = nullptr;
   int nsum_tasks = 0;
   bool split_fp32 = false;
   int tile = kern::kGemmTile;  // FP64 tile edge
@@ -267,7 +265,7 @@ void td_pack(Context* ctx, const TdPlan::Launch& l, bool timed) {
   if (!l.nptasks) return;
   std::unique_ptr<KernelTimer> kt;
   if (timed) kt = std::make_unique<KernelTimer>(*ctx, "pack_permute");
-  kern::permute_copy(ctx->stream(), reinterpret_cast<double*>(ctx->arena().base()), l.pdesc, l.ptasks, l.nptasks);
+  kern::permute_copy(ctx->stream(), reinterpret_cast<double*>(ctx->arena().base()), l.pack, l.nptasks);
 }
 
 void td_run(Context* ctx, const TdPlan::Launch& l, bool timed) {
@@ -278,18 +276,18 @@ void td_run(Context* ctx, const TdPlan::Launch& l, bool timed) {
   td_pack(ctx, l, timed);
   if (l.nrows) {
     auto kt = timer("gemm_rows");
-    kern::gemm_rows(ctx->stream(), ab, l.rows, l.nrows, l.task_rows, l.outs, l.pairs, 1.0, 0.0);
+    kern::gemm_rows(ctx->stream(), ab, l.lists, l.nrows, l.task_rows, 1.0, 0.0);
   }
   if (l.split_fp32) {
     auto kt = timer(l.gemm_name);
-    kern::gemm_split(ctx->stream(), ab, l.tiles, l.ntiles, l.outs, l.pairs, 1.0, 0.0);
+    kern::gemm_split(ctx->stream(), ab, l.lists, l.ntiles, 1.0, 0.0);
   } else {
     auto kt = timer(l.gemm_name);
-    kern::gemm_f64(ctx->stream(), l.tile, l.lay, ab, l.tiles, l.ntiles, l.outs, l.pairs, 1.0, 0.0);
+    kern::gemm_f64(ctx->stream(), l.tile, l.lay, ab, l.lists, l.ntiles, 1.0, 0.0);
   }
   if (l.nsum_tasks) {
     auto kt = timer("gemm_split_k_sum");
-    kern::sum_parts(ctx->stream(), ab, l.sums, l.sum_tasks, l.nsum_tasks);
+    kern::sum_parts(ctx->stream(), ab, l.lists, l.nsum_tasks, 4);
   }
 }
 
@@ -607,7 +605,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     for (auto& v : vb)
       if (v.need_pack) v.off += soff;
     HostTimer ht(*ctx, work.timed() ? "host_td_upload" : nullptr);
-    std::tie(lch.pdesc, lch.ptasks) = put_pack(work, pdesc, ptasks);
+    lch.pack = put_lists(work, pdesc, ptasks);
     lch.nptasks = int(ptasks.size());
   }
 
@@ -822,19 +820,18 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     td_pack(ctx, lch, true);
     if (one.empty()) return out;
     const kern::GemmLayout lay = kern::gemm_layout(gpairs.data(), gpairs.size(), one.data(), one.size());
-    auto [d_one, d_tl, d_pairs] = ctx->upload_pack(one, tl, gpairs);
-    for (size_t l = 0; l < launches.size(); ++l) {
-      const bool first = l == 0 || one[l].c_off != one[l - 1].c_off;
+    kern::Lists l = ctx->device_lists(tl, one, gpairs);
+    for (size_t q = 0; q < launches.size(); ++q) {
+      const bool first = q == 0 || one[q].c_off != one[q - 1].c_off;
       KernelTimer kt(*ctx, "gemm_per_block");
-      kern::gemm_f64(ctx->stream(), kern::kGemmTile, lay, ab, d_tl + launches[l].first, launches[l].second, d_one,
-                     d_pairs, 1.0, first ? 0.0 : 1.0);
+      l.at[0] = uint32_t(launches[q].first * sizeof(kern::GemmTile));
+      kern::gemm_f64(ctx->stream(), kern::kGemmTile, lay, ab, l, launches[q].second, 1.0, first ? 0.0 : 1.0);
     }
     return out;
   }
   ht_plan.stop();
   HostTimer ht_up(*ctx, work.timed() ? "host_td_upload" : nullptr);
-  std::tie(lch.tiles, lch.outs, lch.pairs, lch.rows, lch.sums, lch.sum_tasks) =
-      put_pack(work, tiles, launch_outs, gpairs, row_tasks, sums, sum_tasks);
+  lch.lists = put_lists(work, tiles, launch_outs, gpairs, row_tasks, sums, sum_tasks);
   ht_up.stop();
   lch.ntiles = int(tiles.size());
   lch.nrows = int(row_tasks.size());
@@ -854,11 +851,11 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     for (int v : {kern::kTile64, kern::kTile32}) {
       const int T = kern::variant_tile(v);
       std::vector<kern::GemmTile> tl = tiles_of(T);
-      const kern::GemmTile* dt = ctx->upload_vec(tl);
+      const kern::Lists l = put_lists(work, tl, launch_outs, gpairs, row_tasks, sums, sum_tasks);
       float ms = 0.f;
       for (int rep = 0; rep < 2; ++rep) {
         QTT_HIP(hipEventRecord(e0, ctx->stream()));
-        kern::gemm_f64(ctx->stream(), T, lch.lay, ab, dt, int(tl.size()), lch.outs, lch.pairs, 1.0, 0.0);
+        kern::gemm_f64(ctx->stream(), T, lch.lay, ab, l, int(tl.size()), 1.0, 0.0);
         QTT_HIP(hipEventRecord(e1, ctx->stream()));
         QTT_HIP(hipEventSynchronize(e1));
         QTT_HIP(hipEventElapsedTime(&ms, e0, e1));
@@ -867,7 +864,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
         best_ms = ms;
         best = v;
         lch.tile = T;
-        lch.tiles = dt;
+        lch.lists = l;
         lch.ntiles = int(tl.size());
       }
     }
