@@ -56,19 +56,19 @@ __device__ __forceinline__ int circle_block(int pos, int round, int nb) {
   return pos == 0 ? 0 : 1 + ((pos - 1 + round) % (nb - 1));
 }
 
-// Reciprocal square root and reciprocal by the hardware estimates refined by
-// two Newton steps (each doubles the correct bits), well inside the rounding
-// of the rotations they feed; the division and square root the compiler
-// expands to correctly rounded sequences cost several times more latency.
+// Reciprocal square root and reciprocal: the hardware estimates (relative error
+// up to 2^-24 measured) and one third-order step, 2^-72 before rounding and a
+// shorter chain than two Newton steps; the division and square root the
+// compiler expands to correctly rounded sequences take several times longer.
 __device__ __forceinline__ double fast_rsqrt(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = y * (1.5 - 0.5 * x * y * y);
-  return y * (1.5 - 0.5 * x * y * y);
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 __device__ __forceinline__ double fast_rcp(double x) {
-  double z = __builtin_amdgcn_rcp(x);
-  z = z * (2.0 - x * z);
-  return z * (2.0 - x * z);
+  const double z = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, z, 1.0);
+  return fma(z, fma(e, e, e), z);
 }
 
 // Jacobi rotation (c, s) annihilating the off-diagonal h/2 of the symmetric
@@ -670,28 +670,18 @@ __device__ __forceinline__ double dpp_ror8(double v) {  // lane i <- lane i ^ 8 
   return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
 }
 
-// Lane permutations without index registers where the hardware allows:
-// xor 8 by a DPP row rotation, xor 16 / 24 by ds_swizzle (bit-mask mode,
-// and 0x1F, xor in bits 10-14), xor 32 by ds_bpermute.
-template <int PATTERN>
-__device__ __forceinline__ double swizzle64(double v) {
+// Lane permutations without index registers where the hardware allows: xor 8
+// by a DPP row rotation, xor 16 by ds_swizzle (bit-mask mode), xor 32 by
+// ds_bpermute.  The vector unit's row swaps (v_permlane16_swap and 32) take
+// five instructions a word against one: the steps below are bound by issue.
+__device__ __forceinline__ int xor16(int v) { return __builtin_amdgcn_ds_swizzle(v, 0x401F); }
+__device__ __forceinline__ double xor16(double v) {
   const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_ds_swizzle(int(b & 0xffffffffLL), PATTERN);
-  const int hi = __builtin_amdgcn_ds_swizzle(int(b >> 32), PATTERN);
+  const int lo = xor16(int(b & 0xffffffffLL)), hi = xor16(int(b >> 32));
   return __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
 }
+__device__ __forceinline__ int xor32(int v) { return __shfl_xor(v, 32); }
 __device__ __forceinline__ double xor32(double v) { return __shfl_xor(v, 32); }
-
-template <int M>
-__device__ __forceinline__ double xor_groups(double v) {  // lane i <- lane i ^ (8 M)
-  if constexpr (M == 1) return dpp_ror8(v);
-  if constexpr (M == 2) return swizzle64<0x401F>(v);
-  if constexpr (M == 3) return swizzle64<0x601F>(v);
-  if constexpr (M == 4) return xor32(v);
-  if constexpr (M == 5) return xor32(dpp_ror8(v));
-  if constexpr (M == 6) return xor32(swizzle64<0x401F>(v));
-  return xor32(swizzle64<0x601F>(v));
-}
 
 __device__ __forceinline__ void sum8(double& a) {
 #pragma unroll
@@ -699,14 +689,16 @@ __device__ __forceinline__ void sum8(double& a) {
 }
 
 // A column in registers: true column = d * v (rows li + 8j), n = its squared
-// norm.  Rotations in the scaled form move two FMAs per row (x' = x - t r y
-// with r a ratio of scales) and fold the cosine into d; n follows the exact
-// identities |x'|^2 = |x|^2 - t x.y, |y'|^2 = |y|^2 + t x.y and is recomputed
-// from the rows when it falls below a quarter of its value (cancellation).
-// The scales start at 1 when a column is loaded, so with at most 15
-// rotations between a load and a store they stay above 0.7^15.
+// norm.  Short columns (R <= 8) keep d = 1 and rotate both by c and s, 4 R
+// operations; longer ones rotate in the scaled form, two FMAs per row (x' = x -
+// t r y with r a ratio of scales) with the cosine folded into d.  n follows the
+// exact identities |x'|^2 = |x|^2 - t x.y, |y'|^2 = |y|^2 + t x.y and is
+// recomputed from the rows when it falls below a quarter of its value
+// (cancellation).  The scales start at 1 when a column is loaded, so with at
+// most 15 rotations between a load and a store they stay above 0.7^15.
 template <int R>
 struct WlCol {
+  static constexpr bool kScaled = R > 8;
   double v[R];
   double d, n;
 };
@@ -717,7 +709,7 @@ __device__ __forceinline__ double wl_norm(const WlCol<R>& x) {
 #pragma unroll
   for (int j = 0; j < R; ++j) s += x.v[j] * x.v[j];
   sum8(s);
-  return s * x.d * x.d;
+  return WlCol<R>::kScaled ? s * x.d * x.d : s;
 }
 
 // Column c of X (pitch k) into rows li + 8j.  Rows past k read the next
@@ -743,147 +735,208 @@ __device__ __forceinline__ void wl_store(double* X, int k, int c, int li, const 
   double* col = X + c * k + li;
 #pragma unroll
   for (int j = 0; j < R; ++j)
-    if (li + 8 * j < k) col[8 * j] = x.v[j] * x.d;
+    if (li + 8 * j < k) col[8 * j] = WlCol<R>::kScaled ? x.v[j] * x.d : x.v[j];
 }
 
-// Rotation of the column pair (x, y) from their squared norms and product:
-// t = tan(angle), c = cos(angle) as in jacobi_cs (x' = c x - s y,
-// y' = s x + c y, s = c t); false when the pair is orthogonal to tol_rot.
-__device__ __forceinline__ bool wl_rotation(double xx, double yy, double xy, double tol_rot, double& t, double& c) {
-  if (xx > 0.0 && yy > 0.0 && xy * xy > (tol_rot * xx) * (tol_rot * yy)) {
-    const double d = yy - xx, h = 2.0 * xy;
-    const double q2 = d * d + h * h;
-    const double r = q2 * fast_rsqrt(q2);
-    t = (d >= 0.0 ? h : -h) * fast_rcp(fabs(d) + r);
-    c = fast_rsqrt(1.0 + t * t);
-    return true;
-  }
-  return false;
+// The rotation of a column pair (x, y) from its squared norms and product:
+// x' = c (x - t y), y' = c (y + t x) with c = 1 / sqrt(1 + t^2).  It is
+// orthogonal for any t, so t comes from the bare estimates (2^-23 of the
+// coupling is left, well below tol_rot once couplings are small); c is exact.
+// big: the rotation could leave couplings over tol_rot, see wl_sweeps (t^2
+// (xx^2 + yy^2) / (xx yy) bounds the tangent times the ratio of the lengths).
+constexpr double kWlSmall = 1e-9;
+struct WlRot {
+  double t, c;
+  bool big;
+};
+__device__ __forceinline__ WlRot wl_rotation(double xx, double yy, double xx_yy, double xy, double xy2) {
+  WlRot r;
+  const double d = yy - xx, h = xy + xy;
+  const double q2 = fma(d, d, 4.0 * xy2);
+  const double den = fma(q2, __builtin_amdgcn_rsq(q2), fabs(d));
+  r.t = h * copysign(__builtin_amdgcn_rcp(den), d);
+  const double t2 = r.t * r.t, lim = (kWlSmall * kWlSmall) * xx_yy;
+  r.c = fast_rsqrt(1.0 + t2);
+  r.big = (xy2 > lim) | (t2 * fma(2.0, xx_yy, q2) > lim);
+  return r;
 }
 
-// Squared norm after a rotation, recomputed from the rows on cancellation.
 template <int R>
-__device__ __forceinline__ double wl_next_norm(const WlCol<R>& x, double n_old, double n_new) {
-  if (n_new < 0.25 * n_old) n_new = wl_norm<R>(x);  // uniform in the group
-  return n_new;
+__device__ __forceinline__ double wl_dot(const double* x, const double* y) {
+  double r0 = 0.0, r1 = 0.0;
+#pragma unroll
+  for (int j = 0; j < R; j += 2) {
+    r0 = fma(x[j], y[j], r0);
+    r1 = fma(x[j + 1], y[j + 1], r1);
+  }
+  r0 += r1;
+  sum8(r0);
+  return r0;
 }
 
-// Pairs (g, g ^ M) inside one block: x is the lower group's column.  Both
+// x from the lanes of group (own group) ^ m, m uniform.
+template <int R>
+__device__ __forceinline__ void wl_xor(WlCol<R>& x, int m) {
+  if (m & 1) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) x.v[j] = dpp_ror8(x.v[j]);
+    if constexpr (WlCol<R>::kScaled) x.d = dpp_ror8(x.d);
+    x.n = dpp_ror8(x.n);
+  }
+  if (m & 2) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) x.v[j] = xor16(x.v[j]);
+    if constexpr (WlCol<R>::kScaled) x.d = xor16(x.d);
+    x.n = xor16(x.n);
+  }
+  if (m & 4) {
+#pragma unroll
+    for (int j = 0; j < R; ++j) x.v[j] = xor32(x.v[j]);
+    if constexpr (WlCol<R>::kScaled) x.d = xor32(x.d);
+    x.n = xor32(x.n);
+  }
+}
+
+// Squared norms after a rotation (an, bn by the identities), recomputed from
+// the rows on cancellation.
+template <int R>
+__device__ __forceinline__ void wl_norms(WlCol<R>& a, WlCol<R>& b, double an, double bn) {
+  const bool lost = (an < 0.25 * a.n) | (bn < 0.25 * b.n);
+  a.n = an;
+  b.n = bn;
+  if (lost) {  // uniform in the group
+    a.n = wl_norm<R>(a);
+    b.n = wl_norm<R>(b);
+  }
+}
+
+// Pairs (g, g ^ m) inside one block: x is the lower group's column.  Both
 // groups form the same sums (the products commute and the reduction order is
 // the same), so they compute the same rotation and each updates its own
-// column.
-template <int R, int M>
-__device__ __forceinline__ void wl_intra(WlCol<R>& x, int grp, double tol_rot, int& cnt) {
-  const bool lower = grp < (grp ^ M);
-  double p[R];
+// column.  Without a branch, so that the chains of two blocks interleave.
+template <int R>
+__device__ __forceinline__ void wl_intra(WlCol<R>& x, int m, int grp, double tol2, unsigned long long& big) {
+  const bool lower = grp < (grp ^ m);
+  WlCol<R> p = x;
+  wl_xor<R>(p, m);
+  double xy = wl_dot<R>(x.v, p.v), ratio = 1.0;
+  if constexpr (WlCol<R>::kScaled) {
+    ratio = p.d * fast_rcp(x.d);
+    xy *= x.d * p.d;
+  }
+  const double xy2 = xy * xy, w = x.n * p.n;
+  WlRot r = wl_rotation(lower ? x.n : p.n, lower ? p.n : x.n, w, xy, xy2);
+  const bool rot = xy2 > tol2 * w;
+  big |= __ballot(rot & r.big);
+  // lower: x' = x - t (d_y / d_x) y;  upper: y' = y + t (d_x / d_y) x
+  const double t = rot ? (lower ? -r.t : r.t) : 0.0;
+  const double c = rot ? r.c : 1.0;
+  if constexpr (WlCol<R>::kScaled) {
 #pragma unroll
-  for (int j = 0; j < R; ++j) p[j] = xor_groups<M>(x.v[j]);
-  const double pd = xor_groups<M>(x.d), pn = xor_groups<M>(x.n);
-  double r = 0.0;
-#pragma unroll
-  for (int j = 0; j < R; ++j) r += x.v[j] * p[j];
-  sum8(r);
-  const double xy = (x.d * pd) * r;
-  double t, c;
-  if (wl_rotation(lower ? x.n : pn, lower ? pn : x.n, xy, tol_rot, t, c)) {
-    // lower: x' = x - t (d_y / d_x) y;  upper: y' = y + t (d_x / d_y) x
-    const double f = (lower ? -t : t) * pd * fast_rcp(x.d);
-#pragma unroll
-    for (int j = 0; j < R; ++j) x.v[j] += f * p[j];
+    for (int j = 0; j < R; ++j) x.v[j] = fma(t * ratio, p.v[j], x.v[j]);
     x.d *= c;
-    x.n = wl_next_norm<R>(x, x.n, x.n + (lower ? -t : t) * xy);
-    cnt += lower ? 1 : 0;
+  } else {
+    const double sn = t * c;
+#pragma unroll
+    for (int j = 0; j < R; ++j) x.v[j] = fma(sn, p.v[j], c * x.v[j]);
   }
+  const double n = fma(t, xy, x.n);
+  const bool lost = n < 0.25 * x.n;
+  x.n = n;
+  if (lost) x.n = wl_norm<R>(x);
 }
 
 template <int R>
-__device__ __forceinline__ void wl_intra_all(WlCol<R>& x, int grp, double tol_rot, int& cnt) {
-  wl_intra<R, 1>(x, grp, tol_rot, cnt);
-  wl_intra<R, 2>(x, grp, tol_rot, cnt);
-  wl_intra<R, 3>(x, grp, tol_rot, cnt);
-  wl_intra<R, 4>(x, grp, tol_rot, cnt);
-  wl_intra<R, 5>(x, grp, tol_rot, cnt);
-  wl_intra<R, 6>(x, grp, tol_rot, cnt);
-  wl_intra<R, 7>(x, grp, tol_rot, cnt);
-}
-
-template <int R>
-__device__ __forceinline__ void wl_cross(WlCol<R>& a, WlCol<R>& b, double tol_rot, int& cnt) {
-  double r = 0.0;
+__device__ __forceinline__ void wl_cross(WlCol<R>& a, WlCol<R>& b, double tol2, unsigned long long& big) {
+  double ab = wl_dot<R>(a.v, b.v), ra, rb;
+  if constexpr (WlCol<R>::kScaled) {
+    ra = b.d * fast_rcp(a.d);
+    rb = a.d * fast_rcp(b.d);
+    ab *= a.d * b.d;
+  }
+  const double ab2 = ab * ab, w = a.n * b.n;
+  if (ab2 > tol2 * w) {
+    const WlRot r = wl_rotation(a.n, b.n, w, ab, ab2);
+    big |= __ballot(r.big);
+    if constexpr (WlCol<R>::kScaled) {
+      const double fa = -r.t * ra, fb = r.t * rb;
 #pragma unroll
-  for (int j = 0; j < R; ++j) r += a.v[j] * b.v[j];
-  sum8(r);
-  const double ab = (a.d * b.d) * r;
-  double t, c;
-  if (wl_rotation(a.n, b.n, ab, tol_rot, t, c)) {
-    const double fa = -t * b.d * fast_rcp(a.d), fb = t * a.d * fast_rcp(b.d);
+      for (int j = 0; j < R; ++j) {
+        const double x = a.v[j], y = b.v[j];
+        a.v[j] = fma(fa, y, x);
+        b.v[j] = fma(fb, x, y);
+      }
+      a.d *= r.c;
+      b.d *= r.c;
+    } else {
+      const double sn = r.t * r.c;
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      const double x = a.v[j], y = b.v[j];
-      a.v[j] = x + fa * y;
-      b.v[j] = y + fb * x;
+      for (int j = 0; j < R; ++j) {
+        const double x = a.v[j], y = b.v[j];
+        a.v[j] = fma(-sn, y, r.c * x);
+        b.v[j] = fma(sn, x, r.c * y);
+      }
     }
-    a.d *= c;
-    b.d *= c;
-    a.n = wl_next_norm<R>(a, a.n, a.n - t * ab);
-    b.n = wl_next_norm<R>(b, b.n, b.n + t * ab);
-    ++cnt;
+    wl_norms<R>(a, b, fma(-r.t, ab, a.n), fma(r.t, ab, b.n));
   }
 }
 
-template <int R, int M>
-__device__ __forceinline__ void wl_shift(WlCol<R>& b) {
-#pragma unroll
-  for (int j = 0; j < R; ++j) b.v[j] = xor_groups<M>(b.v[j]);
-  b.d = xor_groups<M>(b.d);
-  b.n = xor_groups<M>(b.n);
-}
-
-// Sweeps until one rotates nothing (or max_sweeps); nrot[2] are shared
+// Sweeps until one has no big rotation (or max_sweeps); nrot[2] are shared
 // counters, zero on entry.  Every thread of the block calls this.
+//
+// A rotation adds to a coupling that is already zeroed at most the product of
+// its own size (the coupling, or for columns of about equal length the
+// tangent, times the ratio of the lengths) and another coupling.  After a
+// sweep in which both stayed below kWlSmall = 1e-9 every pair is below k 1e-18
+// + 2^-23 1e-9, inside tol_rot: a sweep more would only confirm it.  For k =
+// 24 .. 130 that is one of 3 .. 9 sweeps.
 template <int R>
 __device__ __forceinline__ void wl_sweeps(double* X, int k, double tol_rot, int max_sweeps, int* nrot) {
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, grp = lane >> 3, li = lane & 7;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, grp = lane >> 3, li = lane & 7;
   const int NB = 2 * ((k + 15) / 16);
   const bool active = wave < NB / 2;
+  const double tol2 = tol_rot * tol_rot;
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    int cnt = 0;
+    unsigned long long big = 0;
     for (int t = 0; t < NB - 1; ++t) {
       if (active) {
         const int P = circle_block(wave, t, NB), Q = circle_block(NB - 1 - wave, t, NB);
         WlCol<R> a, b;
+        wl_load<R>(X, k, P * 8 + grp, li, a);
         if (t == 0) {  // round 0 holds every block once: pairs inside the blocks
-          wl_load<R>(X, k, P * 8 + grp, li, a);
-          wl_intra_all<R>(a, grp, tol_rot, cnt);
-          wl_store<R>(X, k, P * 8 + grp, li, a);
+          if constexpr (R <= 10) {
+            wl_load<R>(X, k, Q * 8 + grp, li, b);
+#pragma unroll 1
+            for (int m = 1; m < 8; ++m) {
+              wl_intra<R>(a, m, grp, tol2, big);
+              wl_intra<R>(b, m, grp, tol2, big);
+            }
+          } else {  // one block at a time: two with their partners' copies would spill
+#pragma unroll 1
+            for (int m = 1; m < 8; ++m) wl_intra<R>(a, m, grp, tol2, big);
+            wl_load<R>(X, k, Q * 8 + grp, li, b);
+#pragma unroll 1
+            for (int m = 1; m < 8; ++m) wl_intra<R>(b, m, grp, tol2, big);
+          }
+        } else {
           wl_load<R>(X, k, Q * 8 + grp, li, b);
-          wl_intra_all<R>(b, grp, tol_rot, cnt);
-          wl_store<R>(X, k, Q * 8 + grp, li, b);
         }
-        wl_load<R>(X, k, P * 8 + grp, li, a);  // the same lanes wrote these rows: in order
-        wl_load<R>(X, k, Q * 8 + grp, li, b);
-        // group g pairs its P column with the Q column of group g ^ gray(u)
-        wl_cross<R>(a, b, tol_rot, cnt);
-        wl_shift<R, 1>(b);
-        wl_cross<R>(a, b, tol_rot, cnt);
-        wl_shift<R, 2>(b);
-        wl_cross<R>(a, b, tol_rot, cnt);
-        wl_shift<R, 1>(b);
-        wl_cross<R>(a, b, tol_rot, cnt);
-        wl_shift<R, 4>(b);
-        wl_cross<R>(a, b, tol_rot, cnt);
-        wl_shift<R, 1>(b);
-        wl_cross<R>(a, b, tol_rot, cnt);
-        wl_shift<R, 2>(b);
-        wl_cross<R>(a, b, tol_rot, cnt);
-        wl_shift<R, 1>(b);
-        wl_cross<R>(a, b, tol_rot, cnt);
+        // group g pairs its P column with the Q column of group g ^ gray(u);
+        // a loop of two steps, as eight unrolled overflow the instruction cache
+#pragma unroll 1
+        for (int u = 0; u < 4; ++u) {
+          wl_cross<R>(a, b, tol2, big);
+          wl_xor<R>(b, 1);
+          wl_cross<R>(a, b, tol2, big);
+          wl_xor<R>(b, (u & 1) ? 4 : 2);
+        }
         wl_store<R>(X, k, P * 8 + grp, li, a);
-        wl_store<R>(X, k, Q * 8 + (grp ^ 4), li, b);  // gray(7) = 4
+        wl_store<R>(X, k, Q * 8 + grp, li, b);  // the eight moves of b have come round
       }
       __syncthreads();
     }
-    if (li == 0 && cnt) atomicAdd(&nrot[sweep & 1], cnt);
+    if (lane == 0 && big) atomicAdd(&nrot[sweep & 1], 1);
     __syncthreads();
     const int n = nrot[sweep & 1];
     if (tid == 0) nrot[(sweep + 1) & 1] = 0;
@@ -892,73 +945,96 @@ __device__ __forceinline__ void wl_sweeps(double* X, int k, double tol_rot, int 
   }
 }
 
-// Pivoted Cholesky of G (in X, k x k column-major, k <= KM <= 64) by one
-// wave: lane i keeps row i of the trailing matrix in registers, so a step
-// takes no work-group barrier.  The trailing matrix stays symmetric to the
-// bit (both halves take the same products), so the pivot column is lane p's
-// row, which lane p writes to LDS (every index static: an index chosen at
-// run time would move the row to scratch).  Pivot rule, keys and arithmetic
-// are those of the register-tile form (the largest remaining diagonal,
-// smallest index on ties; l = G(:, p) / sqrt(G(p, p)); every update the same
-// fused multiply-add), so L is the same to the bit; column j of X receives l
-// in the original row order, pivoted[i] whether row i was a pivot.  Returns the rank.
-template <int KM>
-__device__ __forceinline__ int chol_wave(double* X, int* pivoted, int k) {
-  __shared__ double lb[64];  // the step's column l, one entry per lane
-  __shared__ double cp[64];  // the pivot's row of the trailing matrix
-  const int lane = threadIdx.x & 63;
-  const bool row = lane < k;
-  double g[KM];
+// Pivoted Cholesky of G (in X, k x k column-major, k <= 8 R <= 64): column j
+// of X receives column j of L in the original row order (X X^T = G), pivoted[i]
+// whether row i was a pivot; returns the rank.  Every thread of the block calls
+// this.
+//
+// Left-looking, eight lanes to a row: a step forms the pivot's column only,
+// G(:, p) minus the product of the columns of L so far, so its chain is one
+// read of the pivot, one of the pivot's row of L (in X), an eight-lane sum and
+// one barrier.  Lane li keeps the entries li, li + 8, ... of its row of G and
+// of L.  The pivot is the largest remaining diagonal up to 2^-12 of it (the key
+// has 20 bits of the value's mantissa less the row's eight), the smallest row
+// on ties; wkey, wval: shared, the waves' candidates by step parity.  k = 12,
+// 24, 40: 6, 14, 31 us against 9, 17, 43 for one wave that updates the trailing
+// matrix in its registers.
+template <int R>
+__device__ __forceinline__ int chol_rows(double* X, int* pivoted, int k, int (*wkey)[16], double (*wval)[16]) {
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = tid & 7;
+  const int nwv = (k + 7) >> 3;  // waves that hold rows
+  const bool has = (tid >> 3) < k;
+  const int row = has ? tid >> 3 : 0;  // reads stay inside X
+  double g[R], lr[R];
 #pragma unroll
-  for (int c = 0; c < KM; ++c) g[c] = (row && c < k) ? X[c * k + lane] : 0.0;
-  double dg = row ? X[lane * k + lane] : 0.0;
-  bool used = !row;
+  for (int q = 0; q < R; ++q) {
+    const int c = li + 8 * q;
+    g[q] = has && c < k ? X[c * k + row] : 0.0;
+    lr[q] = 0.0;
+  }
+  double dg = X[row * k + row];
+  bool out = !has;  // no row, or a pivoted one
+  auto publish = [&](int slot) {
+    const int hi = int(__double_as_longlong(dg) >> 32);
+    const int key = out ? INT_MIN : (hi & ~0xFF) | (255 - row);
+    int top = max(key, __builtin_amdgcn_mov_dpp(key, 0x128, 0xF, 0xF, false));
+    top = max(top, xor16(top));
+    top = max(top, xor32(top));
+    if (key == top && li == 0) {
+      wkey[slot][wave] = top;
+      wval[slot][wave] = dg;
+    }
+  };
+  if (wave < nwv) publish(0);
+  __syncthreads();  // also: every read of G precedes the columns of L
   int rk = k;
   for (int j = 0; j < k; ++j) {
-    long long key = used ? LLONG_MIN : ((__double_as_longlong(dg) & ~0x3FFLL) | (1023 - lane));
-#pragma unroll
-    for (int st = 0; st < 4; ++st) {
-      const long long o = __double_as_longlong(dpp_bits(__longlong_as_double(key), st));
-      key = o > key ? o : key;
-    }
-    long long o = __double_as_longlong(swizzle64<0x401F>(__longlong_as_double(key)));
-    key = o > key ? o : key;
-    o = __double_as_longlong(xor32(__longlong_as_double(key)));
-    key = o > key ? o : key;
-    const int p = __builtin_amdgcn_readfirstlane(key == LLONG_MIN ? -1 : 1023 - int(key & 0x3FF));
-    double pv = 0.0;
-    if (p >= 0) {
-      const long long b = __double_as_longlong(dg);
-      const int lo = __builtin_amdgcn_readlane(int(b & 0xffffffffLL), p);
-      const int hi = __builtin_amdgcn_readlane(int(b >> 32), p);
-      pv = __longlong_as_double((long long)(unsigned)lo | ((long long)hi << 32));
-    }
-    if (!(pv > 0.0)) {  // uniform: the rest of the matrix is zero or negative noise
+    // lane w < nwv looks at wave w's candidate
+    const int cand = lane < nwv ? wkey[j & 1][lane] : INT_MIN;
+    const double cval = lane < nwv ? wval[j & 1][lane] : -1.0;
+    int top = max(cand, __builtin_amdgcn_mov_dpp(cand, 0xB1, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_mov_dpp(top, 0x4E, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_mov_dpp(top, 0x141, 0xF, 0xF, false));
+    top = __builtin_amdgcn_readfirstlane(top);
+    const int who = __ffsll((unsigned long long)__ballot(cand == top)) - 1;
+    const long long cb = __double_as_longlong(cval);
+    const int plo = __builtin_amdgcn_readlane(int(cb & 0xffffffffLL), who);
+    const int phi = __builtin_amdgcn_readlane(int(cb >> 32), who);
+    const double pv = __longlong_as_double((long long)(unsigned)plo | ((long long)phi << 32));
+    const int p = 255 - (top & 0xFF);
+    if (top == INT_MIN || !(pv > 0.0)) {  // uniform: the rest is zero or negative noise
       rk = j;
       break;
     }
-    const double isq = fast_rsqrt(pv), sq = pv * isq;
-    if (lane == p) {
+    if (wave < nwv) {
+      double s = 0.0;
 #pragma unroll
-      for (int c = 0; c < KM; ++c) cp[c] = g[c];
-    }
-    __builtin_amdgcn_wave_barrier();  // one wave: its LDS accesses complete in order
-    const double gp = cp[lane];
-    const double l = lane == p ? sq : (used ? 0.0 : gp * isq);
-    if (lane == p) {
-      used = true;
-      dg = -1.0;
-    } else {
-      dg -= l * l;  // pivoted rows hold -1 and l = 0
-    }
-    if (row) X[j * k + lane] = l;
-    lb[lane] = l;
-    __builtin_amdgcn_wave_barrier();  // one wave: its LDS accesses complete in order
+      for (int q = 0; q < R; ++q)
+        if (q == (p >> 3)) s = g[q];
+      s = li == (p & 7) ? s : 0.0;
+      // entries of L past the j that exist meet zeros of lr
 #pragma unroll
-    for (int c = 0; c < KM; ++c) g[c] -= l * lb[c];
-    __builtin_amdgcn_wave_barrier();  // every read of lb precedes the next step's writes
+      for (int q0 = 0; q0 < R; q0 += 2)
+        if (8 * q0 < j) {
+          const double l0 = X[min(li + 8 * q0, j - 1) * k + p], l1 = X[min(li + 8 * q0 + 8, j - 1) * k + p];
+          s = fma(-lr[q0], l0, s);
+          s = fma(-lr[q0 + 1], l1, s);
+        }
+      const double isq = fast_rsqrt(pv);
+      sum8(s);
+      const bool here = has && row == p;
+      const double l = here ? pv * isq : (out ? 0.0 : s * isq);
+      if (li == 0 && has) X[j * k + row] = l;
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (q == (j >> 3)) lr[q] = li == (j & 7) ? l : lr[q];
+      dg = here ? -1.0 : dg - l * l;
+      out = out || here;
+      publish((j + 1) & 1);
+    }
+    __syncthreads();
   }
-  if (row) pivoted[lane] = used;
+  if (li == 0 && has) pivoted[row] = out;
   return rk;
 }
 
@@ -1035,24 +1111,23 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
   __syncthreads();
   const bool ident = nviol == 0 || k < 2;
   if (!ident && precond) {
-    // ---- 2. pivoted Cholesky, G held in registers ------------------------------
-    // Up to k = 64 one wave does it (chol_wave).  Wider, thread t owns an 8 x 5
-    // tile of G.  Step j picks the largest remaining diagonal p (smallest
-    // index on ties), the owners of column p publish l = G(:, p) / sqrt(G(p,
-    // p)) (zero on rows already pivoted), every tile takes the rank-one update
-    // and vec keeps the remaining diagonal.  Column j of X receives l in the
-    // original row order, so X X^T = G and the Jacobi below needs no
-    // permutation; perm flags the pivoted rows here and is reset to the
-    // identity afterwards.
-    __shared__ int rk_sh;
+    // ---- 2. pivoted Cholesky --------------------------------------------------
+    // Up to k = 64 by chol_rows.  Wider, thread t owns an 8 x 5 tile of G.
+    // Step j picks the largest remaining diagonal p (smallest index on ties),
+    // the owners of column p publish l = G(:, p) / sqrt(G(p, p)) (zero on rows
+    // already pivoted), every tile takes the rank-one update and vec keeps the
+    // remaining diagonal; column j of X receives l (k = 80: 102 us, 133 for
+    // chol_rows, which reads all columns so far each step).  perm flags the
+    // pivoted rows here and is reset to the identity afterwards.
+    __shared__ int wkey[2][16];
+    __shared__ double wval[2][16];
     int rk = k;
     if (k <= 64) {
-      if (tid < 64) {
-        const int r = k <= 32 ? chol_wave<32>(X, perm, k) : chol_wave<64>(X, perm, k);
-        if (tid == 0) rk_sh = r;
-      }
+      rk = k <= 16   ? chol_rows<2>(X, perm, k, wkey, wval)
+           : k <= 32 ? chol_rows<4>(X, perm, k, wkey, wval)
+           : k <= 48 ? chol_rows<6>(X, perm, k, wkey, wval)
+                     : chol_rows<8>(X, perm, k, wkey, wval);
       __syncthreads();
-      rk = rk_sh;
     } else {
       constexpr int TR = 8, TC = 5;
       const int ntc = (k + TC - 1) / TC;
@@ -1071,9 +1146,9 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
       // value, smallest index on ties; pivoted entries hold -1, and non-positive
       // values never win over positive ones under a signed compare.  Thread i <
       // k keeps row i; each wave holding rows reduces its keys and publishes the
-      // maximum in wkey[parity of the step it serves], which every thread reads
+      // maximum in tkey[parity of the step it serves], which every thread reads
       // after the step's second barrier.
-      __shared__ long long wkey[2][kGramEigThreads / 64];
+      __shared__ long long tkey[2][kGramEigThreads / 64];
       const int nwv = (k + 63) >> 6;  // waves that hold rows
       auto publish = [&](int slot) {
         long long key = LLONG_MIN;
@@ -1083,11 +1158,11 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
           const long long o = __double_as_longlong(dpp_bits(__longlong_as_double(key), st));
           key = o > key ? o : key;
         }
-        long long o = __double_as_longlong(swizzle64<0x401F>(__longlong_as_double(key)));
+        long long o = __double_as_longlong(xor16(__longlong_as_double(key)));
         key = o > key ? o : key;
         o = __double_as_longlong(xor32(__longlong_as_double(key)));
         key = o > key ? o : key;
-        if ((tid & 63) == 0) wkey[slot][tid >> 6] = key;
+        if ((tid & 63) == 0) tkey[slot][tid >> 6] = key;
       };
       if (tid < k) {
         vec[tid] = X[tid * k + tid];
@@ -1102,8 +1177,8 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
       // hh and nrm are written one phase after their last reads, behind a
       // barrier, and the wave maxima alternate between two slots.
       for (int j = 0; j < k; ++j) {
-        long long top = wkey[j & 1][0];
-        for (int w = 1; w < nwv; ++w) top = wkey[j & 1][w] > top ? wkey[j & 1][w] : top;
+        long long top = tkey[j & 1][0];
+        for (int w = 1; w < nwv; ++w) top = tkey[j & 1][w] > top ? tkey[j & 1][w] : top;
         const int p = top == LLONG_MIN ? -1 : 1023 - int(top & 0x3FF);
         const double pmx = p >= 0 ? vec[p] : 0.0;
         if (!(pmx > 0.0)) {  // uniform: the rest of the matrix is zero or negative noise

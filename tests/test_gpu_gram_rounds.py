@@ -54,6 +54,24 @@ def test_svd_sectors_at_tile_edges(ctx, shapes, decades, zeros):
             assert np.abs(w.T @ w - np.eye(w.shape[1])).max() <= 1e-12
 
 
+@pytest.mark.parametrize("decades,null", [(0.5, False), (12, False), (6, True)])
+def test_svd_one_group_sector_widths(ctx, decades, null):
+    """Every width class of the solver that takes a sector in one work-group,
+    at its eight-row, register and Cholesky limits, in one call."""
+    import quantit_amd as qa
+    rng = np.random.default_rng(77)
+    mats = [_graded(rng, k + k % 3, k, decades, k // 3 if null else 0)
+            for k in (1, 2, 3, 7, 8, 9, 15, 16, 17, 25, 31, 32, 33, 47, 48, 49, 57, 63, 64, 65, 72, 73, 97)]
+    U, d, V = (from_dev(x) for x in qa.svd(to_dev(ctx, _diagonal(mats)), 1))
+    for i, a in enumerate(mats):
+        u, s, v = U.blocks[(i, i)], d.blocks[(i,)], V.blocks[(i, i)]
+        assert np.abs(s - np.linalg.svd(a, compute_uv=False)).max() <= 1e-12 * s[0]
+        assert np.linalg.norm((u * s) @ v.T - a) <= 1e-12 * np.linalg.norm(a)
+        keep = s > 1e-10 * s[0]
+        for w in (u[:, keep], v[:, keep]):
+            assert np.abs(w.T @ w - np.eye(w.shape[1])).max() <= 1e-12
+
+
 @pytest.mark.parametrize("m,n,zeros", [(60, 60, 3), (200, 90, 1), (70, 150, 8)])
 def test_svd_few_null_columns_are_completed(ctx, m, n, zeros):
     """Few missing directions: no unit vector lies mostly along them, and the
