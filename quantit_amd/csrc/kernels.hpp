@@ -249,8 +249,9 @@ struct CompleteTask {
   int32_t ell, k, limit, pad;
 };
 void svd_complete(hipStream_t s, double* base, const Lists& tasks, int n);
-// eigh mode: c = ||A||_F per sector, stored at shift_off, and Y += c I.
-void svd_shift(hipStream_t s, double* base, const Lists& secs, int nsec);
+// eigh mode: Y += c I per sector, c = ||A||_F (norm: stored at shift_off) or
+// what shift_off holds.
+void svd_shift(hipStream_t s, double* base, const Lists& secs, int nsec, bool norm);
 void fill_i32(hipStream_t s, int32_t* p, int n, int32_t v);
 
 // One k x k matrix of the one-work-group kernels.
@@ -259,6 +260,7 @@ struct SmallJacobi {
   int32_t ell, k, ldy, ldw;
   int32_t flag_idx;       // flags[flag_idx]: result count of the kernel (-1: none)
   int32_t aux_idx;        // flags[aux_idx]: second count (gram_eig; -1: none)
+  int64_t shift_off = -1;  // >= 0: an eigh, G any symmetric matrix; receives the shift used (gram_eig)
 };
 size_t gram_eig_lds_limit();  // largest dynamic LDS per work-group (bytes)
 // Eigenvectors of k x k Gram matrices (SmallJacobi with ell = k): W written

@@ -1077,6 +1077,50 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
     nrot[0] = nrot[1] = 0;
   }
   __syncthreads();
+  // ---- 0. shift of an eigh -----------------------------------------------------
+  // The solver takes a positive definite matrix.  A density matrix is one up to
+  // its rounding, and its factor is as graded as its spectrum, so the sweeps
+  // are few; shifted by its norm all columns are about equally long and the
+  // rounding of their products keeps the sweeps going to their limit (sectors up
+  // to k = 68, twelve decades: 30 sweeps and 976 us, against 440).  So the shift is first the
+  // rounding a Cholesky factorisation may meet, and the norm only where that
+  // fails.
+  const bool eig = J.shift_off >= 0;
+  double shift = 0.0, fro = 0.0;
+  auto add_shift = [&] {
+    if (tid < k) X[tid * k + tid] += shift;
+    __syncthreads();
+  };
+  if (eig) {
+    __shared__ double red[3][kGramEigThreads / 64];
+    double ss = 0.0, lo = INFINITY, hi = 0.0;
+    for (int e = tid; e < k * k; e += blockDim.x) ss = fma(X[e], X[e], ss);
+    if (tid < k) {
+      lo = X[tid * k + tid];
+      hi = fmax(lo, 0.0);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      ss += __shfl_xor(ss, off);
+      lo = fmin(lo, __shfl_xor(lo, off));
+      hi = fmax(hi, __shfl_xor(hi, off));
+    }
+    if ((tid & 63) == 0) {
+      red[0][tid >> 6] = ss;
+      red[1][tid >> 6] = lo;
+      red[2][tid >> 6] = hi;
+    }
+    __syncthreads();
+    ss = 0.0;
+    for (int w = 0; w < kGramEigThreads / 64; ++w) {
+      ss += red[0][w];
+      lo = fmin(lo, red[1][w]);
+      hi = fmax(hi, red[2][w]);
+    }
+    fro = sqrt(ss);
+    shift = 4.0 * k * DBL_EPSILON * hi;
+    if (!(lo + shift > 0.0)) shift = fro;
+    add_shift();
+  }
   // ---- 1. orthogonality test on G -------------------------------------------
   {
     double dm = 0.0;
@@ -1121,112 +1165,121 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
     // pivoted rows here and is reset to the identity afterwards.
     __shared__ int wkey[2][16];
     __shared__ double wval[2][16];
-    int rk = k;
-    if (k <= 64) {
-      rk = k <= 16   ? chol_rows<2>(X, perm, k, wkey, wval)
-           : k <= 32 ? chol_rows<4>(X, perm, k, wkey, wval)
-           : k <= 48 ? chol_rows<6>(X, perm, k, wkey, wval)
-                     : chol_rows<8>(X, perm, k, wkey, wval);
-      __syncthreads();
-    } else {
-      constexpr int TR = 8, TC = 5;
-      const int ntc = (k + TC - 1) / TC;
-      const bool owner = tid < ((k + TR - 1) / TR) * ntc;
-      const int tr = owner ? tid / ntc : 0, tc = owner ? tid % ntc : 0;
-      double g[TR][TC];
-#pragma unroll
-      for (int a = 0; a < TR; ++a)
-#pragma unroll
-        for (int b = 0; b < TC; ++b) {
-          const int i = tr * TR + a, l = tc * TC + b;
-          g[a][b] = (owner && i < k && l < k) ? X[l * k + i] : 0.0;
-        }
-      // Pivot keys: the top 54 bits of the remaining diagonal and the inverted
-      // index in the low 10 bits (k <= 1023), so the largest key is the largest
-      // value, smallest index on ties; pivoted entries hold -1, and non-positive
-      // values never win over positive ones under a signed compare.  Thread i <
-      // k keeps row i; each wave holding rows reduces its keys and publishes the
-      // maximum in tkey[parity of the step it serves], which every thread reads
-      // after the step's second barrier.
-      __shared__ long long tkey[2][kGramEigThreads / 64];
-      const int nwv = (k + 63) >> 6;  // waves that hold rows
-      auto publish = [&](int slot) {
-        long long key = LLONG_MIN;
-        if (tid < k) key = (__double_as_longlong(vec[tid]) & ~0x3FFLL) | (1023 - tid);
-#pragma unroll
-        for (int st = 0; st < 4; ++st) {
-          const long long o = __double_as_longlong(dpp_bits(__longlong_as_double(key), st));
+    int rk;
+    for (;;) {
+      rk = k;
+      if (k <= 64) {
+        rk = k <= 16   ? chol_rows<2>(X, perm, k, wkey, wval)
+             : k <= 32 ? chol_rows<4>(X, perm, k, wkey, wval)
+             : k <= 48 ? chol_rows<6>(X, perm, k, wkey, wval)
+                       : chol_rows<8>(X, perm, k, wkey, wval);
+        __syncthreads();
+      } else {
+        constexpr int TR = 8, TC = 5;
+        const int ntc = (k + TC - 1) / TC;
+        const bool owner = tid < ((k + TR - 1) / TR) * ntc;
+        const int tr = owner ? tid / ntc : 0, tc = owner ? tid % ntc : 0;
+        double g[TR][TC];
+  #pragma unroll
+        for (int a = 0; a < TR; ++a)
+  #pragma unroll
+          for (int b = 0; b < TC; ++b) {
+            const int i = tr * TR + a, l = tc * TC + b;
+            g[a][b] = (owner && i < k && l < k) ? X[l * k + i] : 0.0;
+          }
+        // Pivot keys: the top 54 bits of the remaining diagonal and the inverted
+        // index in the low 10 bits (k <= 1023), so the largest key is the largest
+        // value, smallest index on ties; pivoted entries hold -1, and non-positive
+        // values never win over positive ones under a signed compare.  Thread i <
+        // k keeps row i; each wave holding rows reduces its keys and publishes the
+        // maximum in tkey[parity of the step it serves], which every thread reads
+        // after the step's second barrier.
+        __shared__ long long tkey[2][kGramEigThreads / 64];
+        const int nwv = (k + 63) >> 6;  // waves that hold rows
+        auto publish = [&](int slot) {
+          long long key = LLONG_MIN;
+          if (tid < k) key = (__double_as_longlong(vec[tid]) & ~0x3FFLL) | (1023 - tid);
+  #pragma unroll
+          for (int st = 0; st < 4; ++st) {
+            const long long o = __double_as_longlong(dpp_bits(__longlong_as_double(key), st));
+            key = o > key ? o : key;
+          }
+          long long o = __double_as_longlong(xor16(__longlong_as_double(key)));
           key = o > key ? o : key;
-        }
-        long long o = __double_as_longlong(xor16(__longlong_as_double(key)));
-        key = o > key ? o : key;
-        o = __double_as_longlong(xor32(__longlong_as_double(key)));
-        key = o > key ? o : key;
-        if ((tid & 63) == 0) tkey[slot][tid >> 6] = key;
-      };
-      if (tid < k) {
-        vec[tid] = X[tid * k + tid];
-        perm[tid] = 0;
-      }
-      if ((tid >> 6) < nwv) publish(0);
-      __syncthreads();  // every read of G from X precedes the L columns written below
-      // Each step: (1) every thread takes the pivot p from the wave maxima and
-      // the owners of column p copy it to hh; (2) thread i forms l_i, writes it
-      // to nrm and to column j of X, updates vec[i] and the waves publish the
-      // next keys; (3) the tiles take the rank-one update.  Two barriers a step:
-      // hh and nrm are written one phase after their last reads, behind a
-      // barrier, and the wave maxima alternate between two slots.
-      for (int j = 0; j < k; ++j) {
-        long long top = tkey[j & 1][0];
-        for (int w = 1; w < nwv; ++w) top = tkey[j & 1][w] > top ? tkey[j & 1][w] : top;
-        const int p = top == LLONG_MIN ? -1 : 1023 - int(top & 0x3FF);
-        const double pmx = p >= 0 ? vec[p] : 0.0;
-        if (!(pmx > 0.0)) {  // uniform: the rest of the matrix is zero or negative noise
-          rk = j;
-          break;
-        }
-        const double isq = fast_rsqrt(pmx), sq = pmx * isq;
-        if (owner && tc == p / TC) {
-          // column p - tc TC of the tile by 0/1 weights: a select on the index
-          // would be folded into an indexed load and move the tile to scratch
-          double m[TC];
-#pragma unroll
-          for (int b = 0; b < TC; ++b) m[b] = (p - tc * TC == b) ? 1.0 : 0.0;
-#pragma unroll
-          for (int a = 0; a < TR; ++a) {
-            double v = 0.0;
-#pragma unroll
-            for (int b = 0; b < TC; ++b) v += g[a][b] * m[b];
-            if (tr * TR + a < k) hh[tr * TR + a] = v;
-          }
-        }
-        __syncthreads();
+          o = __double_as_longlong(xor32(__longlong_as_double(key)));
+          key = o > key ? o : key;
+          if ((tid & 63) == 0) tkey[slot][tid >> 6] = key;
+        };
         if (tid < k) {
-          const int i = tid;
-          const double l = i == p ? sq : (perm[i] ? 0.0 : hh[i] * isq);
-          nrm[i] = l;
-          X[j * k + i] = l;
-          if (i == p) {
-            vec[p] = -1.0;
-            perm[p] = 1;
-          } else {
-            vec[i] -= l * l;  // pivoted rows hold -1 and l = 0
+          vec[tid] = X[tid * k + tid];
+          perm[tid] = 0;
+        }
+        if ((tid >> 6) < nwv) publish(0);
+        __syncthreads();  // every read of G from X precedes the L columns written below
+        // Each step: (1) every thread takes the pivot p from the wave maxima and
+        // the owners of column p copy it to hh; (2) thread i forms l_i, writes it
+        // to nrm and to column j of X, updates vec[i] and the waves publish the
+        // next keys; (3) the tiles take the rank-one update.  Two barriers a step:
+        // hh and nrm are written one phase after their last reads, behind a
+        // barrier, and the wave maxima alternate between two slots.
+        for (int j = 0; j < k; ++j) {
+          long long top = tkey[j & 1][0];
+          for (int w = 1; w < nwv; ++w) top = tkey[j & 1][w] > top ? tkey[j & 1][w] : top;
+          const int p = top == LLONG_MIN ? -1 : 1023 - int(top & 0x3FF);
+          const double pmx = p >= 0 ? vec[p] : 0.0;
+          if (!(pmx > 0.0)) {  // uniform: the rest of the matrix is zero or negative noise
+            rk = j;
+            break;
+          }
+          const double isq = fast_rsqrt(pmx), sq = pmx * isq;
+          if (owner && tc == p / TC) {
+            // column p - tc TC of the tile by 0/1 weights: a select on the index
+            // would be folded into an indexed load and move the tile to scratch
+            double m[TC];
+  #pragma unroll
+            for (int b = 0; b < TC; ++b) m[b] = (p - tc * TC == b) ? 1.0 : 0.0;
+  #pragma unroll
+            for (int a = 0; a < TR; ++a) {
+              double v = 0.0;
+  #pragma unroll
+              for (int b = 0; b < TC; ++b) v += g[a][b] * m[b];
+              if (tr * TR + a < k) hh[tr * TR + a] = v;
+            }
+          }
+          __syncthreads();
+          if (tid < k) {
+            const int i = tid;
+            const double l = i == p ? sq : (perm[i] ? 0.0 : hh[i] * isq);
+            nrm[i] = l;
+            X[j * k + i] = l;
+            if (i == p) {
+              vec[p] = -1.0;
+              perm[p] = 1;
+            } else {
+              vec[i] -= l * l;  // pivoted rows hold -1 and l = 0
+            }
+          }
+          if ((tid >> 6) < nwv) publish((j + 1) & 1);
+          __syncthreads();
+          if (owner) {
+            double li[TR], lc[TC];
+  #pragma unroll
+            for (int a = 0; a < TR; ++a) li[a] = tr * TR + a < k ? nrm[tr * TR + a] : 0.0;
+  #pragma unroll
+            for (int b = 0; b < TC; ++b) lc[b] = tc * TC + b < k ? nrm[tc * TC + b] : 0.0;
+  #pragma unroll
+            for (int a = 0; a < TR; ++a)
+  #pragma unroll
+              for (int b = 0; b < TC; ++b) g[a][b] -= li[a] * lc[b];
           }
         }
-        if ((tid >> 6) < nwv) publish((j + 1) & 1);
-        __syncthreads();
-        if (owner) {
-          double li[TR], lc[TC];
-#pragma unroll
-          for (int a = 0; a < TR; ++a) li[a] = tr * TR + a < k ? nrm[tr * TR + a] : 0.0;
-#pragma unroll
-          for (int b = 0; b < TC; ++b) lc[b] = tc * TC + b < k ? nrm[tc * TC + b] : 0.0;
-#pragma unroll
-          for (int a = 0; a < TR; ++a)
-#pragma unroll
-            for (int b = 0; b < TC; ++b) g[a][b] -= li[a] * lc[b];
-        }
       }
+      if (!eig || rk == k || shift == fro) break;
+      __syncthreads();  // not definite: again under the norm
+      for (int e = tid; e < k * k; e += blockDim.x) X[e] = Gg[int64_t(e / k) * J.ldy + e % k];
+      __syncthreads();
+      shift = fro;
+      add_shift();
     }
     // Columns from the rank on: small multiples of the unit vectors of the rows
     // without a pivot, the factor of G + delta^2 I there with delta^2 = 2^-54
@@ -1250,7 +1303,8 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
     __syncthreads();
   }
   // ---- 3. one-sided Jacobi on the columns of X ------------------------------
-  const double tol_rot = tol * (1.0 / 16.0);
+  // (under a shift by the norm, tol / 16 is below the products' rounding)
+  const double tol_rot = tol * (eig && shift == fro ? 0.5 : 1.0 / 16.0);
   const int pi = tid / gsz, li = tid % gsz;
   if (!ident) {
     if (k <= 16)
@@ -1347,6 +1401,7 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
     else
       Wg[int64_t(c) * J.ldw + perm[r]] = X[e];
   }
+  if (tid == 0 && eig) base[J.shift_off] = shift;
   if (tid == 0 && J.flag_idx >= 0) flags[J.flag_idx] = nviol;
   if (tid == 0 && J.aux_idx >= 0) flags[J.aux_idx] = nabs;
 }
@@ -1632,21 +1687,26 @@ void svd_finalize(hipStream_t st, double* base, const Lists& l, const SvdSector*
 }
 
 template <class L>
-__global__ __launch_bounds__(256) void k_svd_shift(double* __restrict__ base, L l) {
+__global__ __launch_bounds__(256) void k_svd_shift(double* __restrict__ base, L l, int norm) {
   __shared__ double sh[256];
   const SvdSector s = l.template list<SvdSector>()[blockIdx.x];
   double* Y = base + s.y_off;
-  const int64_t n = int64_t(s.ell) * s.k;
-  double acc = 0.0;
-  for (int64_t e = threadIdx.x; e < n; e += blockDim.x) acc += Y[e] * Y[e];
-  const double c = sqrt(wg_sum(acc, sh));
+  double c;
+  if (norm) {
+    const int64_t n = int64_t(s.ell) * s.k;
+    double acc = 0.0;
+    for (int64_t e = threadIdx.x; e < n; e += blockDim.x) acc += Y[e] * Y[e];
+    c = sqrt(wg_sum(acc, sh));
+  } else {
+    c = base[s.shift_off];
+  }
   for (int i = threadIdx.x; i < s.k; i += blockDim.x) Y[int64_t(i) * s.ell + i] += c;
-  if (threadIdx.x == 0) base[s.shift_off] = c;
+  if (norm && threadIdx.x == 0) base[s.shift_off] = c;
 }
 
-void svd_shift(hipStream_t st, double* base, const Lists& secs, int nsec) {
+void svd_shift(hipStream_t st, double* base, const Lists& secs, int nsec, bool norm) {
   if (nsec <= 0) return;
-  launch_lists(k_svd_shift<DevLists>, k_svd_shift<ArgLists>, secs, dim3(nsec), dim3(256), 0, st, base);
+  launch_lists(k_svd_shift<DevLists>, k_svd_shift<ArgLists>, secs, dim3(nsec), dim3(256), 0, st, base, int(norm));
 }
 
 __global__ void k_fill_i32(int32_t* p, int n, int32_t v) {

@@ -504,7 +504,6 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
     const kern::Lists d_secs = ctx->lists(B.secs);
     KernelTimer kt(*ctx, "svd_init");
     kern::svd_init_w(ctx->stream(), ab, d_secs, ns);
-    if (eigh_mode) kern::svd_shift(ctx->stream(), ab, d_secs, ns);
   }
   int max_ell = 0;
   for (auto& s : B.secs) max_ell = std::max(max_ell, s.ell);
@@ -540,6 +539,15 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       wide.push_back(i);
       large[i] = 1;
       B.wide[i] = 1;
+    }
+  }
+  if (eigh_mode) {  // the one-group solver chooses its sectors' shifts itself
+    std::vector<kern::SvdSector> by_norm;
+    for (int i = 0; i < ns; ++i)
+      if (large[i] || std::find(wide.begin(), wide.end(), i) == wide.end()) by_norm.push_back(B.secs[i]);
+    if (!by_norm.empty()) {
+      KernelTimer kt(*ctx, "svd_init");
+      kern::svd_shift(ctx->stream(), ab, ctx->lists(by_norm), int(by_norm.size()), true);
     }
   }
   if (!wide.empty()) {
@@ -786,7 +794,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
     };
     // eigh: A + c I is positive (semi-)definite, so it takes the Gram matrix's
     // place once: its eigenvectors are A's, and the column norms of (A + c I) W
-    // are the shifted eigenvalues.
+    // are the shifted eigenvalues.  Small sectors' c comes with the solve.
     const int max_it = eigh_mode ? 1 : env_int("QTT_SVD_GRAM_ITERS", 6);
     for (int it = 0; it < max_it && !act.empty(); ++it) {
       if (eigh_mode) {
@@ -821,7 +829,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         std::vector<kern::SmallJacobi> jd;
         for (int q : act_s) {
           const auto& s = B.secs[wide[q]];
-          jd.push_back({gb + go[q], gb + gwo[q], s.k, s.k, s.k, s.k, q, nw + q});
+          jd.push_back({gb + go[q], gb + gwo[q], s.k, s.k, s.k, s.k, q, nw + q, eigh_mode ? s.shift_off : -1});
         }
         // widest first, so that the longest solves start in the first wave of
         // work-groups when there are more sectors than the device holds
@@ -857,6 +865,12 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         solve_large(act_l);
       }
       if (overlap) ctx->join();
+      if (eigh_mode && !act_s.empty()) {
+        std::vector<kern::SvdSector> own;
+        for (int q : act_s) own.push_back(B.secs[wide[q]]);
+        KernelTimer kt(*ctx, "svd_init");
+        kern::svd_shift(ctx->stream(), ab, ctx->lists(own), int(own.size()), false);
+      }
       if (it >= 1) {  // the small solver's test of this iteration's G
         if (!act_s.empty() && ((act_l.empty() && cd_launched == 0) || overlap)) read_flags();
         retire(act_s);

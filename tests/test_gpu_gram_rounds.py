@@ -99,3 +99,28 @@ def test_eigh_sector_widths(ctx, k, kind):
     assert np.abs(vals - np.linalg.eigvalsh(a)).max() <= 1e-12 * nrm
     assert np.abs(a @ vec - vec * vals).max() <= 1e-11 * nrm
     assert np.abs(vec.T @ vec - np.eye(k)).max() <= 1e-12
+
+
+@pytest.mark.parametrize("low", [0.0, -1e-16, -1e-14, -1e-9, -1.0])
+def test_eigh_around_the_definite(ctx, low):
+    """Matrices just on either side of positive definite, where the solver's
+    shift changes, one with zero rows among them: all in one call."""
+    import quantit_amd as qa
+    rng = np.random.default_rng(3)
+    mats = []
+    for k in (2, 7, 33, 64, 65, 130):
+        q = np.linalg.qr(rng.standard_normal((k, k)))[0]
+        w = 10.0 ** (-12.0 * np.arange(k) / k)
+        w[k // 2:] = np.where(np.arange(k - k // 2) % 2, low, 0.0)
+        a = (q * w) @ q.T
+        mats.append(0.5 * (a + a.T))
+    z = np.zeros((20, 20))
+    z[:9, :9] = mats[1][0, 0] * np.eye(9) + 0.01
+    mats.append(z)
+    d, U = (from_dev(x) for x in qa.eigh(to_dev(ctx, _diagonal(mats)), 1))
+    for i, a in enumerate(mats):
+        vals, vec = d.blocks[(i,)], U.blocks[(i, i)]
+        nrm = np.abs(a).max() * a.shape[0]
+        assert np.abs(np.sort(vals) - np.linalg.eigvalsh(a)).max() <= 1e-12 * nrm
+        assert np.abs(vec.T @ vec - np.eye(a.shape[0])).max() <= 1e-12
+        assert np.abs(a @ vec - vec * vals).max() <= 1e-12 * nrm
