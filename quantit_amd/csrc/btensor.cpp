@@ -376,7 +376,8 @@ BTensor permute(const BTensor& t, const std::vector<int64_t>& in_perm) {
         d.sstride[i] = st[perm[i]];
       }
     }
-    chunk_tasks(tasks, int(descs.size()), sb.numel);
+    const int64_t nt = kern::permute_plan(d);
+    for (int64_t c = 0; c < nt; ++c) tasks.push_back({int32_t(descs.size()), int32_t(c)});
     descs.push_back(d);
   }
   if (!tasks.empty()) {

@@ -124,10 +124,14 @@ void gemm_rows(hipStream_t s, double* base, const Lists& l, int ntasks, int task
 // dims[0..rank) (row-major) reads src[sum_k j_k * sstride[k]].
 struct PermDesc {
   int64_t src_off, dst_off, numel;
-  int32_t rank, pad;
+  int32_t rank;
+  int32_t tj, tn;  // set by permute_plan: tiled dim (-1: none) and its tiles' length along the last dim
   int32_t dims[8];
   int64_t sstride[8];
 };
+// Merges the dims of a descriptor where it can, chooses how it is copied and
+// returns its number of tasks (chunks 0 .. of the descriptor).
+int64_t permute_plan(PermDesc& d);
 struct ChunkTask {
   int32_t desc;
   int32_t chunk;

@@ -589,7 +589,8 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     v.off = pack_elems;
     v.rs = v.K;
     v.cs = 1;
-    add_chunks(ptasks, int(pdesc.size()), blk.numel);
+    const int64_t nt = kern::permute_plan(d);
+    for (int64_t c = 0; c < nt; ++c) ptasks.push_back({int32_t(pdesc.size()), int32_t(c)});
     pdesc.push_back(d);
     pack_elems += blk.numel;
   };
