@@ -51,7 +51,8 @@ __device__ __forceinline__ void pair_side(int p, int round, int nb, int& pair, i
 
 // Rotations (c, s) of two symmetric 2 x 2 blocks [[a, q], [q, b]], their two
 // chains of dependent operations side by side (stage by stage; left to itself
-// the compiler puts one after the other, 1040 cycles a step against 690).  The
+// the compiler puts one after the other, 1040 cycles a step against 990, and 840
+// with the diagonal blocks written without a branch).  The
 // tangent needs only a few digits (the next meeting of the pair removes what
 // is left: a numpy model of the sweeps with tangents rounded to 24 bits takes
 // the same number of sweeps), so it comes from the bare hardware estimates;

@@ -52,11 +52,11 @@ __device__ double block_sum(double v, double* sh) {
   return r;
 }
 
-// 1/sqrt(x) by the hardware estimate and two Newton steps.
+// 1/sqrt(x) by the hardware estimate (2^-24) and one third-order step.
 __device__ __forceinline__ double fast_rsqrt_pc(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  y = y * (1.5 - 0.5 * x * y * y);
-  return y * (1.5 - 0.5 * x * y * y);
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-(x * y), y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
 }  // namespace
@@ -147,46 +147,23 @@ void gram_check(hipStream_t st, double* base, const Lists& descs, int n, int* fl
 // panel's columns are also written to Lp (k x nb, column-major) for the
 // trailing update.  LDS: the nb panel columns, the running diagonal dg
 // (G_ii less this panel's columns so far) and the pivoted flags, k each.
-// A step: per-thread best key over its indices, wave maxima by DPP and lane
-// swizzles, one barrier, every thread reduces the wave maxima itself.  The
-// key is the value's top 51 bits with the inverted index in the low 13
-// (k <= 8192): the largest diagonal wins, the smallest index among values
-// equal to 2^-39 relative; non-positive values never beat positive ones.
-__device__ __forceinline__ long long pc_dpp(long long key, int ctrl) {
-  int lo = int(key & 0xffffffffLL), hi = int(key >> 32);
-  switch (ctrl) {
-    case 0:
-      lo = __builtin_amdgcn_mov_dpp(lo, 0xB1, 0xF, 0xF, false);
-      hi = __builtin_amdgcn_mov_dpp(hi, 0xB1, 0xF, 0xF, false);
-      break;
-    case 1:
-      lo = __builtin_amdgcn_mov_dpp(lo, 0x4E, 0xF, 0xF, false);
-      hi = __builtin_amdgcn_mov_dpp(hi, 0x4E, 0xF, 0xF, false);
-      break;
-    case 2:
-      lo = __builtin_amdgcn_mov_dpp(lo, 0x141, 0xF, 0xF, false);
-      hi = __builtin_amdgcn_mov_dpp(hi, 0x141, 0xF, 0xF, false);
-      break;
-    case 3:
-      lo = __builtin_amdgcn_mov_dpp(lo, 0x140, 0xF, 0xF, false);
-      hi = __builtin_amdgcn_mov_dpp(hi, 0x140, 0xF, 0xF, false);
-      break;
-    case 4:  // lane xor 16 (ds_swizzle bit-mask mode)
-      lo = __builtin_amdgcn_ds_swizzle(lo, 0x401F);
-      hi = __builtin_amdgcn_ds_swizzle(hi, 0x401F);
-      break;
-    default:  // lane xor 32
-      lo = __shfl_xor(lo, 32);
-      hi = __shfl_xor(hi, 32);
-      break;
-  }
-  return (long long)(unsigned)lo | ((long long)hi << 32);
-}
-
+// The pivot is the largest remaining diagonal up to 2^-7 of it, the smallest
+// index on ties: the key is the value's upper word with the inverted index in
+// its low 13 bits (k <= 8192); non-positive values never beat positive ones.
+//
+// A step is bound by its chain (the waves' candidates, the pivot's column of G,
+// one barrier) and by LDS reads, which cost the same for one address as for 64
+// (a candidate per lane, not all by every thread).  ONE: one row to a thread (k
+// <= 1024), whose panel entries, diagonal and flag stay in registers; only the
+// pivot's row comes from LDS.  k = 544: 44 us a panel of 32, against 58 for
+// 64-bit keys and rows read from LDS.
+constexpr int kPanelMax = 32;
+template <bool ONE>
 __global__ __launch_bounds__(kLargeThreads) void k_pchol_panel(double* __restrict__ base,
                                                                const CholPanel* __restrict__ ps, int j0, int nb) {
   extern __shared__ double lds[];
-  __shared__ long long wkey[2][kLargeThreads / 64];  // wave maxima, by step parity
+  __shared__ int wkey[2][kLargeThreads / 64];  // the waves' candidates, by step parity
+  __shared__ double wval[2][kLargeThreads / 64];
   const CholPanel P = ps[blockIdx.x];
   const int k = P.k;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -201,32 +178,50 @@ __global__ __launch_bounds__(kLargeThreads) void k_pchol_panel(double* __restric
     for (int64_t e = tid; e < int64_t(k) * nb; e += blockDim.x) Lp[e] = 0.0;
     return;
   }
-  // the key of index i: the diagonal's top bits with the inverted index below
-  auto key_of = [&](int i) {
-    return used[i] ? LLONG_MIN : ((__double_as_longlong(dg[i]) & ~0x1FFFLL) | (8191 - i));
+  const int nwv = min(int(blockDim.x) >> 6, (k + 63) >> 6);  // waves that hold rows
+  auto key_of = [&](double d, int i) { return (int(__double_as_longlong(d) >> 32) & ~0x1FFF) | (8191 - i); };
+  // the wave's best row, from each lane's best (key, diagonal)
+  auto publish = [&](int key, double d, int slot) {
+    int top = max(key, __builtin_amdgcn_mov_dpp(key, 0xB1, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_mov_dpp(top, 0x4E, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_mov_dpp(top, 0x141, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_mov_dpp(top, 0x140, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_ds_swizzle(top, 0x401F));
+    top = max(top, __shfl_xor(top, 32));
+    if (key == top) {  // one lane, or all of a wave without a row left
+      wkey[slot][wave] = top;
+      wval[slot][wave] = d;
+    }
   };
-  auto publish = [&](long long key, int slot) {
+  double lr[ONE ? kPanelMax : 1], mydg = -1.0;
+  bool out = true;  // ONE: no row, or a pivoted one
 #pragma unroll
-    for (int st = 0; st < 6; ++st) {
-      const long long o = pc_dpp(key, st);
-      key = o > key ? o : key;
-    }
-    if (lane == 0) wkey[slot][wave] = key;
-  };
-  {
-    long long key = LLONG_MIN;
+  for (int t = 0; t < (ONE ? kPanelMax : 1); ++t) lr[t] = 0.0;
+  if (wave < nwv) {
+    int key = INT_MIN;
+    double d = -1.0;
     for (int i = tid; i < k; i += blockDim.x) {
-      dg[i] = G[int64_t(i) * k + i];
-      used[i] = state[1 + i];
-      const long long kk = key_of(i);
-      key = kk > key ? kk : key;
+      const double di = G[int64_t(i) * k + i];
+      const int u = state[1 + i];
+      const int ki = u ? INT_MIN : key_of(di, i);
+      if (ki > key) {
+        key = ki;
+        d = di;
+      }
+      if constexpr (ONE) {
+        mydg = di;
+        out = u != 0;
+      } else {
+        dg[i] = di;
+        used[i] = u;
+      }
     }
-    publish(key, 0);
+    publish(key, d, 0);
   }
   __syncthreads();
   // One barrier per step: a thread forms the next step's key from its own
-  // diagonal entries right after updating them, and the wave maxima go to
-  // the other parity's slots (last read before the previous barrier).
+  // diagonal entries right after updating them, and the candidates go to the
+  // other parity's slots (last read before the previous barrier).
   int rank = k;
   for (int jj = 0; jj < nb; ++jj) {
     const int j = j0 + jj;
@@ -234,53 +229,93 @@ __global__ __launch_bounds__(kLargeThreads) void k_pchol_panel(double* __restric
       for (int i = tid; i < k; i += blockDim.x) col[jj * k + i] = 0.0;
       continue;
     }
-    long long key = LLONG_MIN;
-    // the launch has kLargeThreads threads: a fixed trip count lets the
-    // sixteen reads be issued together
-#pragma unroll
-    for (int w = 0; w < kLargeThreads / 64; ++w) key = wkey[jj & 1][w] > key ? wkey[jj & 1][w] : key;
-    const int p = key == LLONG_MIN ? -1 : 8191 - int(key & 0x1FFF);
-    const double pv = p >= 0 ? dg[p] : 0.0;
-    if (!(pv > 0.0)) {  // uniform: the rest is zero or negative noise
+    // lane w < nwv looks at wave w's candidate
+    const int cand = lane < nwv ? wkey[jj & 1][lane] : INT_MIN;
+    const double cval = lane < nwv ? wval[jj & 1][lane] : -1.0;
+    int top = max(cand, __builtin_amdgcn_mov_dpp(cand, 0xB1, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_mov_dpp(top, 0x4E, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_mov_dpp(top, 0x141, 0xF, 0xF, false));
+    top = max(top, __builtin_amdgcn_mov_dpp(top, 0x140, 0xF, 0xF, false));
+    top = __builtin_amdgcn_readfirstlane(top);
+    const int who = __ffsll((unsigned long long)__ballot(cand == top)) - 1;
+    const long long cb = __double_as_longlong(cval);
+    const int plo = __builtin_amdgcn_readlane(int(cb & 0xffffffffLL), who);
+    const int phi = __builtin_amdgcn_readlane(int(cb >> 32), who);
+    const double pv = __longlong_as_double((long long)(unsigned)plo | ((long long)phi << 32));
+    const int p = 8191 - (top & 0x1FFF);
+    if (top == INT_MIN || !(pv > 0.0)) {  // uniform: the rest is zero or negative noise
       for (int t = jj; t < nb; ++t)
         for (int i = tid; i < k; i += blockDim.x) col[t * k + i] = 0.0;
       rank = j;
       break;
     }
-    const double isq = fast_rsqrt_pc(pv), ljj = pv * isq;
-    long long nkey = LLONG_MIN;
-    for (int i = tid; i < k; i += blockDim.x) {
-      double v = 0.0;
-      if (i == p) {
-        v = ljj;
-        used[p] = 1;
-      } else if (!used[i]) {
-        // the load of G's column p is independent of the dot product over the
-        // panel's earlier columns, so its latency overlaps that sum
-        const double gpi = G[int64_t(p) * k + i];
-        double acc = 0.0;
-        // unrolled so that the LDS reads of several terms are in flight at
-        // once; the FMA chain keeps its order
+    if (wave < nwv) {
+      const double isq = fast_rsqrt_pc(pv), ljj = pv * isq;
+      int key = INT_MIN;
+      double d = -1.0;
+      if constexpr (ONE) {
+        // the load of G's column p does not depend on the sum over the panel's
+        // earlier columns, so its latency overlaps that
+        const double gpi = out ? 0.0 : G[int64_t(p) * k + tid];
+        double acc[2] = {0.0, 0.0};
+#pragma unroll
+        for (int t0 = 0; t0 < kPanelMax; t0 += 8)
+          if (t0 < jj) {  // entries past jj meet zeros of lr
+            double lp[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) lp[u] = col[min(t0 + u, jj - 1) * k + p];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc[u & 1] = fma(lr[t0 + u], lp[u], acc[u & 1]);
+          }
+        const bool here = tid == p;
+        const double v = here ? ljj : out ? 0.0 : (gpi - (acc[0] + acc[1])) * isq;
+        mydg = here ? -1.0 : fma(-v, v, mydg);
+        out = out || here;
+        if (tid < k) col[jj * k + tid] = v;
+#pragma unroll
+        for (int t0 = 0; t0 < kPanelMax; t0 += 8)
+          if (t0 == (jj & ~7))
+#pragma unroll
+            for (int u = 0; u < 8; ++u) lr[t0 + u] = u == (jj & 7) ? v : lr[t0 + u];
+        key = out ? INT_MIN : key_of(mydg, tid);
+        d = mydg;
+      } else {
+        for (int i = tid; i < k; i += blockDim.x) {
+          double v = 0.0;
+          if (i == p) {
+            v = ljj;
+            used[p] = 1;
+          } else if (!used[i]) {
+            const double gpi = G[int64_t(p) * k + i];
+            double acc = 0.0;
 #pragma unroll 8
-        for (int t = 0; t < jj; ++t) acc = fma(col[t * k + i], col[t * k + p], acc);
-        v = (gpi - acc) * isq;
-        dg[i] -= v * v;
+            for (int t = 0; t < jj; ++t) acc = fma(col[t * k + i], col[t * k + p], acc);
+            v = (gpi - acc) * isq;
+            dg[i] -= v * v;
+          }
+          col[jj * k + i] = v;
+          const int ki = used[i] ? INT_MIN : key_of(dg[i], i);
+          if (ki > key) {
+            key = ki;
+            d = dg[i];
+          }
+        }
       }
-      col[jj * k + i] = v;
-      const long long kk = key_of(i);
-      nkey = kk > nkey ? kk : nkey;
+      publish(key, d, (jj + 1) & 1);
     }
-    publish(nkey, (jj + 1) & 1);
     __syncthreads();
   }
+  if constexpr (ONE)
+    if (tid < k) used[tid] = out;
   __syncthreads();  // the copies below read other threads' column entries
   for (int i = tid; i < k; i += blockDim.x) state[1 + i] = used[i];
   if (tid == 0 && rank < k) state[0] = rank;
-  for (int64_t e = tid; e < int64_t(k) * nb; e += blockDim.x) {
-    const int t = int(e / k), i = int(e % k);
-    Lp[e] = col[e];
-    if (j0 + t < k) L[int64_t(j0 + t) * k + i] = col[e];
-  }
+  for (int t = wave; t < nb; t += int(blockDim.x) >> 6)
+    for (int i = lane; i < k; i += 64) {
+      const double v = col[t * k + i];
+      Lp[int64_t(t) * k + i] = v;
+      if (j0 + t < k) L[int64_t(j0 + t) * k + i] = v;
+    }
   if (rank > 0 && rank < k) {
     // the factor of G + delta^2 I on the rows without a pivot, as in k_gram_eig
     __syncthreads();  // the zero columns copied above are overwritten
@@ -310,9 +345,13 @@ void pchol_init(hipStream_t st, double* base, const void* descs, int n) {
 
 void pchol_panel(hipStream_t st, double* base, const void* descs, int n, int j0, int nb, int kmax) {
   if (n <= 0) return;
+  if (nb > kPanelMax) throw std::runtime_error("Cholesky panel wider than 32 columns");
   const size_t lds = size_t(kmax) * (nb + kPcholExtra) * sizeof(double);
-  hipLaunchKernelGGL(k_pchol_panel, dim3(n), dim3(kLargeThreads), lds, st, base,
-                     static_cast<const CholPanel*>(descs), j0, nb);
+  const auto* ps = static_cast<const CholPanel*>(descs);
+  if (kmax <= kLargeThreads)
+    hipLaunchKernelGGL(k_pchol_panel<true>, dim3(n), dim3((kmax + 63) / 64 * 64), lds, st, base, ps, j0, nb);
+  else
+    hipLaunchKernelGGL(k_pchol_panel<false>, dim3(n), dim3(kLargeThreads), lds, st, base, ps, j0, nb);
 }
 
 size_t pchol_lds_limit() {
@@ -321,8 +360,9 @@ size_t pchol_lds_limit() {
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) v = 65536;
     const size_t l = size_t(v) - 1024;  // static arrays of the kernel
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pchol_panel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, int(l));
+    for (const void* f : {reinterpret_cast<const void*>(&k_pchol_panel<true>),
+                          reinterpret_cast<const void*>(&k_pchol_panel<false>)})
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, int(l));
     return l;
   }();
   return limit;
