@@ -207,9 +207,18 @@ void krylov_axpy(hipStream_t s, double* base, int64_t v_off, int64_t ld, int m, 
                  int64_t src_off, int64_t dst_off, int64_t n, int64_t scale_off);
 // alpha[j] = c1[j] + c2[j], beta[j] = sqrt(nrm2) into T (alpha T[0..K), beta
 // T[K..2K)), then the lowest eigenpair of the leading (j+1)-square
-// tridiagonal: out = {eigenvalue, residual beta[j] |y[j]|, beta[j], y...}.
+// tridiagonal: out = {eigenvalue, residual beta[j] |y[j]|, beta[j], y...};
+// host (pinned): the first three, then 1 when a NaN appeared, else 0.
 void lanczos_tridiag(hipStream_t s, double* base, int64_t t_off, int K, int j, int64_t c1_off, int64_t c2_off,
-                     int64_t nrm2_off, int64_t out_off, int* flags);
+                     int64_t nrm2_off, int64_t out_off, double* host);
+// A Lanczos step after the matvec in one launch, for short vectors
+// (krylov_step_fits): w orthogonalised twice against rows 0 .. j of V, nrm2 =
+// |w|^2, row j + 1 = w / |w| (when j + 1 < K), and lanczos_tridiag's results.  w
+// itself is left as it was.
+constexpr int kKrylovStepMaxN = 8192;
+inline bool krylov_step_fits(int64_t n, int m) { return n <= kKrylovStepMaxN && n * m <= 65536; }
+void krylov_step(hipStream_t s, double* base, int64_t v_off, int64_t ld, int j, int K, int64_t w_off, int64_t n,
+                 int64_t t_off, int64_t nrm2_off, int64_t out_off, double* host);
 
 // ---- block SVD ----------------------------------------------------------
 // Sector work matrices: Y (ell x k, column-major, ld = ell) is orthogonalised

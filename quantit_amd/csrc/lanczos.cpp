@@ -162,13 +162,11 @@ LanczosResult lanczos_ground(const BTensor& theta, const BTensor& W, const BTens
   std::vector<char> present(lay.idx.size(), 1);  // blocks some Krylov vector so far has
   if (lay.n == 0) throw DomainError("two-site state without elements");
 
-  // scalars: c1[K], c2[K], nrm2, T[2K], out[3 + K], then the NaN flag (an
-  // int32 in a double slot), so one read per step brings both back
+  // scalars: c1[K], c2[K], nrm2, T[2K], out[3 + K]
   BufPtr sc = ctx->alloc(size_t(6 * K + 8) * sizeof(double));
   const int64_t s0 = sc->dptr() - ab;
   const int64_t c1 = s0, c2 = s0 + K, nrm2 = s0 + 2 * K, t_off = s0 + 2 * K + 1, out = s0 + 4 * K + 1;
-  int32_t* d_flag = reinterpret_cast<int32_t*>(ab + out + 3 + K);
-  kern::fill_i32(ctx->stream(), d_flag, 1, 0);
+  double* const host = ctx->pinned_doubles();  // eigenvalue, residual, beta, NaN flag of the last step
   BufPtr V, w, part;
   auto alloc_vectors = [&](int64_t n) {
     V = ctx->alloc(size_t(K) * size_t(n) * sizeof(double));
@@ -274,7 +272,11 @@ LanczosResult lanczos_ground(const BTensor& theta, const BTensor& W, const BTens
         }
       launch_copies(ctx, ab, cp, tasks, "lanczos_scatter");
     }
-    {
+    const bool one_launch = kern::krylov_step_fits(lay.n, j + 1);
+    if (one_launch) {
+      KernelTimer kt(*ctx, "lanczos_step");
+      kern::krylov_step(ctx->stream(), ab, voff(0), lay.n, j, K, woff(), lay.n, t_off, nrm2, out, host);
+    } else {
       // two classical Gram-Schmidt passes against v_0..v_j, then |w|^2 and
       // the tridiagonal eigensolve (alpha_j = <v_j|H v_j> with its correction)
       KernelTimer kt(*ctx, "lanczos_vec");
@@ -285,22 +287,20 @@ LanczosResult lanczos_ground(const BTensor& theta, const BTensor& W, const BTens
       kern::krylov_axpy(ctx->stream(), ab, voff(0), lay.n, mj, c2, -1.0, woff(), woff(), lay.n, -1);
       kern::krylov_dot(ctx->stream(), ab, woff(), lay.n, 1, woff(), lay.n, poff(), nrm2);
     }
-    {
+    if (!one_launch) {
       KernelTimer kt(*ctx, "lanczos_tridiag");
-      kern::lanczos_tridiag(ctx->stream(), ab, t_off, K, j, c1, c2, nrm2, out, d_flag);
+      kern::lanczos_tridiag(ctx->stream(), ab, t_off, K, j, c1, c2, nrm2, out, host);
     }
-    double host_all[3 + kern::kMaxKrylov + 1];
-    ctx->read_small(host_all, ab + out, size_t(3 + K + 1) * sizeof(double));
-    int32_t hflag = 0;
-    std::memcpy(&hflag, host_all + 3 + K, sizeof(int32_t));
-    if (hflag) throw LogicError("nan found in output tensor");
-    std::copy(host_all, host_all + 3, host_out);
+    ctx->sync();
+    if (host[3] != 0.0) throw LogicError("nan found in output tensor");
+    std::copy(host, host + 3, host_out);
     const double lam = host_out[0], resid = host_out[1], beta = host_out[2];
     m = j + 1;
     const bool done = resid <= tol * std::fabs(lam) || !(beta > 1e-15 * std::fabs(lam)) || m == K;
     if (done) break;
     for (size_t q = 0; q < o.blocks.size(); ++q)
       if (o.blocks[q].numel) present[where[q]] = 1;
+    if (one_launch) continue;
     KernelTimer kt(*ctx, "lanczos_vec");
     kern::krylov_axpy(ctx->stream(), ab, voff(0), lay.n, 0, nrm2, 0.0, woff(), voff(j + 1), lay.n, nrm2);
   }

@@ -128,6 +128,8 @@ class Context {
   // A pinned word that a device-to-host copy may target without waiting;
   // valid after the next synchronization of the stream.
   int32_t* pinned_flag() { return host_small_; }
+  // Four pinned doubles that a kernel may store to; valid likewise.
+  double* pinned_doubles() { return reinterpret_cast<double*>(host_small_) + 4; }
   void reserve_read(size_t n_per_slot);
   int32_t* read_slot(int slot) const { return host_read_ + size_t(slot) * read_cap_; }
   hipEvent_t read_event(int slot) const { return read_ev_[slot]; }
@@ -186,7 +188,7 @@ class Context {
     hipEvent_t a, b;
   };
   std::vector<Pending> pending_;
-  int32_t* host_small_ = nullptr;  // word 0: pinned_flag; from byte 256: read_small
+  int32_t* host_small_ = nullptr;  // word 0: pinned_flag; byte 32: pinned_doubles; from byte 256: read_small
   static constexpr size_t kSmallBytes = size_t(64) << 10;
   int32_t* host_read_ = nullptr;
   size_t read_cap_ = 0;  // words per slot
