@@ -151,7 +151,7 @@ LanczosStep one_step_lanczos(const BTensor& theta, const BTensor& W, const BTens
   return r;
 }
 
-Eig2x2 eig2x2_dev(const BTensor& a0, const BTensor& a1, const BTensor& b) {
+Eig2x2 eig2x2_dev(const BTensor& a0, const BTensor& a1, const BTensor& b, int* flag) {
   Context* ctx = a0.ctx;
   Shape s0;
   s0.g = a0.shape.g;
@@ -165,11 +165,13 @@ Eig2x2 eig2x2_dev(const BTensor& a0, const BTensor& a1, const BTensor& b) {
   }
   r.o.blocks[0].off = 1;
   r.n.blocks[0].off = 2;
-  r.flag = ctx->alloc(sizeof(int));
-  kern::fill_i32(ctx->stream(), reinterpret_cast<int32_t*>(r.flag->cptr()), 1, 0);
+  if (!flag) {
+    r.flag = ctx->alloc(sizeof(int));
+    flag = reinterpret_cast<int*>(r.flag->cptr());
+  }
   KernelTimer kt(*ctx, "eig2x2");
   kern::eig2x2(ctx->stream(), ab, a0.ptr(a0.blocks[0]) - ab, a1.ptr(a1.blocks[0]) - ab, b.ptr(b.blocks[0]) - ab,
-               trio->dptr() - ab, reinterpret_cast<int*>(r.flag->cptr()));
+               trio->dptr() - ab, flag);
   return r;
 }
 
@@ -214,19 +216,17 @@ BTensor dmrg_update(DmrgState& st, const DmrgOptions& opt, DmrgLog* log) {
   }
   // one_step_lanczos (dmrg.cpp:584-608), eig2x2Mat (dmrg.cpp:543-572) on device
   LanczosStep ls = one_step_lanczos(theta, W, Lenv, Renv, &cs);
-  Eig2x2 eg = eig2x2_dev(ls.a0, ls.a1, ls.b);
+  // the flag lands in pinned memory without a wait; the truncation's read of
+  // its kept counts synchronizes the stream after it
+  int32_t* h_flag = ctx->pinned_flag();
+  Eig2x2 eg = eig2x2_dev(ls.a0, ls.a1, ls.b, h_flag);
   const BTensor& psi = ls.Hpsi;
   const BTensor& E = eg.E;
   const BTensor& o = eg.o;
   const BTensor& n = eg.n;
-  // the flag lands in pinned memory without a wait; the truncation's read of
-  // its kept counts synchronizes the stream after it
-  int32_t* h_flag = ctx->pinned_flag();
-  *h_flag = 0;
-  QTT_HIP(hipMemcpyAsync(h_flag, eg.flag->cptr(), sizeof(int), hipMemcpyDeviceToHost, ctx->stream()));
   BTensor theta2 = axpby_dev(theta, o, psi, n);
   SvdResult r = svd_truncated(theta2, 2, opt.cutoff, opt.minimum_bond, opt.maximum_bond, 2.0, &ss);
-  ctx->sync();  // normally already done by the truncation; the flag copy is complete
+  ctx->sync();  // normally already done by the truncation; the flag is there
   if (*h_flag) throw LogicError("nan found in output tensor");
   absorb(st, r, oc);
   if (log) {

@@ -82,7 +82,8 @@ struct Eig2x2 {
   BTensor E, o, n;
   BufPtr flag;
 };
-Eig2x2 eig2x2_dev(const BTensor& a0, const BTensor& a1, const BTensor& b);
+// flag: where the NaN flag goes (null: device memory, kept in the result).
+Eig2x2 eig2x2_dev(const BTensor& a0, const BTensor& a1, const BTensor& b, int* flag = nullptr);
 
 // k-step Lanczos with full reorthogonalisation (FP64, on device) for the
 // lowest eigenpair of the two-site Hamiltonian L.W.R: stops when the residual

@@ -258,7 +258,7 @@ BTensor full_dot(const BTensor& x, const BTensor& y, bool sqrt_out) {
   BufPtr partial = ctx->alloc(std::max<size_t>(tasks.size(), 1) * sizeof(double));
   KernelTimer kt(*ctx, "dot");
   kern::dot(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), partial->dptr() - ab,
-            out.ptr(out.blocks[0]) - ab, sqrt_out);
+            out.ptr(out.blocks[0]) - ab, sqrt_out, ctx->dot_counter());
   return out;
 }
 

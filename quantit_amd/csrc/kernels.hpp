@@ -184,10 +184,10 @@ void axpby(hipStream_t s, double* base, const Lists& l, int ntasks, int64_t a_of
 struct DotDesc {
   int64_t x_off, y_off, numel;
 };
-void dot(hipStream_t s, double* base, const Lists& l, int ntasks,
-         int64_t partial_off, int64_t out_off, bool sqrt_out);
+void dot(hipStream_t s, double* base, const Lists& l, int ntasks, int64_t partial_off, int64_t out_off, bool sqrt_out,
+         int* done);
 // eig2x2Mat (sources/dmrg.cpp:543-572) on device scalars a0, a1, b; writes
-// E, o, n to out[0..3) and sets flags[0] = 1 on NaN.
+// E, o, n to out[0..3) and 1 to flags[0] on NaN, else 0.
 void eig2x2(hipStream_t s, double* base, int64_t a0_off, int64_t a1_off, int64_t b_off, int64_t out_off,
             int* flags);
 // d /= sqrt(sum d^2) over n contiguous values.
@@ -212,11 +212,10 @@ void krylov_axpy(hipStream_t s, double* base, int64_t v_off, int64_t ld, int m, 
 void lanczos_tridiag(hipStream_t s, double* base, int64_t t_off, int K, int j, int64_t c1_off, int64_t c2_off,
                      int64_t nrm2_off, int64_t out_off, double* host);
 // A Lanczos step after the matvec in one launch, for short vectors
-// (krylov_step_fits): w orthogonalised twice against rows 0 .. j of V, nrm2 =
+// (kKrylovStepMaxN): w orthogonalised twice against rows 0 .. j of V, nrm2 =
 // |w|^2, row j + 1 = w / |w| (when j + 1 < K), and lanczos_tridiag's results.  w
 // itself is left as it was.
 constexpr int kKrylovStepMaxN = 8192;
-inline bool krylov_step_fits(int64_t n, int m) { return n <= kKrylovStepMaxN && n * m <= 65536; }
 void krylov_step(hipStream_t s, double* base, int64_t v_off, int64_t ld, int j, int K, int64_t w_off, int64_t n,
                  int64_t t_off, int64_t nrm2_off, int64_t out_off, double* host);
 
@@ -236,7 +235,13 @@ struct SvdSector {
   int64_t shift_off;        // device double holding c (eigh mode)
 };
 constexpr int kSvdBlock = 16;  // columns per Jacobi block
-void svd_init_w(hipStream_t s, double* base, const Lists& secs, int nsec);
+// Start of a decomposition: the work matrices Y (ell x kp) and their partners
+// zero, W (kp x kp) and its partner the identity (offsets < 0: none).
+struct SvdPrep {
+  int64_t y_off, w_off, y2_off, w2_off;
+  int32_t ell, kp;
+};
+void svd_prepare(hipStream_t s, double* base, const Lists& secs, int nsec, int64_t max_elems);
 // One round of the block Jacobi tournament; max_ell = largest row count
 // among the sectors (picks the LDS-resident kernel when the block pair fits).
 // cross_after0: rounds after the first of a sweep rotate only the pairs

@@ -37,19 +37,26 @@ constexpr int GP = NB2 + 1;         // LDS pitch of G and Q
 // W = I (kp x kp) for every sector; gridDim.y work-groups share a sector,
 // one column per wave-step.
 template <class L>
-__global__ void k_svd_init_w(double* __restrict__ base, L l) {
-  const SvdSector s = l.template list<SvdSector>()[blockIdx.x];
-  const int kp = s.nb * kSvdBlock;
-  double* W = base + s.w_off;
-  const int wave = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int nw = gridDim.y * (blockDim.x >> 6);
-  for (int c = wave; c < kp; c += nw)
-    for (int r = lane; r < kp; r += 64) W[int64_t(c) * kp + r] = (r == c) ? 1.0 : 0.0;
+__global__ __launch_bounds__(256) void k_svd_prepare(double* __restrict__ base, L l) {
+  const SvdPrep s = l.template list<SvdPrep>()[blockIdx.x];
+  const int t0 = blockIdx.y * blockDim.x + threadIdx.x, step = gridDim.y * blockDim.x;
+  const int64_t ny = int64_t(s.ell) * s.kp;
+  for (int64_t e = t0; e < ny; e += step) {
+    base[s.y_off + e] = 0.0;
+    if (s.y2_off >= 0) base[s.y2_off + e] = 0.0;
+  }
+  const uint32_t kp = s.kp, nw = kp * kp;  // k is far below 2^16
+  for (uint32_t e = t0; e < nw; e += step) {
+    const double v = e % (kp + 1) == 0 ? 1.0 : 0.0;
+    base[s.w_off + e] = v;
+    if (s.w2_off >= 0) base[s.w2_off + e] = v;
+  }
 }
 
-void svd_init_w(hipStream_t st, double* base, const Lists& secs, int nsec) {
+void svd_prepare(hipStream_t st, double* base, const Lists& secs, int nsec, int64_t max_elems) {
   if (nsec <= 0) return;
-  launch_lists(k_svd_init_w<DevLists>, k_svd_init_w<ArgLists>, secs, dim3(nsec, 16), dim3(256), 0, st, base);
+  const int ny = int(std::min<int64_t>(std::max<int64_t>(max_elems / 2048, 4), 128));  // about 8 elements a thread
+  launch_lists(k_svd_prepare<DevLists>, k_svd_prepare<ArgLists>, secs, dim3(nsec, ny), dim3(256), 0, st, base);
 }
 
 __device__ __forceinline__ int circle_block(int pos, int round, int nb) {

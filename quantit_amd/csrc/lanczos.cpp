@@ -272,7 +272,7 @@ LanczosResult lanczos_ground(const BTensor& theta, const BTensor& W, const BTens
         }
       launch_copies(ctx, ab, cp, tasks, "lanczos_scatter");
     }
-    const bool one_launch = kern::krylov_step_fits(lay.n, j + 1);
+    const bool one_launch = lay.n <= kern::kKrylovStepMaxN;
     if (one_launch) {
       KernelTimer kt(*ctx, "lanczos_step");
       kern::krylov_step(ctx->stream(), ab, voff(0), lay.n, j, K, woff(), lay.n, t_off, nrm2, out, host);

@@ -445,28 +445,9 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
     s.v_off = ob + B.v_off[i];
     s.s_off = ob + B.s_off[i];
   }
-  // gather: zero the Y matrices, then copy every block into its sector slot
+  // gather: every block into its sector slot (the Y matrices are zeroed before)
   std::vector<kern::Copy2D> cp;
   std::vector<kern::ChunkTask> tasks;
-  for (int i = 0; i < ns; ++i) {
-    const auto& s = B.secs[i];
-    const int64_t kp = int64_t(s.nb) * kern::kSvdBlock;
-    kern::Copy2D z{};
-    z.src_off = -1;
-    z.dst_off = s.y_off;
-    z.rows = 1;
-    z.cols = int32_t(int64_t(s.ell) * kp);
-    z.dst_rs = 0;
-    z.dst_cs = 1;
-    add_chunks(tasks, int(cp.size()), int64_t(z.cols));
-    cp.push_back(z);
-  }
-  if (!tasks.empty()) {
-    KernelTimer kt(*ctx, "svd_zero");
-    kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
-  }
-  cp.clear();
-  tasks.clear();
   for (int i = 0; i < ns; ++i) {
     const auto& p = plans[i];
     const auto& s = B.secs[i];
@@ -495,16 +476,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       cp.push_back(c);
     }
   }
-  if (!tasks.empty()) {
-    KernelTimer kt(*ctx, "svd_gather");
-    kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
-  }
   if (ns == 0) return B;
-  {
-    const kern::Lists d_secs = ctx->lists(B.secs);
-    KernelTimer kt(*ctx, "svd_init");
-    kern::svd_init_w(ctx->stream(), ab, d_secs, ns);
-  }
   int max_ell = 0;
   for (auto& s : B.secs) max_ell = std::max(max_ell, s.ell);
   const double tol = 8.0 * std::sqrt(double(std::max(max_ell, 16))) * DBL_EPSILON;
@@ -541,15 +513,35 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       B.wide[i] = 1;
     }
   }
-  if (eigh_mode) {  // the one-group solver chooses its sectors' shifts itself
-    std::vector<kern::SvdSector> by_norm;
+  // every launch of the start: work matrices cleared, blocks gathered
+  auto start = [&](const std::vector<int64_t>& y2, const std::vector<int64_t>& w2) {
+    std::vector<kern::SvdPrep> prep;
+    int64_t most = 0;
+    for (int i = 0; i < ns; ++i) {
+      const auto& s = B.secs[i];
+      const int kp = s.nb * kern::kSvdBlock;
+      prep.push_back({s.y_off, s.w_off, y2[i], w2[i], s.ell, kp});
+      most = std::max(most, int64_t(std::max(s.ell, kp)) * kp);
+    }
+    {
+      KernelTimer kt(*ctx, "svd_init");
+      kern::svd_prepare(ctx->stream(), ab, ctx->lists(prep), ns, most);
+    }
+    if (!tasks.empty()) {
+      KernelTimer kt(*ctx, "svd_gather");
+      kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
+    }
+    if (!eigh_mode) return;
+    std::vector<kern::SvdSector> by_norm;  // the one-group solver chooses its sectors' shifts itself
     for (int i = 0; i < ns; ++i)
       if (large[i] || std::find(wide.begin(), wide.end(), i) == wide.end()) by_norm.push_back(B.secs[i]);
     if (!by_norm.empty()) {
       KernelTimer kt(*ctx, "svd_init");
       kern::svd_shift(ctx->stream(), ab, ctx->lists(by_norm), int(by_norm.size()), true);
     }
-  }
+  };
+  std::vector<int64_t> y2_of(ns, -1), w2_of(ns, -1);
+  if (wide.empty()) start(y2_of, w2_of);
   if (!wide.empty()) {
     const int nw = int(wide.size());
     int kmax_large = 0;
@@ -595,37 +587,18 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
     BufPtr gbuf = ctx->alloc(size_t(elems) * sizeof(double));
     keep.push_back(gbuf);
     const int64_t gb = gbuf->dptr() - ab;
-    {  // ping-pong partners: Y2 zero (padding columns stay zero), W2 identity
-      std::vector<kern::Copy2D> z;
-      std::vector<kern::ChunkTask> zt;
-      std::vector<kern::SvdSector> wi;
-      for (int q = 0; q < nw; ++q) {
-        const auto& s = B.secs[wide[q]];
-        const int64_t kp = int64_t(s.nb) * kern::kSvdBlock;
-        kern::Copy2D c{};
-        c.src_off = -1;
-        c.dst_off = gb + y2o[q];
-        c.rows = 1;
-        c.cols = int32_t(int64_t(s.ell) * kp);
-        c.dst_cs = 1;
-        add_chunks(zt, int(z.size()), int64_t(c.cols));
-        z.push_back(c);
-        kern::SvdSector w = s;
-        w.w_off = gb + w2o[q];
-        wi.push_back(w);
-      }
-      KernelTimer kt(*ctx, "svd_init");
-      kern::copy2d(ctx->stream(), ab, ctx->lists(z, zt), int(zt.size()));
-      kern::svd_init_w(ctx->stream(), ab, ctx->lists(wi), nw);
-    }
     std::vector<int64_t> alt_y(nw), alt_w(nw);
     for (int q = 0; q < nw; ++q) {
-      alt_y[q] = gb + y2o[q];
-      alt_w[q] = gb + w2o[q];
+      alt_y[q] = y2_of[wide[q]] = gb + y2o[q];  // ping-pong partners
+      alt_w[q] = w2_of[wide[q]] = gb + w2o[q];
     }
-    BufPtr fbuf = ctx->alloc(size_t(2 * nw) * sizeof(int32_t));
+    start(y2_of, w2_of);
+    // the one-group solver stores its flags where the host reads them; the wide
+    // sectors' test adds its counts up, in device memory
+    int32_t* const h_pin = kmax_large ? nullptr : ctx->pinned_ints(size_t(2 * nw));
+    BufPtr fbuf = h_pin ? nullptr : ctx->alloc(size_t(2 * nw) * sizeof(int32_t));
     keep.push_back(fbuf);
-    int32_t* d_flags = reinterpret_cast<int32_t*>(fbuf->cptr());
+    int32_t* d_flags = h_pin ? h_pin : reinterpret_cast<int32_t*>(fbuf->cptr());
     std::vector<int32_t> h_flags(size_t(2 * nw), 0);
     std::vector<int> act(nw), corr;
     std::iota(act.begin(), act.end(), 0);
@@ -677,7 +650,11 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         kern::sum_parts(ctx->stream(), ab, ctx->lists(sums, st), int(st.size()));
       }
     };
-    auto read_flags = [&] { ctx->read_small(h_flags.data(), d_flags, size_t(2 * nw) * sizeof(int32_t)); };
+    auto read_flags = [&] {
+      if (!h_pin) return ctx->read_small(h_flags.data(), d_flags, size_t(2 * nw) * sizeof(int32_t));
+      ctx->sync();
+      std::copy(h_pin, h_pin + 2 * nw, h_flags.begin());
+    };
     auto retire = [&](std::vector<int>& qs) {  // drop converged sectors after a flag read
       std::vector<int> next;
       for (int q : qs) {
@@ -1177,7 +1154,8 @@ BTensor truncate_units(BTensor&& d_in, const std::vector<BTensor*>& units, size_
   int64_t n2 = 1;
   while (n2 < total) n2 <<= 1;
   BufPtr scratch = ctx->alloc(size_t(n2 + 1) * sizeof(double) + size_t(nd) * sizeof(int32_t) + 256);
-  int32_t* d_kept = reinterpret_cast<int32_t*>(scratch->cptr() + size_t(n2 + 1) * sizeof(double));
+  int32_t* const h_pin = ctx->pinned_ints(size_t(nd));
+  int32_t* d_kept = h_pin ? h_pin : reinterpret_cast<int32_t*>(scratch->cptr() + size_t(n2 + 1) * sizeof(double));
   double* d_thr = scratch->dptr() + n2;
   const int64_t clamp = std::numeric_limits<int64_t>::max();
   {
@@ -1186,7 +1164,12 @@ BTensor truncate_units(BTensor&& d_in, const std::vector<BTensor*>& units, size_
                           int64_t(std::min<size_t>(max_size, size_t(clamp))), d_kept, d_thr);
   }
   std::vector<int32_t> kept(nd);
-  ctx->read_small(kept.data(), d_kept, size_t(nd) * sizeof(int32_t));
+  if (h_pin) {
+    ctx->sync();
+    std::copy(h_pin, h_pin + nd, kept.begin());
+  } else {
+    ctx->read_small(kept.data(), d_kept, size_t(nd) * sizeof(int32_t));
+  }
   if (before_copy) {
     std::vector<int32_t> kept_sec(d.shape.secs[0].size(), 0);
     for (int i = 0; i < nd; ++i) kept_sec[d.blocks[i].idx.i[0]] = kept[i];

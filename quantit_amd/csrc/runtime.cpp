@@ -87,7 +87,11 @@ Context::Context(int device, size_t arena_bytes, size_t stage_bytes) : device_(d
   dev_stage_ = alloc(stage_cap_);
   for (auto& e : read_ev_) QTT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   QTT_HIP(hipEventCreateWithFlags(&sync_ev_, hipEventDisableTiming));
-  QTT_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_small_), kSmallBytes, hipHostMallocDefault));
+  QTT_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_small_), kSmallBytes + kResultInts * sizeof(int32_t),
+                        hipHostMallocDefault));
+  counter_buf_ = alloc(sizeof(int));
+  dot_counter_ = reinterpret_cast<int*>(counter_buf_->cptr());
+  kern::fill_i32(stream_, dot_counter_, 1, 0);
 }
 
 Context::~Context() {
@@ -103,6 +107,7 @@ Context::~Context() {
   if (host_read_) (void)hipHostFree(host_read_);
   if (host_small_) (void)hipHostFree(host_small_);
   dev_stage_.reset();
+  counter_buf_.reset();
   arena_.reset();
   if (host_stage_) (void)hipHostFree(host_stage_);
   if (side_) (void)hipStreamDestroy(side_);

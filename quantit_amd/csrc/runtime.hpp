@@ -130,6 +130,14 @@ class Context {
   int32_t* pinned_flag() { return host_small_; }
   // Four pinned doubles that a kernel may store to; valid likewise.
   double* pinned_doubles() { return reinterpret_cast<double*>(host_small_) + 4; }
+  // Pinned words that kernels store results to for the host to read after its
+  // next wait (null: more than there are); each use ends with that read.
+  int32_t* pinned_ints(size_t n) {
+    return n <= kResultInts ? host_small_ + kSmallBytes / sizeof(int32_t) : nullptr;
+  }
+  // Device counter of the one-launch reductions (zero between launches of the
+  // main stream).
+  int* dot_counter() const { return dot_counter_; }
   void reserve_read(size_t n_per_slot);
   int32_t* read_slot(int slot) const { return host_read_ + size_t(slot) * read_cap_; }
   hipEvent_t read_event(int slot) const { return read_ev_[slot]; }
@@ -190,6 +198,9 @@ class Context {
   std::vector<Pending> pending_;
   int32_t* host_small_ = nullptr;  // word 0: pinned_flag; byte 32: pinned_doubles; from byte 256: read_small
   static constexpr size_t kSmallBytes = size_t(64) << 10;
+  static constexpr size_t kResultInts = size_t(16) << 10;  // pinned_ints, behind the small reads
+  BufPtr counter_buf_;
+  int* dot_counter_ = nullptr;
   int32_t* host_read_ = nullptr;
   size_t read_cap_ = 0;  // words per slot
   hipEvent_t read_ev_[2] = {nullptr, nullptr};

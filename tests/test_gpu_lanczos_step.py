@@ -1,9 +1,9 @@
 """The Lanczos step in one launch against exact diagonalisation: vectors of
 each width class (at full bond the two-site space of the middle bond is the
-whole charge sector: 252, 924, 3432 states), and counts of Krylov vectors at
-which one solve goes on from the single launch to the launches over all CUs
-(n m > 2^16 at 20 vectors of 3432).  A converged solve's energy is the lowest
-eigenvalue; the bound is the other solves' 1e-10."""
+whole charge sector: 252, 924, 3432 states) with few and many Krylov vectors,
+and of more than 8192 elements at the last, where the steps of wide bonds go in
+launches over all CUs and those of the others in one.  A converged solve's energy
+is the lowest eigenvalue; the bound is the other solves' 1e-10."""
 import itertools
 
 import numpy as np
@@ -37,7 +37,7 @@ def _exact(L, delta, fields):
     return eigsh(h, k=1, which="SA", tol=0)[0][0]
 
 
-@pytest.mark.parametrize("L,bond,krylov", [(10, 32, 4), (12, 64, 9), (14, 128, 6), (14, 128, 40)])
+@pytest.mark.parametrize("L,bond,krylov", [(10, 32, 4), (12, 64, 9), (14, 128, 6), (14, 128, 40), (16, 256, 8)])
 def test_converged_solve_is_exact(ctx, L, bond, krylov):
     import quantit_amd as qa
     rng = np.random.default_rng(L + krylov)
