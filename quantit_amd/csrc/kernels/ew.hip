@@ -122,26 +122,46 @@ void permute_copy(hipStream_t s, double* base, const Lists& l, int ntasks) {
   launch_lists(k_permute<DevLists>, k_permute<ArgLists>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[1]);
 }
 
+// A task's elements: thread i takes start + i, + 256, ...  Its kPer loads are
+// issued before the first result is used (an element past the end repeats the
+// last): one after the other they are a chain of memory latencies, which is
+// what bounds launches of this size.  At the products of a D = 1024 cylinder
+// site sum_parts took 18.9 us and takes 9.0, copies and sums 5.2 -> 4.9 and a
+// dot's partials 5.7 -> 4.5; a dot of 20 k elements in one launch 7.4 -> 5.3
+// (together with block_sum, whose tree in LDS had eight barriers).
+// No task has no elements: a descriptor of numel elements has ceil(numel /
+// kChunk) of them.
+constexpr int kPer = kChunk / 256;
+struct Chunk {
+  int64_t first, end;
+  __device__ Chunk(const ChunkTask& t, int64_t numel)
+      : first(int64_t(t.chunk) * kChunk + threadIdx.x), end(min(int64_t(t.chunk + 1) * kChunk, numel)) {}
+  __device__ bool has(int u) const { return first + u * 256 < end; }
+  __device__ int64_t at(int u) const { return min(first + u * 256, end - 1); }
+};
+
 template <class L>
 __global__ __launch_bounds__(256) void k_copy2d(double* __restrict__ base, L l, uint32_t tasks) {
   const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
   const Copy2D d = l.template list<Copy2D>()[t.desc];
   const int64_t numel = int64_t(d.rows) * d.cols;
-  const int64_t start = int64_t(t.chunk) * kChunk;
-  const int64_t end = min(start + int64_t(kChunk), numel);
+  const Chunk c(t, numel);
   double* dst = base + d.dst_off;
-  if (d.src_off < 0) {
-    for (int64_t e = start + threadIdx.x; e < end; e += blockDim.x) {
-      const int64_t r = e / d.cols, c = e - r * d.cols;
-      dst[r * d.dst_rs + c * d.dst_cs] = d.alpha;
-    }
-    return;
+  const double* src = base + (d.src_off < 0 ? 0 : d.src_off);
+  int64_t to[kPer];
+  double v[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int64_t e = c.at(u);
+    int64_t r = 0;
+    if (d.rows > 1) r = numel < (int64_t(1) << 31) ? int64_t(uint32_t(e) / uint32_t(d.cols)) : e / d.cols;
+    const int64_t q = e - r * d.cols;
+    to[u] = r * d.dst_rs + q * d.dst_cs;
+    v[u] = d.src_off < 0 ? 1.0 : src[r * d.src_rs + q * d.src_cs];
   }
-  const double* src = base + d.src_off;
-  for (int64_t e = start + threadIdx.x; e < end; e += blockDim.x) {
-    const int64_t r = e / d.cols, c = e - r * d.cols;
-    dst[r * d.dst_rs + c * d.dst_cs] = d.alpha * src[r * d.src_rs + c * d.src_cs];
-  }
+#pragma unroll
+  for (int u = 0; u < kPer; ++u)
+    if (c.has(u)) dst[to[u]] = d.alpha * v[u];
 }
 
 // dst[i] = sum over s < parts of src[s * n + i] (fixed order): the reduction of
@@ -151,13 +171,22 @@ __global__ __launch_bounds__(256) void k_sum_parts(double* __restrict__ base, L 
                                                    uint32_t tasks) {
   const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
   const SumParts d = l.template list<SumParts>(descs)[t.desc];
-  const int64_t i0 = int64_t(t.chunk) * kChunk;
-  const int64_t i1 = i0 + kChunk < d.n ? i0 + kChunk : d.n;
-  for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-    double v = 0.0;
-    for (int p = 0; p < d.parts; ++p) v += base[d.src_off + p * d.n + i];
-    base[d.dst_off + i] = v;
+  const Chunk c(t, d.n);
+  double v[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) v[u] = 0.0;
+  const double* src = base + d.src_off;
+#pragma unroll 2
+  for (int p = 0; p < d.parts; ++p, src += d.n) {
+    double x[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) x[u] = src[c.at(u)];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) v[u] += x[u];
   }
+#pragma unroll
+  for (int u = 0; u < kPer; ++u)
+    if (c.has(u)) base[d.dst_off + c.at(u)] = v[u];
 }
 
 void sum_parts(hipStream_t s, double* base, const Lists& l, int ntasks, int first) {
@@ -175,24 +204,26 @@ template <class L>
 __global__ __launch_bounds__(256) void k_ew_binary(double* __restrict__ base, L l, uint32_t tasks, int op, double min_abs) {
   const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
   const EwDesc d = l.template list<EwDesc>()[t.desc];
-  const int64_t start = int64_t(t.chunk) * kChunk;
-  const int64_t end = min(start + int64_t(kChunk), d.numel);
+  const Chunk c(t, d.numel);
   const double* x = base + d.x_off;
   const double* y = base + d.y_off;
   double* out = base + d.out_off;
-  if (d.mode == 0) {
-    const double yv = y[0];
-    const bool skip = (op == 1) && (fabs(yv) < min_abs);
-    for (int64_t e = start + threadIdx.x; e < end; e += blockDim.x)
-      out[e] = skip ? x[e] : (op == 0 ? x[e] * yv : x[e] / yv);
-  } else if (d.mode == 1) {
-    for (int64_t e = start + threadIdx.x; e < end; e += blockDim.x) {
-      const double yv = y[e % d.ncol];
-      out[e] = op == 0 ? x[e] * yv : x[e] / yv;
-    }
-  } else {
-    for (int64_t e = start + threadIdx.x; e < end; e += blockDim.x) out[e] = op == 0 ? x[e] * y[e] : x[e] / y[e];
+  double xv[kPer], yv[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int64_t e = c.at(u);
+    xv[u] = x[e];
+    if (d.mode == 0)
+      yv[u] = y[0];
+    else if (d.mode == 1)
+      yv[u] = y[d.numel < (int64_t(1) << 31) ? int64_t(uint32_t(e) % uint32_t(d.ncol)) : e % d.ncol];
+    else
+      yv[u] = y[e];
   }
+  const bool skip = d.mode == 0 && op == 1 && fabs(yv[0]) < min_abs;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u)
+    if (c.has(u)) out[c.at(u)] = skip ? xv[u] : op == 0 ? xv[u] * yv[u] : xv[u] / yv[u];
 }
 
 void ew_binary(hipStream_t s, double* base, const Lists& l, int ntasks, int op,
@@ -206,25 +237,23 @@ __global__ __launch_bounds__(256) void k_axpby(double* __restrict__ base, L l, u
                                                int64_t b_off, double b) {
   const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
   const AxpbyDesc d = l.template list<AxpbyDesc>()[t.desc];
-  const int64_t start = int64_t(t.chunk) * kChunk;
-  const int64_t end = min(start + int64_t(kChunk), d.numel);
+  const Chunk c(t, d.numel);
   const double av = a_off >= 0 ? base[a_off] : a;
   const double bv = b_off >= 0 ? base[b_off] : b;
   double* out = base + d.out_off;
   const double* x = d.x_off >= 0 ? base + d.x_off : nullptr;
   const double* y = d.y_off >= 0 ? base + d.y_off : nullptr;
-  for (int64_t e = start + threadIdx.x; e < end; e += blockDim.x) {
-    double v;
-    if (x && y) {
-      const double px = av * x[e];
-      const double py = bv * y[e];
-      v = px + py;
-    } else if (x) {
-      v = av * x[e];
-    } else {
-      v = bv * y[e];
-    }
-    out[e] = v;
+  double xv[kPer], yv[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const int64_t e = c.at(u);
+    xv[u] = x ? x[e] : 0.0;
+    yv[u] = y ? y[e] : 0.0;
+  }
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const double px = av * xv[u], py = bv * yv[u];
+    if (c.has(u)) out[c.at(u)] = x && y ? px + py : x ? px : py;
   }
 }
 
@@ -234,38 +263,45 @@ void axpby(hipStream_t s, double* base, const Lists& l, int ntasks, int64_t a_of
   launch_lists(k_axpby<DevLists>, k_axpby<ArgLists>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[1], a_off, a, b_off, b);
 }
 
-// Block-wide sum in fixed order (deterministic).
+// Block-wide sum in fixed order (deterministic): the waves' sums by lane
+// exchanges, then the four of them.
 __device__ double block_sum(double v, double* sh) {
-  const int tid = threadIdx.x;
-  sh[tid] = v;
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if (tid < w) sh[tid] += sh[tid + w];
-    __syncthreads();
-  }
-  const double r = sh[0];
+  const double r = (sh[0] + sh[1]) + (sh[2] + sh[3]);
   __syncthreads();
   return r;
 }
 
+// A thread's part of a task of a dot product.
+__device__ __forceinline__ double chunk_dot(const double* __restrict__ base, const DotDesc& d, const ChunkTask& t) {
+  const Chunk c(t, d.numel);
+  double x[kPer], y[kPer], acc = 0.0;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    x[u] = base[d.x_off + c.at(u)];
+    y[u] = base[d.y_off + c.at(u)];
+  }
+#pragma unroll
+  for (int u = 0; u < kPer; ++u)
+    if (c.has(u)) acc += x[u] * y[u];
+  return acc;
+}
+
 template <class L>
 __global__ __launch_bounds__(256) void k_dot_partial(double* __restrict__ base, L l, uint32_t tasks, int64_t partial_off) {
-  __shared__ double sh[256];
+  __shared__ double sh[4];
   const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
   const DotDesc d = l.template list<DotDesc>()[t.desc];
-  const int64_t start = int64_t(t.chunk) * kChunk;
-  const int64_t end = min(start + int64_t(kChunk), d.numel);
-  const double* x = base + d.x_off;
-  const double* y = base + d.y_off;
-  double acc = 0.0;
-  for (int64_t e = start + threadIdx.x; e < end; e += blockDim.x) acc += x[e] * y[e];
+  const double acc = chunk_dot(base, d, t);
   const double r = block_sum(acc, sh);
   if (threadIdx.x == 0) base[partial_off + blockIdx.x] = r;
 }
 
 __global__ __launch_bounds__(256) void k_dot_final(double* __restrict__ base, int64_t partial_off, int n,
                                                    int64_t out_off, int sqrt_out) {
-  __shared__ double sh[256];
+  __shared__ double sh[4];
   double acc = 0.0;
   for (int i = threadIdx.x; i < n; i += blockDim.x) acc += base[partial_off + i];
   const double r = block_sum(acc, sh);
@@ -282,20 +318,19 @@ constexpr int kDotOneLaunch = 64;
 template <class L>
 __global__ __launch_bounds__(256) void k_dot(double* __restrict__ base, L l, uint32_t tasks, int64_t partial_off,
                                              int64_t out_off, int sqrt_out, int* __restrict__ done) {
-  __shared__ double sh[256];
+  __shared__ double sh[4];
   __shared__ int last;
   const int n = gridDim.x;
   double* partial = base + partial_off;
   {
     const ChunkTask t = l.template list<ChunkTask>(tasks)[blockIdx.x];
     const DotDesc d = l.template list<DotDesc>()[t.desc];
-    const int64_t start = int64_t(t.chunk) * kChunk;
-    const int64_t end = min(start + int64_t(kChunk), d.numel);
-    const double* x = base + d.x_off;
-    const double* y = base + d.y_off;
-    double acc = 0.0;
-    for (int64_t e = start + threadIdx.x; e < end; e += blockDim.x) acc += x[e] * y[e];
+    const double acc = chunk_dot(base, d, t);
     const double r = block_sum(acc, sh);
+    if (n == 1) {  // uniform
+      if (threadIdx.x == 0) base[out_off] = sqrt_out ? sqrt(r) : r;
+      return;
+    }
     if (threadIdx.x == 0) {
       __hip_atomic_store(&partial[blockIdx.x], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       last = __hip_atomic_fetch_add(done, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
@@ -353,7 +388,7 @@ void eig2x2(hipStream_t s, double* base, int64_t a0_off, int64_t a1_off, int64_t
 }
 
 __global__ __launch_bounds__(256) void k_normalize(double* __restrict__ base, int64_t off, int64_t n) {
-  __shared__ double sh[256];
+  __shared__ double sh[4];
   double* d = base + off;
   double acc = 0.0;
   for (int64_t i = threadIdx.x; i < n; i += blockDim.x) acc += d[i] * d[i];
