@@ -281,18 +281,12 @@ BTensor inverse_cvals(const BTensor& t) {
 
 BTensor conj(const BTensor& t) { return inverse_cvals(t); }
 
-static void chunk_tasks(std::vector<kern::ChunkTask>& tasks, int desc, int64_t numel) {
-  const int64_t nch = (numel + kern::kChunk - 1) / kern::kChunk;
-  for (int64_t c = 0; c < nch; ++c) tasks.push_back({desc, int32_t(c)});
-}
-
 BTensor clone(const BTensor& t) {
   BTensor out(t.ctx, t.shape);
   std::vector<BIdx> idx;
   for (auto& b : t.blocks) idx.push_back(b.idx);
   out.allocate(idx);
   std::vector<kern::Copy2D> cp;
-  std::vector<kern::ChunkTask> tasks;
   double* ab = reinterpret_cast<double*>(t.ctx->arena().base());
   for (size_t k = 0; k < t.blocks.size(); ++k) {
     const auto& b = t.blocks[k];
@@ -305,10 +299,10 @@ BTensor clone(const BTensor& t) {
     c.src_rs = c.dst_rs = b.numel;
     c.src_cs = c.dst_cs = 1;
     c.alpha = 1.0;
-    chunk_tasks(tasks, int(cp.size()), b.numel);
-    cp.push_back(c);
+    kern::add_run(cp, c);
   }
-  if (!tasks.empty()) {
+  if (!cp.empty()) {
+    const std::vector<kern::ChunkTask> tasks = kern::chunk_tasks(cp);
     KernelTimer kt(*t.ctx, "copy2d");
     kern::copy2d(t.ctx->stream(), ab, t.ctx->lists(cp, tasks), int(tasks.size()));
   }

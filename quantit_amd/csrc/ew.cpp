@@ -12,11 +12,6 @@ namespace {
 
 double* arena_base(Context* c) { return reinterpret_cast<double*>(c->arena().base()); }
 
-void add_chunks(std::vector<kern::ChunkTask>& tasks, int desc, int64_t numel) {
-  const int64_t nch = (numel + kern::kChunk - 1) / kern::kChunk;
-  for (int64_t c = 0; c < nch; ++c) tasks.push_back({desc, int32_t(c)});
-}
-
 void require_same_layout(const Shape& x, const Shape& y) {
   // add_tensor_check (sources/btensor.cpp:2320-2328)
   if (x.g != y.g || x.cvals != y.cvals)
@@ -75,7 +70,6 @@ BTensor mul(const BTensor& x_in, const BTensor& y_in) {
   out.allocate(idx);
   double* ab = arena_base(ctx);
   std::vector<kern::EwDesc> descs;
-  std::vector<kern::ChunkTask> tasks;
   for (size_t k = 0; k < pairs.size(); ++k) {
     const Block& xb = x.blocks[pairs[k].xi];
     const Block& yb = y.blocks[pairs[k].yi];
@@ -96,10 +90,10 @@ BTensor mul(const BTensor& x_in, const BTensor& y_in) {
       if (sr != lr) throw InvalidArgument("unsupported broadcast");
       d.mode = 2;
     }
-    add_chunks(tasks, int(descs.size()), xb.numel);
-    descs.push_back(d);
+    kern::add_run(descs, d);
   }
-  if (!tasks.empty()) {
+  if (!descs.empty()) {
+    const std::vector<kern::ChunkTask> tasks = kern::chunk_tasks(descs);
     KernelTimer kt(*ctx, "ew_mul");
     kern::ew_binary(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), 0, 0.0);
   }
@@ -122,7 +116,6 @@ BTensor div_scalar_tensor(const BTensor& x, const BTensor& s, double min_abs) {
   }
   double* ab = arena_base(ctx);
   std::vector<kern::EwDesc> descs;
-  std::vector<kern::ChunkTask> tasks;
   for (size_t k = 0; k < x.blocks.size(); ++k) {
     if (!x.blocks[k].numel) continue;
     kern::EwDesc d{};
@@ -131,10 +124,10 @@ BTensor div_scalar_tensor(const BTensor& x, const BTensor& s, double min_abs) {
     d.out_off = out.ptr(out.blocks[k]) - ab;
     d.numel = x.blocks[k].numel;
     d.mode = 0;
-    add_chunks(tasks, int(descs.size()), d.numel);
-    descs.push_back(d);
+    kern::add_run(descs, d);
   }
-  if (!tasks.empty()) {
+  if (!descs.empty()) {
+    const std::vector<kern::ChunkTask> tasks = kern::chunk_tasks(descs);
     KernelTimer kt(*ctx, "ew_div");
     kern::ew_binary(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), 1,
                     min_abs);
@@ -176,7 +169,6 @@ BTensor merge_axpby(const BTensor& x, int64_t a_off, double a, const BTensor& y,
   out.allocate(idx);
   double* ab = arena_base(ctx);
   std::vector<kern::AxpbyDesc> descs;
-  std::vector<kern::ChunkTask> tasks;
   for (size_t k = 0; k < ents.size(); ++k) {
     const int64_t n = out.blocks[k].numel;
     if (!n) continue;
@@ -185,10 +177,10 @@ BTensor merge_axpby(const BTensor& x, int64_t a_off, double a, const BTensor& y,
     d.y_off = ents[k].yi >= 0 ? y.ptr(y.blocks[ents[k].yi]) - ab : -1;
     d.out_off = out.ptr(out.blocks[k]) - ab;
     d.numel = n;
-    add_chunks(tasks, int(descs.size()), n);
-    descs.push_back(d);
+    kern::add_run(descs, d);
   }
-  if (!tasks.empty()) {
+  if (!descs.empty()) {
+    const std::vector<kern::ChunkTask> tasks = kern::chunk_tasks(descs);
     KernelTimer kt(*ctx, "axpby");
     kern::axpby(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), a_off, a,
                 b_off, b);
@@ -233,7 +225,6 @@ BTensor full_dot(const BTensor& x, const BTensor& y, bool sqrt_out) {
   BTensor out(ctx, o);
   double* ab = arena_base(ctx);
   std::vector<kern::DotDesc> descs;
-  std::vector<kern::ChunkTask> tasks;
   const int r = x.rank();
   size_t i = 0, j = 0;
   bool any = false;
@@ -245,9 +236,7 @@ BTensor full_dot(const BTensor& x, const BTensor& y, bool sqrt_out) {
     } else {
       any = true;
       if (x.blocks[i].numel) {
-        kern::DotDesc d{x.ptr(x.blocks[i]) - ab, y.ptr(y.blocks[j]) - ab, x.blocks[i].numel};
-        add_chunks(tasks, int(descs.size()), d.numel);
-        descs.push_back(d);
+        kern::add_run(descs, kern::DotDesc{x.ptr(x.blocks[i]) - ab, y.ptr(y.blocks[j]) - ab, x.blocks[i].numel});
       }
       ++i;
       ++j;
@@ -255,6 +244,7 @@ BTensor full_dot(const BTensor& x, const BTensor& y, bool sqrt_out) {
   }
   if (!any) return out;
   out.allocate({BIdx{}});
+  const std::vector<kern::ChunkTask> tasks = kern::chunk_tasks(descs);
   BufPtr partial = ctx->alloc(std::max<size_t>(tasks.size(), 1) * sizeof(double));
   KernelTimer kt(*ctx, "dot");
   kern::dot(ctx->stream(), ab, ctx->lists(descs, tasks), int(tasks.size()), partial->dptr() - ab,
@@ -289,8 +279,7 @@ BTensor fill_like(Context* ctx, const Shape& s, double value) {
     c.dst_cs = 1;
     c.alpha = value;
     std::vector<kern::Copy2D> cp{c};
-    std::vector<kern::ChunkTask> tasks;
-    add_chunks(tasks, 0, n);
+    const std::vector<kern::ChunkTask> tasks = kern::chunk_tasks(cp);
     KernelTimer kt(*ctx, "fill");
     kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
   }

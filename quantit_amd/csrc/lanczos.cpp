@@ -24,11 +24,6 @@ BTensor matvec_labelled(const BTensor& x, const BTensor& W, const BTensor& Lenv,
 
 namespace {
 
-void add_chunks(std::vector<kern::ChunkTask>& tasks, int desc, int64_t numel) {
-  const int64_t nch = (numel + kern::kChunk - 1) / kern::kChunk;
-  for (int64_t c = 0; c < nch; ++c) tasks.push_back({desc, int32_t(c)});
-}
-
 struct Layout {
   int rank = 0;
   std::vector<BIdx> idx;  // sorted
@@ -65,8 +60,8 @@ struct Layout {
   }
 };
 
-void launch_copies(Context* ctx, double* ab, const std::vector<kern::Copy2D>& cp,
-                   const std::vector<kern::ChunkTask>& tasks, const char* name) {
+void launch_copies(Context* ctx, double* ab, const std::vector<kern::Copy2D>& cp, const char* name) {
+  const std::vector<kern::ChunkTask> tasks = kern::chunk_tasks(cp);
   if (tasks.empty()) return;
   KernelTimer kt(*ctx, name);
   kern::copy2d(ctx->stream(), ab, ctx->lists(cp, tasks), int(tasks.size()));
@@ -181,14 +176,12 @@ LanczosResult lanczos_ground(const BTensor& theta, const BTensor& W, const BTens
   // v0 = theta / |theta|
   {
     std::vector<kern::Copy2D> cp;
-    std::vector<kern::ChunkTask> tasks;
     for (auto& b : theta.blocks) {
       if (!b.numel) continue;
       const int k = lay.find(b.idx);
-      add_chunks(tasks, int(cp.size()), b.numel);
-      cp.push_back(flat_copy(theta.ptr(b) - ab, voff(0) + lay.off[k], b.numel));
+      kern::add_run(cp, flat_copy(theta.ptr(b) - ab, voff(0) + lay.off[k], b.numel));
     }
-    launch_copies(ctx, ab, cp, tasks, "lanczos_scatter");
+    launch_copies(ctx, ab, cp, "lanczos_scatter");
     KernelTimer kt(*ctx, "lanczos_vec");
     kern::krylov_dot(ctx->stream(), ab, voff(0), lay.n, 1, voff(0), lay.n, poff(), nrm2);
     kern::krylov_axpy(ctx->stream(), ab, voff(0), lay.n, 0, nrm2, 0.0, voff(0), voff(0), lay.n, nrm2);
@@ -237,18 +230,16 @@ LanczosResult lanczos_ground(const BTensor& theta, const BTensor& W, const BTens
       const int64_t oldv = oldV->dptr() - ab;
       alloc_vectors(nl.n);
       std::vector<kern::Copy2D> cp;
-      std::vector<kern::ChunkTask> tasks;
       std::vector<char> np(nl.idx.size(), 0);
       for (size_t b = 0; b < nl.idx.size(); ++b) {
         const int k = lay.find(nl.idx[b]);
         if (k >= 0) np[b] = present[k];
         for (int r = 0; r <= j; ++r) {
-          add_chunks(tasks, int(cp.size()), nl.numel[b]);
-          cp.push_back(flat_copy(k >= 0 ? oldv + int64_t(r) * old_n + lay.off[k] : -1,
-                                 V->dptr() - ab + int64_t(r) * nl.n + nl.off[b], nl.numel[b]));
+          kern::add_run(cp, flat_copy(k >= 0 ? oldv + int64_t(r) * old_n + lay.off[k] : -1,
+                                      V->dptr() - ab + int64_t(r) * nl.n + nl.off[b], nl.numel[b]));
         }
       }
-      launch_copies(ctx, ab, cp, tasks, "lanczos_regrow");
+      launch_copies(ctx, ab, cp, "lanczos_regrow");
       lay = nl;
       present.swap(np);
       for (size_t q = 0; q < o.blocks.size(); ++q) where[q] = o.blocks[q].numel ? lay.find(o.blocks[q].idx) : 0;
@@ -256,21 +247,18 @@ LanczosResult lanczos_ground(const BTensor& theta, const BTensor& W, const BTens
     // w = H v_j in the layout (absent blocks zero)
     {
       std::vector<kern::Copy2D> cp;
-      std::vector<kern::ChunkTask> tasks;
       std::vector<char> hit(lay.idx.size(), 0);
       for (size_t q = 0; q < o.blocks.size(); ++q) {
         if (!o.blocks[q].numel) continue;
         const int k = where[q];
         hit[k] = 1;
-        add_chunks(tasks, int(cp.size()), lay.numel[k]);
-        cp.push_back(flat_copy(o.ptr(o.blocks[q]) - ab, woff() + lay.off[k], lay.numel[k]));
+        kern::add_run(cp, flat_copy(o.ptr(o.blocks[q]) - ab, woff() + lay.off[k], lay.numel[k]));
       }
       for (size_t k = 0; k < lay.idx.size(); ++k)
         if (!hit[k]) {
-          add_chunks(tasks, int(cp.size()), lay.numel[k]);
-          cp.push_back(flat_copy(-1, woff() + lay.off[k], lay.numel[k]));
+          kern::add_run(cp, flat_copy(-1, woff() + lay.off[k], lay.numel[k]));
         }
-      launch_copies(ctx, ab, cp, tasks, "lanczos_scatter");
+      launch_copies(ctx, ab, cp, "lanczos_scatter");
     }
     const bool one_launch = lay.n <= kern::kKrylovStepMaxN;
     if (one_launch) {
@@ -320,13 +308,11 @@ LanczosResult lanczos_ground(const BTensor& theta, const BTensor& W, const BTens
   t2.allocate(keep);
   {
     std::vector<kern::Copy2D> cp;
-    std::vector<kern::ChunkTask> tasks;
     for (auto& b : t2.blocks) {
       const int k = lay.find(b.idx);
-      add_chunks(tasks, int(cp.size()), b.numel);
-      cp.push_back(flat_copy(woff() + lay.off[k], t2.ptr(b) - ab, b.numel));
+      kern::add_run(cp, flat_copy(woff() + lay.off[k], t2.ptr(b) - ab, b.numel));
     }
-    launch_copies(ctx, ab, cp, tasks, "lanczos_scatter");
+    launch_copies(ctx, ab, cp, "lanczos_scatter");
   }
   res.theta = std::move(t2);
   Shape rank0;

@@ -38,3 +38,26 @@ def test_sums_of_split_products(ctx, m, n, k):
     a, b = _tensor(rng, (k, m)), _tensor(rng, (k, n))
     got = from_dev(to_dev(ctx, a).tensordot(to_dev(ctx, b), [0], [0]))
     assert np.array_equal(got.blocks[(0, 0)], bo.tensordot(a, b, [0], [0]).blocks[(0, 0)])
+
+
+# blocks that only one operand has break a run, at its ends and inside
+@pytest.mark.parametrize("has_x,has_y", [("11111111", "11111111"), ("11111111", "01111110"), ("10110111", "11101101"),
+                                         ("10101010", "01010101"), ("00001111", "11111111"), ("10000000", "00000001")])
+@pytest.mark.parametrize("size", [(3, 2), (40, 30)])
+def test_runs_of_blocks(ctx, has_x, has_y, size):
+    rng = np.random.default_rng(int(has_x, 2) * 256 + int(has_y, 2))
+    ops = []
+    for has in (has_x, has_y):
+        t = BTensor((0,), [[size[0]] * 8, [size[1]] * 8], [[(i,) for i in range(8)], [(-i,) for i in range(8)]], (0,))
+        for i in range(8):
+            if has[i] == "1":
+                t.blocks[(i, i)] = rng.integers(-9, 10, size).astype(float)
+        ops.append(t)
+    x, y = ops
+    one = _tensor(rng, ())
+    dx, dy, done = to_dev(ctx, x), to_dev(ctx, y), to_dev(ctx, one)
+    for got, want in [(dx.add(dy, 3.0), bo.add(x, y, 3.0)), (dx.mul(dy), bo.mul(x, y)), (dx.mul(done), bo.mul(x, one))]:
+        got = from_dev(got)
+        assert sorted(got.blocks) == sorted(want.blocks)
+        assert all(np.array_equal(got.blocks[k], want.blocks[k]) for k in want.blocks)
+    assert dx.full_dot(dy) == sum(float((x.blocks[k] * y.blocks[k]).sum()) for k in x.blocks if k in y.blocks)
