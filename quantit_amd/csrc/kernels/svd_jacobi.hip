@@ -1477,6 +1477,7 @@ size_t gram_eig_lds_limit() {
 }
 
 // ---- finalize ----------------------------------------------------------------
+constexpr int kFinishMaxK = 64, kFinishMaxEll = 256, kFinishMaxTasks = 256;
 // aux = base + w_off + kp*kp holds 2*kp + ell doubles: column norms, ranks and
 // the completion vector.
 
@@ -1615,6 +1616,94 @@ __global__ __launch_bounds__(256) void k_svd_write(double* __restrict__ base, L 
   }
 }
 
+// Norms, ranks and the scatter in one launch for calls whose sectors are all
+// narrow (kFinishMaxK columns, kFinishMaxEll rows): every tile's work-group
+// forms the norms and ranks it needs itself from Y, which it or a neighbour
+// reads anyway, and the tile's own loads are in flight meanwhile.  The same
+// bits in every work-group; the first tile of a sector stores its values.
+// Bound by one chain of memory latencies instead of three with two launches
+// between them: 7 sectors of 30 x 60 7.6 us against 12.1, 9 of 64 x 64 8.0
+// against 15.3, of 64 x 256 9.8 against 15.7.  More tiles than work-groups
+// run at once pay for the repeated norms (60 sectors of 64 x 256, 300 tiles:
+// 16.3 against 17.7; 200, 1000 tiles: 34.6 against 27.7): kFinishMaxTasks.
+template <class L>
+__global__ __launch_bounds__(256) void k_svd_finish(double* __restrict__ base, L l, uint32_t tasks) {
+  __shared__ double tile[64][65];
+  __shared__ double sig[kFinishMaxK], scl[kFinishMaxK], smax;
+  __shared__ int less[4][kFinishMaxK], perm[kFinishMaxK];
+  const int4 t = l.template list<int4>(tasks)[blockIdx.x];
+  const SvdSector s = l.template list<SvdSector>()[t.x];
+  const int k = s.k, ell = s.ell, kp = s.nb * kSvdBlock;
+  const bool zpart = t.y == 0;
+  const int rows = zpart ? ell : k, ld = zpart ? ell : kp;
+  const double* Y = base + s.y_off;
+  const double* src = base + (zpart ? s.y_off : s.w_off);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r0 = t.z;
+  double v[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = src[min(wave + 4 * i, k - 1) * ld + min(r0 + lane, rows - 1)];
+  // columns 16 wave .. + 15: lane sums, then a butterfly that halves the
+  // columns a lane holds; column 16 wave + (lane >> 2) is left
+  double acc[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) acc[c] = 0.0;
+  if (16 * wave < k)
+    for (int r = lane; r < ell; r += 64) {
+      double x[16];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) x[c] = Y[min(16 * wave + c, k - 1) * ell + r];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) acc[c] = fma(x[c], x[c], acc[c]);
+    }
+#pragma unroll
+  for (int h = 8; h > 0; h >>= 1) {
+    const bool up = lane & (4 * h);
+#pragma unroll
+    for (int c = 0; c < h; ++c) {
+      const double keep = up ? acc[c + h] : acc[c], give = up ? acc[c] : acc[c + h];
+      acc[c] = keep + __shfl_xor(give, 4 * h);
+    }
+  }
+  acc[0] += __shfl_xor(acc[0], 2);
+  acc[0] += __shfl_xor(acc[0], 1);
+  if ((lane & 3) == 0) {
+    const int c = 16 * wave + (lane >> 2);
+    sig[c] = c < k ? sqrt(acc[0]) : -1.0;  // behind every norm
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) tile[wave + 4 * i][lane] = v[i];
+  __syncthreads();
+  const double sj = sig[lane];
+  int r = 0;
+#pragma unroll
+  for (int u = 0; u < 16; ++u) {
+    const int i = 16 * wave + u;
+    const double si = sig[i];
+    r += int(si > sj) | (int(si == sj) & int(i < lane));
+  }
+  less[wave][lane] = r;
+  __syncthreads();
+  r = less[0][lane] + less[1][lane] + less[2][lane] + less[3][lane];
+  if (wave == 0 && lane < k) {
+    perm[lane] = s.eig_shift ? k - 1 - r : r;
+    if (r == 0) smax = sj;
+    if (r0 == 0 && (zpart || s.eig_shift)) base[s.s_off + perm[lane]] = s.eig_shift ? sj - base[s.shift_off] : sj;
+  }
+  __syncthreads();
+  if (wave == 0 && lane < k) {
+    const double thr = (s.eig_shift ? 0.0 : smax) * double(ell) * DBL_EPSILON;
+    scl[lane] = !zpart ? 1.0 : sj > thr && sj > 0.0 ? 1.0 / sj : 0.0;
+  }
+  __syncthreads();
+  double* dst = base + (s.eig_shift || zpart == (s.transposed == 0) ? s.u_off : s.v_off);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int q = r0 + wave + 4 * i;
+    if (q < rows && lane < k) dst[int64_t(q) * k + perm[lane]] = tile[lane][wave + 4 * i] * scl[lane];
+  }
+}
+
 // Orthonormal completion of the Z-side columns whose singular value is
 // numerically zero, columns t < limit: starting from unit vectors, classical
 // Gram-Schmidt twice against all earlier columns (the dot products of one
@@ -1684,8 +1773,16 @@ void svd_complete(hipStream_t st, double* base, const Lists& tasks, int n) {
 
 void svd_finalize(hipStream_t st, double* base, const Lists& l, const SvdSector* host_secs, int nsec, int ntasks) {
   if (nsec <= 0) return;
-  int kmax = 1;
-  for (int i = 0; i < nsec; ++i) kmax = std::max(kmax, host_secs[i].k);
+  int kmax = 1, ellmax = 1;
+  for (int i = 0; i < nsec; ++i) {
+    kmax = std::max(kmax, host_secs[i].k);
+    ellmax = std::max(ellmax, host_secs[i].ell);
+  }
+  if (kmax <= kFinishMaxK && ellmax <= kFinishMaxEll && ntasks <= kFinishMaxTasks) {
+    if (ntasks > 0)
+      launch_lists(k_svd_finish<DevLists>, k_svd_finish<ArgLists>, l, dim3(ntasks), dim3(256), 0, st, base, l.at[1]);
+    return;
+  }
   launch_lists(k_svd_colnorms<DevLists>, k_svd_colnorms<ArgLists>, l, dim3(nsec, (kmax + 15) / 16), dim3(256), 0, st, base);
   launch_lists(k_svd_norms<DevLists>, k_svd_norms<ArgLists>, l, dim3(nsec, (kmax + kNormsWave - 1) / kNormsWave),
                dim3(kNormsWave), 0, st, base);

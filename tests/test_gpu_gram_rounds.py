@@ -124,3 +124,35 @@ def test_eigh_around_the_definite(ctx, low):
         assert np.abs(np.sort(vals) - np.linalg.eigvalsh(a)).max() <= 1e-12 * nrm
         assert np.abs(vec.T @ vec - np.eye(a.shape[0])).max() <= 1e-12
         assert np.abs(a @ vec - vec * vals).max() <= 1e-12 * nrm
+
+
+# the last pass over narrow sectors is one launch up to 64 columns, 256 rows
+# and 256 tiles: both sides of each limit, its quarters of 16 columns and its
+# 64-row tiles, values that are zero and values that tie
+@pytest.mark.parametrize("shapes,zeros", [
+    ([(1, 1)], 0), ([(16, 64), (17, 65), (4, 5)], 0), ([(63, 128), (130, 64)], 2), ([(64, 256), (255, 33)], 5),
+    ([(64, 257)], 0), ([(65, 65), (3, 3)], 0), ([(20, 190)] * 64, 3), ([(20, 190)] * 65, 0)])
+def test_svd_narrow_sectors_at_the_last_pass(ctx, shapes, zeros):
+    import quantit_amd as qa
+    rng = np.random.default_rng(len(shapes) * 1000 + shapes[0][1])
+    mats = [_graded(rng, m, n, 0 if i % 3 == 2 else 3, zeros) for i, (m, n) in enumerate(shapes)]
+    U, d, V = (from_dev(x) for x in qa.svd(to_dev(ctx, _diagonal(mats)), 1))
+    for i, a in enumerate(mats):
+        u, s, v = U.blocks[(i, i)], d.blocks[(i,)], V.blocks[(i, i)]
+        assert np.abs(s - np.linalg.svd(a, compute_uv=False)).max() <= 1e-12 * s[0]
+        assert np.linalg.norm((u * s) @ v.T - a) <= 1e-12 * np.linalg.norm(a)
+        for w in (u, v):
+            assert np.abs(w.T @ w - np.eye(w.shape[1])).max() <= 1e-12
+
+
+@pytest.mark.parametrize("sizes", [(1, 2, 16), (17, 48, 63, 64), (65, 7)])
+def test_eigh_narrow_sectors_at_the_last_pass(ctx, sizes):
+    import quantit_amd as qa
+    rng = np.random.default_rng(sum(sizes))
+    mats = [(lambda a: a + a.T)(rng.standard_normal((k, k))) for k in sizes]
+    e, U = (from_dev(x) for x in qa.eigh(to_dev(ctx, _diagonal(mats)), 1))
+    for i, a in enumerate(mats):
+        w, u = e.blocks[(i,)], U.blocks[(i, i)]
+        assert np.abs(w - np.linalg.eigvalsh(a)).max() <= 1e-12 * np.linalg.norm(a)
+        assert np.linalg.norm((u * w) @ u.T - a) <= 1e-12 * np.linalg.norm(a)
+        assert np.abs(u.T @ u - np.eye(len(w))).max() <= 1e-12
