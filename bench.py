@@ -147,15 +147,15 @@ def dmrg_opts(qa, w, sweeps):
 
 # Timers that time one kernel each (host_* are host phases; the rest group
 # several kernels behind one name or are host waits).
-SVD_WIDE_TIMERS = ("svd_round",)
+SVD_WIDE_TIMERS = ("svd_gram_round", "svd_round")
 SVD_ALL_TIMERS = ("svd_eig", "svd_eig_it1", "svd_eig_it2", "svd_eig_it3+")
 
 
 def kernel_roofline(kt, contract_flops, svd_flops, svd_flops_wide, traffic_summary):
     """Roofline object of the timer with the largest share.  Algorithmic work
     per launch: contraction timers -> sum 2 M N K of the solve over their
-    launches; k_svd_round -> the SVD model FLOPs of the sectors it rotates
-    (14 m n^2 + 8 n^3 each) over its launches; k_gram_eig -> the model FLOPs
+    launches; k_gram_round and k_svd_round -> the SVD model FLOPs of the sectors
+    they rotate (14 m n^2 + 8 n^3 each) over their launches; k_gram_eig -> the model FLOPs
     of all sectors over its launches."""
     kernels = {k: v for k, v in kt.items() if not k.startswith("host_")}
     if not kernels:
@@ -165,7 +165,8 @@ def kernel_roofline(kt, contract_flops, svd_flops, svd_flops_wide, traffic_summa
         group = [k for k in kernels if k.startswith("gemm") and k != "gemm_split_k_sum" and k != "gemm_rows"]
         work, kname, peak = contract_flops, "k_gemm_f64", PEAK_FP64_TFLOPS
     elif dom in SVD_WIDE_TIMERS:
-        group, work, kname, peak = list(SVD_WIDE_TIMERS), svd_flops_wide, "k_svd_round", PEAK_FP64_TFLOPS
+        group, work, kname, peak = [k for k in SVD_WIDE_TIMERS if k in kernels], svd_flops_wide, \
+            "k_gram_round" if dom == "svd_gram_round" else "k_svd_round", PEAK_FP64_TFLOPS
     elif dom in SVD_ALL_TIMERS:
         group, work, kname, peak = [k for k in SVD_ALL_TIMERS if k in kernels], svd_flops, "k_gram_eig", \
             PEAK_FP64_TFLOPS
