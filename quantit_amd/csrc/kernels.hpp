@@ -333,6 +333,14 @@ size_t gram_eig_lds_limit();  // largest dynamic LDS per work-group (bytes)
 // failing the orthogonality test (0: W = I).  precond: pivoted-Cholesky
 // preconditioning.
 constexpr int kGramEigMaxK = 140;
+// Up to kGramEigFew sectors of more than kGramEigFewK columns in an SVD take the
+// rounds of gram_rounds.hip instead: one work-group each leaves the chip idle,
+// while a round's launches cost the same for one sector as for several.  One
+// work-group against rounds (values over 3 and 10 decades, us): 7 sectors of
+// k = 140 1941 / 1496 and 3002 / 2592, of 113 1322 / 1227 and 2110 / 2101, of
+// 105 1363 / 1448 and 1617 / 1911; 10 of 121 over 8 decades 1951 / 2012; 24 of
+// 121 over 12 decades 2334 / 2506.
+constexpr int kGramEigFewK = 112, kGramEigFew = 8;
 void gram_eig(hipStream_t s, double* base, const Lists& descs, int n, int* flags, double tol, int max_sweeps,
               int precond, size_t lds_bytes);
 size_t gram_eig_lds_bytes(int k);

@@ -82,7 +82,7 @@ struct Batched {
   std::vector<int64_t> u_off, v_off, s_off;  // element offsets into outbuf
   int sweeps = 0;
   int unconverged = 0;  // sectors still rotating when a sweep cap was reached
-  std::vector<char> wide;  // sectors whose rotations ran as multi-work-group rounds (k_svd_round)
+  std::vector<char> wide;  // sectors whose rotations ran as multi-work-group rounds
   // defer_complete: the orthonormal completion of null columns, one task per
   // sector (scratch offsets unset), left to the caller
   std::vector<kern::CompleteTask> complete;
@@ -494,20 +494,25 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
   // W <- W W_g until G is diagonal to the tolerance (relative, or absolute
   // with respect to the largest singular value; the second case ends with
   // two Gram-Schmidt passes on the short columns).  Sectors with k <=
-  // kGramEigMaxK solve for W_g in one work-group (LDS); wider ones run the
-  // pivoted Cholesky by panels, block Jacobi rounds on L = R^T and a
-  // normalisation pass, all with G in device memory.
+  // kGramEigMaxK (a few of them: kGramEigFewK) solve for W_g in one work-group
+  // (LDS); wider ones run the pivoted Cholesky by panels, block Jacobi rounds
+  // on L = R^T and a normalisation pass, all with G in device memory.
   const size_t pchol_limit = kern::pchol_lds_limit();
   std::vector<int> wide;
   std::vector<char> large(ns, 0);
-  const int eig_max_k = std::min(kern::kGramEigMaxK, env_int("QTT_SVD_EIG_MAX_K", kern::kGramEigMaxK));
+  const bool large_gram = env_int("QTT_SVD_LARGE_GRAM", 1) != 0;
+  int eig_max_k = std::min(kern::kGramEigMaxK, env_int("QTT_SVD_EIG_MAX_K", kern::kGramEigMaxK));
+  if (!eigh_mode && large_gram) {
+    int few = 0;
+    for (auto& s : B.secs) few += s.k > kern::kGramEigFewK && s.k <= eig_max_k;
+    if (few <= kern::kGramEigFew) eig_max_k = std::min(eig_max_k, kern::kGramEigFewK);
+  }
   for (int i = 0; i < ns; ++i) {
     const auto& s = B.secs[i];
     if (!use_small || s.k < 1) continue;
     if (s.k <= eig_max_k && kern::gram_eig_lds_bytes(s.k) + lds_margin <= lds_limit) {
       wide.push_back(i);
-    } else if (size_t(s.k) * (4 + kern::kPcholExtra) * sizeof(double) <= pchol_limit &&
-               env_int("QTT_SVD_LARGE_GRAM", 1)) {
+    } else if (large_gram && size_t(s.k) * (4 + kern::kPcholExtra) * sizeof(double) <= pchol_limit) {
       wide.push_back(i);
       large[i] = 1;
       B.wide[i] = 1;

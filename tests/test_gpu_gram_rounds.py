@@ -156,3 +156,23 @@ def test_eigh_narrow_sectors_at_the_last_pass(ctx, sizes):
         assert np.abs(w - np.linalg.eigvalsh(a)).max() <= 1e-12 * np.linalg.norm(a)
         assert np.linalg.norm((u * w) @ u.T - a) <= 1e-12 * np.linalg.norm(a)
         assert np.abs(u.T @ u - np.eye(len(w))).max() <= 1e-12
+
+
+# more than eight sectors of 113 .. 140 columns stay with the solver that takes
+# a sector in one work-group, up to eight take the rounds; narrower ones beside
+# them stay
+@pytest.mark.parametrize("count", [1, 8, 9])
+@pytest.mark.parametrize("decades,zeros", [(3, 0), (12, 0), (5, 30)])
+def test_svd_few_sectors_of_medium_width(ctx, count, decades, zeros):
+    import quantit_amd as qa
+    rng = np.random.default_rng(count * 100 + decades)
+    widths = [(113, 128, 129, 140)[i % 4] for i in range(count)] + [112, 40]
+    mats = [_graded(rng, k + i % 3, k + 5 * (i % 2), decades, zeros) for i, k in enumerate(widths)]
+    U, d, V = (from_dev(x) for x in qa.svd(to_dev(ctx, _diagonal(mats)), 1))
+    for i, a in enumerate(mats):
+        u, s, v = U.blocks[(i, i)], d.blocks[(i,)], V.blocks[(i, i)]
+        assert np.abs(s - np.linalg.svd(a, compute_uv=False)).max() <= 1e-12 * s[0]
+        assert np.linalg.norm((u * s) @ v.T - a) <= 1e-12 * np.linalg.norm(a)
+        keep = s > 1e-10 * s[0]
+        for w in (u[:, keep], v[:, keep]):
+            assert np.abs(w.T @ w - np.eye(w.shape[1])).max() <= 1e-12
