@@ -8,9 +8,9 @@
 //                   P^T G P = R^T R (left-looking inside the panel; the
 //                   trailing matrix is updated by a GEMM G -= Lp Lp^T after
 //                   each panel).  L = R^T is kept with its rows in the
-//                   original order, so L L^T = G and the one-sided Jacobi on
-//                   the columns of L (block rounds of k_svd_round) yields G's
-//                   eigenvectors as the normalised columns,
+//                   original order, so L L^T = G and the Jacobi rounds on the
+//                   columns of L (gram_rounds.hip) yield G's eigenvectors
+//                   as the normalised columns,
 //   k_gram_vectors  normalises the columns of the rotated L into W and
 //                   completes zero columns from the unit vector with the
 //                   largest residual (two projection passes).
