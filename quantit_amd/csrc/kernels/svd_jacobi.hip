@@ -1827,6 +1827,13 @@ void fill_i32(hipStream_t st, int32_t* p, int n, int32_t v) {
 // The values of all sectors are gathered, sorted descending (bitonic, in LDS
 // when 2^ceil(log2 total) doubles fit, else in the scratch area) and the cut
 // is found by the reference's sequential tail accumulation.
+//
+// Up to kRankSort values are put in order by counting, for each, the values
+// before it: reads of LDS that do not wait for each other and two barriers,
+// where the bitonic sort has a barrier of 16 waves at each of its steps (36 of
+// them at 256 values): the whole kernel at the 150 values of a D = 48 update
+// 12.7 -> 8.9 us.
+constexpr int kRankSort = 512;
 template <class L, bool IN_LDS>
 __global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, L l, uint32_t at_pos, uint32_t at_ks,
                                                    int nsec, int64_t scratch_off,
@@ -1835,6 +1842,7 @@ __global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, L 
                                                    double* __restrict__ thr_out) {
   extern __shared__ double vl[];
   __shared__ double thr_sh;
+  __shared__ int before[kRankSort];
   const int64_t* s_offs = l.template list<int64_t>();
   const int64_t* s_pos = l.template list<int64_t>(at_pos);
   const int32_t* ks = l.template list<int32_t>(at_ks);
@@ -1852,10 +1860,28 @@ __global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, L 
     for (int j = lane; j < n; j += 64) v[pos + j] = src[j];
   }
   for (int64_t j = total + tid; j < n2; j += blockDim.x) v[j] = -INFINITY;
+  if (tid < kRankSort) before[tid] = 0;
   __syncthreads();
+  const bool by_rank = IN_LDS && total <= kRankSort;
+  if (by_rank) {  // value j by blockDim.x / n2 threads, each counting a part
+    const int n = int(total), m = int(n2), parts = blockDim.x / m;
+    const int j = tid & (m - 1), step = (n + parts - 1) / parts;
+    const int i0 = tid / m * step, i1 = min(i0 + step, n);
+    const double x = v[j];
+    int r = 0;
+#pragma unroll 8
+    for (int i = i0; i < i1; ++i) r += int(v[i] > x) | (int(v[i] == x) & int(i < j));
+    double* sorted = vl + m;
+    if (tid < m) sorted[tid] = x;  // no hole where a NaN has no place
+    if (j < n) atomicAdd(&before[j], r);
+    __syncthreads();
+    if (tid < n) sorted[before[tid]] = x;
+    __syncthreads();
+    v = sorted;
+  }
   // bitonic sort, descending (n2 < 2^31; strides are powers of two, so the
   // pair index is formed with masks, not divisions)
-  const int m2 = int(n2);
+  const int m2 = by_rank ? 0 : int(n2);
   for (int size = 2; size <= m2; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
       for (int i = tid; i < m2 / 2; i += blockDim.x) {
@@ -1927,15 +1953,15 @@ void truncate_select(hipStream_t st, double* base, const Lists& l, int nsec, int
   int64_t n2 = 1;
   while (n2 < total) n2 <<= 1;
   if (n2 > (int64_t(1) << 30)) throw std::runtime_error("truncation: more than 2^30 values");
-  const size_t lds = size_t(n2) * sizeof(double);
+  const size_t lds = size_t(n2) * sizeof(double) * (total <= kRankSort ? 2 : 1);
   static const size_t limit = [] {
     int dev = 0, v = 0;
     (void)hipGetDevice(&dev);
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess) v = 65536;
     for (const void* f : {reinterpret_cast<const void*>(&k_truncate<DevLists, true>),
                           reinterpret_cast<const void*>(&k_truncate<ArgLists, true>)})
-      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, v - 256);
-    return size_t(v) - 256;
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, v - 256 - kRankSort * int(sizeof(int)));
+    return size_t(v) - 256 - kRankSort * sizeof(int);
   }();
   if (lds <= limit)
     launch_lists(k_truncate<DevLists, true>, k_truncate<ArgLists, true>, l, dim3(1), dim3(1024), lds, st, base, l.at[1],
