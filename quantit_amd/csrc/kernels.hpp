@@ -391,10 +391,11 @@ void gram_vectors(hipStream_t s, double* base, const Lists& descs, int n, int km
 // Global truncation (sources/btensor_linalg.cpp:657-755,
 // sources/LinearAlgebra.cpp:57-75): singular values of nsec sectors stored
 // descending at s_off[i] with k[i] entries, s_pos[i] = k[0] + ... + k[i-1];
-// writes kept[i].
+// writes kept[i], and to kept[nsec] whether some sector keeps a value that is
+// not above null_scale times its first.
 // lists: s_off, s_pos, k
 void truncate_select(hipStream_t s, double* base, const Lists& l, int nsec, int64_t scratch_off, int64_t total, double tol, double pow, int64_t min_size,
-                     int64_t max_size, int32_t* kept, double* thr_out);
+                     int64_t max_size, double null_scale, int32_t* kept, double* thr_out);
 
 }  // namespace kern
 }  // namespace qtt

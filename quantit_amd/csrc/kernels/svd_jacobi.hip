@@ -1838,11 +1838,11 @@ template <class L, bool IN_LDS>
 __global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, L l, uint32_t at_pos, uint32_t at_ks,
                                                    int nsec, int64_t scratch_off,
                                                    int64_t total, double tol, double pw, int64_t min_size,
-                                                   int64_t max_size, int32_t* __restrict__ kept,
-                                                   double* __restrict__ thr_out) {
+                                                   int64_t max_size, double null_scale,
+                                                   int32_t* __restrict__ kept, double* __restrict__ thr_out) {
   extern __shared__ double vl[];
   __shared__ double thr_sh;
-  __shared__ int before[kRankSort];
+  __shared__ int before[kRankSort], null_sh;
   const int64_t* s_offs = l.template list<int64_t>();
   const int64_t* s_pos = l.template list<int64_t>(at_pos);
   const int32_t* ks = l.template list<int32_t>(at_ks);
@@ -1943,6 +1943,7 @@ __global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, L 
     const double sl = v[last];
     thr_sh = sl - 2.0 * sl * DBL_EPSILON;
     thr_out[0] = thr_sh;
+    null_sh = 0;
   }
   __syncthreads();
   const double thr = thr_sh;
@@ -1959,12 +1960,17 @@ __global__ __launch_bounds__(1024) void k_truncate(double* __restrict__ base, L 
       const unsigned long long m = __ballot(j < n && !(src[j < n ? j : 0] > thr));
       if (m && c == n) c = j0 + __ffsll((long long)m) - 1;
     }
-    if (lane == 0) kept[i] = c;
+    if (lane == 0) {
+      kept[i] = c;
+      if (c > 0 && !(src[c - 1] > src[0] * null_scale)) null_sh = 1;
+    }
   }
+  __syncthreads();
+  if (tid == 0) kept[nsec] = null_sh;
 }
 
 void truncate_select(hipStream_t st, double* base, const Lists& l, int nsec, int64_t scratch_off, int64_t total, double tol, double pw, int64_t min_size,
-                     int64_t max_size, int32_t* kept, double* thr_out) {
+                     int64_t max_size, double null_scale, int32_t* kept, double* thr_out) {
   int64_t n2 = 1;
   while (n2 < total) n2 <<= 1;
   if (n2 > (int64_t(1) << 30)) throw std::runtime_error("truncation: more than 2^30 values");
@@ -1980,10 +1986,10 @@ void truncate_select(hipStream_t st, double* base, const Lists& l, int nsec, int
   }();
   if (lds <= limit)
     launch_lists(k_truncate<DevLists, true>, k_truncate<ArgLists, true>, l, dim3(1), dim3(1024), lds, st, base, l.at[1],
-                 l.at[2], nsec, scratch_off, total, tol, pw, min_size, max_size, kept, thr_out);
+                 l.at[2], nsec, scratch_off, total, tol, pw, min_size, max_size, null_scale, kept, thr_out);
   else
     launch_lists(k_truncate<DevLists, false>, k_truncate<ArgLists, false>, l, dim3(1), dim3(1024), 0, st, base, l.at[1],
-                 l.at[2], nsec, scratch_off, total, tol, pw, min_size, max_size, kept, thr_out);
+                 l.at[2], nsec, scratch_off, total, tol, pw, min_size, max_size, null_scale, kept, thr_out);
 }
 
 }  // namespace kern

@@ -1137,10 +1137,12 @@ namespace {
 // *units are replaced and the truncated d is returned.
 // before_copy (may be empty) runs once the kept counts are known, before any
 // block is copied, with the kept count of every section of d (0 for sections
-// without a block).
+// without a block) and whether a section keeps a value that is not above
+// null_scale times its largest.
 BTensor truncate_units(BTensor&& d_in, const std::vector<BTensor*>& units, size_t max_size, size_t min_size,
                        double tol, double pw,
-                       const std::function<void(const std::vector<int32_t>&)>& before_copy = {}) {
+                       const std::function<void(const std::vector<int32_t>&, bool)>& before_copy = {},
+                       double null_scale = 0.0) {
   BTensor d = std::move(d_in);
   Context* ctx = d.ctx;
   double* ab = arena_base(ctx);
@@ -1158,27 +1160,27 @@ BTensor truncate_units(BTensor&& d_in, const std::vector<BTensor*>& units, size_
   if (total == 0) return d;
   int64_t n2 = 1;
   while (n2 < total) n2 <<= 1;
-  BufPtr scratch = ctx->alloc(size_t(n2 + 1) * sizeof(double) + size_t(nd) * sizeof(int32_t) + 256);
-  int32_t* const h_pin = ctx->pinned_ints(size_t(nd));
+  BufPtr scratch = ctx->alloc(size_t(n2 + 1) * sizeof(double) + size_t(nd + 1) * sizeof(int32_t) + 256);
+  int32_t* const h_pin = ctx->pinned_ints(size_t(nd) + 1);
   int32_t* d_kept = h_pin ? h_pin : reinterpret_cast<int32_t*>(scratch->cptr() + size_t(n2 + 1) * sizeof(double));
   double* d_thr = scratch->dptr() + n2;
   const int64_t clamp = std::numeric_limits<int64_t>::max();
   {
     KernelTimer kt(*ctx, "truncate_select");
     kern::truncate_select(ctx->stream(), ab, ctx->lists(s_offs, s_pos, ks), nd, scratch->dptr() - ab, total, tol, pw, int64_t(std::min<size_t>(min_size, size_t(clamp))),
-                          int64_t(std::min<size_t>(max_size, size_t(clamp))), d_kept, d_thr);
+                          int64_t(std::min<size_t>(max_size, size_t(clamp))), null_scale, d_kept, d_thr);
   }
-  std::vector<int32_t> kept(nd);
+  std::vector<int32_t> kept(nd + 1);
   if (h_pin) {
     ctx->sync();
-    std::copy(h_pin, h_pin + nd, kept.begin());
+    std::copy(h_pin, h_pin + nd + 1, kept.begin());
   } else {
-    ctx->read_small(kept.data(), d_kept, size_t(nd) * sizeof(int32_t));
+    ctx->read_small(kept.data(), d_kept, size_t(nd + 1) * sizeof(int32_t));
   }
   if (before_copy) {
     std::vector<int32_t> kept_sec(d.shape.secs[0].size(), 0);
     for (int i = 0; i < nd; ++i) kept_sec[d.blocks[i].idx.i[0]] = kept[i];
-    before_copy(kept_sec);
+    before_copy(kept_sec, kept[nd] != 0);
   }
 
   const size_t nu = units.size();
@@ -1323,13 +1325,15 @@ SvdResult svd_matrix(const BTensor& t, bool some, bool compute_uv) {
 
 // The truncation drops every column whose singular value is numerically zero
 // unless min_size keeps it, so the orthonormal completion of such columns runs
-// after the cut and only for the columns that are kept.
+// after the cut and only for the columns that are kept, and is launched only
+// when the cut kept such a column (a launch of its own found that out before).
 SvdResult svd_truncated(const BTensor& t, size_t split, double tol, size_t min_size, size_t max_size, double pw,
                         SvdStats* stats) {
   std::vector<kern::CompleteTask> pend;
   SvdResult out = svd_impl(t, split, stats, &pend);
   Context* ctx = t.ctx;
-  auto complete_kept = [&](const std::vector<int32_t>& kept_sec) {
+  auto complete_kept = [&](const std::vector<int32_t>& kept_sec, bool nulls) {
+    if (!nulls) return;
     std::vector<kern::CompleteTask> run;
     int64_t elems = 0;
     for (size_t i = 0; i < pend.size() && i < kept_sec.size(); ++i) {
@@ -1352,7 +1356,11 @@ SvdResult svd_truncated(const BTensor& t, size_t split, double tol, size_t min_s
     KernelTimer kt(*ctx, "svd_complete");
     kern::svd_complete(ctx->stream(), arena_base(ctx), ctx->lists(run), int(run.size()));
   };
-  out.d = truncate_units(std::move(out.d), {&out.U, &out.V}, max_size, min_size, tol, pw, complete_kept);
+  // the completion's own test is against S[0] * ell * eps of each sector
+  int ell = 0;
+  for (const auto& c : pend) ell = std::max(ell, c.ell);
+  const double null_scale = 1.001 * double(ell) * DBL_EPSILON;
+  out.d = truncate_units(std::move(out.d), {&out.U, &out.V}, max_size, min_size, tol, pw, complete_kept, null_scale);
   return out;
 }
 
