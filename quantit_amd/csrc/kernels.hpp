@@ -138,8 +138,8 @@ struct ChunkTask {
   int32_t chunk;
 };
 // Elements per work-group task of the element-wise kernels: 8 per thread of
-// a 256-thread group, so a task is a few dependent memory round trips and a
-// launch spreads over many work-groups.
+// a 256-thread group, loaded together, so a task is one memory round trip and
+// a launch spreads over many work-groups.
 constexpr int kChunk = 2048;
 // The lists of these launches: descriptors, ChunkTasks.
 void permute_copy(hipStream_t s, double* base, const Lists& l, int ntasks);
