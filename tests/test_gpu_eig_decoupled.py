@@ -1,0 +1,66 @@
+"""eigh and SVD of sectors whose columns do not all couple (hidden symmetries,
+direct sums): in the one-work-group solver eight lanes rotate a pair, the eight
+pairs of a wave independently of each other, and a sweep may only be the last
+when no pair of any of them rotated far.  Vectors orthonormal, values and
+residuals within 1e-12 of the norm (the bound of the other eigensolver tests)."""
+import numpy as np
+import pytest
+
+from oracle.btensor_oracle import BTensor
+from tests.helpers import from_dev, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _sector(m):
+    A = BTensor((0,), [[m.shape[0]], [m.shape[1]]], [[(0,)], [(0,)]], (0,))
+    A.blocks[(0, 0)] = m
+    return A
+
+
+def _matrix(kind, k):
+    """A positive definite k x k matrix."""
+    if kind == "random beside a lone state":
+        x = np.random.default_rng(k).standard_normal((k - 1, k - 1))
+        g = np.zeros((k, k))
+        g[0, 0] = 10.0 * k
+        g[1:, 1:] = x @ x.T + np.eye(k - 1)
+        return g
+    # diagonals that fall so evenly that pivoting keeps the order, column c
+    # coupled to c + 8 in every sixteen
+    d = 2.0 - 0.05 * np.arange(k) if kind == "even steps" else 2.0 ** (-0.2 * np.arange(k))
+    g = np.diag(d)
+    for c in range(k - 8):
+        if c // 8 % 2 == 0 and (kind == "all in pairs" or c % 8):
+            g[c, c + 8] = g[c + 8, c] = 0.3 if kind == "even steps" else 0.3 * np.sqrt(d[c] * d[c + 8])
+    return g
+
+
+CASES = [("even steps", 16)] + [(kind, k) for kind in ("first of eight alone", "all in pairs",
+                                                       "random beside a lone state") for k in (16, 32, 64, 130)]
+
+
+@pytest.mark.parametrize("kind,k", CASES)
+def test_eigh_of_decoupled_columns(ctx, kind, k):
+    import quantit_amd as qa
+    g = _matrix(kind, k)
+    e, U = (from_dev(x) for x in qa.eigh(to_dev(ctx, _sector(g)), 1))
+    w, u = e.blocks[(0,)], U.blocks[(0, 0)]
+    nrm = np.linalg.norm(g, 2)
+    assert np.abs(u.T @ u - np.eye(k)).max() <= 1e-12
+    assert np.abs(w - np.linalg.eigvalsh(g)).max() <= 1e-12 * nrm
+    assert np.abs(g @ u - u * w).max() <= 1e-12 * nrm
+
+
+@pytest.mark.parametrize("kind,k", CASES)
+def test_svd_of_decoupled_columns(ctx, kind, k):
+    import quantit_amd as qa
+    g = _matrix(kind, k)
+    q = np.linalg.qr(np.random.default_rng(k).standard_normal((k + 5, k)))[0]
+    a = q @ np.linalg.cholesky(g).T  # a^T a = g
+    U, d, V = (from_dev(x) for x in qa.svd(to_dev(ctx, _sector(a)), 1))
+    u, s, v = U.blocks[(0, 0)], d.blocks[(0,)], V.blocks[(0, 0)]
+    for w in (u, v):
+        assert np.abs(w.T @ w - np.eye(k)).max() <= 1e-12
+    assert np.abs(s - np.linalg.svd(a, compute_uv=False)).max() <= 1e-12 * s[0]
+    assert np.linalg.norm((u * s) @ v.T - a) <= 1e-12 * np.linalg.norm(a)
