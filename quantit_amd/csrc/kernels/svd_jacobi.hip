@@ -1095,6 +1095,7 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
   // fails.
   const bool eig = J.shift_off >= 0;
   double shift = 0.0, fro = 0.0;
+  bool by_norm = false;  // counted, not compared: the norm may be a NaN
   auto add_shift = [&] {
     if (tid < k) X[tid * k + tid] += shift;
     __syncthreads();
@@ -1126,7 +1127,8 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
     }
     fro = sqrt(ss);
     shift = 4.0 * k * DBL_EPSILON * hi;
-    if (!(lo + shift > 0.0)) shift = fro;
+    by_norm = !(lo + shift > 0.0);
+    if (by_norm) shift = fro;
     add_shift();
   }
   // ---- 1. orthogonality test on G -------------------------------------------
@@ -1282,10 +1284,11 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
           }
         }
       }
-      if (!eig || rk == k || shift == fro) break;
+      if (!eig || rk == k || by_norm) break;
       __syncthreads();  // not definite: again under the norm
       for (int e = tid; e < k * k; e += blockDim.x) X[e] = Gg[int64_t(e / k) * J.ldy + e % k];
       __syncthreads();
+      by_norm = true;
       shift = fro;
       add_shift();
     }
@@ -1312,7 +1315,7 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
   }
   // ---- 3. one-sided Jacobi on the columns of X ------------------------------
   // (under a shift by the norm, tol / 16 is below the products' rounding)
-  const double tol_rot = tol * (eig && shift == fro ? 0.5 : 1.0 / 16.0);
+  const double tol_rot = tol * (by_norm ? 0.5 : 1.0 / 16.0);
   const int pi = tid / gsz, li = tid % gsz;
   if (!ident) {
     if (k <= 16)
