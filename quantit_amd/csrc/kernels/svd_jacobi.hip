@@ -1127,7 +1127,8 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
     }
     fro = sqrt(ss);
     shift = 4.0 * k * DBL_EPSILON * hi;
-    by_norm = !(lo + shift > 0.0);
+    // without the factorisation nothing would tell that the shift is too small
+    by_norm = !precond || !(lo + shift > 0.0);
     if (by_norm) shift = fro;
     add_shift();
   }

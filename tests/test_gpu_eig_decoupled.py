@@ -64,3 +64,23 @@ def test_svd_of_decoupled_columns(ctx, kind, k):
         assert np.abs(w.T @ w - np.eye(k)).max() <= 1e-12
     assert np.abs(s - np.linalg.svd(a, compute_uv=False)).max() <= 1e-12 * s[0]
     assert np.linalg.norm((u * s) @ v.T - a) <= 1e-12 * np.linalg.norm(a)
+
+
+@pytest.mark.parametrize("precond", ["0", "1"])
+@pytest.mark.parametrize("k", [2, 16, 65, 130])
+def test_eigh_of_indefinite_matrices_with_a_positive_diagonal(ctx, k, precond, monkeypatch):
+    """Nothing but the factorisation shows that these are not definite, and
+    QTT_SVD_PRECOND=0 does without it."""
+    import quantit_amd as qa
+    monkeypatch.setenv("QTT_SVD_PRECOND", precond)
+    x = np.random.default_rng(k).uniform(-1.0, 1.0, (k, k))
+    g = x + x.T
+    np.fill_diagonal(g, 0.5)
+    g[0, 1] = g[1, 0] = 0.8
+    e, U = (from_dev(x) for x in qa.eigh(to_dev(ctx, _sector(g)), 1))
+    w, u = e.blocks[(0,)], U.blocks[(0, 0)]
+    nrm = np.linalg.norm(g)
+    assert w[0] < 0.0
+    assert np.abs(w - np.linalg.eigvalsh(g)).max() <= 1e-12 * nrm
+    assert np.abs(g @ u - u * w).max() <= 1e-12 * nrm
+    assert np.abs(u.T @ u - np.eye(k)).max() <= 1e-12
