@@ -5,8 +5,12 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <string>
 #include <vector>
+
+#include "qtt_common.hpp"
 
 namespace qtt {
 namespace kern {
@@ -73,9 +77,21 @@ struct GemmPair {
 };
 struct GemmTile {
   int32_t out;
-  int16_t tm, tn;  // tile coordinates inside the output block
+  uint16_t tm, tn;  // tile coordinates inside the output block
 };
 constexpr int kGemmTile = 64;
+// Rows or columns of an output block that tiles of edge T can address: 2.1 M
+// for T = 32, 4.2 M for 64.
+constexpr int64_t gemm_tile_reach(int T) { return int64_t(T) << 16; }
+// Adds the tiles of one M x N output block to a list, row by row.
+inline void add_tiles(std::vector<GemmTile>& tiles, int out, int64_t M, int64_t N, int T) {
+  if (std::max(M, N) > gemm_tile_reach(T))
+    throw InvalidArgument("output block of " + std::to_string(M) + " x " + std::to_string(N) +
+                          " elements: more than " + std::to_string(gemm_tile_reach(T)) + " rows or columns");
+  const int64_t tm = (M + T - 1) / T, tn = (N + T - 1) / T;
+  for (int64_t i = 0; i < tm; ++i)
+    for (int64_t j = 0; j < tn; ++j) tiles.push_back({int32_t(out), uint16_t(i), uint16_t(j)});
+}
 // How the operands of a launch are contiguous: bit 0 A in k (else in m), bit 1
 // B in n (else in k), common to all its pairs; kLayoutAny: in no common way.
 enum GemmLayout : int { kLayoutAny = -1 };

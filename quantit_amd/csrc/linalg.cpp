@@ -109,11 +109,7 @@ GemmLaunch prepare_gemm(Context* ctx, const std::vector<kern::GemmOut>& outs,
   if (g.lay != kern::kLayoutAny && count(64) < kern::kTile64Min) g.tile = 32;
   std::vector<kern::GemmTile> tiles;
   tiles.reserve(size_t(count(g.tile)));
-  for (size_t o = 0; o < outs.size(); ++o) {
-    const int tm = (outs[o].M + g.tile - 1) / g.tile, tn = (outs[o].N + g.tile - 1) / g.tile;
-    for (int i = 0; i < tm; ++i)
-      for (int j = 0; j < tn; ++j) tiles.push_back({int32_t(o), int16_t(i), int16_t(j)});
-  }
+  for (size_t o = 0; o < outs.size(); ++o) kern::add_tiles(tiles, int(o), outs[o].M, outs[o].N, g.tile);
   if (tiles.empty()) return g;
   g.lists = repeated ? ctx->device_lists(tiles, outs, pairs) : ctx->lists(tiles, outs, pairs);
   g.ntiles = int(tiles.size());

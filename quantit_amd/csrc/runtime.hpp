@@ -104,6 +104,7 @@ class Context {
   kern::Lists device_lists(const std::vector<T>&... v) {
     return make_lists(false, v...);
   }
+  size_t stage_bytes() const { return stage_cap_; }
   // Copies host bytes through the pinned staging ring to any device address
   // (stream-ordered; no allocation).
   void stage_to(void* dev_dst, const void* data, size_t bytes);

@@ -146,6 +146,8 @@ class TdWork {
   // device copy of host bytes, ordered on the context stream before the
   // work enqueued afterwards
   virtual void* put(const void* src, size_t bytes) = 0;
+  // the most that one put can take now
+  virtual size_t room() const = 0;
   // the context, when the launch follows at once and is not repeated
   virtual Context* launches_once() const { return nullptr; }
   virtual bool timed() const = 0;
@@ -160,6 +162,7 @@ class ArenaWork : public TdWork {
     return keep_.back()->dptr() - reinterpret_cast<double*>(ctx_->arena().base());
   }
   void* put(const void* src, size_t bytes) override { return ctx_->upload(src, bytes); }
+  size_t room() const override { return ctx_->stage_bytes(); }
   Context* launches_once() const override { return ctx_; }
   bool timed() const override { return true; }
 
@@ -189,6 +192,7 @@ class StaticWork : public TdWork {
     ctx_->stage_to(p, src, bytes);
     return p;
   }
+  size_t room() const override { return std::min(kern::kNoAllocScratchBytes - pos_, ctx_->stage_bytes()); }
   bool timed() const override { return false; }
 
  private:
@@ -235,6 +239,7 @@ class PersistWork : public TdWork {
     ctx_->stage_to(keep_->back()->cptr(), src, bytes);
     return keep_->back()->cptr();
   }
+  size_t room() const override { return ctx_->stage_bytes(); }
   bool timed() const override { return false; }
 
  private:
@@ -756,10 +761,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     std::vector<kern::GemmTile> tl;
     for (int o : ord) {
       if (size_t(o) < outs.size() && (narrow[size_t(o)] || split_block[size_t(o)])) continue;
-      const int tm = (launch_outs[o].M + T - 1) / T;
-      const int tn = (launch_outs[o].N + T - 1) / T;
-      for (int i = 0; i < tm; ++i)
-        for (int j = 0; j < tn; ++j) tl.push_back({int32_t(o), int16_t(i), int16_t(j)});
+      kern::add_tiles(tl, o, launch_outs[o].M, launch_outs[o].N, T);
     }
     return tl;
   };
@@ -788,6 +790,21 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
       tune_now = false;
     else
       lch.tile = kern::variant_tile(variant);
+    // no 32 x 32 tiles, not for a timing either, where their coordinates would
+    // not reach or the list, four times as long, would not fit
+    int64_t widest = 0, tiles32 = 0;
+    for (size_t o = 0; o < launch_outs.size(); ++o) {
+      const int64_t M = launch_outs[o].M, N = launch_outs[o].N;
+      widest = std::max({widest, M, N});
+      tiles32 += (M + 31) / 32 * ((N + 31) / 32);
+    }
+    const size_t bytes32 = size_t(tiles32) * sizeof(kern::GemmTile) + launch_outs.size() * sizeof(kern::GemmOut) +
+                           gpairs.size() * sizeof(kern::GemmPair) + sums.size() * sizeof(kern::SumParts) +
+                           sum_tasks.size() * sizeof(kern::ChunkTask) + 512;
+    if (widest > kern::gemm_tile_reach(32) || bytes32 > work.room()) {
+      lch.tile = kern::kGemmTile;
+      tune_now = false;
+    }
   }
   tiles = tiles_of(lch.tile);
   if (stats) {
@@ -804,18 +821,15 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     std::vector<kern::GemmTile> tl;
     std::vector<std::pair<int, int>> launches;  // (first tile, tile count) per pair
     for (size_t o = 0; o < outs.size(); ++o) {
-      const int tm = (gouts[o].M + kern::kGemmTile - 1) / kern::kGemmTile;
-      const int tn = (gouts[o].N + kern::kGemmTile - 1) / kern::kGemmTile;
-      if (tm * tn == 0) continue;
+      if (int64_t(gouts[o].M) * gouts[o].N == 0) continue;
       for (int p = gouts[o].pair_begin; p < gouts[o].pair_end; ++p) {
         const int t0 = int(tl.size());
-        for (int i = 0; i < tm; ++i)
-          for (int j = 0; j < tn; ++j) tl.push_back({int32_t(one.size()), int16_t(i), int16_t(j)});
+        kern::add_tiles(tl, int(one.size()), gouts[o].M, gouts[o].N, kern::kGemmTile);
         kern::GemmOut g1 = gouts[o];
         g1.pair_begin = p;
         g1.pair_end = p + 1;
         one.push_back(g1);
-        launches.push_back({t0, tm * tn});
+        launches.push_back({t0, int(tl.size()) - t0});
       }
     }
     td_pack(ctx, lch, true);
