@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -41,6 +42,7 @@ struct DevLists {
 // The lists of one launch, list i at byte at[i].
 struct Lists {
   const char* dev = nullptr;  // null: in arg
+  std::shared_ptr<void> own;  // device memory of their own, until the launches are enqueued
   uint32_t at[6] = {0, 0, 0, 0, 0, 0};
   ArgLists arg;
   Lists() {}

@@ -189,7 +189,8 @@ int jacobi_sweeps(Context* ctx, double* ab, const std::vector<kern::SvdSector>& 
   // holds at once, the long ones start in the first wave of work-groups
   std::stable_sort(work.begin(), work.end(),
                    [](const kern::RoundWork& a, const kern::RoundWork& b) { return a.ell > b.ell; });
-  const kern::RoundWork* d_work = work.empty() ? nullptr : ctx->upload_vec(work);
+  const kern::Lists l_work = ctx->device_lists(work);  // read by every round
+  const auto* d_work = reinterpret_cast<const kern::RoundWork*>(l_work.dev);
   auto enqueue = [&](int sweep) {
     int max_nb = 0;
     int64_t nactive = 0;
@@ -349,7 +350,8 @@ int gram_sweeps(Context* ctx, double* ab, const std::vector<GramProblem>& ps, do
     outs.push_back({p.g0, p.k, p.k, int32_t(prs.size()), int32_t(prs.size() + 1), p.nb * kern::kSvdBlock, 0});
     prs.push_back(g);
   }
-  const kern::GramRound* d_work = ctx->upload_vec(work);
+  const kern::Lists l_work = ctx->device_lists(work);  // read by every round
+  const auto* d_work = reinterpret_cast<const kern::GramRound*>(l_work.dev);
   const GemmLaunch gram = prepare_gemm(ctx, outs, prs, true);
   constexpr int kAhead = 6;  // launches enqueued before the host waits for the counts
   for (int sweep = 0;; ++sweep) {
@@ -742,7 +744,8 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         outs.push_back({gb + go[q], s.k, s.k, int32_t(prs.size()), int32_t(prs.size() + 1), s.k, 0});
         prs.push_back(gp);
       }
-      const auto* d_pd = ctx->upload_vec(pd);
+      const kern::Lists l_pd = ctx->device_lists(pd);
+      const auto* d_pd = reinterpret_cast<const kern::CholPanel*>(l_pd.dev);
       kern::pchol_init(ctx->stream(), ab, d_pd, int(pd.size()));
       const GemmLaunch upd = prepare_gemm(ctx, outs, prs, true);
       for (int j0 = 0; j0 < kact; j0 += pnb) {
@@ -803,6 +806,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       // stream joins before the rotation.  Profiling keeps one stream so that
       // the event timers stay per kernel.
       const bool overlap = !act_s.empty() && !act_l.empty() && !ctx->profiling && ctx->overlap;
+      kern::Lists d_jd;  // the side stream may read them until the join
       if (!act_s.empty()) {
         std::vector<kern::SmallJacobi> jd;
         for (int q : act_s) {
@@ -814,7 +818,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         std::stable_sort(jd.begin(), jd.end(),
                          [](const kern::SmallJacobi& a, const kern::SmallJacobi& b) { return a.k > b.k; });
         static const char* const kEigNames[] = {"svd_eig", "svd_eig_it1", "svd_eig_it2", "svd_eig_it3+"};
-        const kern::Lists d_jd = ctx->lists(jd);
+        d_jd = ctx->lists(jd);
         if (overlap) ctx->fork();
         KernelTimer kt(*ctx, kEigNames[std::min(it, 3)]);
         kern::gram_eig(overlap ? ctx->side_stream() : ctx->stream(), ab, d_jd, int(jd.size()), d_flags, tol,

@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 
 namespace qtt {
@@ -82,6 +83,8 @@ Context::Context(int device, size_t arena_bytes, size_t stage_bytes) : device_(d
   QTT_HIP(hipEventCreateWithFlags(&join_ev_, hipEventDisableTiming));
   arena_ = std::make_shared<Arena>(arena_bytes);
   // the descriptor staging ring comes out of the arena: at most a quarter of it
+  if (const char* e = std::getenv("QTT_STAGE_BYTES"))
+    stage_bytes = std::max<size_t>(size_t(64) << 10, std::strtoull(e, nullptr, 10));
   stage_cap_ = round_up(std::min(stage_bytes, std::max<size_t>(size_t(1) << 20, arena_bytes / 4)));
   QTT_HIP(hipHostMalloc(reinterpret_cast<void**>(&host_stage_), stage_cap_, hipHostMallocDefault));
   dev_stage_ = alloc(stage_cap_);
@@ -133,32 +136,22 @@ char* Context::stage_host(size_t bytes, size_t* pos) {
 // Above this the copy is a kernel (stage_copy); below, the two are alike.
 static constexpr size_t kStageKernelBytes = size_t(16) << 10;
 
-// The device half of the ring at pos, after the host half's copy to it.
-char* Context::stage_send(size_t pos, size_t bytes) {
-  char* d = dev_stage_->cptr() + pos;
-  if (bytes > kStageKernelBytes)
-    kern::stage_copy(stream_, d, host_stage_ + pos, bytes);
+// Copy of the ring's host half at pos to device memory.
+void Context::stage_send(void* dev_dst, size_t pos, size_t bytes) {
+  if (bytes > kStageKernelBytes && reinterpret_cast<uintptr_t>(dev_dst) % 16 == 0)
+    kern::stage_copy(stream_, dev_dst, host_stage_ + pos, bytes);
   else if (bytes)
-    QTT_HIP(hipMemcpyAsync(d, host_stage_ + pos, bytes, hipMemcpyHostToDevice, stream_));
-  return d;
-}
-
-void* Context::upload(const void* data, size_t bytes) {
-  size_t pos = 0;
-  char* h = stage_host(bytes, &pos);
-  if (bytes) std::memcpy(h, data, bytes);
-  return stage_send(pos, bytes);
+    QTT_HIP(hipMemcpyAsync(dev_dst, host_stage_ + pos, bytes, hipMemcpyHostToDevice, stream_));
 }
 
 void Context::stage_to(void* dev_dst, const void* data, size_t bytes) {
-  if (!bytes) return;
-  size_t pos = 0;
-  char* h = stage_host(bytes, &pos);
-  std::memcpy(h, data, bytes);
-  if (bytes > kStageKernelBytes && reinterpret_cast<uintptr_t>(dev_dst) % 16 == 0)
-    kern::stage_copy(stream_, dev_dst, h, bytes);
-  else
-    QTT_HIP(hipMemcpyAsync(dev_dst, h, bytes, hipMemcpyHostToDevice, stream_));
+  const size_t most = stage_cap_ / 2;  // the next piece is filled while this one is copied
+  for (size_t at = 0; at < bytes; at += most) {
+    const size_t n = std::min(most, bytes - at);
+    size_t pos = 0;
+    std::memcpy(stage_host(n, &pos), static_cast<const char*>(data) + at, n);
+    stage_send(static_cast<char*>(dev_dst) + at, pos, n);
+  }
 }
 
 void Context::fork() {

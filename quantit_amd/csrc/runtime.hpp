@@ -86,16 +86,10 @@ class Context {
   Arena& arena() { return *arena_; }
   BufPtr alloc(size_t bytes) { return std::make_shared<DeviceBuffer>(arena_, bytes); }
 
-  // Copies host descriptors to device memory in stream order; returns a device
-  // pointer valid for kernels enqueued afterwards on this context's stream.
-  void* upload(const void* data, size_t bytes);
-  template <class T>
-  T* upload_vec(const std::vector<T>& v) {
-    return static_cast<T*>(upload(v.data(), v.size() * sizeof(T)));
-  }
-  // The descriptor lists of one launch, each 16-byte aligned: in the launch's
-  // arguments where they fit, else in one staging copy.  device_lists: always
-  // a staging copy, for lists that several launches read.
+  // The descriptor lists of one launch that follows soon, each 16-byte aligned:
+  // in the launch's arguments where they fit, else in one copy to the staging
+  // ring or, above ring_list_bytes(), to arena memory of their own.
+  // device_lists: always of their own, for lists that several launches read.
   template <class... T>
   kern::Lists lists(const std::vector<T>&... v) {
     return make_lists(true, v...);
@@ -104,7 +98,9 @@ class Context {
   kern::Lists device_lists(const std::vector<T>&... v) {
     return make_lists(false, v...);
   }
-  size_t stage_bytes() const { return stage_cap_; }
+  // The longest list that stays in the ring: an eighth of it, so that the list
+  // at hand never lands on one of up to six before it that wait for their launch.
+  size_t ring_list_bytes() const { return stage_cap_ / 8; }
   // Copies host bytes through the pinned staging ring to any device address
   // (stream-ordered; no allocation).
   void stage_to(void* dev_dst, const void* data, size_t bytes);
@@ -208,7 +204,7 @@ class Context {
   hipEvent_t sync_ev_ = nullptr;
   void* noalloc_scratch_ = nullptr;
   char* stage_host(size_t bytes, size_t* pos);
-  char* stage_send(size_t pos, size_t bytes);
+  void stage_send(void* dev_dst, size_t pos, size_t bytes);
   template <class... T>
   kern::Lists make_lists(bool in_args, const std::vector<T>&... v) {
     kern::Lists l;
@@ -221,10 +217,23 @@ class Context {
     }
     if (total > UINT32_MAX) throw OutOfMemory("descriptor lists larger than 4 GiB");
     const bool arg = in_args && total <= kern::kArgListBytes;
-    char* h = arg ? l.arg.b : stage_host(total, &pos);
-    for (size_t i = 0; i < sizeof...(T); ++i)
-      if (sizes[i]) std::memcpy(h + l.at[i], src[i], sizes[i]);
-    if (!arg) l.dev = stage_send(pos, total);
+    const bool in_ring = in_args && total <= ring_list_bytes();
+    char* dst = nullptr;
+    if (!arg && !in_ring) {
+      const BufPtr own = alloc(total);
+      dst = own->cptr();
+      l.own = own;
+    }
+    if (total > ring_list_bytes() && !arg) {
+      for (size_t i = 0; i < sizeof...(T); ++i) stage_to(dst + l.at[i], src[i], sizes[i]);
+    } else {
+      char* h = arg ? l.arg.b : stage_host(total, &pos);
+      for (size_t i = 0; i < sizeof...(T); ++i)
+        if (sizes[i]) std::memcpy(h + l.at[i], src[i], sizes[i]);
+      if (in_ring) dst = dev_stage_->cptr() + pos;
+      if (!arg) stage_send(dst, pos, total);
+    }
+    if (!arg) l.dev = dst;
     return l;
   }
 };

@@ -146,14 +146,14 @@ class TdWork {
   // device copy of host bytes, ordered on the context stream before the
   // work enqueued afterwards
   virtual void* put(const void* src, size_t bytes) = 0;
-  // the most that one put can take now
+  // the most that lists may take without a cost beside their length
   virtual size_t room() const = 0;
   // the context, when the launch follows at once and is not repeated
   virtual Context* launches_once() const { return nullptr; }
   virtual bool timed() const = 0;
 };
 
-// Temporaries from the context arena, descriptors through its staging ring.
+// Temporaries from the context arena.
 class ArenaWork : public TdWork {
  public:
   explicit ArenaWork(Context* c) : ctx_(c) {}
@@ -161,8 +161,8 @@ class ArenaWork : public TdWork {
     keep_.push_back(ctx_->alloc(bytes));
     return keep_.back()->dptr() - reinterpret_cast<double*>(ctx_->arena().base());
   }
-  void* put(const void* src, size_t bytes) override { return ctx_->upload(src, bytes); }
-  size_t room() const override { return ctx_->stage_bytes(); }
+  void* put(const void*, size_t) override { return nullptr; }  // not asked: the lists go with the launch
+  size_t room() const override { return ctx_->ring_list_bytes(); }
   Context* launches_once() const override { return ctx_; }
   bool timed() const override { return true; }
 
@@ -192,7 +192,7 @@ class StaticWork : public TdWork {
     ctx_->stage_to(p, src, bytes);
     return p;
   }
-  size_t room() const override { return std::min(kern::kNoAllocScratchBytes - pos_, ctx_->stage_bytes()); }
+  size_t room() const override { return kern::kNoAllocScratchBytes - pos_; }
   bool timed() const override { return false; }
 
  private:
@@ -239,7 +239,7 @@ class PersistWork : public TdWork {
     ctx_->stage_to(keep_->back()->cptr(), src, bytes);
     return keep_->back()->cptr();
   }
-  size_t room() const override { return ctx_->stage_bytes(); }
+  size_t room() const override { return ctx_->ring_list_bytes(); }
   bool timed() const override { return false; }
 
  private:
@@ -621,6 +621,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
   gpairs.reserve(all_pairs.size());
   std::vector<int64_t> out_work(outs.size());
   double flops = 0, bytes = 0;
+  int64_t widest = 0;
   for (size_t o = 0; o < outs.size(); ++o) {
     const Block& cb_ = out.blocks[o];
     int64_t odims[kMaxRank];
@@ -628,6 +629,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
     int64_t M = 1, N = 1;
     for (int j = 0; j < na; ++j) M *= odims[j];
     for (int j = 0; j < nb; ++j) N *= odims[na + j];
+    widest = std::max({widest, M, N});
     gouts[o].c_off = out.ptr(cb_) - ab;
     gouts[o].M = int32_t(M);
     gouts[o].N = int32_t(N);
@@ -686,6 +688,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
   std::vector<char> split_block(outs.size(), 0);
   std::vector<kern::SumParts> sums;
   std::vector<kern::ChunkTask> sum_tasks;
+  int64_t part_max = 1;  // runs of a block at most
   {
     constexpr int64_t kTargetTiles = 2048, kSplitMinK = 64;
     constexpr int64_t kMaxSplit = 8;
@@ -700,6 +703,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
         const int64_t np = std::min(split, out_work[o] / kSplitMinK);
         if (np < 2) continue;
         nparts[o] = int(np);
+        part_max = std::max(part_max, np);
         part_elems += np * gouts[o].M * gouts[o].N;
       }
     if (part_elems) {
@@ -792,12 +796,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
       lch.tile = kern::variant_tile(variant);
     // no 32 x 32 tiles, not for a timing either, where their coordinates would
     // not reach or the list, four times as long, would not fit
-    int64_t widest = 0, tiles32 = 0;
-    for (size_t o = 0; o < launch_outs.size(); ++o) {
-      const int64_t M = launch_outs[o].M, N = launch_outs[o].N;
-      widest = std::max({widest, M, N});
-      tiles32 += (M + 31) / 32 * ((N + 31) / 32);
-    }
+    const int64_t tiles32 = 4 * mfma_tiles * part_max;  // or fewer
     const size_t bytes32 = size_t(tiles32) * sizeof(kern::GemmTile) + launch_outs.size() * sizeof(kern::GemmOut) +
                            gpairs.size() * sizeof(kern::GemmPair) + sums.size() * sizeof(kern::SumParts) +
                            sum_tasks.size() * sizeof(kern::ChunkTask) + 512;
