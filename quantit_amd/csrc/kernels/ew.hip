@@ -9,7 +9,6 @@ namespace qtt {
 namespace kern {
 
 // A permuted copy whose last dim is not the contiguous one of the source goes
-// A permuted copy whose last dim is not the contiguous one of the source goes
 // through LDS in tiles of up to 32 elements along the source's contiguous dim
 // and as many along the last as make 2048, so that both sides are read and
 // written in order (a tile is read in the source's order: where its two dims
@@ -17,7 +16,14 @@ namespace kern {
 // element by element in the destination's order, offsets by 32-bit divisions.
 // 121 MB in blocks of up to 272 x 272 x 12 with the last two dims exchanged: 22
 // us, against 83 with a 64-bit division per element and dim.
-constexpr int kPermTile = 32, kPermElems = 2048;
+//
+// A tile is a work-group with a task of its own, however little it holds, so
+// tiles are taken where they hold kPermTileMin elements on average.  8 M
+// elements, last dims m and n exchanged, list upload included, tiles against
+// element by element (us): m 4, n 16 617 / 35; 8, 32 77 / 36; 16, 32 46 / 40; 16,
+// 48 35 .. 47 / 41; 8, 128 29 .. 38 / 37; 16, 64 29 .. 38 / 43; 32, 64 26 / 44 (the
+// larger ones where the staging ring's pages are read for the first time).
+constexpr int kPermTile = 32, kPermElems = 2048, kPermTileMin = 1024;
 int64_t permute_plan(PermDesc& d) {
   int r = 0;
   for (int i = 0; i < d.rank; ++i) {
@@ -41,11 +47,14 @@ int64_t permute_plan(PermDesc& d) {
   if (d.sstride[r - 1] != 1 && n >= 16)
     for (int j = 0; j + 1 < r; ++j)
       if (d.sstride[j] == 1 && d.dims[j] >= 4) d.tj = j;
-  if (d.tj < 0) return (d.numel + kChunk - 1) / kChunk;
-  const int mj = std::min(d.dims[d.tj], kPermTile);
-  d.tn = kPermElems / mj / 64 * 64;
-  const int64_t tiles = int64_t((d.dims[d.tj] + kPermTile - 1) / kPermTile) * ((n + d.tn - 1) / d.tn);
-  return d.numel / d.dims[d.tj] / n * tiles;
+  if (d.tj >= 0) {
+    const int m = d.dims[d.tj];
+    d.tn = kPermElems / std::min(m, kPermTile) / 64 * 64;
+    const int64_t tiles = (int64_t(m) + kPermTile - 1) / kPermTile * ((int64_t(n) + d.tn - 1) / d.tn);
+    if (int64_t(m) * n >= tiles * kPermTileMin) return d.numel / m / n * tiles;
+    d.tj = -1;
+  }
+  return (d.numel + kChunk - 1) / kChunk;
 }
 
 template <class L>

@@ -31,7 +31,22 @@ static bool refused(int64_t M, int64_t N, int T) {
   return false;
 }
 
+// Tasks of a copy of (a, n, m) with its last dims exchanged: no more than one
+// for 1024 elements, or one for 2048 where the copy is not tiled.
+static void permute_tasks(int a, int n, int m) {
+  kern::PermDesc d{};
+  d.numel = int64_t(a) * n * m;
+  d.rank = 3;
+  const int dims[3] = {a, m, n};
+  const int64_t st[3] = {int64_t(n) * m, 1, m};
+  for (int i = 0; i < 3; ++i) d.dims[i] = dims[i], d.sstride[i] = st[i];
+  const int64_t tasks = kern::permute_plan(d);
+  CHECK(d.tj < 0 ? tasks == (d.numel + 2047) / 2048 : tasks * 1024 <= d.numel);
+}
+
 int main() {
+  for (int n : {1, 15, 16, 17, 63, 64, 65, 100, 128, 255, 256, 257, 512, 1000})
+    for (int m : {1, 3, 4, 5, 8, 15, 16, 17, 31, 32, 33, 63, 64, 65, 300}) permute_tasks(1000, n, m);
   for (int T : {32, 64}) {
     const int64_t reach = kern::gemm_tile_reach(T);
     for (int64_t m : {int64_t(1), int64_t(T), int64_t(T + 1), int64_t(32767) * T, int64_t(32768) * T,
