@@ -130,7 +130,7 @@ double qtt_last_tensordot_flops(void);
  * (sections, charges, selection rule, block list in order), for instance a
  * previous result of the same contraction; it must not share storage with a
  * or b.  Packed operands, split-K partials and launch descriptors live in a
- * static device scratch of 128 MiB per GPU; a contraction that needs more
+ * static device scratch of 160 MiB per GPU; a contraction that needs more
  * fails with QTT_INVALID_ARGUMENT before any launch.  The call allocates
  * nothing, records no profiling events and always uses the grouped kernels.
  * Every call on one GPU shares that scratch: calls that overlap on one GPU

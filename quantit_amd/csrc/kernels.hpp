@@ -117,7 +117,10 @@ constexpr int64_t kTile64Min = 768;
 // Size of the file-scope device scratch (kernels/gemm.hip) that the
 // allocation-free contraction takes its packed operands, split-K partials
 // and descriptors from.
-constexpr size_t kNoAllocScratchBytes = size_t(128) << 20;
+// 128 MiB beside what lists need: a task of 64 or 128 rows, of a tile of 1024
+// permuted elements or of a 32 x 32 product takes 8 bytes, so that 32 MiB hold
+// those of 2^29 rows.
+constexpr size_t kNoAllocScratchBytes = size_t(160) << 20;
 // Device address of that scratch on `device` (which must be current):
 // hipGetSymbolAddress on the first call per device, cached afterwards.
 hipError_t noalloc_scratch_address(int device, void** out);

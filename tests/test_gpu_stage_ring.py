@@ -77,3 +77,18 @@ def test_dmrg(ctx, small):
                  qa.DmrgOptions(cutoff=1e-8, convergence_criterion=0.0, maximum_bond=24, maximum_iterations=4))[0]
          for c in (ctx, small)]
     assert E[0] == E[1]
+
+
+@pytest.mark.parametrize("j,k", [(32, 64), (20, 40), (4, 16)])
+def test_allocation_free_contraction_that_fills_128_mib(ctx, j, k):
+    """A packed operand that leaves 100 KB of 128 MiB to the lists, however
+    finely the copy and the rows are divided."""
+    import quantit_amd as qa
+    i = ((128 << 20) - 100000) // 8 // (j * k)
+    rng = np.random.default_rng(j)
+    x, v = rng.integers(-8, 9, (i, k, j)).astype(float), rng.integers(-8, 9, (k, 3)).astype(float)
+    a = qa.BTensor.from_parts(ctx, (0,), [[i], [k], [j]], [[(0,)]] * 3, (0,), {(0, 0, 0): x})
+    b = qa.BTensor.from_parts(ctx, (0,), [[k], [3]], [[(0,)]] * 2, (0,), {(0, 0): v})
+    out = qa.BTensor.from_parts(ctx, (0,), [[i], [j], [3]], [[(0,)]] * 3, (0,), {(0, 0, 0): np.zeros((i, j, 3))})
+    a.tensordot_into(b, [1], [0], out)
+    assert np.array_equal(from_dev(out).blocks[(0, 0, 0)], np.matmul(x.transpose(0, 2, 1), v))
