@@ -226,7 +226,11 @@ int jacobi_sweeps(Context* ctx, double* ab, const std::vector<kern::SvdSector>& 
     for (int i = 0; i < ns; ++i)
       if (active[i]) elems += int64_t(secs[i].k) * secs[i].k;
     if (elems == 0) return false;
-    gram = ctx->alloc(size_t(elems) * sizeof(double));
+    try {
+      gram = ctx->alloc(size_t(elems) * sizeof(double));
+    } catch (const OutOfMemory&) {
+      return false;  // a sweep that rotates nothing tells as much
+    }
     int64_t go = gram->dptr() - ab;
     for (int i = 0; i < ns; ++i) {
       if (!active[i]) continue;
@@ -544,28 +548,34 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
     }
   };
   std::vector<int64_t> y2_of(ns, -1), w2_of(ns, -1);
-  if (wide.empty()) start(y2_of, w2_of);
+  // partial Gram matrices of a sector's first iteration (gram_of)
+  auto gram_parts = [](const kern::SvdSector& s) {
+    return int(std::min<int64_t>(16, std::max<int64_t>(1, s.ell / env_int("QTT_GRAM_ROWS_PER_PART", 256))));
+  };
+  BufPtr gbuf;
+  std::vector<int64_t> go, gwo, y2o, w2o, lo, lpo, sco, sto, pqo;
+  size_t lds_need = 0;
+  int pnb = 0, kmax_large = 0;
   if (!wide.empty()) {
     const int nw = int(wide.size());
-    int kmax_large = 0;
     for (int i : wide)
       if (large[i]) kmax_large = std::max(kmax_large, B.secs[i].k);
-    const int pnb =
-        kmax_large
-            ? int(std::min<size_t>(32, pchol_limit / (size_t(kmax_large) * sizeof(double)) - kern::kPcholExtra))
-            : 0;
-    int64_t elems = 0;
-    std::vector<int64_t> go(nw), gwo(nw), y2o(nw), w2o(nw), lo(nw, -1), lpo(nw, -1), sco(nw, -1), sto(nw, -1),
-        pgo(nw, -1), pqo(nw, -1);
-    size_t lds_need = 0;
+    pnb = kmax_large
+              ? int(std::min<size_t>(32, pchol_limit / (size_t(kmax_large) * sizeof(double)) - kern::kPcholExtra))
+              : 0;
+    int64_t elems = 0, parts = 0;
+    for (auto* v : {&go, &gwo, &y2o, &w2o, &lo, &lpo, &sco, &sto, &pqo}) v->assign(nw, -1);
     for (int q = 0; q < nw; ++q) {
       const auto& s = B.secs[wide[q]];
       const int64_t kp = int64_t(s.nb) * kern::kSvdBlock;
       const int64_t k = s.k;
+      // of a large sector also the sweeps' two G buffers: G itself is used up by
+      // the Cholesky factorisation, W_g is written after the sweeps
+      const int64_t ge = large[wide[q]] ? kp * kp : k * k;
       go[q] = elems;
-      elems += k * k;
+      elems += ge;
       gwo[q] = elems;
-      elems += k * k;
+      elems += ge;
       y2o[q] = elems;
       elems += int64_t(s.ell) * kp;
       w2o[q] = elems;
@@ -579,15 +589,27 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         elems += 3 * k;
         sto[q] = elems;  // ints
         elems += (k + 2) / 2 + 1;
-        pgo[q] = elems;  // the sweeps' two G buffers
-        elems += 2 * kp * kp;
         pqo[q] = elems;  // rotations and rotated blocks, two parities each
         elems += int64_t(4) * (s.nb / 2) * 1024;
       } else {
         lds_need = std::max(lds_need, kern::gram_eig_lds_bytes(s.k));
       }
+      if (!eigh_mode && gram_parts(s) > 1) parts += gram_parts(s) * k * k;
     }
-    BufPtr gbuf = ctx->alloc(size_t(elems) * sizeof(double));
+    // Where the arena has no room for these, every sector goes by the rounds on
+    // Y below, which need none of them.
+    try {
+      gbuf = ctx->alloc(size_t(elems) * sizeof(double));
+      if (parts) (void)ctx->alloc(size_t(parts) * sizeof(double));
+    } catch (const OutOfMemory&) {
+      gbuf.reset();
+      wide.clear();
+      std::fill(large.begin(), large.end(), 0);
+    }
+  }
+  if (wide.empty()) start(y2_of, w2_of);
+  if (!wide.empty()) {
+    const int nw = int(wide.size());
     keep.push_back(gbuf);
     const int64_t gb = gbuf->dptr() - ab;
     std::vector<int64_t> alt_y(nw), alt_w(nw);
@@ -614,7 +636,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       int64_t pelems = 0;
       for (size_t j = 0; j < qs.size(); ++j) {
         const auto& s = B.secs[wide[qs[j]]];
-        parts[j] = int(std::min<int64_t>(16, std::max<int64_t>(1, s.ell / env_int("QTT_GRAM_ROWS_PER_PART", 256))));
+        parts[j] = gram_parts(s);
         if (parts[j] > 1) pelems += int64_t(parts[j]) * s.k * s.k;
       }
       BufPtr pbuf = pelems ? ctx->alloc(size_t(pelems) * sizeof(double)) : nullptr;
@@ -715,7 +737,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
           c.dst_cs = 1;
           add_chunks(zt, int(z.size()), int64_t(c.cols));
           z.push_back(c);
-          c.dst_off = gb + pgo[q];  // G's padding stays zero under the sweeps
+          c.dst_off = gb + gwo[q];  // the padding of the sweeps' first G stays zero
           c.cols = int32_t(kp * kp);
           add_chunks(zt, int(z.size()), int64_t(c.cols));
           z.push_back(c);
@@ -759,8 +781,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       std::vector<kern::GramVec> vd;
       for (int q : qs) {
         const auto& s = B.secs[wide[q]];
-        const int64_t kp = int64_t(s.nb) * kern::kSvdBlock;
-        ps.push_back({gb + lo[q], gb + pgo[q], gb + pgo[q] + kp * kp, gb + pqo[q],
+        ps.push_back({gb + lo[q], gb + gwo[q], gb + go[q], gb + pqo[q],
                       gb + pqo[q] + int64_t(2) * (s.nb / 2) * 1024, s.k, s.nb});
         vd.push_back({gb + lo[q], gb + gwo[q], gb + sco[q], s.k, s.k, s.k, 0});
       }
