@@ -683,7 +683,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
     auto retire = [&](std::vector<int>& qs) {  // drop converged sectors after a flag read
       std::vector<int> next;
       for (int q : qs) {
-        if (h_flags[q] == 0) {
+        if (h_flags[q] == 0 && !(eigh_mode && h_flags[nw + q])) {
           done[wide[q]] = 1;
           if (h_flags[nw + q] > 0) corr.push_back(q);  // converged in the absolute sense only
         } else {
@@ -848,9 +848,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       // large sectors: test first (the solve is a long chain of launches); the
       // flag read also covers the small solver launched above
       int cd_launched = 0;
-      if (!act_l.empty() && eigh_mode) {
-        solve_large(act_l);
-      } else if (!act_l.empty()) {
+      if (!act_l.empty()) {
         cd_launched = 1;
         std::vector<kern::SmallJacobi> cd;
         int kc = 0;
@@ -861,7 +859,8 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
         }
         {
           KernelTimer kt(*ctx, "svd_check");
-          kern::gram_check(ctx->stream(), ab, ctx->lists(cd), int(cd.size()), d_flags, tol, kc);
+          // an eigh is not tested again: nothing the sweeps would rotate may pass
+          kern::gram_check(ctx->stream(), ab, ctx->lists(cd), int(cd.size()), d_flags, eigh_mode ? tol / 8.0 : tol, kc);
         }
         read_flags();  // the small sectors' flags may not be written yet when overlapped
         retire(act_l);

@@ -84,3 +84,33 @@ def test_eigh_of_indefinite_matrices_with_a_positive_diagonal(ctx, k, precond, m
     assert np.abs(w - np.linalg.eigvalsh(g)).max() <= 1e-12 * nrm
     assert np.abs(g @ u - u * w).max() <= 1e-12 * nrm
     assert np.abs(u.T @ u - np.eye(k)).max() <= 1e-12
+
+
+@pytest.mark.parametrize("coupling", [0.0, 1e-13, 1e-3])
+def test_eigh_of_wide_almost_diagonal_matrices(ctx, coupling):
+    """A wide sector that is diagonal to the rounding is not factored, whatever
+    the one beside it; couplings above the rounding are solved."""
+    import quantit_amd as qa
+    rng = np.random.default_rng(9)
+    x = rng.standard_normal((150, 150))
+    mats = [np.diag(rng.uniform(-1.0, 1.0, 200)), np.diag(np.full(141, 2.0)), x + x.T]
+    y = rng.standard_normal((200, 200))
+    mats[0] += coupling * (y + y.T)
+    A = BTensor((0,), [[200, 141, 150]] * 2, [[(0,), (1,), (2,)], [(0,), (-1,), (-2,)]], (0,))
+    for i, m in enumerate(mats):
+        A.blocks[(i, i)] = m
+    capped = ctx.svd_stats()["unconverged"]
+    e, U = (from_dev(x) for x in qa.eigh(to_dev(ctx, A), 1))
+    assert ctx.svd_stats()["unconverged"] == capped
+    for i, a in enumerate(mats):
+        w, u, nrm = e.blocks[(i,)], U.blocks[(i, i)], np.linalg.norm(a)
+        assert np.abs(w - np.linalg.eigvalsh(a)).max() <= 1e-12 * nrm
+        assert np.abs(a @ u - u * w).max() <= 1e-13 * nrm
+        assert np.abs(u.T @ u - np.eye(len(a))).max() <= 1e-12
+    del A.blocks[(2, 2)]
+    ctx.set_profiling(True)
+    ctx.kernel_times()
+    qa.eigh(to_dev(ctx, A), 1)
+    names = ctx.kernel_times()
+    ctx.set_profiling(False)
+    assert ("svd_pchol" in names) == (coupling > 0.0)
