@@ -788,7 +788,8 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       // well inside tol: couplings d left between the columns come back in the
       // next Gram matrix as d (sigma_i^2 + sigma_j^2), against tol sigma_i
       // sigma_max; stopping at tol itself repeats the iteration up to its cap
-      gram_sweeps(ctx, ab, ps, tol / 8.0, max_sweeps, &B.unconverged);
+      const int sweeps = gram_sweeps(ctx, ab, ps, tol / 8.0, max_sweeps, &B.unconverged);
+      if (eigh_mode) B.sweeps += sweeps;  // of an SVD the Gram iterations are counted
       int kv = 0;
       for (auto& v : vd) kv = std::max(kv, v.k);
       KernelTimer kt(*ctx, "svd_vectors");
@@ -881,7 +882,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       act.insert(act.end(), act_l.begin(), act_l.end());
       if (act.empty()) break;
       rotate(act);
-      B.sweeps += 1;
+      if (!eigh_mode) B.sweeps += 1;
     }
     if (eigh_mode)
       for (int q : act) done[wide[q]] = 1;

@@ -114,3 +114,15 @@ def test_eigh_of_wide_almost_diagonal_matrices(ctx, coupling):
     names = ctx.kernel_times()
     ctx.set_profiling(False)
     assert ("svd_pchol" in names) == (coupling > 0.0)
+
+
+def test_eigh_counts_its_sweeps():
+    """The largest sweep count of a call: the sweeps over a wide sector, none of
+    those that one work-group makes."""
+    import quantit_amd as qa
+    ctx = qa.Context(0, arena_bytes=256 << 20)
+    for k, sweeps in ((60, range(0, 1)), (200, range(3, 30))):
+        x = np.random.default_rng(k).standard_normal((k, k))
+        qa.eigh(to_dev(ctx, _sector(x + x.T)), 1)
+        assert ctx.svd_stats()["max_sweeps"] in sweeps
+    ctx.close()
