@@ -366,7 +366,7 @@ void gram_eig(hipStream_t s, double* base, const Lists& descs, int n, int* flags
               int precond, size_t lds_bytes);
 size_t gram_eig_lds_bytes(int k);
 // First-order Gram-Schmidt factor T (k x k at w_off) from the Gram matrix at
-// y_off (SmallJacobi with ell = k).
+// y_off (SmallJacobi; ell: rows of the matrix whose columns they are).
 void gs_step(hipStream_t s, double* base, const Lists& descs, int n, int kmax);
 
 // ---- Gram eigenvectors for wide sectors (G in device memory) ---------------

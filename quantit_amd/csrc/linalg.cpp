@@ -896,7 +896,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
       int kg = 0;
       for (int q : corr) {
         const auto& s = B.secs[wide[q]];
-        gd.push_back({gb + go[q], gb + gwo[q], s.k, s.k, s.k, s.k, -1, -1});
+        gd.push_back({gb + go[q], gb + gwo[q], s.ell, s.k, s.k, s.k, -1, -1});
         kg = std::max(kg, s.k);
       }
       {
