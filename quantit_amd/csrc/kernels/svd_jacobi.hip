@@ -822,7 +822,7 @@ __device__ __forceinline__ void wl_norms(WlCol<R>& a, WlCol<R>& b, double an, do
 // the same), so they compute the same rotation and each updates its own
 // column.  Without a branch, so that the chains of two blocks interleave.
 template <int R>
-__device__ __forceinline__ void wl_intra(WlCol<R>& x, int m, int grp, double tol2, bool& big) {
+__device__ __forceinline__ void wl_intra(WlCol<R>& x, int m, int grp, double tol2, int& big) {
   const bool lower = grp < (grp ^ m);
   WlCol<R> p = x;
   wl_xor<R>(p, m);
@@ -834,7 +834,7 @@ __device__ __forceinline__ void wl_intra(WlCol<R>& x, int m, int grp, double tol
   const double xy2 = xy * xy, w = x.n * p.n;
   WlRot r = wl_rotation(lower ? x.n : p.n, lower ? p.n : x.n, w, xy, xy2);
   const bool rot = xy2 > tol2 * w;
-  big |= rot & r.big;
+  big |= int(rot & r.big);
   // lower: x' = x - t (d_y / d_x) y;  upper: y' = y + t (d_x / d_y) x
   const double t = rot ? (lower ? -r.t : r.t) : 0.0;
   const double c = rot ? r.c : 1.0;
@@ -854,7 +854,7 @@ __device__ __forceinline__ void wl_intra(WlCol<R>& x, int m, int grp, double tol
 }
 
 template <int R>
-__device__ __forceinline__ void wl_cross(WlCol<R>& a, WlCol<R>& b, double tol2, bool& big) {
+__device__ __forceinline__ void wl_cross(WlCol<R>& a, WlCol<R>& b, double tol2, int& big) {
   double ab = wl_dot<R>(a.v, b.v), ra, rb;
   if constexpr (WlCol<R>::kScaled) {
     ra = b.d * fast_rcp(a.d);
@@ -864,7 +864,7 @@ __device__ __forceinline__ void wl_cross(WlCol<R>& a, WlCol<R>& b, double tol2, 
   const double ab2 = ab * ab, w = a.n * b.n;
   if (ab2 > tol2 * w) {
     const WlRot r = wl_rotation(a.n, b.n, w, ab, ab2);
-    big |= r.big;
+    big |= int(r.big);
     if constexpr (WlCol<R>::kScaled) {
       const double fa = -r.t * ra, fb = r.t * rb;
 #pragma unroll
@@ -905,7 +905,7 @@ __device__ __forceinline__ void wl_sweeps(double* X, int k, double tol_rot, int 
   const bool active = wave < NB / 2;
   const double tol2 = tol_rot * tol_rot;
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    bool big = false;  // of this lane's group: the groups rotate or not independently
+    int big = 0;  // of this lane's group: the groups rotate or not independently (a vector register: lane masks cost more)
     for (int t = 0; t < NB - 1; ++t) {
       if (active) {
         const int P = circle_block(wave, t, NB), Q = circle_block(NB - 1 - wave, t, NB);
@@ -943,7 +943,7 @@ __device__ __forceinline__ void wl_sweeps(double* X, int k, double tol_rot, int 
       }
       __syncthreads();
     }
-    const bool any = __any(big);
+    const bool any = __any(big != 0);
     if (lane == 0 && any) atomicAdd(&nrot[sweep & 1], 1);
     __syncthreads();
     const int n = nrot[sweep & 1];
