@@ -955,8 +955,8 @@ __device__ __forceinline__ void wl_sweeps(double* X, int k, double tol_rot, int 
 
 // Pivoted Cholesky of G (in X, k x k column-major, k <= 8 R <= 64): column j
 // of X receives column j of L in the original row order (X X^T = G), pivoted[i]
-// whether row i was a pivot; returns the rank.  Every thread of the block calls
-// this.
+// whether row i was a pivot; returns the rank, pv0 and pv1 the first and the
+// last pivot.  Every thread of the block calls this.
 //
 // Left-looking, eight lanes to a row: a step forms the pivot's column only,
 // G(:, p) minus the product of the columns of L so far, so its chain is one
@@ -968,7 +968,8 @@ __device__ __forceinline__ void wl_sweeps(double* X, int k, double tol_rot, int 
 // 24, 40: 6, 14, 31 us against 9, 17, 43 for one wave that updates the trailing
 // matrix in its registers.
 template <int R>
-__device__ __forceinline__ int chol_rows(double* X, int* pivoted, int k, int (*wkey)[16], double (*wval)[16]) {
+__device__ __forceinline__ int chol_rows(double* X, int* pivoted, int k, int (*wkey)[16], double (*wval)[16],
+                                         double& pv0, double& pv1) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, li = tid & 7;
   const int nwv = (k + 7) >> 3;  // waves that hold rows
   const bool has = (tid >> 3) < k;
@@ -1014,6 +1015,8 @@ __device__ __forceinline__ int chol_rows(double* X, int* pivoted, int k, int (*w
       rk = j;
       break;
     }
+    if (j == 0) pv0 = pv;
+    pv1 = pv;
     if (wave < nwv) {
       double s = 0.0;
 #pragma unroll
@@ -1177,13 +1180,14 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
     __shared__ int wkey[2][16];
     __shared__ double wval[2][16];
     int rk;
+    double pv0 = 0.0, pv1 = 0.0;  // first and last pivot
     for (;;) {
       rk = k;
       if (k <= 64) {
-        rk = k <= 16   ? chol_rows<2>(X, perm, k, wkey, wval)
-             : k <= 32 ? chol_rows<4>(X, perm, k, wkey, wval)
-             : k <= 48 ? chol_rows<6>(X, perm, k, wkey, wval)
-                       : chol_rows<8>(X, perm, k, wkey, wval);
+        rk = k <= 16   ? chol_rows<2>(X, perm, k, wkey, wval, pv0, pv1)
+             : k <= 32 ? chol_rows<4>(X, perm, k, wkey, wval, pv0, pv1)
+             : k <= 48 ? chol_rows<6>(X, perm, k, wkey, wval, pv0, pv1)
+                       : chol_rows<8>(X, perm, k, wkey, wval, pv0, pv1);
         __syncthreads();
       } else {
         constexpr int TR = 8, TC = 5;
@@ -1242,6 +1246,8 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
             rk = j;
             break;
           }
+          if (j == 0) pv0 = pmx;
+          pv1 = pmx;
           const double isq = fast_rsqrt(pmx), sq = pmx * isq;
           if (owner && tc == p / TC) {
             // column p - tc TC of the tile by 0/1 weights: a select on the index
@@ -1294,21 +1300,23 @@ __global__ __launch_bounds__(kGramEigThreads) void k_gram_eig(double* __restrict
       add_shift();
     }
     // Columns from the rank on: small multiples of the unit vectors of the rows
-    // without a pivot, the factor of G + delta^2 I there with delta^2 = 2^-54
-    // of the largest diagonal, below the rounding of G.  The Jacobi sweeps
-    // then make the null space's basis with all others (a numpy model takes
-    // the same number of sweeps or one more); completing zero columns one by
-    // one took 640 of 1780 us for two sectors of k = 98 with spectra over ten
-    // decades.  G = 0 leaves zero columns.
+    // without a pivot, the factor of G + delta^2 I there with delta^2 the last
+    // pivot, 2^-54 of the largest diagonal at most: below the rounding of G,
+    // which is that small for the short columns of a graded matrix.  The Jacobi
+    // sweeps then make the null space's basis with all others (a numpy model
+    // takes the same number of sweeps or one more); completing zero columns one
+    // by one took 640 of 1780 us for two sectors of k = 98 with spectra over ten
+    // decades.  (2^-54 of the largest diagonal throughout left couplings among
+    // short columns when the spectrum fell below 1e-16, and the iteration ran to
+    // its cap: 300 columns over 30 decades 61 ms and V^T V - I = 4e-13, now 38 ms
+    // and 3e-15.)  G = 0 leaves zero columns.
     for (int e = rk * k + tid; e < k * k; e += blockDim.x) X[e] = 0.0;
-    double top = 0.0;
-    if (rk > 0 && rk < k)
-      for (int i = 0; i < k; ++i) top = fmax(top, fabs(X[i]));  // sqrt of the largest diagonal
+    const double delta = sqrt(fmin(pv0 * 0x1p-54, pv1));
     __syncthreads();
     if (rk > 0 && tid < k && !perm[tid]) {
       int c = rk;
       for (int i = 0; i < tid; ++i) c += perm[i] ? 0 : 1;
-      X[c * k + tid] = top * 0x1p-27;
+      X[c * k + tid] = delta;
     }
     __syncthreads();
     for (int i = tid; i < ke; i += blockDim.x) perm[i] = i;

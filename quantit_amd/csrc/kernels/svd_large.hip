@@ -320,14 +320,22 @@ __global__ __launch_bounds__(kLargeThreads) void k_pchol_panel(double* __restric
     // the factor of G + delta^2 I on the rows without a pivot, as in k_gram_eig
     __syncthreads();  // the zero columns copied above are overwritten
     const double* first = j0 == 0 ? col : L;
-    double top = 0.0;
-    for (int i = lane; i < k; i += 64) top = fmax(top, fabs(first[i]));
-    for (int off = 32; off > 0; off >>= 1) top = fmax(top, __shfl_xor(top, off));
+    const double* end = rank > j0 ? col + (rank - 1 - j0) * k : L + int64_t(rank - 1) * k;
+    double top = 0.0, last = 0.0;
+    for (int i = lane; i < k; i += 64) {
+      top = fmax(top, fabs(first[i]));
+      last = fmax(last, fabs(end[i]));
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      top = fmax(top, __shfl_xor(top, off));
+      last = fmax(last, __shfl_xor(last, off));
+    }
+    top = fmin(top * 0x1p-27, last);
     for (int i = tid; i < k; i += blockDim.x) {
       if (used[i]) continue;
       int c = rank;
       for (int j = 0; j < i; ++j) c += used[j] ? 0 : 1;
-      L[int64_t(c) * k + i] = top * 0x1p-27;
+      L[int64_t(c) * k + i] = top;
     }
   }
 }

@@ -42,3 +42,20 @@ def test_null_values_and_vectors(ctx, m, k, kind):
     assert np.abs(got - np.sort(s)[::-1]).max() <= 1e-14 * s.max()
     for w in (u, v):
         assert np.abs(w.T @ w - np.eye(k)).max() <= 1e-12
+
+
+@pytest.mark.parametrize("m,k", [(24, 24), (64, 64), (400, 130), (160, 160), (300, 300)])
+@pytest.mark.parametrize("decades", [20, 30])
+def test_spectra_below_the_rounding(ctx, m, k, decades):
+    """The Gram iterations converge: V is the product of two to four orthogonal
+    factors, each within sqrt(k) roundings of one."""
+    import quantit_amd as qa
+    s = 10.0 ** (-decades * np.arange(k) / k)
+    own = qa.Context(0, arena_bytes=256 << 20)
+    u, got, v = _svd(own, _matrix(m, k, s))
+    assert own.svd_stats()["max_sweeps"] <= 5
+    own.close()
+    assert np.abs(got - s).max() <= 1e-14
+    assert np.abs(v.T @ v - np.eye(k)).max() <= 4 * np.sqrt(k) * 2.3e-16 + 1e-14
+    keep = got > 1e-10
+    assert np.abs(u[:, keep].T @ u[:, keep] - np.eye(keep.sum())).max() <= 1e-12
