@@ -129,16 +129,22 @@ hipError_t noalloc_scratch_address(int device, void** out);
 // chunk and are folded into FP64 accumulators after every chunk.
 void gemm_split(hipStream_t s, double* base, const Lists& l, int ntiles, double alpha, double beta);
 // Output blocks with at most kRowsMaxN columns and a short summed K.  A task is
-// 64 or 128 (task_rows) consecutive rows of one output block: 64 while the
-// work-groups all fit on the chip at once (30 blocks of 300 rows, K 128: 8.6 us
-// against 9.9; 72 k rows 4.1 against 4.2), above that 128, whose longer streams
-// hide more (760 k rows of 7 and 12 columns, K 33: 46.8 us against 52.3, 85.6
-// for one thread a row; 1 M rows, N 3, K 5: 16.2 against 21.6 and 18.2).
+// 64, 128 or a multiple of 128 (task_rows) consecutive rows of one output
+// block: 64 while the work-groups all fit on the chip at once (30 blocks of 300
+// rows, K 128: 8.6 us against 9.9; 72 k rows 4.1 against 4.2), above that 128,
+// whose longer streams hide more (760 k rows of 7 and 12 columns, K 33: 46.8 us
+// against 52.3, 85.6 for one thread a row).  Up to K = 16 the rows are soon done
+// and the list of tasks counts, so from 2^19 rows on a task takes several 128,
+// about 4096 tasks in all: 1 M rows, N 3, K 5 26 us a call against 39, 8 M rows,
+// N 2, K 2 72 against 99.  (Longer K: 600 k rows, N 16, K 100 133 us against 124.)
 constexpr int kRowsMaxN = 16, kRowsMaxK = 128;
 struct RowTask {
   int32_t out, row0;
 };
-inline int rows_per_task(int64_t rows) { return rows < 64 * 2048 ? 64 : 128; }
+inline int rows_per_task(int64_t rows, int64_t longest_k) {
+  if (rows < 64 * 2048) return 64;
+  return longest_k > 16 ? 128 : 128 * int(std::min<int64_t>((rows + (int64_t(1) << 19) - 1) >> 19, 64));
+}
 void gemm_rows(hipStream_t s, double* base, const Lists& l, int ntasks, int task_rows, double alpha, double beta);
 
 // ---- data movement ----------------------------------------------------------

@@ -640,7 +640,8 @@ struct RowK {
 };
 template <class L, int RT>
 __global__ __launch_bounds__(256) void k_gemm_rows(double* __restrict__ base, L l, uint32_t at_tasks,
-                                                   uint32_t at_outs, uint32_t at_pairs, double alpha, double beta) {
+                                                   uint32_t at_outs, uint32_t at_pairs, int rows, double alpha,
+                                                   double beta) {
   const RowTask* tasks = l.template list<RowTask>(at_tasks);
   const GemmOut* outs = l.template list<GemmOut>(at_outs);
   const GemmPair* pairs = l.template list<GemmPair>(at_pairs);
@@ -660,62 +661,66 @@ __global__ __launch_bounds__(256) void k_gemm_rows(double* __restrict__ base, L 
       ks[pr.k0 + k] = {pr.a_off + k * pr.a_cs, pr.a_rs, pr.b_off + k * pr.b_rs, pr.b_cs};
   }
   __syncthreads();
-  const int m0 = t.row0 + (tid >> 6) * 16 * RT;
-  if (m0 >= o.M || o.N <= 0) return;
+  if (o.N <= 0) return;
   const int cl = lane & 15, kq = lane >> 4;
   const int64_t n = min(cl, o.N - 1);
-  int64_t m[RT];
+  const int64_t end = min(int64_t(t.row0) + rows, int64_t(o.M));
+  for (int64_t first = t.row0; first < end; first += 64 * RT) {
+    const int m0 = int(first) + (tid >> 6) * 16 * RT;
+    if (m0 >= o.M) return;
+    int64_t m[RT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) m[i] = min(m0 + 16 * i + cl, o.M - 1);
-  v4d acc[RT];
+    for (int i = 0; i < RT; ++i) m[i] = min(m0 + 16 * i + cl, o.M - 1);
+    v4d acc[RT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) acc[i] = v4d{0.0, 0.0, 0.0, 0.0};
-  // chunk c: k = 4 c .. 4 c + 3 of the list, one per lane quarter; loads past
-  // the list's end repeat its last k, and their values are dropped
-  auto load = [&](int c, double (&a)[RT], double& b) {
-    const RowK e = ks[min(4 * c + kq, ksum - 1)];
-    b = base[e.b_off + n * e.b_cs];
+    for (int i = 0; i < RT; ++i) acc[i] = v4d{0.0, 0.0, 0.0, 0.0};
+    // chunk c: k = 4 c .. 4 c + 3 of the list, one per lane quarter; loads past
+    // the list's end repeat its last k, and their values are dropped
+    auto load = [&](int c, double (&a)[RT], double& b) {
+      const RowK e = ks[min(4 * c + kq, ksum - 1)];
+      b = base[e.b_off + n * e.b_cs];
 #pragma unroll
-    for (int i = 0; i < RT; ++i) a[i] = base[e.a_off + m[i] * e.a_rs];
-  };
-  auto multiply = [&](int c, double (&a)[RT], double b) {
-    if (4 * c + 4 > ksum) {
-      const bool in = 4 * c + kq < ksum;
-      b = in ? b : 0.0;
+      for (int i = 0; i < RT; ++i) a[i] = base[e.a_off + m[i] * e.a_rs];
+    };
+    auto multiply = [&](int c, double (&a)[RT], double b) {
+      if (4 * c + 4 > ksum) {
+        const bool in = 4 * c + kq < ksum;
+        b = in ? b : 0.0;
 #pragma unroll
-      for (int i = 0; i < RT; ++i) a[i] = in ? a[i] : 0.0;
-    }
+        for (int i = 0; i < RT; ++i) a[i] = in ? a[i] : 0.0;
+      }
 #pragma unroll
-    for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a[i], acc[i], 0, 0, 0);
-  };
-  if (ksum > 0) {
-    const int nc = (ksum + 3) / 4;
-    double a0[RT], a1[RT], b0, b1;
-    load(0, a0, b0);
-    load(1, a1, b1);
-    if (nc <= 2) {
-      multiply(0, a0, b0);
-      if (nc == 2) multiply(1, a1, b1);
-    } else {
-      for (int c = 0; c < nc; c += 2) {
-        multiply(c, a0, b0);
-        load(c + 2, a0, b0);
-        if (c + 1 < nc) multiply(c + 1, a1, b1);
-        load(c + 3, a1, b1);
+      for (int i = 0; i < RT; ++i) acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a[i], acc[i], 0, 0, 0);
+    };
+    if (ksum > 0) {
+      const int nc = (ksum + 3) / 4;
+      double a0[RT], a1[RT], b0, b1;
+      load(0, a0, b0);
+      load(1, a1, b1);
+      if (nc <= 2) {
+        multiply(0, a0, b0);
+        if (nc == 2) multiply(1, a1, b1);
+      } else {
+        for (int c = 0; c < nc; c += 2) {
+          multiply(c, a0, b0);
+          load(c + 2, a0, b0);
+          if (c + 1 < nc) multiply(c + 1, a1, b1);
+          load(c + 3, a1, b1);
+        }
       }
     }
-  }
 #pragma unroll
-  for (int i = 0; i < RT; ++i) {
-    const int row = m0 + 16 * i + cl;
-    double* C = base + o.c_off + int64_t(row) * o.ldc;
+    for (int i = 0; i < RT; ++i) {
+      const int row = m0 + 16 * i + cl;
+      double* C = base + o.c_off + int64_t(row) * o.ldc;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int col = 4 * r + kq;  // f64 MFMA output layout, transposed
-      if (row < o.M && col < o.N) {
-        double v = alpha * acc[i][r];
-        if (beta != 0.0) v += beta * C[col];
-        C[col] = v;
+      for (int r = 0; r < 4; ++r) {
+        const int col = 4 * r + kq;  // f64 MFMA output layout, transposed
+        if (row < o.M && col < o.N) {
+          double v = alpha * acc[i][r];
+          if (beta != 0.0) v += beta * C[col];
+          C[col] = v;
+        }
       }
     }
   }
@@ -723,12 +728,12 @@ __global__ __launch_bounds__(256) void k_gemm_rows(double* __restrict__ base, L 
 
 void gemm_rows(hipStream_t s, double* base, const Lists& l, int ntasks, int task_rows, double alpha, double beta) {
   if (ntasks <= 0) return;
-  if (task_rows == 128)
+  if (task_rows % 128 == 0)
     launch_lists(k_gemm_rows<DevLists, 2>, k_gemm_rows<ArgLists, 2>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[3],
-                 l.at[1], l.at[2], alpha, beta);
+                 l.at[1], l.at[2], task_rows, alpha, beta);
   else
     launch_lists(k_gemm_rows<DevLists, 1>, k_gemm_rows<ArgLists, 1>, l, dim3(ntasks), dim3(256), 0, s, base, l.at[3],
-                 l.at[1], l.at[2], alpha, beta);
+                 l.at[1], l.at[2], task_rows, alpha, beta);
 }
 
 GemmLayout gemm_layout(const GemmPair* pairs, size_t n, const GemmOut* outs, size_t nouts) {

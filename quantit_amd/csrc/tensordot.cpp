@@ -772,7 +772,7 @@ BTensor tensordot_impl(const BTensor& a, const BTensor& b, const std::vector<int
   if (all_narrow) {
     int64_t rows = 0;
     for (auto& o : gouts) rows += o.M;
-    lch.task_rows = kern::rows_per_task(rows);
+    lch.task_rows = kern::rows_per_task(rows, *std::max_element(out_work.begin(), out_work.end()));
   }
   for (int o : ord)
     if (size_t(o) < outs.size() && narrow[size_t(o)]) {

@@ -36,3 +36,30 @@ def test_rows_beyond_every_tile_are_refused(ctx):
     b = _matrix(np.random.default_rng(2), 1, 17)
     with pytest.raises(ValueError, match="rows or columns"):
         to_dev(ctx, a).tensordot(to_dev(ctx, b), [1], [0])
+
+
+@pytest.mark.parametrize("rows", [(1 << 19) - 1, 1 << 19, (1 << 19) + 1, (1 << 20) + 129, 3000000])
+@pytest.mark.parametrize("k,n,transposed", [(2, 3, False), (16, 5, True), (17, 5, False)])
+def test_tall_narrow_products_are_exact(ctx, rows, k, n, transposed):
+    """Tasks of several 128 rows from 2^19 rows on, up to K = 16."""
+    rng = np.random.default_rng(rows)
+    a, b = _matrix(rng, *((k, rows) if transposed else (rows, k))), _matrix(rng, k, n)
+    got = from_dev(to_dev(ctx, a).tensordot(to_dev(ctx, b), [0 if transposed else 1], [0])).blocks[(0, 0)]
+    x = a.blocks[(0, 0)]
+    assert np.array_equal(got, (x.T if transposed else x) @ b.blocks[(0, 0)])
+
+
+def test_many_tall_narrow_blocks_are_exact(ctx):
+    """Blocks of a few rows to 300000 beside each other in tasks of 256 rows."""
+    rng = np.random.default_rng(3)
+    rows = [1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 300000, 300001]
+    A = BTensor((0,), [rows, [2] * len(rows)], [[(i,) for i in range(len(rows))], [(-i,) for i in range(len(rows))]], (0,))
+    for i, m in enumerate(rows):
+        A.blocks[(i, i)] = rng.integers(-8, 9, (m, 2)).astype(float)
+    C = BTensor((0,), [[2] * len(rows), [3] * len(rows)],
+                [[(i,) for i in range(len(rows))], [(-i,) for i in range(len(rows))]], (0,))
+    for i in range(len(rows)):
+        C.blocks[(i, i)] = rng.integers(-8, 9, (2, 3)).astype(float)
+    got = from_dev(to_dev(ctx, A).tensordot(to_dev(ctx, C), [1], [0]))
+    for i in range(len(rows)):
+        assert np.array_equal(got.blocks[(i, i)], A.blocks[(i, i)] @ C.blocks[(i, i)])
