@@ -25,11 +25,12 @@ constexpr int BM = 64, BN = 64, BK = 16;
 constexpr int LDP = BM + 16;  // LDS row pitch (doubles)
 
 // Loads the A tile (BM x BK, element (m,k) at A[m*rs + k*cs]) into As[k][m]
-// and the B tile (BK x BN, element (k,n) at B[k*rs + n*cs]) into Bs[k][n].
-template <class T>
+// and the B tile (BK x BN, element (k,n) at B[k*rs + n*cs]) into Bs[k][n], as
+// high parts and, in As2 and Bs2, what they leave.
 __device__ __forceinline__ void load_tiles(const double* __restrict__ A, const double* __restrict__ B,
                                            const GemmPair& pr, int M, int N, int m0, int n0, int k0, int tid,
-                                           T (*As)[LDP], T (*Bs)[LDP], T (*As2)[LDP], T (*Bs2)[LDP]) {
+                                           float (*As)[LDP], float (*Bs)[LDP], float (*As2)[LDP],
+                                           float (*Bs2)[LDP]) {
   const int K = pr.K;
   if (pr.a_cs == 1) {  // row-major A: 4 consecutive k per thread
     const int m = tid >> 2, kq = (tid & 3) * 4;
@@ -38,13 +39,9 @@ __device__ __forceinline__ void load_tiles(const double* __restrict__ A, const d
     for (int j = 0; j < 4; ++j) {
       const int gk = k0 + kq + j;
       double v = (gm < M && gk < K) ? A[int64_t(gm) * pr.a_rs + gk] : 0.0;
-      if constexpr (sizeof(T) == 8) {
-        As[kq + j][m] = v;
-      } else {
-        float hi = float(v);
-        As[kq + j][m] = hi;
-        As2[kq + j][m] = float(v - double(hi));
-      }
+      float hi = float(v);
+      As[kq + j][m] = hi;
+      As2[kq + j][m] = float(v - double(hi));
     }
   } else {  // column-major or general strides: 4 consecutive m per thread
     const int k = tid >> 4, mq = (tid & 15) * 4;
@@ -53,13 +50,9 @@ __device__ __forceinline__ void load_tiles(const double* __restrict__ A, const d
     for (int j = 0; j < 4; ++j) {
       const int gm = m0 + mq + j;
       double v = (gm < M && gk < K) ? A[int64_t(gm) * pr.a_rs + int64_t(gk) * pr.a_cs] : 0.0;
-      if constexpr (sizeof(T) == 8) {
-        As[k][mq + j] = v;
-      } else {
-        float hi = float(v);
-        As[k][mq + j] = hi;
-        As2[k][mq + j] = float(v - double(hi));
-      }
+      float hi = float(v);
+      As[k][mq + j] = hi;
+      As2[k][mq + j] = float(v - double(hi));
     }
   }
   if (pr.b_cs == 1) {  // row-major B: 4 consecutive n per thread
@@ -69,13 +62,9 @@ __device__ __forceinline__ void load_tiles(const double* __restrict__ A, const d
     for (int j = 0; j < 4; ++j) {
       const int gn = n0 + nq + j;
       double v = (gn < N && gk < K) ? B[int64_t(gk) * pr.b_rs + gn] : 0.0;
-      if constexpr (sizeof(T) == 8) {
-        Bs[k][nq + j] = v;
-      } else {
-        float hi = float(v);
-        Bs[k][nq + j] = hi;
-        Bs2[k][nq + j] = float(v - double(hi));
-      }
+      float hi = float(v);
+      Bs[k][nq + j] = hi;
+      Bs2[k][nq + j] = float(v - double(hi));
     }
   } else {  // column-major or general: 4 consecutive k per thread
     const int n = tid >> 2, kq = (tid & 3) * 4;
@@ -84,13 +73,9 @@ __device__ __forceinline__ void load_tiles(const double* __restrict__ A, const d
     for (int j = 0; j < 4; ++j) {
       const int gk = k0 + kq + j;
       double v = (gn < N && gk < K) ? B[int64_t(gk) * pr.b_rs + int64_t(gn) * pr.b_cs] : 0.0;
-      if constexpr (sizeof(T) == 8) {
-        Bs[kq + j][n] = v;
-      } else {
-        float hi = float(v);
-        Bs[kq + j][n] = hi;
-        Bs2[kq + j][n] = float(v - double(hi));
-      }
+      float hi = float(v);
+      Bs[kq + j][n] = hi;
+      Bs2[kq + j][n] = float(v - double(hi));
     }
   }
 }
@@ -98,8 +83,7 @@ __device__ __forceinline__ void load_tiles(const double* __restrict__ A, const d
 // Output element (row, col) of 16x16 MFMA tile register r in lane l:
 //   v_mfma_f64_16x16x4_f64: row = 4*r + l/16, col = l%16
 //   v_mfma_f32_16x16x4_f32: row = 4*(l/16) + r, col = l%16
-// (measured on gfx950; the two layouts differ).
-template <bool F64Layout>
+// (measured on gfx950; the two layouts differ).  This stores the second.
 __device__ __forceinline__ void store_tile(double* __restrict__ C, const GemmOut& o, int m0, int n0, int wm, int wn,
                                            int lane, const v4d (&acc)[2][2], double alpha, double beta) {
 #pragma unroll
@@ -108,7 +92,7 @@ __device__ __forceinline__ void store_tile(double* __restrict__ C, const GemmOut
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm + i * 16 + (F64Layout ? 4 * r + (lane >> 4) : 4 * (lane >> 4) + r);
+        const int row = m0 + wm + i * 16 + 4 * (lane >> 4) + r;
         const int col = n0 + wn + j * 16 + (lane & 15);
         if (row < o.M && col < o.N) {
           double* p = C + int64_t(row) * o.ldc + col;
@@ -375,28 +359,26 @@ __global__ __launch_bounds__(256) void k_gemm_f64c(double* __restrict__ base, L 
 // The same tile for launches whose pairs are not contiguous in one common way
 // (blocks with unit-length legs beside permuted ones): 8-byte loads with a
 // bounds check each, double-buffered LDS k by k.
-template <int TM, int TN, int KD>
 struct TileRegs {
-  double a[TM * KD / 256], b[TN * KD / 256];
+  double a[BM * BK / 256], b[BN * BK / 256];
 };
 
-template <int TM, int TN, int KD>
 __device__ __forceinline__ void fetch_t(const double* __restrict__ base, const GemmPair& pr, int M, int N, int m0,
-                                        int n0, int k0, int tid, TileRegs<TM, TN, KD>& r) {
-  constexpr int EA = TM * KD / 256, EB = TN * KD / 256;  // elements per thread
+                                        int n0, int k0, int tid, TileRegs& r) {
+  constexpr int EA = BM * BK / 256, EB = BN * BK / 256;  // elements per thread
   const double* A = base + pr.a_off;
   const double* B = base + pr.b_off;
   const int K = pr.K;
-  if (pr.a_cs == 1) {  // k contiguous: KD/EA threads per row, EA consecutive k each
-    constexpr int TPR = KD / EA;
+  if (pr.a_cs == 1) {  // k contiguous: BK/EA threads per row, EA consecutive k each
+    constexpr int TPR = BK / EA;
     const int m = tid / TPR, kq = (tid % TPR) * EA, gm = m0 + m;
 #pragma unroll
     for (int j = 0; j < EA; ++j) {
       const int gk = k0 + kq + j;
       r.a[j] = (gm < M && gk < K) ? A[int64_t(gm) * pr.a_rs + gk] : 0.0;
     }
-  } else {  // m contiguous (or general): TM/EA threads per k, EA consecutive m each
-    constexpr int TPK = TM / EA;
+  } else {  // m contiguous (or general): BM/EA threads per k, EA consecutive m each
+    constexpr int TPK = BM / EA;
     const int k = tid / TPK, mq = (tid % TPK) * EA, gk = k0 + k;
 #pragma unroll
     for (int j = 0; j < EA; ++j) {
@@ -404,16 +386,16 @@ __device__ __forceinline__ void fetch_t(const double* __restrict__ base, const G
       r.a[j] = (gm < M && gk < K) ? A[int64_t(gm) * pr.a_rs + int64_t(gk) * pr.a_cs] : 0.0;
     }
   }
-  if (pr.b_cs == 1) {  // n contiguous: TN/EB threads per k, EB consecutive n each
-    constexpr int TPK = TN / EB;
+  if (pr.b_cs == 1) {  // n contiguous: BN/EB threads per k, EB consecutive n each
+    constexpr int TPK = BN / EB;
     const int k = tid / TPK, nq = (tid % TPK) * EB, gk = k0 + k;
 #pragma unroll
     for (int j = 0; j < EB; ++j) {
       const int gn = n0 + nq + j;
       r.b[j] = (gn < N && gk < K) ? B[int64_t(gk) * pr.b_rs + gn] : 0.0;
     }
-  } else {  // k contiguous (or general): KD/EB threads per column
-    constexpr int TPC = KD / EB;
+  } else {  // k contiguous (or general): BK/EB threads per column
+    constexpr int TPC = BK / EB;
     const int n = tid / TPC, kq = (tid % TPC) * EB, gn = n0 + n;
 #pragma unroll
     for (int j = 0; j < EB; ++j) {
@@ -423,46 +405,45 @@ __device__ __forceinline__ void fetch_t(const double* __restrict__ base, const G
   }
 }
 
-template <int TM, int TN, int KD>
-__device__ __forceinline__ void stash_t(const GemmPair& pr, int tid, const TileRegs<TM, TN, KD>& r,
-                                        double (*As)[TM + 16], double (*Bs)[TN + 16]) {
-  constexpr int EA = TM * KD / 256, EB = TN * KD / 256;
+__device__ __forceinline__ void stash_t(const GemmPair& pr, int tid, const TileRegs& r,
+                                        double (*As)[LDP], double (*Bs)[LDP]) {
+  constexpr int EA = BM * BK / 256, EB = BN * BK / 256;
   if (pr.a_cs == 1) {
-    constexpr int TPR = KD / EA;
+    constexpr int TPR = BK / EA;
     const int m = tid / TPR, kq = (tid % TPR) * EA;
 #pragma unroll
     for (int j = 0; j < EA; ++j) As[kq + j][m] = r.a[j];
   } else {
-    constexpr int TPK = TM / EA;
+    constexpr int TPK = BM / EA;
     const int k = tid / TPK, mq = (tid % TPK) * EA;
 #pragma unroll
     for (int j = 0; j < EA; ++j) As[k][mq + j] = r.a[j];
   }
   if (pr.b_cs == 1) {
-    constexpr int TPK = TN / EB;
+    constexpr int TPK = BN / EB;
     const int k = tid / TPK, nq = (tid % TPK) * EB;
 #pragma unroll
     for (int j = 0; j < EB; ++j) Bs[k][nq + j] = r.b[j];
   } else {
-    constexpr int TPC = KD / EB;
+    constexpr int TPC = BK / EB;
     const int n = tid / TPC, kq = (tid % TPC) * EB;
 #pragma unroll
     for (int j = 0; j < EB; ++j) Bs[kq + j][n] = r.b[j];
   }
 }
 
-template <class L, int TM, int TN, int KD>
+template <class L>
 __global__ __launch_bounds__(256) void k_gemm_f64t(double* __restrict__ base, L l, uint32_t at_tiles,
                                                    uint32_t at_outs, uint32_t at_pairs, double alpha, double beta) {
   const GemmTile* tiles = l.template list<GemmTile>(at_tiles);
   const GemmOut* outs = l.template list<GemmOut>(at_outs);
   const GemmPair* pairs = l.template list<GemmPair>(at_pairs);
-  constexpr int WM = TM / 2, WN = TN / 2, FI = WM / 16, FJ = WN / 16;
-  __shared__ double As[2][KD][TM + 16];
-  __shared__ double Bs[2][KD][TN + 16];
+  constexpr int WM = BM / 2, WN = BN / 2, FI = WM / 16, FJ = WN / 16;
+  __shared__ double As[2][BK][LDP];
+  __shared__ double Bs[2][BK][LDP];
   const GemmTile t = tiles[blockIdx.x];
   const GemmOut o = outs[t.out];
-  const int m0 = t.tm * TM, n0 = t.tn * TN;
+  const int m0 = t.tm * BM, n0 = t.tn * BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
   v4d acc[FI][FJ];
@@ -476,13 +457,13 @@ __global__ __launch_bounds__(256) void k_gemm_f64t(double* __restrict__ base, L 
   if (p < o.pair_end) {
     GemmPair pr = pairs[p];
     int k0 = 0, buf = 0;
-    TileRegs<TM, TN, KD> regs;
-    fetch_t<TM, TN, KD>(base, pr, o.M, o.N, m0, n0, 0, tid, regs);
-    stash_t<TM, TN, KD>(pr, tid, regs, As[0], Bs[0]);
+    TileRegs regs;
+    fetch_t(base, pr, o.M, o.N, m0, n0, 0, tid, regs);
+    stash_t(pr, tid, regs, As[0], Bs[0]);
     __syncthreads();
     // the step after (p, k0)
     auto advance = [&](int& q, int& k, GemmPair& g) {
-      k += KD;
+      k += BK;
       if (k >= g.K) {
         k = 0;
         ++q;
@@ -494,10 +475,10 @@ __global__ __launch_bounds__(256) void k_gemm_f64t(double* __restrict__ base, L 
     GemmPair npr = pr;
     advance(np, nk, npr);
     bool more = np < o.pair_end;
-    if (more) fetch_t<TM, TN, KD>(base, npr, o.M, o.N, m0, n0, nk, tid, regs);
+    if (more) fetch_t(base, npr, o.M, o.N, m0, n0, nk, tid, regs);
     while (true) {
 #pragma unroll
-      for (int kk = 0; kk < KD; kk += 4) {
+      for (int kk = 0; kk < BK; kk += 4) {
         const int kr = kk + (lane >> 4), c = lane & 15;
         double a[FI], b[FJ];
 #pragma unroll
@@ -512,22 +493,20 @@ __global__ __launch_bounds__(256) void k_gemm_f64t(double* __restrict__ base, L 
       if (!more) break;
       // regs hold step (np, nk): into the other buffer (its last readers
       // passed the barrier of the previous step), then fetch the step after
-      stash_t<TM, TN, KD>(npr, tid, regs, As[buf ^ 1], Bs[buf ^ 1]);
-      GemmPair cur = npr;
+      stash_t(npr, tid, regs, As[buf ^ 1], Bs[buf ^ 1]);
       int q = np, k = nk;
       advance(q, k, npr);
       more = q < o.pair_end;
       np = q;
       nk = k;
-      if (more) fetch_t<TM, TN, KD>(base, npr, o.M, o.N, m0, n0, nk, tid, regs);
-      (void)cur;
+      if (more) fetch_t(base, npr, o.M, o.N, m0, n0, nk, tid, regs);
       __syncthreads();
       buf ^= 1;
       // the step in buffer buf is complete; one more compute round if it
       // was the last one loaded
       if (!more) {
 #pragma unroll
-        for (int kk = 0; kk < KD; kk += 4) {
+        for (int kk = 0; kk < BK; kk += 4) {
           const int kr = kk + (lane >> 4), c = lane & 15;
           double a[FI], b[FJ];
 #pragma unroll
@@ -586,7 +565,7 @@ __global__ __launch_bounds__(256) void k_gemm_split(double* __restrict__ base, L
     const double* A = base + pr.a_off;
     const double* B = base + pr.b_off;
     for (int k0 = 0; k0 < pr.K; k0 += BK) {
-      load_tiles<float>(A, B, pr, o.M, o.N, m0, n0, k0, tid, Ah, Bh, Al, Bl);
+      load_tiles(A, B, pr, o.M, o.N, m0, n0, k0, tid, Ah, Bh, Al, Bl);
       __syncthreads();
       v4f hh[2][2], cr[2][2];
 #pragma unroll
@@ -622,7 +601,7 @@ __global__ __launch_bounds__(256) void k_gemm_split(double* __restrict__ base, L
       __syncthreads();
     }
   }
-  store_tile<false>(base + o.c_off, o, m0, n0, wm, wn, lane, acc, alpha, beta);
+  store_tile(base + o.c_off, o, m0, n0, wm, wn, lane, acc, alpha, beta);
 }
 
 // Narrow outputs (N <= kRowsMaxN, summed K <= kRowsMaxK): an MFMA tile of the
@@ -775,7 +754,7 @@ void gemm_f64(hipStream_t s, int tile, GemmLayout lay, double* base, const Lists
               double beta) {
   if (ntiles <= 0) return;
   if (lay == kLayoutAny)
-    launch_lists(k_gemm_f64t<DevLists, 64, 64, 16>, k_gemm_f64t<ArgLists, 64, 64, 16>, l, dim3(ntiles), dim3(256), 0,
+    launch_lists(k_gemm_f64t<DevLists>, k_gemm_f64t<ArgLists>, l, dim3(ntiles), dim3(256), 0,
                  s, base, l.at[0], l.at[1], l.at[2], alpha, beta);
   else if (tile == 32)
     gemm_contiguous<32>(s, lay, base, l, ntiles, alpha, beta);

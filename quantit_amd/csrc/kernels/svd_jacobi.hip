@@ -34,8 +34,8 @@ constexpr int YC = 128;             // rows of Y staged per chunk
 constexpr int YP = YC + 2;          // LDS pitch of the staged Y chunk
 constexpr int GP = NB2 + 1;         // LDS pitch of G and Q
 
-// W = I (kp x kp) for every sector; gridDim.y work-groups share a sector,
-// one column per wave-step.
+// Y and its partner zero, W and its partner the identity, for every sector;
+// gridDim.y work-groups share a sector.
 template <class L>
 __global__ __launch_bounds__(256) void k_svd_prepare(double* __restrict__ base, L l) {
   const SvdPrep s = l.template list<SvdPrep>()[blockIdx.x];
@@ -511,8 +511,7 @@ __global__ __launch_bounds__(RESIDENT ? 1024 : 256) void k_svd_round(double* __r
   } else {
     apply_rotation(Y, ld, ell, cols, Ys, Q[cur]);
   }
-  if (s.w_off < 0) return;  // caller keeps no right rotation
-  __syncthreads();           // the staging area below aliases the resident block
+  __syncthreads();  // the staging area below aliases the resident block
   const int kp = nb * kSvdBlock;
   apply_rotation(base + s.w_off, kp, kp, cols, Ys, Q[cur]);
 }

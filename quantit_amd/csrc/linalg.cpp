@@ -135,10 +135,9 @@ int env_int(const char* name, int dflt) {
 }
 
 // Cyclic block Jacobi sweeps over the sectors listed in `which` until a sweep
-// rotates nothing (or max_sweeps).  first_rot[i] receives the number of
-// rotating work-groups of the first sweep of sector which[i].  Returns the
-// number of sweeps run; *capped (if given) is raised by the number of
-// sectors still rotating when max_sweeps ran out.
+// rotates nothing (or max_sweeps).  Returns the number of sweeps run; *capped
+// (if given) is raised by the number of sectors still rotating when max_sweeps
+// ran out.
 //
 // The sweeps are pipelined one deep while they rotate much: sweep s+1 is
 // enqueued before the host waits for the rotation counts of sweep s, so the
@@ -158,7 +157,7 @@ int env_int(const char* name, int dflt) {
 // (k_gram_check).  A sector whose pairs all pass has converged: the sweep
 // after would have rotated nothing.
 int jacobi_sweeps(Context* ctx, double* ab, const std::vector<kern::SvdSector>& secs, const std::vector<int>& which,
-                  double tol, int inner, int max_sweeps, std::vector<int>* first_rot, int* capped) {
+                  double tol, int inner, int max_sweeps, int* capped) {
   const int ns = int(secs.size());
   if (which.empty() || max_sweeps <= 0) return 0;
   BufPtr cnt = ctx->alloc(size_t(4 * ns) * sizeof(int32_t));  // counts of two sweeps, check flags
@@ -167,7 +166,6 @@ int jacobi_sweeps(Context* ctx, double* ab, const std::vector<kern::SvdSector>& 
   ctx->reserve_read(size_t(ns));
   std::vector<char> active(ns, 0);
   for (int i : which) active[i] = 1;
-  if (first_rot) first_rot->assign(which.size(), 0);
   // Rounds after the first of a sweep rotate only the pairs across their two
   // blocks (the first round holds every block once and takes all its pairs,
   // so a sweep still meets every column pair).  QTT_SVD_CROSS_INNER: 1 (the
@@ -271,8 +269,6 @@ int jacobi_sweeps(Context* ctx, double* ab, const std::vector<kern::SvdSector>& 
     ctx->wait_event(ctx->read_event(sweep & 1));
     const int32_t* h_cnt = ctx->read_slot(sweep & 1);
     sweeps = sweep + 1;
-    if (sweep == 0 && first_rot)
-      for (size_t q = 0; q < which.size(); ++q) (*first_rot)[q] = h_cnt[which[q]];
     bool any = false;
     int64_t rotated = 0;
     for (int i = 0; i < ns; ++i) {
@@ -928,7 +924,7 @@ Batched run_batched(const BTensor& t, const std::vector<SectorPlan>& plans, bool
   for (int i = 0; i < ns; ++i)
     if (!done[i] && B.secs[i].k > 0) rest.push_back(i);
   for (int i : rest) B.wide[i] = 1;
-  B.sweeps += jacobi_sweeps(ctx, ab, B.secs, rest, tol, inner, max_sweeps, nullptr, &B.unconverged);
+  B.sweeps += jacobi_sweeps(ctx, ab, B.secs, rest, tol, inner, max_sweeps, &B.unconverged);
   // ---- finalize --------------------------------------------------------------
   std::vector<int4> wt;
   for (int i = 0; i < ns; ++i) {
