@@ -138,12 +138,12 @@ double qtt_last_tensordot_flops(void);
 int qtt_tensordot_into(const qtt_btensor* a, const qtt_btensor* b, int ndims, const int64_t* dims_a,
                        const int64_t* dims_b, qtt_btensor* out);
 
-/* The FP64 contraction GEMM has tile variants (64x64 single-buffered, and
-   64x64, 128x64, 64x128, 128x128 with double-buffered LDS); they give the
-   same bits.  A contraction's shape class (work-weighted mean block size and
-   tile count) picks its variant from a process-wide table that is filled by
-   timing every variant the first time a class is met; the table persists as
-   JSON through these calls.  No counterpart in the reference. */
+/* The FP64 contraction GEMM has 64x64 and 32x32 tiles; they give the same
+   bits.  A contraction's shape class (work-weighted mean block size and tile
+   count) picks its tile from a process-wide table that is filled by timing
+   both the first time a class is met; the table persists as JSON through
+   these calls (entries of older builds whose kernel is gone are timed anew).
+   No counterpart in the reference. */
 int qtt_gemm_tuning_save(const char* path);
 int qtt_gemm_tuning_load(const char* path);
 int qtt_gemm_tuning_size(int64_t* entries);

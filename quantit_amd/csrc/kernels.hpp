@@ -105,7 +105,8 @@ void gemm_f64(hipStream_t s, int tile, GemmLayout lay, double* base, const Lists
               double beta);
 // Tile choices of the tuning table and of QTT_GEMM_VARIANT, by number: 5 is
 // the 32 x 32 tile, every other number the 64 x 64 one (0 the general kernel;
-// 2 to 4 are numbers of wider tiles in tables of older builds).
+// 2 to 4 are numbers of wider tiles in tables of older builds, whose 0 and 5
+// are not taken over).
 enum GemmVariant : int { kTileAny = 0, kTile64 = 1, kTile32 = 5, kGemmVariants = 6 };
 inline int variant_tile(int v) { return v == kTile32 ? 32 : 64; }
 // Tile of a launch that is not timed: 32 x 32 below this many 64 x 64 tiles

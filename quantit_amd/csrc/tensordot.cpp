@@ -298,13 +298,13 @@ void td_run(Context* ctx, const TdPlan::Launch& l, bool timed) {
 
 }  // namespace
 
-// The tuning table as JSON: {"gemm_variants": {"<class>": <variant>, ...}}.
+// The tuning table as JSON: {"tiles": [64, 32], "gemm_variants": {"<class>": <variant>, ...}}.
 void gemm_tuning_save(const std::string& path) {
   TuneTable& t = tune_table();
   std::lock_guard<std::mutex> lk(t.mu);
   std::FILE* f = std::fopen(path.c_str(), "w");
   if (!f) throw InvalidArgument("cannot write " + path);
-  std::fprintf(f, "{\"gemm_variants\": {");
+  std::fprintf(f, "{\"tiles\": [64, 32], \"gemm_variants\": {");
   bool first = true;
   for (auto& kv : t.best) {
     std::fprintf(f, "%s\n  \"%s\": %d", first ? "" : ",", kv.first.c_str(), kv.second);
@@ -324,6 +324,9 @@ void gemm_tuning_load(const std::string& path) {
   std::fclose(f);
   const size_t start = text.find("\"gemm_variants\"");
   if (start == std::string::npos) throw InvalidArgument(path + ": no gemm_variants table");
+  // tables without the line of tiles are of builds where 0 and 5 stood for other
+  // kernels: their classes are timed anew
+  const bool current = text.rfind("\"tiles\": [64, 32]", start) != std::string::npos;
   size_t pos = text.find('{', start);
   std::map<std::string, int> got;
   while (pos != std::string::npos) {
@@ -335,7 +338,7 @@ void gemm_tuning_load(const std::string& path) {
     if (q1 == std::string::npos || colon == std::string::npos) throw InvalidArgument(path + ": malformed table");
     const int v = std::atoi(text.c_str() + colon + 1);
     if (v < 0 || v >= kern::kGemmVariants) throw InvalidArgument(path + ": unknown variant");
-    got[text.substr(q0 + 1, q1 - q0 - 1)] = v;
+    if (current || (v != kern::kTileAny && v != kern::kTile32)) got[text.substr(q0 + 1, q1 - q0 - 1)] = v;
     pos = text.find_first_of(",}", colon);
     if (pos == std::string::npos || text[pos] == '}') break;
   }
