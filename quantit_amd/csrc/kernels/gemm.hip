@@ -609,8 +609,9 @@ __global__ __launch_bounds__(256) void k_gemm_split(double* __restrict__ base, L
 // the chain of dependent loads decides, then the streaming of A.  A wave takes
 // RT x 16 rows and all columns as v_mfma_f64_16x16x4 products of the transposed
 // operands (a store then holds four columns of 16 rows, contiguous for N <= 4),
-// the operands straight from global memory, the next two chunks in flight.  The k of all pairs form one list, so a
-// pair of one or two k wastes nothing; where each k lives goes to LDS first.
+// the operands straight from global memory, the next two chunks in flight.  The
+// k of all pairs form one list, so a pair of one or two k wastes nothing; where
+// each k lives goes to LDS first.  A group takes its rows 64 RT at a time.
 // Twelve blocks of 4 .. 15 rows and columns, K 48: 4.7 us against 34.7 for a
 // thread per row with B in LDS, whose loads came four at a time.
 // Every element is one chain over the pairs in order, k ascending.

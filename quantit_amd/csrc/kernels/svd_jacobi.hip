@@ -904,7 +904,9 @@ __device__ __forceinline__ void wl_sweeps(double* X, int k, double tol_rot, int 
   const bool active = wave < NB / 2;
   const double tol2 = tol_rot * tol_rot;
   for (int sweep = 0; sweep < max_sweeps; ++sweep) {
-    int big = 0;  // of this lane's group: the groups rotate or not independently (a vector register: lane masks cost more)
+    // of this lane's group: the groups rotate or not independently (an integer,
+    // in a vector register: lane masks cost more)
+    int big = 0;
     for (int t = 0; t < NB - 1; ++t) {
       if (active) {
         const int P = circle_block(wave, t, NB), Q = circle_block(NB - 1 - wave, t, NB);
